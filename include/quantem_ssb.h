@@ -124,6 +124,17 @@ int ssb_normalize_scan_typed(const void* src, int dtype, int H, int W, int det_r
                              int T, void* stream);
 
 /*
+ * ssb_normalize_scan_typed in a device workspace of the caller's, of at
+ * least ssb_normalize_workspace_bytes (negative: a QSSB_ERR_* code) and
+ * 16-byte aligned: enqueued on the stream without an allocation or a
+ * synchronisation.  The workspace is free again once the stream has run the
+ * call.  The same results.
+ */
+int64_t ssb_normalize_workspace_bytes(int dtype, int H, int W, int det_rows, int det_cols);
+int ssb_normalize_scan_ws(const void* src, int dtype, int H, int W, int det_rows, int det_cols, void* dst, int T,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * ssb_normalize_scan_u16 without any device allocation or synchronisation.
  * No counterpart in the reference: it is for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid

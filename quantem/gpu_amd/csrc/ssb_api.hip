@@ -150,6 +150,7 @@ int ssb_plan_create(int scan_n, int det_rows, int det_cols, int max_bf, double w
   p->D = det_rows * det_cols;
   p->max_bf = max_bf;
   p->nbf_hint = max_bf;
+  p->max_ranges = dp_max_ranges(p->D);
   p->max_groups = trotter_groups_max(scan_n);
   p->wavelength = wavelength_A;
   p->semiangle = semiangle_rad;
@@ -730,24 +731,56 @@ int ssb_scan_target(int H, int W) {
   return longest <= 128 ? 128 : (longest <= 256 ? 256 : (longest <= 512 ? 512 : 1024));
 }
 
+// shared argument check of the scan normalisation; T < 0 leaves the target out
+static int check_normalize(int dtype, int H, int W, int det_rows, int det_cols, int T) {
+  if (!dtype_size(dtype)) return fail(QSSB_ERR_ARG, "unknown sample type " + std::to_string(dtype));
+  if (H < 1 || W < 1 || det_rows < 1 || det_cols < 1) return fail(QSSB_ERR_ARG, "shapes must be positive");
+  if (T >= 0 && T != ssb_scan_target(H, W))
+    return fail(QSSB_ERR_ARG, "target scan size " + std::to_string(T) + " is not the supported size for a " +
+                                  std::to_string(H) + " x " + std::to_string(W) + " scan (" +
+                                  std::to_string(ssb_scan_target(H, W)) + ")");
+  if ((long long)det_rows * det_cols > (1 << 24)) return fail(QSSB_ERR_UNSUPPORTED, "detector too large");
+  return QSSB_OK;
+}
+
+int64_t ssb_normalize_workspace_bytes(int dtype, int H, int W, int det_rows, int det_cols) {
+  g_last_error.clear();
+  const int rc = check_normalize(dtype, H, W, det_rows, det_cols, -1);
+  if (rc) return rc;
+  return (int64_t)normalize_workspace_bytes(dtype, H, ssb_scan_target(H, W), W, det_rows * det_cols, 0, nullptr);
+}
+
+int ssb_normalize_scan_ws(const void* src, int dtype, int H, int W, int det_rows, int det_cols, void* dst, int T,
+                          void* workspace, int64_t workspace_bytes, void* stream) {
+  g_last_error.clear();
+  if (!src || !dst) return fail(QSSB_ERR_ARG, "source and destination must not be NULL");
+  const int rc = check_normalize(dtype, H, W, det_rows, det_cols, T);
+  if (rc) return rc;
+  const int D = det_rows * det_cols;
+  size_t mean_off = 0;
+  const size_t need = normalize_workspace_bytes(dtype, H, T, W, D, 0, &mean_off);
+  if (!workspace || workspace_bytes < (int64_t)need || (reinterpret_cast<uintptr_t>(workspace) & 15u))
+    return fail(QSSB_ERR_ARG, "the scan normalisation needs a 16-byte aligned workspace of " + std::to_string(need) +
+                                  " bytes");
+  uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
+  HIP_TRY(launch_normalize_scan_typed(dtype, src, H, W, D, dst, T, ws, mean_off, ws + mean_off, as_stream(stream)),
+          "normalize_scan");
+  return QSSB_OK;
+}
+
 static int normalize_scan_typed(const void* src, int dtype, int H, int W, int det_rows, int det_cols, void* dst,
                                 int T, void* stream) {
   g_last_error.clear();
   if (!src || !dst) return fail(QSSB_ERR_ARG, "source and destination must not be NULL");
-  if (!dtype_size(dtype)) return fail(QSSB_ERR_ARG, "unknown sample type " + std::to_string(dtype));
-  if (H < 1 || W < 1 || det_rows < 1 || det_cols < 1) return fail(QSSB_ERR_ARG, "shapes must be positive");
-  if (T != ssb_scan_target(H, W))
-    return fail(QSSB_ERR_ARG, "target scan size " + std::to_string(T) + " is not the supported size for a " +
-                                  std::to_string(H) + " x " + std::to_string(W) + " scan (" +
-                                  std::to_string(ssb_scan_target(H, W)) + ")");
-  const long long D = (long long)det_rows * det_cols;
-  if (D > (1 << 24)) return fail(QSSB_ERR_UNSUPPORTED, "detector too large");
+  const int rc = check_normalize(dtype, H, W, det_rows, det_cols, T);
+  if (rc) return rc;
+  const int D = det_rows * det_cols;
   hipStream_t s = as_stream(stream);
   size_t mean_off = 0;
-  const size_t bytes = normalize_workspace_bytes(dtype, H, T, (int)D, &mean_off);
+  const size_t bytes = normalize_workspace_bytes(dtype, H, T, W, D, 0, &mean_off);
   uint8_t* ws = nullptr;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&ws), bytes);
-  if (e == hipSuccess) e = launch_normalize_scan_typed(dtype, src, H, W, (int)D, dst, T, ws, ws + mean_off, s);
+  if (e == hipSuccess) e = launch_normalize_scan_typed(dtype, src, H, W, D, dst, T, ws, mean_off, ws + mean_off, s);
   hipError_t e2 = hipStreamSynchronize(s);
   dfree(ws);
   if (e != hipSuccess) return hip_fail(e, "normalize_scan");
@@ -1025,7 +1058,7 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
     p->ev_stream_recorded = true;
   }
   mark(2);
-  HIP_TRY(launch_mean_dp_reduce(dtype, data, frames, p->D, partial, p->max_ranges, p->tune_stream_wg, p->gain,
+  HIP_TRY(launch_mean_dp_reduce(dtype, frames, p->D, partial, p->max_ranges, p->tune_stream_wg, p->gain,
                                 p->dp_sums, p->dp_mean, p->dp_dcpix, s),
           "mean_dp");
   p->dp_dtype = dtype;

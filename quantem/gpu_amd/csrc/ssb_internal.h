@@ -138,7 +138,7 @@ int dtype_size(int dtype);
 bool dtype_wide_partials(int dtype);
 
 // Mean DP of `frames` frames of D samples of type `dtype`.  partial holds
-// max_ranges * D partial sums (32-bit, or 64-bit when dtype_wide_partials);
+// max_ranges (dp_max_ranges) * D partial sums (32-bit, or 64-bit when dtype_wide_partials);
 // target_wg: workgroups of the stream pass (0 = default 1536).  gain (D
 // floats) may be NULL.  sums: exact uint64 sums (integer samples; 0 for
 // float32), mean: f32(sum)/f32(frames) * gain, dcpix: f32(sum) * gain
@@ -146,10 +146,11 @@ bool dtype_wide_partials(int dtype);
 hipError_t launch_mean_dp(int dtype, const void* data, long long frames, int D, void* partial, int max_ranges,
                           int target_wg, const float* gain, unsigned long long* sums, float* mean, float* dcpix,
                           hipStream_t s);
+int dp_max_ranges(int D);
 // the two passes of launch_mean_dp, separately (stage timing)
 hipError_t launch_mean_dp_stream(int dtype, const void* data, long long frames, int D, void* partial, int max_ranges,
                                  int target_wg, hipStream_t s);
-hipError_t launch_mean_dp_reduce(int dtype, const void* data, long long frames, int D, const void* partial,
+hipError_t launch_mean_dp_reduce(int dtype, long long frames, int D, const void* partial,
                                  int max_ranges, int target_wg, const float* gain, unsigned long long* sums,
                                  float* mean, float* dcpix, hipStream_t s);
 // exact_dc: dc from the exact unsigned integer sums (no gain); otherwise
@@ -198,16 +199,14 @@ hipError_t launch_max_u16(const uint16_t* data, long long n, unsigned int* parti
                           hipStream_t s);
 int max_u16_parts();
 
-// Scan normalisation: crop/pad the H x W scan to T x T (partial holds
-// normalize_partial_groups(QSSB_DTYPE_U16, H, T, D) * D uint32, mean D uint16).
-hipError_t launch_normalize_scan(const uint16_t* src, int H, int W, int D, uint16_t* dst, int T,
-                                 uint32_t* partial, uint16_t* mean, hipStream_t s);
-int normalize_partial_groups(int dtype, int H, int T, int D);
-// The same for any QSSB_DTYPE_* sample type; partial and mean as laid out by
-// normalize_workspace_bytes (mean at *mean_offset of the workspace).
+// Scan normalisation: crop/pad the H x W scan of any QSSB_DTYPE_* sample type
+// to T x T; partial (partial_bytes) and mean as laid out by
+// normalize_workspace_bytes, the mean at *mean_offset of the workspace.
 hipError_t launch_normalize_scan_typed(int dtype, const void* src, int H, int W, int D, void* dst, int T,
-                                       void* partial, void* mean, hipStream_t s);
-size_t normalize_workspace_bytes(int dtype, int H, int T, int D, size_t* mean_offset);
+                                       void* partial, size_t partial_bytes, void* mean, hipStream_t s);
+// limit: size of a workspace that cannot grow (0 = none); a result above it
+// means the shape does not fit.
+size_t normalize_workspace_bytes(int dtype, int H, int T, int W, int D, size_t limit, size_t* mean_offset);
 
 // Constants of the isotropic aperture evaluated from d = Rout^2 - |u|^2.
 struct ApIso {

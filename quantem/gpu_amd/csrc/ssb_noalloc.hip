@@ -52,7 +52,7 @@ extern "C" int ssb_normalize_scan_u16_noalloc(const uint16_t* src, int H, int W,
   const long long D = (long long)det_rows * det_cols;
   if (D > (1 << 24)) return report_error(QSSB_ERR_UNSUPPORTED, "detector too large");
   size_t mean_off = 0;
-  const size_t need = normalize_workspace_bytes(QSSB_DTYPE_U16, H, T, (int)D, &mean_off);
+  const size_t need = normalize_workspace_bytes(QSSB_DTYPE_U16, H, T, W, (int)D, QSSB_NOALLOC_SCRATCH_BYTES, &mean_off);
   if (need > (size_t)QSSB_NOALLOC_SCRATCH_BYTES)
     return report_error(QSSB_ERR_ARG, "scan " + std::to_string(H) + " x " + std::to_string(W) + " with a " +
                                           std::to_string(det_rows) + " x " + std::to_string(det_cols) +
@@ -63,8 +63,8 @@ extern "C" int ssb_normalize_scan_u16_noalloc(const uint16_t* src, int H, int W,
   uint8_t* ws = nullptr;
   const int rc = scratch_of_current_device(&ws);
   if (rc) return rc;
-  const hipError_t e = launch_normalize_scan_typed(QSSB_DTYPE_U16, src, H, W, (int)D, dst, T, ws, ws + mean_off,
-                                                   reinterpret_cast<hipStream_t>(stream));
+  const hipError_t e = launch_normalize_scan_typed(QSSB_DTYPE_U16, src, H, W, (int)D, dst, T, ws, mean_off,
+                                                   ws + mean_off, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return report_hip_error(e, "normalize_scan_noalloc");
   return QSSB_OK;
 }

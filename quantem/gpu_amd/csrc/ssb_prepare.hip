@@ -14,67 +14,6 @@ namespace qssb {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// ------------------------------------------------------------------------
-// Mean DP, pass 1: per frame-range partial sums.
-// grid = (pixel tiles of 256*VEC, frame ranges).  Every workgroup streams a
-// contiguous 256*VEC-pixel slice of `frames_per_range` consecutive frames,
-// so each wave issues 16-byte coalesced non-temporal loads.  A range holds
-// at most 65536 frames, so the 32-bit partials of 8- and 16-bit samples
-// cannot overflow (65536 * 65535 < 2^32, 65536 * 32768 = 2^31); 32-bit
-// samples keep 64-bit partials (signed ones sign-extended, modulo 2^64, as
-// the reference's uint64 accumulator), float32 samples double-float pairs.
-// ------------------------------------------------------------------------
-template <int VEC>
-__global__ void __launch_bounds__(256)
-k_dp_partial(const uint16_t* __restrict__ data, long long frames, int D, int frames_per_range,
-             uint32_t* __restrict__ partial) {
-  const int pix0 = (blockIdx.x * 256 + threadIdx.x) * VEC;
-  const long long f0 = (long long)blockIdx.y * frames_per_range;
-  long long f1 = f0 + frames_per_range;
-  if (f1 > frames) f1 = frames;
-  if (pix0 >= D) return;
-  uint32_t acc[VEC];
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) acc[e] = 0u;
-  const uint16_t* p = data + f0 * (long long)D + pix0;
-  if constexpr (VEC == 8) {
-    long long f = f0;
-    for (; f + 2 <= f1; f += 2) {
-      u32x4 v[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-        v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + (long long)u * D));
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          acc[2 * w] += v[u][w] & 0xFFFFu;
-          acc[2 * w + 1] += v[u][w] >> 16;
-        }
-      }
-      p += 2LL * D;
-    }
-    for (; f < f1; ++f) {
-      u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        acc[2 * w] += v[w] & 0xFFFFu;
-        acc[2 * w + 1] += v[w] >> 16;
-      }
-      p += D;
-    }
-    uint32_t* out = partial + (long long)blockIdx.y * D + pix0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = acc[e];
-  } else {
-    for (long long f = f0; f < f1; ++f) {
-      acc[0] += p[0];
-      p += D;
-    }
-    partial[(long long)blockIdx.y * D + pix0] = acc[0];
-  }
-}
-
 // The uint16 stream pass of a reconstruction: the same partial sums, and
 // every frame's superset box copied compactly to C[frame][row - r0][col - c0]
 // (bh * bw uint16 per frame), so the BF gather reads contiguous box rows
@@ -170,40 +109,63 @@ __device__ __forceinline__ void dp_add(P& a, T v) {
   }
 }
 
-// Generic stream pass for the non-uint16 sample types: VEC samples of 16
-// bytes per thread and frame when the detector row allows it, else one.
-template <typename T, int VEC>
+// V samples of one frame, 16 bytes when V = 16 / sizeof(T).  Aligned to the
+// sample only: a detector whose pixel count is no multiple of V puts most
+// frames off 16 bytes, and global memory takes such a 16-byte access whole.
+template <typename T, int V> struct FrameVec {
+  typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+};
+
+// ------------------------------------------------------------------------
+// Mean DP, pass 1: per frame-range partial sums.  Bound by the one read of
+// the raw frames.  A thread owns V adjacent pixels (16 bytes) of a range of
+// consecutive frames, two frames in flight, non-temporal; the (range, lane)
+// pairs are dealt out linearly over the grid, so no lane idles whatever the
+// detector size, and the last lane of a frame steps back to D - V when V does
+// not divide D (the pixels it shares with its neighbour are summed by both to
+// the same value).  256 x 256 frames of 128 x 128 uint16: 311 us, 6.9 TB/s;
+// 61 x 83 uint16 pixels went one 2-byte load a thread before.  A range holds at most 65536 frames, so the 32-bit
+// partials of 8- and 16-bit samples cannot overflow (65536 * 65535 < 2^32,
+// 65536 * 32768 = 2^31); 32-bit samples keep 64-bit partials (signed ones
+// sign-extended, modulo 2^64, as the reference's uint64 accumulator), float32
+// samples double-float pairs.
+// ------------------------------------------------------------------------
+template <typename T, int V>
 __global__ void __launch_bounds__(256)
-k_dp_partial_t(const T* __restrict__ data, long long frames, int D, int frames_per_range,
-               typename DpElem<T>::P* __restrict__ partial) {
+k_dp_partial(const T* __restrict__ data, long long frames, int D, int lanes, int ranges, int frames_per_range,
+             typename DpElem<T>::P* __restrict__ partial) {
   typedef typename DpElem<T>::P P;
-  const int pix0 = (blockIdx.x * 256 + threadIdx.x) * VEC;
-  const long long f0 = (long long)blockIdx.y * frames_per_range;
-  long long f1 = f0 + frames_per_range;
-  if (f1 > frames) f1 = frames;
-  if (pix0 >= D) return;
-  P acc[VEC];
+  typedef typename FrameVec<T, V>::type Vec;
+  const unsigned gid = blockIdx.x * 256u + threadIdx.x;
+  const int r = (int)(gid / (unsigned)lanes);
+  if (r >= ranges) return;
+  const int pix0 = min((int)(gid - (unsigned)r * (unsigned)lanes) * V, D - V);
+  const long long f0 = (long long)r * frames_per_range;
+  const int n = (int)min((long long)frames_per_range, frames - f0);
+  P acc[V];
 #pragma unroll
-  for (int e = 0; e < VEC; ++e) dp_zero(acc[e]);
+  for (int e = 0; e < V; ++e) dp_zero(acc[e]);
   const T* p = data + f0 * (long long)D + pix0;
-  for (long long f = f0; f < f1; ++f) {
-    if constexpr (VEC * sizeof(T) == 16) {
-      union {
-        u32x4 v;
-        T e[VEC];
-      } u;
-      u.v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  int f = 0;
+  if constexpr (sizeof(T) == 2) {   // wider and narrower samples spend more on the sums and gain nothing here
+    for (; f + 2 <= n; f += 2) {
+      const Vec v0 = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(p));
+      const Vec v1 = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(p + D));
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) dp_add<T, P>(acc[e], u.e[e]);
-    } else {
+      for (int e = 0; e < V; ++e) dp_add<T, P>(acc[e], (T)v0[e]);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) dp_add<T, P>(acc[e], p[e]);
+      for (int e = 0; e < V; ++e) dp_add<T, P>(acc[e], (T)v1[e]);
+      p += 2LL * D;
     }
-    p += D;
   }
-  P* out = partial + (long long)blockIdx.y * D + pix0;
+  for (; f < n; ++f, p += D) {
+    const Vec v = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(p));
 #pragma unroll
-  for (int e = 0; e < VEC; ++e) out[e] = acc[e];
+    for (int e = 0; e < V; ++e) dp_add<T, P>(acc[e], (T)v[e]);
+  }
+  P* out = partial + (long long)r * D + pix0;
+#pragma unroll
+  for (int e = 0; e < V; ++e) out[e] = acc[e];
 }
 
 // Pass 2: fold the frame ranges into exact uint64 sums (integer samples) or
@@ -242,15 +204,12 @@ k_dp_reduce(const P* __restrict__ partial, int ranges, int D, long long frames, 
   dp_zero(s);
   if (i < D) {
     int r = quarter;
-    for (; r + 3 * LANES < ranges; r += 4 * LANES) {
-      const P a = partial[(long long)r * D + i];
-      const P b = partial[(long long)(r + LANES) * D + i];
-      const P c = partial[(long long)(r + 2 * LANES) * D + i];
-      const P d = partial[(long long)(r + 3 * LANES) * D + i];
-      dp_fold<P>(s, a);
-      dp_fold<P>(s, b);
-      dp_fold<P>(s, c);
-      dp_fold<P>(s, d);
+    for (; r + 7 * LANES < ranges; r += 8 * LANES) {
+      P v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = partial[(long long)(r + k * LANES) * D + i];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) dp_fold<P>(s, v[k]);
     }
     for (; r < ranges; r += LANES) dp_fold<P>(s, partial[(long long)r * D + i]);
   }
@@ -896,8 +855,8 @@ k_gather_rowfft(const T* __restrict__ data, int D, int det_cols,
 // frames per range so the 32-bit partial sums cannot overflow.  `vec` is
 // the pixels per thread of the stream kernel.
 static void range_split(long long frames, int D, int vec, int max_ranges, int target_wg, int& ranges, int& fpr) {
-  const long long tiles = (D / vec + 255) / 256;
-  long long r = (target_wg > 0 ? target_wg : 1536) / (tiles > 0 ? tiles : 1);
+  const long long lanes = (D + vec - 1) / vec;
+  long long r = (target_wg > 0 ? target_wg : 1536) * 256LL / lanes;
   const long long min_r = (frames + 65535) / 65536;
   if (r < min_r) r = min_r;
   if (r > max_ranges) r = max_ranges;
@@ -905,6 +864,15 @@ static void range_split(long long frames, int D, int vec, int max_ranges, int ta
   if (r < 1) r = 1;
   fpr = (int)((frames + r - 1) / r);
   ranges = (int)((frames + fpr - 1) / fpr);
+}
+
+// Ranges a plan keeps partial sums for.  256 ranges of a 128 x 128 detector
+// are 2048 workgroups; smaller detectors need more ranges to fill the chip
+// (64 x 64 at scan 128: 512 workgroups, 4.7 TB/s), up to 768, where the
+// reduction over them starts to cost what the stream gains.
+int dp_max_ranges(int D) {
+  const int r = (256 * 16384) / (D > 0 ? D : 1);
+  return r < 256 ? 256 : (r > 768 ? 768 : r);
 }
 
 int dtype_size(int dtype) {
@@ -920,12 +888,10 @@ bool dtype_wide_partials(int dtype) {
   return dtype == QSSB_DTYPE_U32 || dtype == QSSB_DTYPE_I32 || dtype == QSSB_DTYPE_F32;
 }
 
-// pixels per thread of the stream pass for this dtype, detector and base address
-static int stream_vec(int dtype, int D, const void* data) {
-  const int es = dtype_size(dtype);
-  const int v = 16 / es;
-  const bool aligned = (reinterpret_cast<uintptr_t>(data) & 15u) == 0;
-  return (D % v == 0 && aligned) ? v : 1;
+// pixels per thread of the stream and copy passes: 16 bytes of any detector that holds them
+static int stream_vec(int dtype, int D) {
+  const int v = 16 / dtype_size(dtype);
+  return D >= v ? v : 1;
 }
 
 template <typename T>
@@ -933,34 +899,24 @@ static void launch_partial_t(const void* data, long long frames, int D, int vec,
                              hipStream_t s) {
   typedef typename DpElem<T>::P P;
   constexpr int V = 16 / sizeof(T);
-  if (vec == V) {
-    dim3 grid((D / V + 255) / 256, ranges);
-    hipLaunchKernelGGL((k_dp_partial_t<T, V>), grid, dim3(256), 0, s, reinterpret_cast<const T*>(data), frames, D,
-                       fpr, reinterpret_cast<P*>(partial));
-  } else {
-    dim3 grid((D + 255) / 256, ranges);
-    hipLaunchKernelGGL((k_dp_partial_t<T, 1>), grid, dim3(256), 0, s, reinterpret_cast<const T*>(data), frames, D,
-                       fpr, reinterpret_cast<P*>(partial));
-  }
+  const int lanes = (D + vec - 1) / vec;
+  const dim3 grid((unsigned)(((long long)lanes * ranges + 255) / 256));
+  if (vec == V)
+    hipLaunchKernelGGL((k_dp_partial<T, V>), grid, dim3(256), 0, s, reinterpret_cast<const T*>(data), frames, D,
+                       lanes, ranges, fpr, reinterpret_cast<P*>(partial));
+  else
+    hipLaunchKernelGGL((k_dp_partial<T, 1>), grid, dim3(256), 0, s, reinterpret_cast<const T*>(data), frames, D,
+                       lanes, ranges, fpr, reinterpret_cast<P*>(partial));
 }
 
 hipError_t launch_mean_dp_stream(int dtype, const void* data, long long frames, int D, void* partial, int max_ranges,
                                  int target_wg, hipStream_t s) {
-  const int vec = stream_vec(dtype, D, data);
+  if (!dtype_size(dtype)) return hipErrorInvalidValue;
+  const int vec = stream_vec(dtype, D);
   int ranges, fpr;
   range_split(frames, D, vec, max_ranges, target_wg, ranges, fpr);
   switch (dtype) {
-    case QSSB_DTYPE_U16:
-      if (vec == 8) {
-        dim3 grid((D / 8 + 255) / 256, ranges);
-        hipLaunchKernelGGL(k_dp_partial<8>, grid, dim3(256), 0, s, reinterpret_cast<const uint16_t*>(data), frames,
-                           D, fpr, reinterpret_cast<uint32_t*>(partial));
-      } else {
-        dim3 grid((D + 255) / 256, ranges);
-        hipLaunchKernelGGL(k_dp_partial<1>, grid, dim3(256), 0, s, reinterpret_cast<const uint16_t*>(data), frames,
-                           D, fpr, reinterpret_cast<uint32_t*>(partial));
-      }
-      break;
+    case QSSB_DTYPE_U16: launch_partial_t<uint16_t>(data, frames, D, vec, ranges, fpr, partial, s); break;
     case QSSB_DTYPE_U8: launch_partial_t<uint8_t>(data, frames, D, vec, ranges, fpr, partial, s); break;
     case QSSB_DTYPE_I8: launch_partial_t<int8_t>(data, frames, D, vec, ranges, fpr, partial, s); break;
     case QSSB_DTYPE_I16: launch_partial_t<int16_t>(data, frames, D, vec, ranges, fpr, partial, s); break;
@@ -974,7 +930,7 @@ hipError_t launch_mean_dp_stream(int dtype, const void* data, long long frames, 
 
 hipError_t launch_mean_dp_stream_sup(const uint16_t* data, long long frames, int D, int det_cols, uint32_t* partial,
                                      int max_ranges, int target_wg, const SupBox* box, uint16_t* C, hipStream_t s) {
-  if (det_cols % 8 != 0 || stream_vec(QSSB_DTYPE_U16, D, data) != 8) return hipErrorInvalidValue;
+  if (det_cols % 8 != 0 || (reinterpret_cast<uintptr_t>(data) & 15u) != 0) return hipErrorInvalidValue;
   int ranges, fpr;
   range_split(frames, D, 8, max_ranges, target_wg, ranges, fpr);
   dim3 grid((D / 8 + 255) / 256, ranges);
@@ -982,12 +938,12 @@ hipError_t launch_mean_dp_stream_sup(const uint16_t* data, long long frames, int
   return hipGetLastError();
 }
 
-hipError_t launch_mean_dp_reduce(int dtype, const void* data, long long frames, int D, const void* partial,
+hipError_t launch_mean_dp_reduce(int dtype, long long frames, int D, const void* partial,
                                  int max_ranges, int target_wg, const float* gain, unsigned long long* sums,
                                  float* mean, float* dcpix, hipStream_t s) {
-  const int vec = stream_vec(dtype, D, data);
+  if (!dtype_size(dtype)) return hipErrorInvalidValue;
   int ranges, fpr;
-  range_split(frames, D, vec, max_ranges, target_wg, ranges, fpr);
+  range_split(frames, D, stream_vec(dtype, D), max_ranges, target_wg, ranges, fpr);
   // 16 range lanes per pixel column: 1024-thread workgroups keep enough
   // loads in flight for a reduction that has only D / 64 workgroups
   const dim3 grid((D + 63) / 64), block(1024);
@@ -1011,7 +967,7 @@ hipError_t launch_mean_dp(int dtype, const void* data, long long frames, int D, 
                           hipStream_t s) {
   hipError_t e = launch_mean_dp_stream(dtype, data, frames, D, partial, max_ranges, target_wg, s);
   if (e != hipSuccess) return e;
-  return launch_mean_dp_reduce(dtype, data, frames, D, partial, max_ranges, target_wg, gain, sums, mean, dcpix, s);
+  return launch_mean_dp_reduce(dtype, frames, D, partial, max_ranges, target_wg, gain, sums, mean, dcpix, s);
 }
 
 // ------------------------------------------------------------------------
@@ -1243,255 +1199,264 @@ hipError_t launch_gather_rowfft(int N, int dtype, const void* data, int D, int d
 // ------------------------------------------------------------------------
 // Scan normalisation (cuda/backend.py:229-269): centre-crop oversize axes to
 // the window (r0, c0, h, w) of the source, pad to T x T with the window's
-// mean frame floor(sum / (h*w)) -- the reference's int64 sum, float64 divide
-// and truncating cast give exactly the integer floor for these ranges --
-// placed at pad_top = (T - h)/2, pad_left = (T - w)/2.
+// mean frame -- integer sums divided with truncation toward zero (the
+// reference's int64 sum, float64 quotient and truncating cast give exactly
+// that integer for these ranges), float32 frames a double-float mean rounded
+// once -- placed at pad_top = (T - h)/2, pad_left = (T - w)/2.
+//
+// Bound by the copy: each window frame is read once and written once, its
+// sums taken on the way (k_window_copy), then the mean frame goes to the
+// border (k_pad_fill).  203 x 178 frames of 93 x 96 uint16 into 256 x 256:
+// the separate sum and copy passes, which read the frames twice, took 331 +
+// 424 us; these take 228 (1.29 GB copied, 5.7 TB/s) + 7 + 105.
 // ------------------------------------------------------------------------
-constexpr int kWindowRows = 64;   // window rows per partial sum: 64*1024*65535 < 2^32
+struct Window {
+  int W, D;            // source scan columns, pixels per frame
+  int r0, c0, h, w;    // the window in the source
+  int T, top, left;    // target size and the window's place in it
+};
 
-// Window rows per partial sum: at most kWindowRows; integer samples split
-// further so that a small detector still spreads over ~256 workgroups
-// (integer sums are exact in any split); float32 keeps kWindowRows, since
-// its double-float sums depend on the split.
-static int window_rows(int dtype, int h, int D) {
-  if (dtype == QSSB_DTYPE_F32) return kWindowRows;
-  const int tiles = (D + 255) / 256;
-  const int want = (256 + tiles - 1) / tiles;
-  const int rows = (h + want - 1) / want;
-  return rows < 1 ? 1 : (rows > kWindowRows ? kWindowRows : rows);
-}
-
+template <typename T, int V, bool SUM>
 __global__ void __launch_bounds__(256)
-k_window_partial(const uint16_t* __restrict__ src, int W, int D, int r0, int c0, int h, int w, int rows,
-                 uint32_t* __restrict__ partial) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= D) return;
-  const int ra = blockIdx.y * rows;
-  const int rb = min(h, ra + rows);
-  uint32_t acc = 0u;
-  for (int r = ra; r < rb; ++r) {
-    const uint16_t* row = src + ((long long)(r0 + r) * W + c0) * D + p;
-#pragma unroll 8
-    for (int c = 0; c < w; ++c) acc += row[(long long)c * D];
-  }
-  partial[(long long)blockIdx.y * D + p] = acc;
-}
-
-__global__ void __launch_bounds__(256)
-k_window_mean(const uint32_t* __restrict__ partial, int groups, int D, unsigned long long count,
-              uint16_t* __restrict__ mean) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= D) return;
-  unsigned long long s = 0ull;
-  for (int g = 0; g < groups; ++g) s += partial[(long long)g * D + p];
-  mean[p] = (uint16_t)(s / count);
-}
-
-template <int VEC>
-__global__ void __launch_bounds__(256)
-k_pad_copy(const uint16_t* __restrict__ src, int W, int D, int r0, int c0, int h, int w, int T, int pad_top,
-           int pad_left, const uint16_t* __restrict__ mean, uint16_t* __restrict__ dst) {
-  const long long frame = blockIdx.y + (long long)blockIdx.z * 65535;
-  if (frame >= (long long)T * T) return;
-  const int i = (int)(frame / T), j = (int)(frame % T);
-  const int si = i - pad_top, sj = j - pad_left;
-  const bool inside = si >= 0 && si < h && sj >= 0 && sj < w;
-  const uint16_t* from = inside ? src + ((long long)(r0 + si) * W + (c0 + sj)) * D : mean;
-  uint16_t* to = dst + frame * D;
-  const int e = (blockIdx.x * 256 + threadIdx.x) * VEC;
-  if (e >= D) return;
-  if constexpr (VEC == 8) {
-    *reinterpret_cast<u32x4*>(to + e) = *reinterpret_cast<const u32x4*>(from + e);
-  } else {
-    to[e] = from[e];
-  }
-}
-
-hipError_t launch_normalize_scan(const uint16_t* src, int H, int W, int D, uint16_t* dst, int T,
-                                 uint32_t* partial, uint16_t* mean, hipStream_t s) {
-  const int r0 = H > T ? (H - T) / 2 : 0;
-  const int c0 = W > T ? (W - T) / 2 : 0;
-  const int h = H < T ? H : T;
-  const int w = W < T ? W : T;
-  const int pad_top = (T - h) / 2, pad_left = (T - w) / 2;
-  if (h < T || w < T) {
-    const int rows = window_rows(QSSB_DTYPE_U16, h, D);
-    const int groups = (h + rows - 1) / rows;
-    hipLaunchKernelGGL(k_window_partial, dim3((D + 255) / 256, groups), dim3(256), 0, s, src, W, D, r0, c0, h, w,
-                       rows, partial);
-    hipLaunchKernelGGL(k_window_mean, dim3((D + 255) / 256), dim3(256), 0, s, partial, groups, D,
-                       (unsigned long long)h * (unsigned long long)w, mean);
-  }
-  const long long frames = (long long)T * T;
-  const dim3 grid_f(1, (unsigned)(frames < 65535 ? frames : 65535), (unsigned)((frames + 65534) / 65535));
-  const bool vec = (D % 8 == 0) && ((reinterpret_cast<uintptr_t>(src) & 15u) == 0) &&
-                   ((reinterpret_cast<uintptr_t>(dst) & 15u) == 0) && ((reinterpret_cast<uintptr_t>(mean) & 15u) == 0);
-  if (vec) {
-    dim3 g = grid_f;
-    g.x = (D / 8 + 255) / 256;
-    hipLaunchKernelGGL(k_pad_copy<8>, g, dim3(256), 0, s, src, W, D, r0, c0, h, w, T, pad_top, pad_left, mean, dst);
-  } else {
-    dim3 g = grid_f;
-    g.x = (D + 255) / 256;
-    hipLaunchKernelGGL(k_pad_copy<1>, g, dim3(256), 0, s, src, W, D, r0, c0, h, w, T, pad_top, pad_left, mean, dst);
-  }
-  return hipGetLastError();
-}
-
-int normalize_partial_groups(int dtype, int H, int T, int D) {
-  const int h = H < T ? H : T;
-  const int rows = window_rows(dtype, h, D);
-  return (h + rows - 1) / rows;
-}
-
-// Scan normalisation of the other sample types: per 64-row group int64
-// sums (integers) or double-float sums (float32) of the window, then the
-// pad frame sum / count truncated toward zero (the float64 quotient of an
-// int64 sum below 2^53 truncates to the same integer) or rounded to float32.
-template <typename T> struct WinSum { typedef long long S; };
-template <> struct WinSum<float> { typedef float2 S; };
-
-template <typename T>
-__global__ void __launch_bounds__(256)
-k_window_partial_t(const T* __restrict__ src, int W, int D, int r0, int c0, int h, int w, int rows,
-                   typename WinSum<T>::S* __restrict__ partial) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= D) return;
-  const int ra = blockIdx.y * rows;
-  const int rb = min(h, ra + rows);
-  if constexpr (std::is_same<T, float>::value) {
-    float hi = 0.0f, lo = 0.0f;
-    for (int r = ra; r < rb; ++r) {
-      const T* row = src + ((long long)(r0 + r) * W + c0) * D + p;
-      for (int c = 0; c < w; ++c) {
-        const df t = two_sum(hi, row[(long long)c * D]);
-        hi = t.hi;
-        lo += t.lo;
+k_window_copy(const T* __restrict__ src, Window g, int lanes, int ranges, int frames_per_range, T* __restrict__ dst,
+              typename DpElem<T>::P* __restrict__ partial) {
+  typedef typename DpElem<T>::P P;
+  typedef typename FrameVec<T, V>::type Vec;
+  constexpr int U = 4;   // frames in flight
+  const unsigned gid = blockIdx.x * 256u + threadIdx.x;
+  const int r = (int)(gid / (unsigned)lanes);
+  if (r >= ranges) return;
+  const int pix0 = min((int)(gid - (unsigned)r * (unsigned)lanes) * V, g.D - V);
+  const int f0 = r * frames_per_range;
+  const int n = min(frames_per_range, g.h * g.w - f0);
+  int i = f0 / g.w, j = f0 - (f0 / g.w) * g.w;
+  const T* from = src + ((long long)(g.r0 + i) * g.W + g.c0 + j) * g.D + pix0;
+  T* to = dst + ((long long)(g.top + i) * g.T + g.left + j) * g.D + pix0;
+  P acc[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) dp_zero(acc[e]);
+  // both pointers to the next frame of the window: past a row's end they skip what lies outside it
+  const long long srow = (long long)(g.W - g.w) * g.D, drow = (long long)(g.T - g.w) * g.D;
+  auto step = [&](const T*& a, T*& b) {
+    const bool wrap = ++j == g.w;
+    j = wrap ? 0 : j;
+    a += g.D + (wrap ? srow : 0);
+    b += g.D + (wrap ? drow : 0);
+  };
+  int f = 0;
+  for (; f + U <= n; f += U) {
+    Vec v[U];
+    T* at[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      v[u] = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(from));
+      at[u] = to;
+      step(from, to);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      *reinterpret_cast<Vec*>(at[u]) = v[u];
+      if constexpr (SUM) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) dp_add<T, P>(acc[e], (T)v[u][e]);
       }
     }
-    partial[(long long)blockIdx.y * D + p] = make_float2(hi, lo);
-  } else {
-    long long acc = 0;
-    for (int r = ra; r < rb; ++r) {
-      const T* row = src + ((long long)(r0 + r) * W + c0) * D + p;
-#pragma unroll 8
-      for (int c = 0; c < w; ++c) acc += (long long)row[(long long)c * D];
-    }
-    partial[(long long)blockIdx.y * D + p] = acc;
   }
+  for (; f < n; ++f) {
+    const Vec v = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(from));
+    *reinterpret_cast<Vec*>(to) = v;
+    if constexpr (SUM) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) dp_add<T, P>(acc[e], (T)v[e]);
+    }
+    step(from, to);
+  }
+  if constexpr (SUM) {
+    P* out = partial + (long long)r * g.D + pix0;
+#pragma unroll
+    for (int e = 0; e < V; ++e) out[e] = acc[e];
+  }
+}
+
+// The pad frame from the ranges' sums: a workgroup owns 64 pixels, its 16
+// waves fold interleaved shares of the ranges and combine in wave order.
+template <typename T>
+__global__ void __launch_bounds__(1024)
+k_window_mean(const typename DpElem<T>::P* __restrict__ partial, int ranges, int D, long long count,
+              T* __restrict__ mean) {
+  typedef typename DpElem<T>::P P;
+  typedef typename std::conditional<std::is_same<T, float>::value, df, long long>::type S;
+  __shared__ S part[16][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + lane;
+  S s{};
+  auto fold = [&](P v) {
+    if constexpr (std::is_same<T, float>::value) s = df_add(s, df{v.x, v.y});
+    else s += (long long)v;
+  };
+  if (p < D) {
+    int r = wv;
+    for (; r + 3 * 16 < ranges; r += 4 * 16) {
+      P v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = partial[(long long)(r + 16 * k) * D + p];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) fold(v[k]);
+    }
+    for (; r < ranges; r += 16) fold(partial[(long long)r * D + p]);
+  }
+  part[wv][lane] = s;
+  __syncthreads();
+  if (wv == 0 && p < D) {
+    S t{};
+    for (int k = 0; k < 16; ++k) {
+      if constexpr (std::is_same<T, float>::value) t = df_add(t, part[k][lane]);
+      else t += part[k][lane];
+    }
+    if constexpr (std::is_same<T, float>::value) {
+      const df q = df_div(t, df{(float)count, (float)(count - (long long)(float)count)});
+      mean[p] = q.hi + q.lo;
+    } else {
+      mean[p] = (T)(t / count);
+    }
+  }
+}
+
+// The mean frame into every frame outside the window: a thread keeps its V
+// pixels and stores them to a range of border frames, taken in the order top
+// rows, the rows beside the window, bottom rows.
+template <typename T, int V>
+__global__ void __launch_bounds__(256)
+k_pad_fill(const T* __restrict__ mean, Window g, int lanes, int ranges, int frames_per_range, T* __restrict__ dst) {
+  typedef typename FrameVec<T, V>::type Vec;
+  const unsigned gid = blockIdx.x * 256u + threadIdx.x;
+  const int r = (int)(gid / (unsigned)lanes);
+  if (r >= ranges) return;
+  const int pix0 = min((int)(gid - (unsigned)r * (unsigned)lanes) * V, g.D - V);
+  const Vec v = *reinterpret_cast<const Vec*>(mean + pix0);
+  const int above = g.top * g.T, side = g.T - g.w;
+  const int beside = above + g.h * side;
+  const int total = g.T * g.T - g.h * g.w;
+  const int k1 = min(total, (r + 1) * frames_per_range);
+  for (int k = r * frames_per_range; k < k1; ++k) {
+    int frame;
+    if (k < above) {
+      frame = k;
+    } else if (k < beside) {
+      const int i = (k - above) / side, c = (k - above) - i * side;
+      frame = (g.top + i) * g.T + (c < g.left ? c : c + g.w);
+    } else {
+      frame = k - beside + (g.top + g.h) * g.T;
+    }
+    *reinterpret_cast<Vec*>(dst + (long long)frame * g.D + pix0) = v;
+  }
+}
+
+static Window window_of(int H, int W, int D, int T) {
+  Window g;
+  g.W = W;
+  g.D = D;
+  g.r0 = H > T ? (H - T) / 2 : 0;
+  g.c0 = W > T ? (W - T) / 2 : 0;
+  g.h = H < T ? H : T;
+  g.w = W < T ? W : T;
+  g.T = T;
+  g.top = (T - g.h) / 2;
+  g.left = (T - g.w) / 2;
+  return g;
+}
+
+static size_t window_sum_bytes(int dtype) { return dtype_wide_partials(dtype) ? 8 : 4; }
+
+// Ranges of window frames whose sums fit `room` bytes: the stream pass's
+// share of workgroups, and never over 65536 frames a range.
+static void window_split(int dtype, const Window& g, size_t room, int& ranges, int& fpr) {
+  const long long fit = (long long)(room / ((size_t)g.D * window_sum_bytes(dtype)));
+  const int most = (int)(fit < 1 ? 1 : (fit > 1024 ? 1024 : fit));
+  range_split((long long)g.h * g.w, g.D, stream_vec(dtype, g.D), most, 0, ranges, fpr);
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256)
-k_window_mean_t(const typename WinSum<T>::S* __restrict__ partial, int groups, int D, long long count,
-                T* __restrict__ mean) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= D) return;
-  if constexpr (std::is_same<T, float>::value) {
-    df s{0.0f, 0.0f};
-    for (int g = 0; g < groups; ++g) {
-      const float2 v = partial[(long long)g * D + p];
-      s = df_add(s, df{v.x, v.y});
-    }
-    const df q = df_div(s, df{(float)count, (float)(count - (long long)(float)count)});
-    mean[p] = q.hi + q.lo;
-  } else {
-    long long s = 0;
-    for (int g = 0; g < groups; ++g) s += partial[(long long)g * D + p];
-    mean[p] = (T)(s / count);
-  }
-}
-
-// Copy (or pad) one frame of `fbytes` bytes per grid row, in 16-byte words
-// when every frame is 16-byte aligned, else in elements of `es` bytes.
-template <int ES>
-__global__ void __launch_bounds__(256)
-k_pad_copy_bytes(const uint8_t* __restrict__ src, int W, long long fbytes, int r0, int c0, int h, int w, int T,
-                 int pad_top, int pad_left, const uint8_t* __restrict__ mean, uint8_t* __restrict__ dst) {
-  const long long frame = blockIdx.y + (long long)blockIdx.z * 65535;
-  if (frame >= (long long)T * T) return;
-  const int i = (int)(frame / T), j = (int)(frame % T);
-  const int si = i - pad_top, sj = j - pad_left;
-  const bool inside = si >= 0 && si < h && sj >= 0 && sj < w;
-  const uint8_t* from = inside ? src + ((long long)(r0 + si) * W + (c0 + sj)) * fbytes : mean;
-  uint8_t* to = dst + frame * fbytes;
-  const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * ES;
-  if (e >= fbytes) return;
-  if constexpr (ES == 16) {
-    *reinterpret_cast<u32x4*>(to + e) = *reinterpret_cast<const u32x4*>(from + e);
-  } else if constexpr (ES == 4) {
-    *reinterpret_cast<uint32_t*>(to + e) = *reinterpret_cast<const uint32_t*>(from + e);
-  } else if constexpr (ES == 2) {
-    *reinterpret_cast<uint16_t*>(to + e) = *reinterpret_cast<const uint16_t*>(from + e);
-  } else {
-    to[e] = from[e];
-  }
-}
-
-template <typename T>
-static hipError_t normalize_typed(const void* src_v, int H, int W, int D, void* dst_v, int T_, void* partial_v,
-                                  void* mean_v, hipStream_t s) {
-  typedef typename WinSum<T>::S S;
-  const int r0 = H > T_ ? (H - T_) / 2 : 0;
-  const int c0 = W > T_ ? (W - T_) / 2 : 0;
-  const int h = H < T_ ? H : T_;
-  const int w = W < T_ ? W : T_;
-  const int pad_top = (T_ - h) / 2, pad_left = (T_ - w) / 2;
+static hipError_t normalize_typed(int dtype, const void* src_v, const Window& g, void* dst_v, void* partial_v,
+                                  size_t partial_bytes, void* mean_v, hipStream_t s) {
+  typedef typename DpElem<T>::P P;
+  constexpr int V = 16 / sizeof(T);
+  const int vec = stream_vec(dtype, g.D);
+  const int lanes = (g.D + vec - 1) / vec;
   const T* src = reinterpret_cast<const T*>(src_v);
+  T* dst = reinterpret_cast<T*>(dst_v);
   T* mean = reinterpret_cast<T*>(mean_v);
-  if (h < T_ || w < T_) {
-    const int rows = window_rows(std::is_same<T, float>::value ? QSSB_DTYPE_F32 : QSSB_DTYPE_I32, h, D);
-    const int groups = (h + rows - 1) / rows;
-    S* partial = reinterpret_cast<S*>(partial_v);
-    hipLaunchKernelGGL(k_window_partial_t<T>, dim3((D + 255) / 256, groups), dim3(256), 0, s, src, W, D, r0, c0, h,
-                       w, rows, partial);
-    hipLaunchKernelGGL(k_window_mean_t<T>, dim3((D + 255) / 256), dim3(256), 0, s, partial, groups, D,
-                       (long long)h * w, mean);
+  P* partial = reinterpret_cast<P*>(partial_v);
+  const bool pad = g.h < g.T || g.w < g.T;
+  int ranges, fpr;
+  window_split(dtype, g, pad ? partial_bytes : ~(size_t)0, ranges, fpr);
+  const dim3 grid((unsigned)(((long long)lanes * ranges + 255) / 256));
+#define QSSB_COPY(VV, SUM)                                                                                       \
+  hipLaunchKernelGGL((k_window_copy<T, VV, SUM>), grid, dim3(256), 0, s, src, g, lanes, ranges, fpr, dst, partial)
+  if (!pad) {
+    if (vec == V) QSSB_COPY(V, false);
+    else QSSB_COPY(1, false);
+    return hipGetLastError();
   }
-  const long long frames = (long long)T_ * T_;
-  const long long fbytes = (long long)D * sizeof(T);
-  dim3 grid(1, (unsigned)(frames < 65535 ? frames : 65535), (unsigned)((frames + 65534) / 65535));
-  auto al = [](const void* q, int a) { return (reinterpret_cast<uintptr_t>(q) % a) == 0; };
-  const uint8_t* sb = reinterpret_cast<const uint8_t*>(src_v);
-  const uint8_t* mb = reinterpret_cast<const uint8_t*>(mean_v);
-  uint8_t* db = reinterpret_cast<uint8_t*>(dst_v);
-  if (fbytes % 16 == 0 && al(sb, 16) && al(db, 16) && al(mb, 16)) {
-    grid.x = (unsigned)((fbytes / 16 + 255) / 256);
-    hipLaunchKernelGGL(k_pad_copy_bytes<16>, grid, dim3(256), 0, s, sb, W, fbytes, r0, c0, h, w, T_, pad_top,
-                       pad_left, mb, db);
-  } else {
-    constexpr int ES = sizeof(T);
-    grid.x = (unsigned)((fbytes / ES + 255) / 256);
-    hipLaunchKernelGGL(k_pad_copy_bytes<ES>, grid, dim3(256), 0, s, sb, W, fbytes, r0, c0, h, w, T_, pad_top,
-                       pad_left, mb, db);
-  }
+  if (vec == V) QSSB_COPY(V, true);
+  else QSSB_COPY(1, true);
+#undef QSSB_COPY
+  hipLaunchKernelGGL(k_window_mean<T>, dim3((g.D + 63) / 64), dim3(1024), 0, s, partial, ranges, g.D,
+                     (long long)g.h * g.w, mean);
+  const int border = g.T * g.T - g.h * g.w;
+  int fr, ff;
+  range_split(border, g.D, vec, 65536, 0, fr, ff);
+  const dim3 fgrid((unsigned)(((long long)lanes * fr + 255) / 256));
+  if (vec == V)
+    hipLaunchKernelGGL((k_pad_fill<T, V>), fgrid, dim3(256), 0, s, mean, g, lanes, fr, ff, dst);
+  else
+    hipLaunchKernelGGL((k_pad_fill<T, 1>), fgrid, dim3(256), 0, s, mean, g, lanes, fr, ff, dst);
   return hipGetLastError();
 }
 
 hipError_t launch_normalize_scan_typed(int dtype, const void* src, int H, int W, int D, void* dst, int T,
-                                       void* partial, void* mean, hipStream_t s) {
+                                       void* partial, size_t partial_bytes, void* mean, hipStream_t s) {
+  const Window g = window_of(H, W, D, T);
   switch (dtype) {
-    case QSSB_DTYPE_U16:
-      return launch_normalize_scan(reinterpret_cast<const uint16_t*>(src), H, W, D, reinterpret_cast<uint16_t*>(dst),
-                                   T, reinterpret_cast<uint32_t*>(partial), reinterpret_cast<uint16_t*>(mean), s);
-    case QSSB_DTYPE_U8: return normalize_typed<uint8_t>(src, H, W, D, dst, T, partial, mean, s);
-    case QSSB_DTYPE_I8: return normalize_typed<int8_t>(src, H, W, D, dst, T, partial, mean, s);
-    case QSSB_DTYPE_I16: return normalize_typed<int16_t>(src, H, W, D, dst, T, partial, mean, s);
-    case QSSB_DTYPE_U32: return normalize_typed<uint32_t>(src, H, W, D, dst, T, partial, mean, s);
-    case QSSB_DTYPE_I32: return normalize_typed<int32_t>(src, H, W, D, dst, T, partial, mean, s);
-    case QSSB_DTYPE_F32: return normalize_typed<float>(src, H, W, D, dst, T, partial, mean, s);
+#define QSSB_NORM(CODE, TT) case CODE: return normalize_typed<TT>(dtype, src, g, dst, partial, partial_bytes, mean, s);
+    QSSB_NORM(QSSB_DTYPE_U16, uint16_t)
+    QSSB_NORM(QSSB_DTYPE_U8, uint8_t)
+    QSSB_NORM(QSSB_DTYPE_I8, int8_t)
+    QSSB_NORM(QSSB_DTYPE_I16, int16_t)
+    QSSB_NORM(QSSB_DTYPE_U32, uint32_t)
+    QSSB_NORM(QSSB_DTYPE_I32, int32_t)
+    QSSB_NORM(QSSB_DTYPE_F32, float)
+#undef QSSB_NORM
     default: return hipErrorInvalidValue;
   }
 }
 
-// bytes of the partial sums and of the pad frame of launch_normalize_scan_typed
-size_t normalize_workspace_bytes(int dtype, int H, int T, int D, size_t* mean_offset) {
-  const int groups = normalize_partial_groups(dtype, H, T, D);
-  const size_t per = dtype == QSSB_DTYPE_U16 ? 4 : 8;
-  size_t part = (size_t)groups * D * per;
-  part = (part + 255) & ~(size_t)255;
+// Bytes of the partial sums (`*mean_offset` of them, a multiple of 256) and
+// of the pad frame.  Without a limit: the ranges window_split would take.
+// With one (a workspace that cannot grow): as many as fit, at least one range
+// per 64 window rows, or per as many as spread a small detector over 256
+// workgroups; a shape whose sums in that split pass the limit is the
+// caller's to refuse.
+size_t normalize_workspace_bytes(int dtype, int H, int T, int W, int D, size_t limit, size_t* mean_offset) {
+  const Window g = window_of(H, W, D, T);
+  const size_t tail = (size_t)D * dtype_size(dtype) + 256;
+  const size_t per = window_sum_bytes(dtype);
+  const size_t align = ~(size_t)255;
+  size_t part;
+  if (limit == 0) {
+    int ranges, fpr;
+    window_split(dtype, g, ~(size_t)0, ranges, fpr);
+    part = ((size_t)ranges * D * per + 255) & align;
+  } else {
+    const int tiles = (D + 255) / 256;
+    const int want = (256 + tiles - 1) / tiles;
+    int rows = (g.h + want - 1) / want;
+    rows = rows < 1 ? 1 : (rows > 64 ? 64 : rows);
+    part = ((size_t)((g.h + rows - 1) / rows) * D * per + 255) & align;
+    if (part + tail <= limit) part = (limit - tail) & align;
+  }
   if (mean_offset) *mean_offset = part;
-  return part + (size_t)D * dtype_size(dtype) + 256;
+  return part + tail;
 }
 
 // ------------------------------------------------------------------------

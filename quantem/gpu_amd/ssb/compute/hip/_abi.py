@@ -84,6 +84,8 @@ SIGNATURES: dict[str, list] = {
                         _vp, _vp],
     "ssb_normalize_scan_typed": [_vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _vp],
     "ssb_bf_columns_u8": [_vp, _vp, _c_int, _c_int, _vp, _vp],
+    "ssb_normalize_workspace_bytes": [_c_int, _c_int, _c_int, _c_int, _c_int],
+    "ssb_normalize_scan_ws": [_vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _vp, _i64, _vp],
     "ssb_normalize_scan_u16_noalloc": [_vp, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _vp],
     "ssb_batch_phase_loss_graph": [_vp, _c_int, _dp, _dp, _dp, _vp, _vp],
     "ssb_trials_create": [_pp, _c_int, _c_int, _pp],
@@ -121,7 +123,8 @@ def lib() -> ctypes.CDLL:
     handle.ssb_last_error.restype = ctypes.c_char_p
     handle.ssb_stage_name.argtypes = [_c_int]
     handle.ssb_stage_name.restype = ctypes.c_char_p
-    for name in ("ssb_bslz4_workspace_bytes", "ssb_bslz4_encode_bound", "ssb_bslz4_encode_u16"):
+    for name in ("ssb_bslz4_workspace_bytes", "ssb_bslz4_encode_bound", "ssb_bslz4_encode_u16",
+                 "ssb_normalize_workspace_bytes"):
         if hasattr(handle, name):
             getattr(handle, name).restype = ctypes.c_longlong
     _lib = handle

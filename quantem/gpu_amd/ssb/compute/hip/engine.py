@@ -91,9 +91,16 @@ def normalize_scan(data):
         return data
     src = data.contiguous()
     out = torch.empty((T, T, kr, kc), dtype=data.dtype, device=data.device)
+    need = int(_abi.lib().ssb_normalize_workspace_bytes(code, H, W, kr, kc))
+    if need < 0:
+        _abi.check(need, "ssb_normalize_workspace_bytes")
+    # src, out and the workspace go back to the caching allocator, which
+    # reuses them only for later work on this same stream
+    ws = torch.empty(need, dtype=torch.uint8, device=data.device)
     with torch.cuda.device(data.device):
         stream = _abi.stream_handle(torch.cuda.current_stream(data.device))
-        _abi.call("ssb_normalize_scan_typed", _abi.ptr(src), code, H, W, kr, kc, _abi.ptr(out), T, stream)
+        _abi.call("ssb_normalize_scan_ws", _abi.ptr(src), code, H, W, kr, kc, _abi.ptr(out), T, _abi.ptr(ws), need,
+                  stream)
     return out
 
 
