@@ -57,6 +57,20 @@ int qnn_mse(const float* pred, const float* target, int n, float* grad, float* l
 int qnn_adam(float* p, const float* g, float* m, float* v, long long n, float lr, float b1, float b2, float eps,
              int step, uint16_t* ph, void* stream);
 
+/* The same step on up to QNN_ADAM_MAX tensors in one launch (items_host: host
+ * memory, read before the call returns; ph may be NULL per item). */
+#define QNN_ADAM_MAX 16
+typedef struct {
+  float* p;
+  const float* g;
+  float* m;
+  float* v;
+  uint16_t* ph;
+  long long n;
+} qnn_adam_item;
+int qnn_adam_multi(const qnn_adam_item* items_host, int count, float lr, float b1, float b2, float eps, int step,
+                   void* stream);
+
 /* Forward-model training features: S samples theta[s] = (C10 A, C30 A,
  * rotation rad), noise sigma snr[s], detector reciprocal sampling recip
  * (1/A per pixel), semiangle and angular sampling (rad), wavelength (A),

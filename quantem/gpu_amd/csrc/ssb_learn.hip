@@ -13,6 +13,7 @@
 // Also here: the synthetic training features (trotter values of the SSB
 // forward model G_b(Q) = Gamma_b(Q; theta) Phi(Q) + noise at fixed Q) and
 // the same features read from a resident Fourier stack.
+#include "../../../include/quantem_nn.h"
 #include "ssb_internal.h"
 #include "ssb_overlap.h"
 
@@ -104,44 +105,238 @@ k_gemm_bf16(const uint16_t* __restrict__ A, long long sam, long long sak, const 
       }
 }
 
-// C[m][n] = sum_z P[z][m][n] in order (split-K partial planes, contiguous M x N)
+// The same product where each operand is contiguous along m or along k (A)
+// and along n or along k (B) with 16-byte rows: 64 x TN tiles, four waves of
+// 16 x TN, K in steps of 64 through LDS (k contiguous, so an MFMA operand is
+// one 8-byte read; rows contiguous along m or n are transposed on the way in,
+// two k at a time), the next step's rows loaded while this one is multiplied.
+// Every output sums its products in the order of the general kernel, 16 at a
+// time from the slice's start: the same bits.  Bound by the wait on its
+// loads: the general kernel loads one 16-bit element a lane and waits twice
+// per 16 k.  M 65536, N 32, K 144: 25 -> 9.9 us; M 4096, N 64, K 576: 48 -> 11;
+// the weight gradient M 32, N 144, K 65536 in 64 slices: 109 -> 21 us.
+constexpr int kGemmK = 64;
+constexpr int kGemmLd = kGemmK + 8;   // 144-byte rows: 16-byte aligned, and 16 rows spread over the banks
+
+// ROWS rows (m or n) x 64 k of one operand into LDS.  KC: rows contiguous
+// along k (row r at src + r * ld), else contiguous along the row index
+// (k at src + k * ld).  Two steps, so that a step's loads can be in flight
+// while the previous one is used.
+template <int ROWS, bool KC>
+struct GemmTile {
+  static constexpr int VECS = KC ? ROWS * 8 / 256 : 2;   // 16-byte loads a thread
+  uint4 v[VECS < 1 ? 1 : VECS];
+
+  __device__ __forceinline__ void load(const uint16_t* __restrict__ src, long long ld, int row0, int rows, int k0,
+                                       int ke, int tid) {
+    if constexpr (KC) {
+#pragma unroll
+      for (int i = 0; i < VECS; ++i) {
+        const int c = tid + i * 256, r = row0 + (c >> 3), k = k0 + (c & 7) * 8;
+        v[i] = (r < rows && k < ke) ? *reinterpret_cast<const uint4*>(src + (long long)r * ld + k)
+                                    : make_uint4(0u, 0u, 0u, 0u);
+      }
+    } else {
+      const int k = k0 + (tid >> 3) * 2, r = row0 + (tid & 7) * 8;   // 8 lanes read 128 bytes of one k
+      const bool in = (tid & 7) * 8 < ROWS && r < rows;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        v[i] = (in && k + i < ke) ? *reinterpret_cast<const uint4*>(src + (long long)(k + i) * ld + r)
+                                  : make_uint4(0u, 0u, 0u, 0u);
+    }
+  }
+
+  __device__ __forceinline__ void store(uint16_t (*sh)[kGemmLd], int tid) const {
+    if constexpr (KC) {
+#pragma unroll
+      for (int i = 0; i < VECS; ++i) {
+        const int c = tid + i * 256;
+        *reinterpret_cast<uint4*>(&sh[c >> 3][(c & 7) * 8]) = v[i];
+      }
+    } else {
+      const int kk = (tid >> 3) * 2, rr = (tid & 7) * 8;
+      if (rr < ROWS) {
+        const unsigned a[4] = {v[0].x, v[0].y, v[0].z, v[0].w}, b[4] = {v[1].x, v[1].y, v[1].z, v[1].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          *reinterpret_cast<unsigned*>(&sh[rr + 2 * i][kk]) = (a[i] & 0xFFFFu) | (b[i] << 16);
+          *reinterpret_cast<unsigned*>(&sh[rr + 2 * i + 1][kk]) = (a[i] >> 16) | (b[i] & 0xFFFF0000u);
+        }
+      }
+    }
+  }
+};
+
+template <int TN, bool AK, bool BK, bool RELU>
 __global__ void __launch_bounds__(256)
+k_gemm_bf16_tile(const uint16_t* __restrict__ A, long long lda, const uint16_t* __restrict__ B, long long ldb,
+                 float* __restrict__ C, long long scm, long long scn, const float* __restrict__ bias, int M, int N,
+                 int K, int accumulate, int kslice, long long pstride) {
+  __shared__ __attribute__((aligned(16))) uint16_t As[64][kGemmLd];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[TN][kGemmLd];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * TN;
+  constexpr int NT = TN / 16;
+  float4v acc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) acc[j] = float4v{0.f, 0.f, 0.f, 0.f};
+  const int kb = blockIdx.z * kslice;
+  const int ke = min(K, kb + kslice);
+  C += (long long)blockIdx.z * pstride;
+  GemmTile<64, AK> ta;
+  GemmTile<TN, BK> tb;
+  ta.load(A, lda, m0, M, kb, ke, tid);
+  tb.load(B, ldb, n0, N, kb, ke, tid);
+  for (int k0 = kb; k0 < ke; k0 += kGemmK) {
+    __syncthreads();                        // the previous step's readers are done
+    ta.store(As, tid);
+    tb.store(Bs, tid);
+    __syncthreads();
+    if (k0 + kGemmK < ke) {
+      ta.load(A, lda, m0, M, k0 + kGemmK, ke, tid);
+      tb.load(B, ldb, n0, N, k0 + kGemmK, ke, tid);
+    }
+    const int ar = w * 16 + (lane & 15), kq = (lane >> 4) * 4;
+#pragma unroll
+    for (int ks = 0; ks < kGemmK; ks += 16) {
+      const short4v a = *reinterpret_cast<const short4v*>(&As[ar][ks + kq]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const short4v b = *reinterpret_cast<const short4v*>(&Bs[j * 16 + (lane & 15)][ks + kq]);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gm = m0 + w * 16 + (lane >> 4) * 4 + r;
+      const int gn = n0 + j * 16 + (lane & 15);
+      if (gm < M && gn < N) {
+        float v = acc[j][r];
+        if (bias) v += bias[gn];
+        if (RELU) v = fmaxf(v, 0.0f);
+        float* c = C + (long long)gm * scm + (long long)gn * scn;
+        *c = accumulate ? *c + v : v;
+      }
+    }
+}
+
+// Which kernel a product takes: the tiled one where both operands have
+// 16-byte rows that end on 16 bytes (every layer of the network except the
+// three-output one), the general one for any other strides.
+static bool gemm_rows16(const uint16_t* p, long long ld, long long len) {
+  return ld % 8 == 0 && len % 8 == 0 && (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
+}
+
+static void launch_gemm(const uint16_t* A, long long sam, long long sak, const uint16_t* B, long long sbk,
+                        long long sbn, float* C, long long scm, long long scn, const float* bias, int M, int N, int K,
+                        bool relu, int accumulate, int kslice, int z, long long pstride, hipStream_t s) {
+  const bool ak = sak == 1, bk = sbk == 1;
+  const long long lda = ak ? sam : sak, ldb = bk ? sbn : sbk;
+  const bool fast = (ak || sam == 1) && (bk || sbn == 1) && lda > 0 && ldb > 0 && kslice % 8 == 0 &&
+                    gemm_rows16(A, lda, ak ? K : M) && gemm_rows16(B, ldb, bk ? K : N);
+  if (!fast) {
+    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)z);
+    if (relu)
+      hipLaunchKernelGGL(k_gemm_bf16<true>, grid, dim3(256), 0, s, A, sam, sak, B, sbk, sbn, C, scm, scn, bias, M, N,
+                         K, accumulate, kslice, pstride);
+    else
+      hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, s, A, sam, sak, B, sbk, sbn, C, scm, scn, bias, M, N,
+                         K, accumulate, kslice, pstride);
+    return;
+  }
+#define QNN_GEMM_ONE(TN, AK, BK)                                                                              \
+  do {                                                                                                        \
+    const dim3 grid((unsigned)((N + TN - 1) / TN), (unsigned)((M + 63) / 64), (unsigned)z);                   \
+    if (relu)                                                                                                 \
+      hipLaunchKernelGGL((k_gemm_bf16_tile<TN, AK, BK, true>), grid, dim3(256), 0, s, A, lda, B, ldb, C, scm, \
+                         scn, bias, M, N, K, accumulate, kslice, pstride);                                    \
+    else                                                                                                      \
+      hipLaunchKernelGGL((k_gemm_bf16_tile<TN, AK, BK, false>), grid, dim3(256), 0, s, A, lda, B, ldb, C, scm, \
+                         scn, bias, M, N, K, accumulate, kslice, pstride);                                    \
+  } while (0)
+#define QNN_GEMM(TN)                                   \
+  do {                                                 \
+    if (ak && bk) QNN_GEMM_ONE(TN, true, true);        \
+    else if (ak) QNN_GEMM_ONE(TN, true, false);        \
+    else if (bk) QNN_GEMM_ONE(TN, false, true);        \
+    else QNN_GEMM_ONE(TN, false, false);               \
+  } while (0)
+  if (N <= 32) QNN_GEMM(32);
+  else QNN_GEMM(64);
+#undef QNN_GEMM
+#undef QNN_GEMM_ONE
+}
+
+// C[m][n] = sum_z P[z][m][n] in order (split-K partial planes, contiguous
+// M x N), 16 planes' loads in flight.
+__global__ void __launch_bounds__(64)
 k_sum_partials(const float* __restrict__ P, int splits, long long n, float* __restrict__ C) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
+  constexpr int U = 16;
+  for (long long i = (long long)blockIdx.x * 64 + threadIdx.x; i < n; i += (long long)gridDim.x * 64) {
     float s = 0.0f;
-    for (int z = 0; z < splits; ++z) s += P[(long long)z * n + i];
+    int z = 0;
+    for (; z + U <= splits; z += U) {
+      float v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = P[(long long)(z + u) * n + i];
+#pragma unroll
+      for (int u = 0; u < U; ++u) s += v[u];
+    }
+    for (; z < splits; ++z) s += P[(long long)z * n + i];
     C[i] = s;
   }
 }
 
 // NHWC fp32 -> im2col bf16 for a 3x3, stride 2, pad 1 convolution:
 // cols[(b, oy, ox)][(ky, kx, c)] = X[b][2 oy + ky - 1][2 ox + kx - 1][c] (0 outside).
+// A thread owns V channels of one tap (V = 8: one 16-byte store).
+template <int V>
 __global__ void __launch_bounds__(256)
 k_im2col_bf16(const float* __restrict__ X, int B, int H, int W, int Cin, int Ho, int Wo, uint16_t* __restrict__ cols) {
-  const long long K = 9LL * Cin;
-  const long long total = (long long)B * Ho * Wo * K;
+  const int groups = Cin / V;
+  const int taps = 9 * groups;
+  const long long total = (long long)B * Ho * Wo * taps;
   for (long long idx = (long long)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (long long)gridDim.x * 256) {
-    const long long m = idx / K;
-    const int k = (int)(idx - m * K);
-    const int c = k % Cin, kxy = k / Cin, kx = kxy % 3, ky = kxy / 3;
+    const long long m = total <= 0x7fffffffLL ? (long long)((unsigned)idx / (unsigned)taps) : idx / taps;
+    const int k = (int)(idx - m * taps);
+    const int kxy = k / groups, c = (k - kxy * groups) * V, ky = kxy / 3, kx = kxy - 3 * ky;
     const int ox = (int)(m % Wo), oy = (int)((m / Wo) % Ho), b = (int)(m / ((long long)Wo * Ho));
     const int y = 2 * oy + ky - 1, x = 2 * ox + kx - 1;
-    float v = 0.0f;
-    if (y >= 0 && y < H && x >= 0 && x < W) v = X[(((long long)b * H + y) * W + x) * Cin + c];
-    cols[idx] = f32_to_bf16(v);
+    const bool in = y >= 0 && y < H && x >= 0 && x < W;
+    const float* src = X + (((long long)b * H + y) * W + x) * Cin + c;
+    uint16_t* dst = cols + m * 9 * Cin + (long long)kxy * Cin + c;
+    if constexpr (V == 8) {
+      float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
+      if (in) {
+        u = reinterpret_cast<const float4*>(src)[0];
+        v = reinterpret_cast<const float4*>(src)[1];
+      }
+      auto two = [](float lo, float hi) { return (unsigned)f32_to_bf16(lo) | ((unsigned)f32_to_bf16(hi) << 16); };
+      *reinterpret_cast<uint4*>(dst) = make_uint4(two(u.x, u.y), two(u.z, u.w), two(v.x, v.y), two(v.z, v.w));
+    } else {
+      dst[0] = f32_to_bf16(in ? src[0] : 0.0f);
+    }
   }
 }
 
 // dX[b][y][x][c] = sum over the output positions whose 3x3 window covers
-// (y, x) of dcols[(b, oy, ox)][(ky, kx, c)], in (ky, kx) order.
+// (y, x) of dcols[(b, oy, ox)][(ky, kx, c)], in (ky, kx) order; V channels a
+// thread (V = 4: 16-byte loads and stores).
+template <int V>
 __global__ void __launch_bounds__(256)
 k_col2im(const float* __restrict__ dcols, int B, int H, int W, int Cin, int Ho, int Wo, float* __restrict__ dX) {
-  const long long total = (long long)B * H * W * Cin;
+  typedef float Vec __attribute__((ext_vector_type(V)));
+  const int groups = Cin / V;
+  const long long total = (long long)B * H * W * groups;
   for (long long idx = (long long)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (long long)gridDim.x * 256) {
-    const int c = (int)(idx % Cin);
-    const int x = (int)((idx / Cin) % W), y = (int)((idx / ((long long)Cin * W)) % H);
-    const int b = (int)(idx / ((long long)Cin * W * H));
-    float s = 0.0f;
+    const long long p = total <= 0x7fffffffLL ? (long long)((unsigned)idx / (unsigned)groups) : idx / groups;
+    const int c = (int)(idx - p * groups) * V;
+    const int x = (int)(p % W), y = (int)((p / W) % H);
+    const int b = (int)(p / ((long long)W * H));
+    Vec s = 0.0f;
     for (int ky = 0; ky < 3; ++ky) {
       const int ty = y + 1 - ky;
       if (ty < 0 || (ty & 1) || (ty >> 1) >= Ho) continue;
@@ -149,10 +344,10 @@ k_col2im(const float* __restrict__ dcols, int B, int H, int W, int Cin, int Ho, 
         const int tx = x + 1 - kx;
         if (tx < 0 || (tx & 1) || (tx >> 1) >= Wo) continue;
         const long long m = ((long long)b * Ho + (ty >> 1)) * Wo + (tx >> 1);
-        s += dcols[m * 9 * Cin + (ky * 3 + kx) * Cin + c];
+        s += *reinterpret_cast<const Vec*>(dcols + m * 9 * Cin + (ky * 3 + kx) * Cin + c);
       }
     }
-    dX[idx] = s;
+    *reinterpret_cast<Vec*>(dX + p * Cin + c) = s;
   }
 }
 
@@ -177,50 +372,56 @@ k_relu_bwd(const float* __restrict__ Y, const float* __restrict__ dY, long long 
 // Pass 1: one workgroup per (64-column tile, chunk of kColsumRows rows),
 // 4 row lanes per column, each a compensated sum, combined in lane order;
 // pass 2: the chunks' partial sums per column, compensated, in chunk order.
+// Bound by the wait on its loads and then by the chain of compensated adds
+// (512 of them, ~20 cycles each): with one load at a time M 65536, N 32 took
+// 132 us, with 64 in flight 12 us.
 constexpr int kColsumRows = 2048;
+
+// s, c continued over x[0], x[step], ... (n of them), U loads in flight
+template <int U>
+__device__ __forceinline__ void compensated_run(const float* __restrict__ x, long long step, int n, float& s,
+                                                float& c) {
+  auto add = [&](float v) {
+    const float y = v - c;
+    const float t = s + y;
+    c = (t - s) - y;
+    s = t;
+  };
+  int i = 0;
+  for (; i + U <= n; i += U) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = x[(i + u) * step];
+#pragma unroll
+    for (int u = 0; u < U; ++u) add(v[u]);
+  }
+  for (; i < n; ++i) add(x[i * step]);
+}
 
 __global__ void __launch_bounds__(256)
 k_colsum_part(const float* __restrict__ dZ, int M, int N, float* __restrict__ part) {
   __shared__ float sh[4][64];
   const int lc = threadIdx.x & 63, lr = threadIdx.x >> 6;
   const int n = blockIdx.x * 64 + lc;
-  const int m0 = blockIdx.y * kColsumRows;
-  const int m1 = min(M, m0 + kColsumRows);
+  const int m0 = blockIdx.y * kColsumRows + lr;
+  const int m1 = min(M, (int)(blockIdx.y + 1) * kColsumRows);
   float s = 0.0f, c = 0.0f;
-  if (n < N) {
-    for (int m = m0 + lr; m < m1; m += 4) {
-      const float y = dZ[(long long)m * N + n] - c;
-      const float t = s + y;
-      c = (t - s) - y;
-      s = t;
-    }
-  }
+  if (n < N && m0 < m1) compensated_run<64>(dZ + (long long)m0 * N + n, 4LL * N, (m1 - m0 + 3) / 4, s, c);
   sh[lr][lc] = s - c;
   __syncthreads();
   if (lr == 0 && n < N) {
-    float s2 = 0.0f, c2 = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float y = sh[r][lc] - c2;
-      const float t = s2 + y;
-      c2 = (t - s2) - y;
-      s2 = t;
-    }
-    part[(long long)blockIdx.y * N + n] = s2 - c2;
+    s = c = 0.0f;
+    compensated_run<4>(&sh[0][lc], 64, 4, s, c);
+    part[(long long)blockIdx.y * N + n] = s - c;
   }
 }
 
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(64)
 k_colsum_finish(const float* __restrict__ part, int chunks, int N, float* __restrict__ out) {
-  const int n = blockIdx.x * 256 + threadIdx.x;
+  const int n = blockIdx.x * 64 + threadIdx.x;
   if (n >= N) return;
   float s = 0.0f, c = 0.0f;
-  for (int k = 0; k < chunks; ++k) {
-    const float y = part[(long long)k * N + n] - c;
-    const float t = s + y;
-    c = (t - s) - y;
-    s = t;
-  }
+  compensated_run<16>(part + n, N, chunks, s, c);
   out[n] = s - c;
 }
 
@@ -244,10 +445,22 @@ k_mse(const float* __restrict__ pred, const float* __restrict__ target, int n, f
   if (threadIdx.x == 0) loss[0] = sm[0] / (float)n;
 }
 
-// Adam on fp32 master weights; refreshes the bf16 copy
+// Adam on fp32 master weights; refreshes the bf16 copy.  One launch over
+// every tensor of a step (row y of the grid: tensor y); a launch each cost
+// more than the arithmetic.
+struct AdamItems {
+  qnn_adam_item t[QNN_ADAM_MAX];
+};
+
 __global__ void __launch_bounds__(256)
-k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v, long long n,
-       float lr, float b1, float b2, float eps, float bc1, float bc2, uint16_t* __restrict__ ph) {
+k_adam(AdamItems items, float lr, float b1, float b2, float eps, float bc1, float bc2) {
+  const qnn_adam_item it = items.t[blockIdx.y];
+  float* __restrict__ p = it.p;
+  const float* __restrict__ g = it.g;
+  float* __restrict__ m = it.m;
+  float* __restrict__ v = it.v;
+  uint16_t* __restrict__ ph = it.ph;
+  const long long n = it.n;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
     const float gi = g[i];
     const float mi = b1 * m[i] + (1.0f - b1) * gi;
@@ -454,14 +667,8 @@ int qnn_gemm_bf16(const uint16_t* A, long long sam, long long sak, const uint16_
                   float* C, long long scm, long long scn, const float* bias, int M, int N, int K, int relu,
                   int accumulate, void* stream) {
   if (!A || !B || !C || M < 1 || N < 1 || K < 1) return -1;
-  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (relu)
-    hipLaunchKernelGGL(k_gemm_bf16<true>, grid, dim3(256), 0, s, A, sam, sak, B, sbk, sbn, C, scm, scn, bias, M, N,
-                       K, accumulate, K, 0LL);
-  else
-    hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, s, A, sam, sak, B, sbk, sbn, C, scm, scn, bias, M, N,
-                       K, accumulate, K, 0LL);
+  launch_gemm(A, sam, sak, B, sbk, sbn, C, scm, scn, bias, M, N, K, relu != 0, accumulate, (K + 15) / 16 * 16, 1, 0LL,
+              reinterpret_cast<hipStream_t>(stream));
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -470,27 +677,35 @@ int qnn_gemm_bf16_splitk(const uint16_t* A, long long sam, long long sak, const 
   if (!A || !B || !C || !workspace || M < 1 || N < 1 || K < 1 || splits < 1) return -1;
   const int kslice = ((K + splits - 1) / splits + 15) / 16 * 16;
   const int z = (K + kslice - 1) / kslice;
-  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)z);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const long long plane = (long long)M * N;
-  hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, s, A, sam, sak, B, sbk, sbn, workspace, (long long)N,
-                     1LL, nullptr, M, N, K, 0, kslice, plane);
-  hipLaunchKernelGGL(k_sum_partials, dim3(grid_of(plane)), dim3(256), 0, s, workspace, z, plane, C);
+  launch_gemm(A, sam, sak, B, sbk, sbn, workspace, (long long)N, 1LL, nullptr, M, N, K, false, 0, kslice, z, plane, s);
+  const long long blocks = (plane + 63) / 64;
+  hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)(blocks < 65535 ? blocks : 65535)), dim3(64), 0, s, workspace, z,
+                     plane, C);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 int qnn_im2col(const float* X, int B, int H, int W, int Cin, uint16_t* cols, void* stream) {
   if (!X || !cols || B < 1 || H < 2 || W < 2 || Cin < 1) return -1;
   const int Ho = H / 2, Wo = W / 2;
-  hipLaunchKernelGGL(k_im2col_bf16, dim3(grid_of((long long)B * Ho * Wo * 9 * Cin)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), X, B, H, W, Cin, Ho, Wo, cols);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const long long total = (long long)B * Ho * Wo * 9 * Cin;
+  if (Cin % 8 == 0 && ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(cols)) & 15u) == 0)
+    hipLaunchKernelGGL(k_im2col_bf16<8>, dim3(grid_of(total / 8)), dim3(256), 0, s, X, B, H, W, Cin, Ho, Wo, cols);
+  else
+    hipLaunchKernelGGL(k_im2col_bf16<1>, dim3(grid_of(total)), dim3(256), 0, s, X, B, H, W, Cin, Ho, Wo, cols);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 int qnn_col2im(const float* dcols, int B, int H, int W, int Cin, float* dX, void* stream) {
   if (!dcols || !dX || B < 1 || H < 2 || W < 2 || Cin < 1) return -1;
-  hipLaunchKernelGGL(k_col2im, dim3(grid_of((long long)B * H * W * Cin)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), dcols, B, H, W, Cin, H / 2, W / 2, dX);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const long long total = (long long)B * H * W * Cin;
+  if (Cin % 4 == 0 && ((reinterpret_cast<uintptr_t>(dcols) | reinterpret_cast<uintptr_t>(dX)) & 15u) == 0)
+    hipLaunchKernelGGL(k_col2im<4>, dim3(grid_of(total / 4)), dim3(256), 0, s, dcols, B, H, W, Cin, H / 2, W / 2, dX);
+  else
+    hipLaunchKernelGGL(k_col2im<1>, dim3(grid_of(total)), dim3(256), 0, s, dcols, B, H, W, Cin, H / 2, W / 2, dX);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -519,7 +734,7 @@ int qnn_colsum(const float* dZ, int M, int N, float* out, float* work, long long
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(k_colsum_part, dim3((unsigned)((N + 63) / 64), (unsigned)chunks), dim3(256), 0, s, dZ, M, N,
                      work);
-  hipLaunchKernelGGL(k_colsum_finish, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, work, chunks, N, out);
+  hipLaunchKernelGGL(k_colsum_finish, dim3((unsigned)((N + 63) / 64)), dim3(64), 0, s, work, chunks, N, out);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -529,13 +744,26 @@ int qnn_mse(const float* pred, const float* target, int n, float* grad, float* l
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
+int qnn_adam_multi(const qnn_adam_item* items_host, int count, float lr, float b1, float b2, float eps, int step,
+                   void* stream) {
+  if (!items_host || count < 1 || count > QNN_ADAM_MAX || step < 1) return -1;
+  AdamItems a{};
+  long long most = 0;
+  for (int i = 0; i < count; ++i) {
+    a.t[i] = items_host[i];
+    if (!a.t[i].p || !a.t[i].g || !a.t[i].m || !a.t[i].v || a.t[i].n < 1) return -1;
+    if (a.t[i].n > most) most = a.t[i].n;
+  }
+  const float bc1 = 1.0f - powf(b1, (float)step), bc2 = 1.0f - powf(b2, (float)step);
+  hipLaunchKernelGGL(k_adam, dim3(grid_of(most), (unsigned)count), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                     a, lr, b1, b2, eps, bc1, bc2);
+  return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
 int qnn_adam(float* p, const float* g, float* m, float* v, long long n, float lr, float b1, float b2, float eps,
              int step, uint16_t* ph, void* stream) {
-  if (!p || !g || !m || !v || n < 1 || step < 1) return -1;
-  const float bc1 = 1.0f - powf(b1, (float)step), bc2 = 1.0f - powf(b2, (float)step);
-  hipLaunchKernelGGL(k_adam, dim3(grid_of(n)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p, g, m, v, n, lr,
-                     b1, b2, eps, bc1, bc2, ph);
-  return hipGetLastError() == hipSuccess ? 0 : -4;
+  const qnn_adam_item it{p, g, m, v, ph, n};
+  return qnn_adam_multi(&it, 1, lr, b1, b2, eps, step, stream);
 }
 
 // theta: [S][3] (C10 A, C30 A, rotation rad); snr: [S] noise sigma (relative to |Phi| ~ 1);

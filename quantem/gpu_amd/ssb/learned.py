@@ -31,8 +31,20 @@ NQ = 8
 SCALE = np.array([500.0, 2.0e5, math.radians(5.0)])
 
 
+class _AdamItem(ctypes.Structure):
+    _fields_ = [("p", ctypes.c_void_p), ("g", ctypes.c_void_p), ("m", ctypes.c_void_p), ("v", ctypes.c_void_p),
+                ("ph", ctypes.c_void_p), ("n", ctypes.c_longlong)]
+
+
+_bound = None
+
+
 def _lib():
+    """The native library with the network's argument types (bound once)."""
+    global _bound
     lib = _abi.lib()
+    if lib is _bound:
+        return lib
     vp, i64, ci, cf = ctypes.c_void_p, ctypes.c_longlong, ctypes.c_int, ctypes.c_float
     sig = {
         "qnn_gemm_bf16": [vp, i64, i64, vp, i64, i64, vp, i64, i64, vp, ci, ci, ci, ci, ci, vp],
@@ -45,6 +57,7 @@ def _lib():
         "qnn_colsum": [vp, ci, ci, vp, vp, ctypes.c_longlong, vp],
         "qnn_mse": [vp, vp, ci, vp, vp, vp],
         "qnn_adam": [vp, vp, vp, vp, i64, cf, cf, cf, cf, ci, vp, vp],
+        "qnn_adam_multi": [vp, ci, cf, cf, cf, cf, ci, vp],
         "qnn_features_synth": [vp, vp, ci, cf, cf, cf, cf, vp, ctypes.c_uint, vp, vp],
     }
     for name, argtypes in sig.items():
@@ -52,6 +65,7 @@ def _lib():
         fn.argtypes = argtypes
         fn.restype = ci
     lib.qnn_colsum_workspace.restype = i64
+    _bound = lib
     return lib
 
 
@@ -247,11 +261,11 @@ class LearnedInit:
 
     def apply(self, grads, lr: float, b1=0.9, b2=0.999, eps=1e-8) -> None:
         self.step += 1
-        for i, ((w, b), (dw, db), (mw, vw, mb, vb)) in enumerate(zip(self.params, grads, self.adam)):
-            _call("qnn_adam", _p(w), _p(dw), _p(mw), _p(vw), int(w.numel()), lr, b1, b2, eps, self.step,
-                  _p(self.half[i]), self._s())
-            _call("qnn_adam", _p(b), _p(db), _p(mb), _p(vb), int(b.numel()), lr, b1, b2, eps, self.step, None,
-                  self._s())
+        items = []
+        for (w, b), (dw, db), (mw, vw, mb, vb), h in zip(self.params, grads, self.adam, self.half):
+            items.append((w.data_ptr(), dw.data_ptr(), mw.data_ptr(), vw.data_ptr(), h.data_ptr(), w.numel()))
+            items.append((b.data_ptr(), db.data_ptr(), mb.data_ptr(), vb.data_ptr(), None, b.numel()))
+        _call("qnn_adam_multi", (_AdamItem * len(items))(*items), len(items), lr, b1, b2, eps, self.step, self._s())
 
     # ---------------------------------------------------------------- data
     def synth_batch(self, cfg: FeatureConfig, rng: np.random.Generator, n: int, ranges=None, seed: int = 0):
