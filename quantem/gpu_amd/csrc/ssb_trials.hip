@@ -16,7 +16,7 @@
 //
 // Pipeline (all parameters read from device memory, so the sequence is
 // captured once in a hipGraph and replayed for every new batch of trials):
-//   k_trial_geometry   per (trial, BF pixel): rotated k, A(k), chi(k), Rout^2-|k|^2
+//   k_trial_geometry   per (trial, BF pixel): rotated k, A(k), Rout^2-|k|^2, chi's terms in k
 //   k_trotter_trials   work queue over (dataset, block of TB trials, 256 points
 //                      of the Hermitian half plane); each workgroup reads the
 //                      stack G_b(Q) once per BF pixel for its TB trials
@@ -38,23 +38,47 @@ namespace qssb {
 // Aberration phase and rotation of one trial, prepared on the host in double
 // precision and rounded once to float32 (double-float for the rotation).
 struct TrialChi {
-  ChiPoly cp;       // even-m terms only (odd-m trials are rejected)
-  int radial;       // only m = 0 terms: chi = r2 (K0 + r2 (K4 + r2 K10))
-  int pad;
-  df cos_a, sin_a;  // cos and sin of -rotation
+  ChiPoly cp;         // even-m terms only (odd-m trials are rejected)
+  int kind;           // kChiRadial ..., by the terms that are not zero
+  float k0, k4;       // C10 and C30 terms in half turns: chi / pi = k0 r2 + k4 r2^2 + ...
+  float m12c, m12s;   // C12 in half turns: + m12c (ux^2 - uy^2) + m12s 2 ux uy
+  int radial;         // only m = 0 terms: chi = r2 (K0 + r2 (K4 + r2 K10))
+  int pad[2];
+  df cos_a, sin_a;    // cos and sin of -rotation
 };
 
-// One (trial, BF pixel): rotated detector k as double-float, A(k), chi(k),
-// and Rout^2 - |k|^2 as double-float.
-struct TrialBf {
-  float kx, kxl, ky, kyl;
-  float ak, chik, cb, cbl;
+enum : int {
+  kChiRadial = 0,    // C10 and C30
+  kChiAstig = 1,     // and C12
+  kChiGeneral = 2,   // any even term: chi evaluated at Q - k and Q + k
+};
+
+constexpr int kTrialBlock = 8;      // trials per workgroup of k_trotter_trials
+
+// One BF pixel of a block of trials, read by whole waves as scalars: what
+// every point needs.  A pixel with A(k) = 0 contributes nothing (cb far below
+// every edge), one with a small A(k) sends all its points through the general
+// form (an unbounded margin).
+struct __attribute__((aligned(32))) TrialBf {
+  float kx2[kTrialBlock], ky2[kTrialBlock];   // 2 k
+  float cb[kTrialBlock];                      // Rout^2 - |k|^2
+  float u[kTrialBlock];                       // d(chi / pi) / d(r2) at |k|^2: k0 + 2 k4 |k|^2
+  float margin[kTrialBlock];                  // kApMargin, or infinity
+};
+
+// What points at an aperture's edge and the other trials need besides.
+struct __attribute__((aligned(32))) TrialBfMore {
+  float ak, chik;      // A(k), chi(k) in radians
+  float cb, cbl;       // Rout^2 - |k|^2 as double-float
+  float kxl, kyl;      // low words of k
+  float vx, vy;        // 2 M k of the C12 matrix, half turns
 };
 
 // One dataset of the work queue.
 struct TrialSet {
   const float2* Gt;      // resident Hermitian stack [nbf][N/2+1][N]
-  const TrialBf* tbf;    // [T][nbf]
+  const TrialBf* tbf;          // [trial block][nbf]
+  const TrialBfMore* more;     // [trial block][nbf][kTrialBlock]
   float2* S;             // corrected Fourier sums [T][trial_points(N)]
   const float* qx;
   const float* qxl;
@@ -65,7 +89,6 @@ struct TrialSet {
   long long item0;       // first queue item of this dataset
 };
 
-constexpr int kTrialBlock = 8;      // trials per workgroup of k_trotter_trials
 // Corrected sums stored per trial: the Hermitian half plane (columns 0..N/2)
 // and the Nyquist row's columns N/2+1..N-1.
 __host__ __device__ constexpr int trial_points(int N) { return (N / 2 + 1) * N + (N / 2 - 1); }
@@ -79,10 +102,19 @@ __device__ __forceinline__ float chi_even(const TrialChi& tc, float ux, float uy
   return e;
 }
 
+// Below this A(k) the overlap's guard |Gamma|^2 > 1e-16 can act away from an
+// exact zero of the sine: such BF pixels take the general form.
+constexpr float kSmallAk = 1e-3f;
+
+// Within this of an aperture's outer edge, d = Rout^2 - |u|^2 as a float32
+// estimate (absolute error far below it) does not decide whether the aperture
+// is zero: d is formed in double-float there.
+constexpr float kApMargin = 1e-4f;
+
 __global__ void __launch_bounds__(256)
 k_trial_geometry(const int* __restrict__ bf_rows, const int* __restrict__ bf_cols, const BfInfo* __restrict__ info,
-                 int nbf, int T, df recip_y, df recip_x, Optics o, df rout2, const TrialChi* __restrict__ chis,
-                 TrialBf* __restrict__ out) {
+                 int nbf, int T, df recip_y, df recip_x, Optics o, df rout2,
+                 const TrialChi* __restrict__ chis, TrialBf* __restrict__ out, TrialBfMore* __restrict__ more) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (long long)T * nbf) return;
   const int t = (int)(idx / nbf), b = (int)(idx - (long long)t * nbf);
@@ -94,26 +126,136 @@ k_trial_geometry(const int* __restrict__ bf_rows, const int* __restrict__ bf_col
   const df kx = df_add(df_mul(kxa, tc.cos_a), df_mul(kya, tc.sin_a));
   const df ky = df_sub(df_mul(kya, tc.cos_a), df_mul(kxa, tc.sin_a));
   const df cb = df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky)));
-  TrialBf r;
-  r.kx = kx.hi;
-  r.kxl = kx.lo;
-  r.ky = ky.hi;
-  r.kyl = ky.lo;
-  r.ak = aperture_band(kx, ky, o);
-  r.chik = chi_even(tc, kx.hi, ky.hi);
-  r.cb = cb.hi;
-  r.cbl = cb.lo;
-  out[idx] = r;
+  const float k2 = kx.hi * kx.hi + ky.hi * ky.hi;
+  const float ak = aperture_band(kx, ky, o);
+  const int i = t % kTrialBlock;
+  const long long slot = (long long)(t / kTrialBlock) * nbf + b;
+  TrialBf& r = out[slot];
+  r.kx2[i] = 2.0f * kx.hi;
+  r.ky2[i] = 2.0f * ky.hi;
+  r.cb[i] = ak == 0.0f ? -1e30f : cb.hi;
+  r.u[i] = fmaf(2.0f * tc.k4, k2, tc.k0);
+  r.margin[i] = ak < kSmallAk && ak > 0.0f ? INFINITY : kApMargin;
+  TrialBfMore m;
+  m.ak = ak;
+  m.chik = chi_even(tc, kx.hi, ky.hi);
+  m.cb = cb.hi;
+  m.cbl = cb.lo;
+  m.kxl = kx.lo;
+  m.kyl = ky.lo;
+  m.vx = 2.0f * (tc.m12c * kx.hi + tc.m12s * ky.hi);
+  m.vy = 2.0f * (tc.m12s * kx.hi - tc.m12c * ky.hi);
+  more[slot * kTrialBlock + i] = m;
 }
 
-// Aperture from d = Rout^2 - |u|^2 given as a float32 estimate `dapprox`
-// (absolute error far below kApMargin): exactly 1 or 0 outside the soft band
-// plus the margin, otherwise -1 (evaluate d in double-float).
-constexpr float kApMargin = 1e-4f;
-__device__ __forceinline__ float aperture_quick(float dapprox, const ApIso& a) {
-  if (dapprox >= a.d_in + kApMargin) return 1.0f;
-  if (dapprox <= a.d_out - kApMargin) return 0.0f;
-  return -1.0f;
+// Data that only kernels before this one write, read through the constant
+// address space: scalar loads.
+template <typename T>
+using Const = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ Const<T> as_const(const T* p) {
+  return (Const<T>)(unsigned long long)p;
+}
+
+// The sums over the BF pixels of one point for the `nt` trials of a block.
+// RADIAL: none of them has a term beyond C10 and C30; otherwise each trial's
+// kind is looked up (the same arithmetic for its terms, so a trial's sums do
+// not depend on the block it is in).
+template <int TB, bool RADIAL>
+__device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* __restrict__ tch, Const<TrialBf> kb,
+                                           Const<TrialBfMore> km, Const<TrialChi> ch, int nt, int q, int c, bool live,
+                                           bool nyq, const float2* __restrict__ gsrc, long long gstep,
+                                           Kahan (&ar)[TB], Kahan (&ai)[TB]) {
+  const int nbf = ds.nbf;
+  const float d_in = ds.ap.d_in;
+  const float qxf = ds.qx[q], qyf = ds.qy[c];
+  float q2f, qa = 0.0f, qb = 0.0f;
+  {
+    const df qx{qxf, ds.qxl[q]}, qy{qyf, ds.qyl[c]};
+    const df q2 = df_add(df_mul(qx, qx), df_mul(qy, qy));
+    q2f = live ? q2.hi + q2.lo : 1e30f;   // idle lanes: outside every aperture
+  }
+  if (!RADIAL) {
+    qa = qxf * qxf - qyf * qyf;
+    qb = 2.0f * qxf * qyf;
+  }
+  float k4[TB];
+#pragma unroll
+  for (int i = 0; i < TB; ++i) k4[i] = ch[i < nt ? i : 0].k4;
+  float2 nextG = gsrc[0];
+  for (int b = 0; b < nbf; ++b, ++kb, km += TB) {
+    // the pixel's scalars in whole loads, before the first use
+    float kx2[TB], ky2[TB], cb[TB], u[TB], edge[TB];
+#pragma unroll
+    for (int i = 0; i < TB; ++i) {
+      kx2[i] = kb->kx2[i];
+      ky2[i] = kb->ky2[i];
+      cb[i] = kb->cb[i];
+      u[i] = kb->u[i];
+      edge[i] = kb->margin[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float2 G = nextG;
+    if (b + 1 < nbf) nextG = gsrc[(long long)(b + 1) * gstep];
+    if (nyq) G.y = -G.y;
+#pragma unroll
+    for (int i = 0; i < TB; ++i) {
+      if (i < nt) {
+        const float B = fmaf(qxf, kx2[i], qyf * ky2[i]);
+        const float base = cb[i] - q2f;
+        // d of Q -/+ k, the larger first: the apertures are zero from 0 down, one from d_in up
+        const float near = base + fabsf(B), far = base - fabsf(B);
+        const float margin = edge[i];
+        if (near > -margin) {
+          const int kind = RADIAL ? kChiRadial : ch[i].kind;
+          const float w = fmaf(k4[i], q2f, u[i]);
+          float t = fabsf(B) * fmaf(k4[i], q2f, w);
+          float s = fmaf(q2f, w, k4[i] * (B * B));
+          if (!RADIAL && kind != kChiRadial) {
+            float ts;                            // t on the side of k itself
+            if (kind == kChiAstig) {
+              ts = fmaf(qxf, km[i].vx, qyf * km[i].vy);
+              ts = B < 0.0f ? ts - t : ts + t;
+              s = fmaf(qa, ch[i].m12c, fmaf(qb, ch[i].m12s, s));
+            } else {
+              const float kxh = 0.5f * kx2[i], kyh = 0.5f * ky2[i], chik = km[i].chik;
+              const float cm = chi_even(tch[i], qxf - kxh, qyf - kyh) - chik;
+              const float cp = chi_even(tch[i], qxf + kxh, qyf + kyh) - chik;
+              constexpr float kTurn = 0.15915494309189535f;   // 1 / 2pi
+              ts = (cp - cm) * kTurn;
+              s = (cp + cm) * kTurn;
+            }
+            t = B < 0.0f ? -ts : ts;
+          }
+          // One phasor where one aperture is zero, whatever the other's value
+          // (normalising takes it out), and where both are one; the general
+          // form at an outer edge, with the smaller aperture in its soft band,
+          // and where the sine vanishes.
+          const bool both = far >= d_in;
+          const bool general = (fabsf(near) < margin) | ((far > -margin) & (far < d_in)) | (both & (s == floorf(s)));
+          float2 z = overlap_unit(G, both, s, t, __float_as_uint(B) & 0x80000000u);
+          if (general) {
+            df dn{near, 0.0f}, dfar{far, 0.0f};
+            if ((fabsf(near) < kApMargin) | (fabsf(far) < kApMargin)) {
+              const df qx = df_in_branch(df{qxf, ds.qxl[q]}), qy = df_in_branch(df{qyf, ds.qyl[c]});
+              const df kx{0.5f * kx2[i], km[i].kxl}, ky{0.5f * ky2[i], km[i].kyl};
+              df qk2 = df_mul(df_add(df_mul(qx, kx), df_mul(qy, ky)), df{2.0f, 0.0f});
+              if (B < 0.0f) qk2 = df_neg(qk2);
+              const df bd = df_sub(df{km[i].cb, km[i].cbl}, df_add(df_mul(qx, qx), df_mul(qy, qy)));
+              dn = df_add(bd, qk2);
+              dfar = df_sub(bd, qk2);
+            }
+            float2 g = gamma_hat_st(km[i].ak, aperture_from_d(dn, ds.ap), aperture_from_d(dfar, ds.ap), s, t);
+            if (B < 0.0f) g.x = -g.x;
+            z = mul_conj(G, g);
+          }
+          ar[i].add(z.x);
+          ai[i].add(z.y);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);   // one trial at a time: their temporaries do not overlap
+    }
+  }
 }
 
 // The persistent workgroups take items from a counter in device memory
@@ -121,10 +263,22 @@ __device__ __forceinline__ float aperture_quick(float dapprox, const ApIso& a) {
 // more points inside the apertures) and the short ones share the CUs evenly;
 // the last workgroup to leave (queue[1]) sets both counters back to zero for
 // the next launch, so a captured graph replays the kernel as it is.
-// Two workgroups per CU (2 waves per SIMD, 256 registers with 2 spilled):
-// unbounded, the kernel took 258 and ran one workgroup per CU at half the rate.
+//
+// Bound by VALU issue.  A point with one aperture zero or both one, and a chi
+// of C10, C12 and C30 terms, needs one phasor (overlap_unit), and with
+// A = |Q|^2 + |k|^2 and B = 2 Q.k the half difference and half sum of the
+// phases are polynomials without cancellation:
+//   t = B (k0 + 2 k4 A),  s = |Q|^2 (k0 + k4 (|Q|^2 + 2 |k|^2)) + k4 B^2,
+// C12 adding bilinear and quadratic forms.  A wave runs the general form as
+// soon as one of its points needs it, so the points lie in square tiles.  512
+// trials of C10, C30 and rotation at 256 x 256, 800 BF pixels: 66.9 ms with
+// two sincosf and a normalisation a point; 32.4 ms with one phasor and the
+// whole soft bands in the general form; 9.0 ms with the general form at the
+// outer edges and the lens' own band alone, on 8 x 8 tiles.  At most 128
+// registers (4 waves per SIMD): the BF pixel's scalars and the next G hide
+// behind the other waves.
 template <int TB>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, 4)
 k_trotter_trials(const TrialSet* __restrict__ sets, int n_sets, long long total_items,
                  const TrialChi* __restrict__ chis, unsigned* __restrict__ queue) {
   __shared__ TrialChi tch[TB];
@@ -134,15 +288,14 @@ k_trotter_trials(const TrialSet* __restrict__ sets, int n_sets, long long total_
     __syncthreads();   // the previous item's readers of tch and s_item are done
     if (tid == 0) s_item = atomicAdd(&queue[0], 1u);
     __syncthreads();
-    const long long item = s_item;
+    const long long item = __builtin_amdgcn_readfirstlane(s_item);
     if (item >= total_items) break;
     int d = 0;
     while (d + 1 < n_sets && item >= sets[d + 1].item0) ++d;
-    const TrialSet ds = sets[d];
-    const int N = ds.N, nbf = ds.nbf;
+    const TrialSet& ds = sets[d];
+    const int N = ds.N;
     const int NPG = (N / 2 + 1) * N;     // points of the Hermitian half plane (the stack's per-pixel size)
     const int NP = trial_points(N);      // plus the Nyquist row's other half
-    const int pblocks = (NP + kTrialPoints - 1) / kTrialPoints;
     const long long loc = item - ds.item0;
     // point-block major: the low columns (the long items) are taken first
     const int tblocks = (ds.T + TB - 1) / TB;
@@ -160,52 +313,38 @@ k_trotter_trials(const TrialSet* __restrict__ sets, int n_sets, long long total_
     // p >= NPG: the Nyquist row q = N/2 at column c > N/2, whose mirror
     // -Q = (+N/2, N - c) is not a grid frequency (fftfreq puts -N/2 on the
     // grid), so it is evaluated directly with G(N/2, c) = conj G(N/2, N - c)
-    const int p = pb * kTrialPoints + tid;
+    int p;
+    if (pb < N * N / (2 * kTrialPoints)) {
+      // 16 x 16 tiles of the columns below N/2, 8 x 8 a wave: few waves hold
+      // points at an aperture's edge, and few points outside beside points
+      // inside (64 points of one column cross an edge in most waves)
+      const int rows = N / 16, w = tid >> 6, l = tid & 63;
+      const int tc = pb / rows, tr = pb - tc * rows;
+      p = (tc * 16 + (w >> 1) * 8 + (l >> 3)) * N + tr * 16 + (w & 1) * 8 + (l & 7);
+    } else {
+      p = pb * kTrialPoints + tid;   // column N/2 and the Nyquist row's other half
+    }
     const bool live = p < NP;
     const bool nyq = live && p >= NPG;
     const int c = nyq ? N / 2 + 1 + (p - NPG) : (live ? p / N : 0);
     const int q = nyq ? N / 2 : (live ? p - c * N : 0);
     const long long gofs = nyq ? (long long)(N - c) * N + N / 2 : (long long)(live ? p : 0);
-    const df qx{ds.qx[q], ds.qxl[q]}, qy{ds.qy[c], ds.qyl[c]};
-    const df q2 = df_add(df_mul(qx, qx), df_mul(qy, qy));
-    const float qxf = qx.hi, qyf = qy.hi, q2f = q2.hi + q2.lo;
     Kahan ar[TB], ai[TB];
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
       ar[i].init();
       ai[i].init();
     }
-    const float2* gsrc = ds.Gt + gofs;
-    for (int b = 0; b < nbf; ++b) {
-      float2 G = live ? gsrc[(long long)b * NPG] : make_float2(0.f, 0.f);
-      if (nyq) G.y = -G.y;
-#pragma unroll
-      for (int i = 0; i < TB; ++i) {
-        if (i < nt) {
-          const TrialBf k = ds.tbf[(long long)(t0 + i) * nbf + b];
-          const float qk = qxf * k.kx + qyf * k.ky;
-          const float base = k.cb - q2f;
-          float am = aperture_quick(base + 2.0f * qk, ds.ap);
-          float ap = aperture_quick(base - 2.0f * qk, ds.ap);
-          if (am < 0.0f || ap < 0.0f) {
-            // inside the soft band: d = (Rout^2 - |k|^2 - |Q|^2) +/- 2 Q.k in double-float
-            const df kx{k.kx, k.kxl}, ky{k.ky, k.kyl};
-            const df qk2 = df_mul(df_add(df_mul(qx, kx), df_mul(qy, ky)), df{2.0f, 0.0f});
-            const df bd = df_sub(df{k.cb, k.cbl}, q2);
-            if (am < 0.0f) am = aperture_from_d(df_add(bd, qk2), ds.ap);
-            if (ap < 0.0f) ap = aperture_from_d(df_sub(bd, qk2), ds.ap);
-          }
-          if (am != 0.0f || ap != 0.0f) {
-            const float cm = chi_even(tch[i], qxf - k.kx, qyf - k.ky);
-            const float cp = chi_even(tch[i], qxf + k.kx, qyf + k.ky);
-            const float2 g = gamma_hat_chi(k.ak, am, ap, cm - k.chik, cp - k.chik);
-            const float2 t = mul_conj(G, g);
-            ar[i].add(t.x);
-            ai[i].add(t.y);
-          }
-        }
-      }
-    }
+    const long long slot = (long long)tb * ds.nbf;
+    const Const<TrialBf> kb = as_const(ds.tbf + slot);
+    const Const<TrialBfMore> km = as_const(ds.more + slot * TB);
+    const Const<TrialChi> ch = as_const(chis + t0);
+    bool radial = true;
+    for (int i = 0; i < nt; ++i) radial = radial && ch[i].kind == kChiRadial;
+    if (radial)
+      trial_sums<TB, true>(ds, tch, kb, km, ch, nt, q, c, live, nyq, ds.Gt + gofs, NPG, ar, ai);
+    else
+      trial_sums<TB, false>(ds, tch, kb, km, ch, nt, q, c, live, nyq, ds.Gt + gofs, NPG, ar, ai);
     if (live) {
 #pragma unroll
       for (int i = 0; i < TB; ++i)
@@ -388,6 +527,7 @@ struct ssb_trials {
   TrialSet* sets = nullptr;
   std::vector<TrialSet> sets_host;
   std::vector<TrialBf*> tbf;
+  std::vector<TrialBfMore*> more;
   std::vector<float2*> S;
   std::vector<float2*> W;
   std::vector<float*> part;
@@ -414,6 +554,7 @@ void trials_free(ssb_trials* tr) {
   (void)hipFree(tr->queue);
   (void)hipFree(tr->sets);
   for (auto* p : tr->tbf) (void)hipFree(p);
+  for (auto* p : tr->more) (void)hipFree(p);
   for (auto* p : tr->S) (void)hipFree(p);
   for (auto* p : tr->W) (void)hipFree(p);
   for (auto* p : tr->part) (void)hipFree(p);
@@ -435,7 +576,7 @@ hipError_t enqueue_trials(ssb_trials* tr, float* out, hipStream_t s) {
     const long long total = (long long)T * p->g_nbf;
     hipLaunchKernelGGL(k_trial_geometry, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p->bf_rows,
                        p->bf_cols, p->info, p->g_nbf, T, to_df(p->recip_y), to_df(p->recip_x), p->optics, rout2,
-                       tr->chis, tr->tbf[i]);
+                       tr->chis, tr->tbf[i], tr->more[i]);
   }
   long long total_items = 0;
   for (auto& ds : tr->sets_host) {
@@ -483,17 +624,21 @@ int ssb_trials_create(ssb_plan* const* plans, int n_plans, int max_trials, ssb_t
   for (int i = 0; i < n_plans && e == hipSuccess; ++i) {
     ssb_plan* p = plans[i];
     const long long NP = trial_points(p->n);
+    const size_t slots = (size_t)((max_trials + kTrialBlock - 1) / kTrialBlock) * p->g_nbf;
     TrialBf* tb = nullptr;
+    TrialBfMore* more = nullptr;
     float2* S = nullptr;
     float2* W = nullptr;
     float* part = nullptr;
-    e = hipMalloc(reinterpret_cast<void**>(&tb), sizeof(TrialBf) * (size_t)max_trials * p->g_nbf);
+    e = hipMalloc(reinterpret_cast<void**>(&tb), sizeof(TrialBf) * slots);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&more), sizeof(TrialBfMore) * kTrialBlock * slots);
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&S), sizeof(float2) * (size_t)max_trials * NP);
     if (e == hipSuccess)
       e = hipMalloc(reinterpret_cast<void**>(&W), sizeof(float2) * (size_t)max_trials * p->n * p->n);
     if (e == hipSuccess)
       e = hipMalloc(reinterpret_cast<void**>(&part), sizeof(float) * 4 * (size_t)max_trials * (p->n / kFinishCount));
     tr->tbf.push_back(tb);
+    tr->more.push_back(more);
     tr->S.push_back(S);
     tr->W.push_back(W);
     tr->part.push_back(part);
@@ -501,6 +646,7 @@ int ssb_trials_create(ssb_plan* const* plans, int n_plans, int max_trials, ssb_t
     TrialSet ds{};
     ds.Gt = p->Gt;
     ds.tbf = tb;
+    ds.more = more;
     ds.S = S;
     ds.qx = p->qx;
     ds.qxl = p->qxl;
@@ -548,6 +694,7 @@ int ssb_trials_set(ssb_trials* tr, int n_trials, const double* mags_host, const 
     const double* m = mags_host + (size_t)t * 14;
     const double* a = angles_host + (size_t)t * 14;
     tc.radial = 1;
+    tc.kind = kChiRadial;
     for (int i = 0; i < 14; ++i) {
       if ((km[i] & 1) && m[i] != 0.0)
         return report_error(QSSB_ERR_UNSUPPORTED, "the batched search evaluates even aberrations only "
@@ -556,7 +703,14 @@ int ssb_trials_set(ssb_trials* tr, int n_trials, const double* mags_host, const 
       tc.cp.ca[i] = (float)std::cos(km[i] * a[i]);
       tc.cp.sa[i] = (float)std::sin(km[i] * a[i]);
       if (km[i] != 0 && tc.cp.K[i] != 0.0f) tc.radial = 0;
+      if (tc.cp.K[i] != 0.0f && i == 1 && tc.kind == kChiRadial) tc.kind = kChiAstig;
+      if (tc.cp.K[i] != 0.0f && i != 0 && i != 1 && i != 4) tc.kind = kChiGeneral;
     }
+    // chi / pi: 2 / lam * lam^(n+1) / (n+1) * C
+    tc.k0 = (float)(lam * m[0]);
+    tc.k4 = (float)(0.5 * lam * lam * lam * m[4]);
+    tc.m12c = (float)(lam * m[1] * std::cos(2.0 * a[1]));
+    tc.m12s = (float)(lam * m[1] * std::sin(2.0 * a[1]));
     tc.cp.odd = 0;
     const double rot = rotation_host ? rotation_host[t] : 0.0;
     tc.cos_a = to_df(std::cos(-rot));
