@@ -1,5 +1,6 @@
 // C ABI of the MI355X SSB engine: plan management and pipeline launches.
 // Declarations and reference citations: include/quantem_ssb.h.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -596,13 +597,31 @@ int ssb_object(ssb_plan* p, double c10, double c12, double phi12, void* obj_out,
   return QSSB_OK;
 }
 
+static ChiPoly chi_poly(const ssb_plan* p, const double* mags, const double* angles) {
+  static const int kn[14] = {1, 1, 2, 2, 3, 3, 3, 4, 4, 4, 5, 5, 5, 5};
+  static const int km[14] = {0, 2, 1, 3, 0, 2, 4, 1, 3, 5, 0, 2, 4, 6};
+  ChiPoly cp{};
+  const double lam = p->wavelength;
+  for (int i = 0; i < 14; ++i) {
+    const int n = kn[i], m = km[i];
+    cp.K[i] = (float)(2.0 * M_PI / lam * std::pow(lam, n + 1) / (n + 1) * mags[i]);
+    cp.ca[i] = (float)std::cos(m * angles[i]);
+    cp.sa[i] = (float)std::sin(m * angles[i]);
+    if ((m & 1) && cp.K[i] != 0.0f) cp.odd = 1;
+  }
+  return cp;
+}
+
+// Workspace of the exact phase path, for its even and its general form alike
+// (a later call of the other form, under capture too, allocates nothing).
 static int alloc_loss(ssb_plan* p) {
   if (p->T) return QSSB_OK;
   const size_t nn = (size_t)p->n * p->n;
-  hipError_t e = dmalloc(&p->T, (size_t)loss_chunk_bf(p->n) * nn);
-  if (e == hipSuccess) e = dmalloc(&p->M1, (size_t)loss_splits(p->n) * nn);
-  if (e == hipSuccess) e = dmalloc(&p->M2, (size_t)loss_splits(p->n) * nn);
-  if (e == hipSuccess) e = dmalloc(&p->var_part, (nn + 255) / 256);
+  const size_t planes = std::max(phase_splits(p->n), loss_splits(p->n));
+  hipError_t e = dmalloc(&p->T, std::max(phase_workspace_floats2(p->n), loss_chunk_bf(p->n) * nn));
+  if (e == hipSuccess) e = dmalloc(&p->M1, planes * nn);
+  if (e == hipSuccess) e = dmalloc(&p->M2, planes * nn);
+  if (e == hipSuccess) e = dmalloc(&p->var_part, nn / 64);
   if (e == hipSuccess) e = dmalloc(&p->loss, 1);
   if (e != hipSuccess) {
     dfree(p->T);
@@ -617,6 +636,47 @@ static int alloc_loss(ssb_plan* p) {
   return QSSB_OK;
 }
 
+// The even part of a chi without odd terms, in half turns; `general` when it
+// has terms besides C10, C12 and C30.
+static EvenChi even_chi(const ssb_plan* p, const double* mags, const double* angles, const ChiPoly& cp) {
+  const double lam = p->wavelength;
+  EvenChi ev{};
+  ev.k0 = (float)(lam * mags[0]);
+  ev.k4 = (float)(0.5 * lam * lam * lam * mags[4]);
+  ev.m12c = (float)(lam * mags[1] * std::cos(2.0 * angles[1]));
+  ev.m12s = (float)(lam * mags[1] * std::sin(2.0 * angles[1]));
+  for (int i = 2; i < 14; ++i)
+    if (i != 4 && cp.K[i] != 0.0f) ev.general = 1;
+  ev.cp = cp;
+  return ev;
+}
+
+// Enqueue one exact evaluation with the plan's cached geometry (the
+// workspace allocated): the even form where it applies, else the general one.
+// `quad`: only mags[0..1] count.  d, when given: the trial's device copy.
+static hipError_t enqueue_phase(ssb_plan* p, const double* mags, const double* angles, bool quad, float* phase_out,
+                                float* loss_out, hipStream_t s, const ExactTrial* d = nullptr) {
+  double m14[14] = {0}, a14[14] = {0};
+  for (int i = 0; i < (quad ? 2 : 14); ++i) {
+    m14[i] = mags[i];
+    a14[i] = angles[i];
+  }
+  const ChiPoly cp = chi_poly(p, m14, a14);
+  if (phase_even_path(p->n, p->gcols, p->optics, cp.odd != 0)) {
+    const EvenChi ev = even_chi(p, m14, a14, cp);
+    return launch_phase_even(p->n, p->Gt, p->info, p->g_nbf, geom_ptrs(p), ev, d ? &d->ev : nullptr, p->optics, p->tw,
+                             p->T, p->M1, p->M2, p->var_part, phase_out, loss_out, s);
+  }
+  hipError_t e = hipSuccess;
+  if (quad)
+    e = launch_phasors(p->n, p->info, p->nbf_hint, geom_ptrs(p), quad_chi(p, mags[0], mags[1], angles[1]), p->rowph,
+                       p->colph, p->echi, s, d ? &d->m : nullptr);
+  if (e != hipSuccess) return e;
+  return launch_phase_moments(p->n, p->Gt, p->gcols, p->info, p->g_nbf, geom_ptrs(p), p->rowph, p->colph, p->echi,
+                              quad ? nullptr : &cp, p->optics, p->tw, p->T, p->M1, p->M2, p->var_part, phase_out,
+                              loss_out, s, d && !quad ? &d->cp : nullptr);
+}
+
 int ssb_phase_loss(ssb_plan* p, double c10, double c12, double phi12, float* phase_out, float* loss_out,
                    void* stream) {
   int rc = check_plan(p);
@@ -629,12 +689,8 @@ int ssb_phase_loss(ssb_plan* p, double c10, double c12, double phi12, float* pha
   }
   rc = alloc_loss(p);
   if (rc) return rc;
-  const QuadChi m = quad_chi(p, c10, c12, phi12);
-  HIP_TRY(launch_phasors(p->n, p->info, p->nbf_hint, geom_ptrs(p), m, p->rowph, p->colph, p->echi, s), "phasors");
-  HIP_TRY(launch_phase_moments(p->n, p->Gt, p->gcols, p->info, p->g_nbf, geom_ptrs(p), p->rowph, p->colph, p->echi,
-                               nullptr, p->optics, p->tw, p->T, p->M1, p->M2, p->var_part, phase_out,
-                               loss_out ? loss_out : p->loss, s),
-          "phase_moments");
+  const double mags[2] = {c10, c12}, angles[2] = {0.0, phi12};
+  HIP_TRY(enqueue_phase(p, mags, angles, true, phase_out, loss_out ? loss_out : p->loss, s), "phase_moments");
   return QSSB_OK;
 }
 
@@ -799,21 +855,6 @@ int ssb_normalize_scan_typed(const void* src, int dtype, int H, int W, int det_r
 }
 
 
-static ChiPoly chi_poly(const ssb_plan* p, const double* mags, const double* angles) {
-  static const int kn[14] = {1, 1, 2, 2, 3, 3, 3, 4, 4, 4, 5, 5, 5, 5};
-  static const int km[14] = {0, 2, 1, 3, 0, 2, 4, 1, 3, 5, 0, 2, 4, 6};
-  ChiPoly cp{};
-  const double lam = p->wavelength;
-  for (int i = 0; i < 14; ++i) {
-    const int n = kn[i], m = km[i];
-    cp.K[i] = (float)(2.0 * M_PI / lam * std::pow(lam, n + 1) / (n + 1) * mags[i]);
-    cp.ca[i] = (float)std::cos(m * angles[i]);
-    cp.sa[i] = (float)std::sin(m * angles[i]);
-    if ((m & 1) && cp.K[i] != 0.0f) cp.odd = 1;
-  }
-  return cp;
-}
-
 int ssb_phase_loss_full(ssb_plan* p, const double* mags_host, const double* angles_host, float* phase_out,
                         float* loss_out, void* stream) {
   int rc = check_plan(p);
@@ -827,10 +868,7 @@ int ssb_phase_loss_full(ssb_plan* p, const double* mags_host, const double* angl
   }
   rc = alloc_loss(p);
   if (rc) return rc;
-  const ChiPoly cp = chi_poly(p, mags_host, angles_host);
-  HIP_TRY(launch_phase_moments(p->n, p->Gt, p->gcols, p->info, p->g_nbf, geom_ptrs(p), p->rowph, p->colph, p->echi,
-                               &cp, p->optics, p->tw, p->T, p->M1, p->M2, p->var_part, phase_out,
-                               loss_out ? loss_out : p->loss, s),
+  HIP_TRY(enqueue_phase(p, mags_host, angles_host, false, phase_out, loss_out ? loss_out : p->loss, s),
           "phase_moments_full");
   return QSSB_OK;
 }
@@ -863,21 +901,7 @@ int ssb_batch_phase_loss(ssb_plan* p, int n_trials, const double* mags_host, con
     }
     bool higher = false;
     for (int i = 2; i < 14; ++i) higher = higher || (m[i] != 0.0);
-    float* lt = losses_out + t;
-    if (higher) {
-      const ChiPoly cp = chi_poly(p, m, a);
-      HIP_TRY(launch_phase_moments(p->n, p->Gt, p->gcols, p->info, p->g_nbf, geom_ptrs(p), p->rowph, p->colph,
-                                   p->echi, &cp, p->optics, p->tw, p->T, p->M1, p->M2, p->var_part, nullptr, lt, s),
-              "batch phase_moments_full");
-    } else {
-      const QuadChi qc = quad_chi(p, m[0], m[1], a[1]);
-      HIP_TRY(launch_phasors(p->n, p->info, p->nbf_hint, geom_ptrs(p), qc, p->rowph, p->colph, p->echi, s),
-              "batch phasors");
-      HIP_TRY(launch_phase_moments(p->n, p->Gt, p->gcols, p->info, p->g_nbf, geom_ptrs(p), p->rowph, p->colph,
-                                   p->echi, nullptr, p->optics, p->tw, p->T, p->M1, p->M2, p->var_part, nullptr, lt,
-                                   s),
-              "batch phase_moments");
-    }
+    HIP_TRY(enqueue_phase(p, m, a, !higher, nullptr, losses_out + t, s), "batch phase_moments");
   }
   // leave the cached rotation as the caller set it
   if (rotation_host && p->rotation != rot0) {
@@ -889,8 +913,8 @@ int ssb_batch_phase_loss(ssb_plan* p, int n_trials, const double* mags_host, con
 }
 
 // Enqueue the captured form of a batch: per trial the geometry (every
-// trial, from the device table), then the phasors and the exact loss of
-// ssb_batch_phase_loss reading their coefficients from the table.
+// trial, from the device table), then the exact loss of ssb_batch_phase_loss
+// reading its coefficients from the table.
 static hipError_t enqueue_exact_batch(ssb_plan* p, int n, float* losses_out, hipStream_t s) {
   hipError_t e = hipSuccess;
   for (int t = 0; t < n && e == hipSuccess; ++t) {
@@ -899,17 +923,7 @@ static hipError_t enqueue_exact_batch(ssb_plan* p, int n, float* losses_out, hip
     e = launch_bf_geometry(p->bf_rows, p->bf_cols, p->info, p->max_bf, to_df(p->recip_y), to_df(p->recip_x),
                            h.cs[0], h.cs[1], p->optics, p->kx, p->kxl, p->ky, p->kyl, p->ak, s, d->cs);
     if (e != hipSuccess) break;
-    if (h.higher) {
-      e = launch_phase_moments(p->n, p->Gt, p->gcols, p->info, p->g_nbf, geom_ptrs(p), p->rowph, p->colph, p->echi,
-                               &h.cp, p->optics, p->tw, p->T, p->M1, p->M2, p->var_part, nullptr, losses_out + t, s,
-                               &d->cp);
-    } else {
-      e = launch_phasors(p->n, p->info, p->nbf_hint, geom_ptrs(p), h.m, p->rowph, p->colph, p->echi, s, &d->m);
-      if (e == hipSuccess)
-        e = launch_phase_moments(p->n, p->Gt, p->gcols, p->info, p->g_nbf, geom_ptrs(p), p->rowph, p->colph,
-                                 p->echi, nullptr, p->optics, p->tw, p->T, p->M1, p->M2, p->var_part, nullptr,
-                                 losses_out + t, s);
-    }
+    e = enqueue_phase(p, h.mags, h.angles, !h.higher, nullptr, losses_out + t, s, d);
   }
   return e;
 }
@@ -958,7 +972,12 @@ int ssb_batch_phase_loss_graph(ssb_plan* p, int n_trials, const double* mags_hos
     x.higher = higher ? 1 : 0;
     x.m = quad_chi(p, m[0], m[1], a[1]);
     x.cp = chi_poly(p, m, a);
-    pattern[t] = x.higher;
+    x.ev = even_chi(p, m, a, x.cp);
+    for (int i = 0; i < 14; ++i) {
+      x.mags[i] = m[i];
+      x.angles[i] = a[i];
+    }
+    pattern[t] = x.higher | (x.cp.odd << 1) | (x.ev.general << 2);
   }
   HIP_TRY(hipMemcpyAsync(p->xt, p->xt_host.data(), sizeof(ExactTrial) * n_trials, hipMemcpyHostToDevice, s),
           "batch table upload");

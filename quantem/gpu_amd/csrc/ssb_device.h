@@ -206,6 +206,15 @@ __device__ __forceinline__ void copy_async16(const void* gptr, void* lds_wave_ba
 }
 __device__ __forceinline__ void wait_async_copies() { __builtin_amdgcn_s_waitcnt(0); }
 
+// Data that only kernels before this one write, read through the constant
+// address space: scalar loads.
+template <typename T>
+using Const = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ Const<T> as_const(const T* p) {
+  return (Const<T>)(unsigned long long)p;
+}
+
 // ---------------------------------------------------------------- double-float
 // Unevaluated sums hi + lo of two floats (~44-bit significand), built from
 // error-free transformations (Dekker / Knuth two-sum, FMA two-product).

@@ -76,6 +76,14 @@ struct ChiPoly {
   int odd;   // any odd-m term (C21, C23, C41, C43, C45) non-zero: chi(-u) != chi(u)
 };
 
+// An even aberration phase: chi / pi = k0 r2 + k4 r2^2 + m12c (ux^2 - uy^2) +
+// m12s 2 ux uy (C10, C30, C12), or with `general` the even part of cp.
+struct EvenChi {
+  float k0, k4, m12c, m12s;
+  int general;
+  ChiPoly cp;
+};
+
 // Matrix of the quadratic aberration phase chi(u) = u^T M u,
 // M = pi*lambda*[[C10 + C12 cos2p, C12 sin2p], [C12 sin2p, C10 - C12 cos2p]].
 struct QuadChi {
@@ -261,8 +269,9 @@ int loss_chunk_bf(int N);
 int loss_splits(int N);
 // Mean of per-BF phases and the phase-variance loss from the resident
 // stack Gt[b][c][q] (gcols = N/2+1 Hermitian, or N full-plane), with the
-// phasor tables of a quadratic chi, or (poly != NULL) the full chi; T holds loss_chunk_bf(N) planes, M1/M2
-// loss_splits(N) planes, var_part N*N/256 floats.  phase may be NULL; loss
+// phasor tables of a quadratic chi, or (poly != NULL) the full chi, where
+// phase_even_path does not hold; T holds loss_chunk_bf(N) planes, M1/M2
+// loss_splits(N) planes, var_part N*N/64 floats.  phase may be NULL; loss
 // is a device scalar.
 hipError_t launch_phase_moments(int N, const float2* Gt, int gcols, const BfInfo* info, int nbf_hint, const GeomPtrs& gp,
                                 const float2* rowph, const float2* colph, const float2* echi, const ChiPoly* poly,
@@ -270,6 +279,20 @@ hipError_t launch_phase_moments(int N, const float2* Gt, int gcols, const BfInfo
                                 const float2* tw, float2* T, float2* M1, float2* M2, float* var_part,
                                 float* phase, float* loss, hipStream_t s,
                                 const ChiPoly* poly_dev = nullptr);
+
+// The same for a Hermitian stack, an even chi and equal detector sampling
+// (phase_even_path): half the columns, rows and bytes.  ws holds
+// phase_workspace_floats2(N) float2, M1/M2 phase_splits(N) planes.  ch_dev,
+// when given, holds the coefficients (ch then only says which form).
+bool phase_even_path(int N, int gcols, const Optics& o, bool odd);
+int phase_splits(int N);
+size_t phase_workspace_floats2(int N);
+hipError_t launch_phase_even(int N, const float2* Gt, const BfInfo* info, int nbf, const GeomPtrs& gp,
+                             const EvenChi& ch, const EvenChi* ch_dev, const Optics& o, const float2* tw, float2* ws,
+                             float2* M1, float2* M2, float* var_part, float* phase, float* loss, hipStream_t s);
+// Splits combined, mean phase (may be NULL), loss (device scalar).
+hipError_t launch_moments_finish(int N, int nsplit, const BfInfo* info, const float2* M1, const float2* M2,
+                                 float* var_part, float* phase, float* loss, hipStream_t s);
 
 // Learned-initializer features of the resident Hermitian stack at the 8
 // scan-frequency grid points (qrow[i], qcol[i]) (device arrays): out is

@@ -1,4 +1,6 @@
-// Exact per-BF phase path of the MI355X SSB engine: for every bright-field
+// Exact per-BF phase path of the MI355X SSB engine, in its general form (full-
+// plane stacks, aberrations with odd terms, unequal detector sampling; the
+// rest is in ssb_phase.hip), and the finishing kernels: for every bright-field
 // pixel b the corrected plane C_b(Q) = G_b(Q) conj(Gamma^_b(Q)) with its DC
 // bin replaced by dc, the inverse 2D FFT O_b = IFFT2(C_b), phi_b = angle(O_b),
 // and the per-pixel moments sum_b phi_b, sum_b phi_b^2.  From them the mean
@@ -170,9 +172,8 @@ k_corr_colifft(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
         }
         eB = cmul(rowA, (j == 0) ? colHalf : cconj(colp));
       }
-      // Mirror points with an even chi (every quadratic chi; a full chi
-      // without odd-m terms): B sees the apertures swapped, the phasors
-      // conjugated and conj(G), so Gamma_B = -conj(Gamma_A) with the same
+      // Mirror points with an even chi (unequal detector sampling): B sees
+      // the apertures swapped, the phasors conjugated and conj(G), so Gamma_B = -conj(Gamma_A) with the same
       // norm and C_B = -conj(C_A) exactly (every operation is
       // sign-symmetric); it is not recomputed.
       const bool same = mirror && !FULL && (!POLY || !cp.odd);
@@ -304,39 +305,40 @@ k_rowifft_moments(const float2* __restrict__ T, const BfInfo* __restrict__ info,
 // Pass 3: combine the splits (fixed order), mean phase, per-pixel variance,
 // per-block variance sums; then one block sums those in fixed order.
 // ------------------------------------------------------------------------
+// A workgroup owns 64 pixels, its four waves a quarter of the splits each.
 __global__ void __launch_bounds__(256)
 k_moments_finish(const float2* __restrict__ M1, const float2* __restrict__ M2, int nsplit, int NN,
                  const BfInfo* __restrict__ info, float* __restrict__ phase, float* __restrict__ var_part) {
-  __shared__ float red_s[4];
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  float var = 0.0f;
-  if (idx < NN) {
-    Kahan s1, s2;
-    s1.init();
-    s2.init();
-    for (int sp = 0; sp < nsplit; ++sp) {
-      const float2 a = M1[(long long)sp * NN + idx];
-      const float2 c = M2[(long long)sp * NN + idx];
-      s1.add(a.x - a.y);
-      s2.add(c.x - c.y);
-    }
-    const float inv = 1.0f / (float)(info->nbf > 0 ? info->nbf : 1);
-    const float mean = (s1.s - s1.c) * inv;
-    var = (s2.s - s2.c) * inv - mean * mean;
-    if (phase) phase[idx] = mean;
-  }
-  // block sum of var: wave tree sums (fixed order), then the 4 waves in order
-  float v = var;
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  __shared__ float2 part[4][64][2];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) red_s[w] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    Kahan k;
-    k.init();
-    for (int i = 0; i < 4; ++i) k.add(red_s[i]);
-    var_part[blockIdx.x] = k.s - k.c;
+  const int idx = blockIdx.x * 64 + lane;   // N * N is a multiple of 64
+  const int s0 = nsplit * w / 4, s1 = nsplit * (w + 1) / 4;
+  Kahan a1, a2;
+  a1.init();
+  a2.init();
+#pragma unroll 4
+  for (int sp = s0; sp < s1; ++sp) {
+    const float2 a = M1[(long long)sp * NN + idx];
+    const float2 c = M2[(long long)sp * NN + idx];
+    a1.add(a.x - a.y);
+    a2.add(c.x - c.y);
   }
+  part[w][lane][0] = make_float2(a1.s, a1.c);
+  part[w][lane][1] = make_float2(a2.s, a2.c);
+  __syncthreads();
+  if (w != 0) return;
+  for (int k = 1; k < 4; ++k) {
+    const float2 u = part[k][lane][0], v = part[k][lane][1];
+    a1.add(u.x - u.y);
+    a2.add(v.x - v.y);
+  }
+  const float inv = 1.0f / (float)(info->nbf > 0 ? info->nbf : 1);
+  const float mean = (a1.s - a1.c) * inv;
+  if (phase) phase[idx] = mean;
+  // the block's variances in a tree of fixed order
+  float v = (a2.s - a2.c) * inv - mean * mean;
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  if (lane == 0) var_part[blockIdx.x] = v;
 }
 
 __global__ void __launch_bounds__(256)
@@ -383,14 +385,17 @@ hipError_t launch_phase_moments(int N, const float2* Gt, int gcols, const BfInfo
   const bool iso = optics_isotropic(o);
   const bool full = (gcols == N);
   if (!full && gcols != N / 2 + 1) return hipErrorInvalidValue;
+  if (iso && !full && !(poly && poly->odd)) return hipErrorInvalidValue;   // launch_phase_even's
   const int chunk = loss_chunk_bf(N);
   const int nsplit = loss_splits(N);
   const int nb = nbf_hint > 0 ? nbf_hint : 1;
+#define QSSB_P1_POLY(NN, SGV, BL, IS, FU)                                                                   \
+  hipLaunchKernelGGL((k_corr_colifft<NN, SGV, BL, IS, FU, true>), dim3(g1), dim3(BL), 0, s, Gt, info, gp,        \
+                     rowph, colph, echi, *poly, poly_dev, ap, rout2, o, tw, b0, cnt, T)
 #define QSSB_P1_ONE(NN, SGV, BL, IS, FU)                                                                    \
   do {                                                                                                       \
     if (poly)                                                                                                \
-      hipLaunchKernelGGL((k_corr_colifft<NN, SGV, BL, IS, FU, true>), dim3(g1), dim3(BL), 0, s, Gt, info, gp,   \
-                         rowph, colph, echi, *poly, poly_dev, ap, rout2, o, tw, b0, cnt, T);                  \
+      QSSB_P1_POLY(NN, SGV, BL, IS, FU);                                                                     \
     else                                                                                                     \
       hipLaunchKernelGGL((k_corr_colifft<NN, SGV, BL, IS, FU, false>), dim3(g1), dim3(BL), 0, s, Gt, info, gp,  \
                          rowph, colph, echi, ChiPoly{}, nullptr, ap, rout2, o, tw, b0, cnt, T);               \
@@ -398,7 +403,7 @@ hipError_t launch_phase_moments(int N, const float2* Gt, int gcols, const BfInfo
 #define QSSB_P1(NN, SGV, BL)                                                    \
   do {                                                                         \
     const unsigned g1 = (unsigned)((long long)cnt * ((NN / 2) / SGV));        \
-    if (iso && !full) QSSB_P1_ONE(NN, SGV, BL, true, false);                   \
+    if (iso && !full) QSSB_P1_POLY(NN, SGV, BL, true, false);                  \
     else if (iso) QSSB_P1_ONE(NN, SGV, BL, true, true);                        \
     else if (!full) QSSB_P1_ONE(NN, SGV, BL, false, false);                    \
     else QSSB_P1_ONE(NN, SGV, BL, false, true);                                \
@@ -436,9 +441,15 @@ hipError_t launch_phase_moments(int N, const float2* Gt, int gcols, const BfInfo
   }
 #undef QSSB_P1
 #undef QSSB_P1_ONE
+#undef QSSB_P1_POLY
 #undef QSSB_P2
+  return launch_moments_finish(N, nsplit, info, M1, M2, var_part, phase, loss, s);
+}
+
+hipError_t launch_moments_finish(int N, int nsplit, const BfInfo* info, const float2* M1, const float2* M2,
+                                 float* var_part, float* phase, float* loss, hipStream_t s) {
   const int NN = N * N;
-  const int parts = (NN + 255) / 256;
+  const int parts = NN / 64;
   hipLaunchKernelGGL(k_moments_finish, dim3(parts), dim3(256), 0, s, M1, M2, nsplit, NN, info, phase, var_part);
   hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(256), 0, s, var_part, parts, NN, loss);
   return hipGetLastError();

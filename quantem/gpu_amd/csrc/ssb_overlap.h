@@ -114,6 +114,11 @@ __device__ __forceinline__ float2 gamma_hat(float ak, float2 eth, float am, floa
   return make_float2(gr * sc, gi * sc);
 }
 
+// G * conj(g)
+__device__ __forceinline__ float2 mul_conj(float2 G, float2 g) {
+  return make_float2(G.x * g.x + G.y * g.y, G.y * g.x - G.x * g.y);
+}
+
 // sin(pi r) and cos(pi r) for |r| <= 1/2: minimax polynomials in r^2 (fitted
 // for these functions by iteratively reweighted least squares; 5.3e-9 and
 // 2.4e-10 before rounding, 1.6e-7 and 1.1e-7 evaluated in float32).
@@ -168,10 +173,63 @@ __device__ __forceinline__ float2 gamma_hat_st(float ak, float am, float app, fl
   turn(s, ss, cc);
   turn(t, st, ct);
   const float wr = (am - app) * cc, wi = -(am + app) * ss;
-  float gr = ak * (ct * wr - st * wi), gi = ak * (ct * wi + st * wr);
-  const float mag2 = gr * gr + gi * gi;
+  // contracted as written: the same bits wherever this is inlined
+  const float gr = ak * fmaf(ct, wr, -(st * wi)), gi = ak * fmaf(ct, wi, st * wr);
+  const float mag2 = fmaf(gr, gr, gi * gi);
   const float sc = (mag2 > 1e-16f) ? rsqrtf(mag2) : 1e8f;
   return make_float2(gr * sc, gi * sc);
+}
+
+// The term G * conj(Gamma^) of one point for an even chi.  near >= far: d =
+// Rout^2 - |u|^2 of Q - k and Q + k, the larger first, as float32 estimates
+// (an aperture is zero from d = 0 down and one from ap.d_in up); B: its sign
+// says which of the two is the nearer (negative: Q + k); s, t as in
+// overlap_unit, t on the nearer side.  One phasor serves where one aperture
+// is zero, whatever the other's value (normalising takes it out), and where
+// both are one; the general form at an outer edge and with the smaller
+// aperture in its soft band, where the sine vanishes, and for a BF pixel whose
+// small A(k) can meet the guard elsewhere (margin = infinity).  There both d
+// come in double-float from exact(dn, df) within kEdgeMargin of an edge and
+// with both apertures in their bands, where their values or their difference
+// decide; inside one aperture and well inside the other's band the estimates
+// give the ratio to 2e-6.  B must not be a negative zero unless t is zero.
+constexpr float kEdgeMargin = 1e-4f;   // far above the estimates' error (2e-5 for terms below 32)
+constexpr float kSmallAk = 1e-3f;
+__device__ __forceinline__ float edge_margin(float ak) { return ak < kSmallAk ? INFINITY : kEdgeMargin; }
+
+template <typename Exact>
+__device__ __forceinline__ float2 overlap_term(float2 G, float near, float far, float B, float s, float t,
+                                               float margin, float ak, const ApIso& ap, Exact exact) {
+  const float inner = ap.d_in + kEdgeMargin;
+  const bool both = far >= inner;
+  const bool general = (fabsf(near) < margin) | ((far > -margin) & (far < inner)) | (both & (s == floorf(s)));
+  float2 z = overlap_unit(G, both, s, t, __float_as_uint(B) & 0x80000000u);
+  if (general) {
+    df dn{near, 0.0f}, dfar{far, 0.0f};
+    // the estimates do away from every edge of a lens whose other aperture is one
+    if (!(both | ((near >= inner) & (far >= kEdgeMargin) & (far <= ap.d_in - kEdgeMargin))) | (margin > kEdgeMargin)) {
+      exact(dn, dfar);
+      if (B < 0.0f) {
+        const df x = dn;
+        dn = dfar;
+        dfar = x;
+      }
+    }
+    float2 g = gamma_hat_st(ak, aperture_from_d(dn, ap), aperture_from_d(dfar, ap), s, t);
+    if (B < 0.0f) g.x = -g.x;
+    z = make_float2(fmaf(G.x, g.x, G.y * g.y), fmaf(G.y, g.x, -(G.x * g.y)));
+  }
+  return z;
+}
+
+// d of Q - k and Q + k in double-float; q and k through the branch they are
+// needed in (nothing of it is formed ahead of it).
+__device__ __forceinline__ void exact_d(df qx, df qy, df kx, df ky, df cb, df& dm, df& dp) {
+  const df x = df_in_branch(qx), y = df_in_branch(qy);
+  const df qk2 = df_mul(df_add(df_mul(x, kx), df_mul(y, ky)), df{2.0f, 0.0f});
+  const df base = df_sub(cb, df_add(df_mul(x, x), df_mul(y, y)));
+  dm = df_add(base, qk2);
+  dp = df_sub(base, qk2);
 }
 
 // chi(u) split into its even part E and odd part O (ChiPoly).
@@ -205,11 +263,6 @@ __device__ __forceinline__ float2 gamma_hat_chi(float ak, float am, float app, f
   const float mag2 = gr * gr + gi * gi;
   const float sc = (mag2 > 1e-16f) ? rsqrtf(mag2) : 1e8f;
   return make_float2(gr * sc, gi * sc);
-}
-
-// G * conj(g)
-__device__ __forceinline__ float2 mul_conj(float2 G, float2 g) {
-  return make_float2(G.x * g.x + G.y * g.y, G.y * g.x - G.x * g.y);
 }
 
 }  // namespace qssb

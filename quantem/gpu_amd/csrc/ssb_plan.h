@@ -12,12 +12,14 @@ using qssb::Optics;
 
 // One trial of a captured exact-objective batch, read by the captured
 // kernels from device memory: {cos, sin} of -rotation, the quadratic chi
-// matrix and the full chi polynomial.
+// matrix, the full chi polynomial and, without odd terms, its even form.
 struct ExactTrial {
   qssb::df cs[2];
   qssb::QuadChi m;
   int higher;
   qssb::ChiPoly cp;
+  qssb::EvenChi ev;
+  double mags[14], angles[14];   // as given (host)
 };
 
 struct ssb_plan {
@@ -89,7 +91,7 @@ struct ssb_plan {
   ExactTrial* xt = nullptr;            // device table [xt_cap]
   int xt_cap = 0;
   std::vector<ExactTrial> xt_host;
-  std::vector<int> xt_pattern;         // per trial: higher-order chi (topology of the graph)
+  std::vector<int> xt_pattern;         // per trial: higher-order chi (the form, topology of the graph)
   hipStream_t gstream = nullptr;       // the graph's own stream
   // second stream of the reconstruction: the gather of the second half of
   // the BF pixels runs on it while the first half's trotter runs on the

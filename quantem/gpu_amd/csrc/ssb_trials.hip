@@ -63,7 +63,7 @@ struct __attribute__((aligned(32))) TrialBf {
   float kx2[kTrialBlock], ky2[kTrialBlock];   // 2 k
   float cb[kTrialBlock];                      // Rout^2 - |k|^2
   float u[kTrialBlock];                       // d(chi / pi) / d(r2) at |k|^2: k0 + 2 k4 |k|^2
-  float margin[kTrialBlock];                  // kApMargin, or infinity
+  float margin[kTrialBlock];                  // edge_margin
 };
 
 // What points at an aperture's edge and the other trials need besides.
@@ -102,15 +102,6 @@ __device__ __forceinline__ float chi_even(const TrialChi& tc, float ux, float uy
   return e;
 }
 
-// Below this A(k) the overlap's guard |Gamma|^2 > 1e-16 can act away from an
-// exact zero of the sine: such BF pixels take the general form.
-constexpr float kSmallAk = 1e-3f;
-
-// Within this of an aperture's outer edge, d = Rout^2 - |u|^2 as a float32
-// estimate (absolute error far below it) does not decide whether the aperture
-// is zero: d is formed in double-float there.
-constexpr float kApMargin = 1e-4f;
-
 __global__ void __launch_bounds__(256)
 k_trial_geometry(const int* __restrict__ bf_rows, const int* __restrict__ bf_cols, const BfInfo* __restrict__ info,
                  int nbf, int T, df recip_y, df recip_x, Optics o, df rout2,
@@ -135,7 +126,7 @@ k_trial_geometry(const int* __restrict__ bf_rows, const int* __restrict__ bf_col
   r.ky2[i] = 2.0f * ky.hi;
   r.cb[i] = ak == 0.0f ? -1e30f : cb.hi;
   r.u[i] = fmaf(2.0f * tc.k4, k2, tc.k0);
-  r.margin[i] = ak < kSmallAk && ak > 0.0f ? INFINITY : kApMargin;
+  r.margin[i] = ak == 0.0f ? kEdgeMargin : edge_margin(ak);
   TrialBfMore m;
   m.ak = ak;
   m.chik = chi_even(tc, kx.hi, ky.hi);
@@ -148,15 +139,6 @@ k_trial_geometry(const int* __restrict__ bf_rows, const int* __restrict__ bf_col
   more[slot * kTrialBlock + i] = m;
 }
 
-// Data that only kernels before this one write, read through the constant
-// address space: scalar loads.
-template <typename T>
-using Const = const __attribute__((address_space(4))) T*;
-template <typename T>
-__device__ __forceinline__ Const<T> as_const(const T* p) {
-  return (Const<T>)(unsigned long long)p;
-}
-
 // The sums over the BF pixels of one point for the `nt` trials of a block.
 // RADIAL: none of them has a term beyond C10 and C30; otherwise each trial's
 // kind is looked up (the same arithmetic for its terms, so a trial's sums do
@@ -167,7 +149,6 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
                                            bool nyq, const float2* __restrict__ gsrc, long long gstep,
                                            Kahan (&ar)[TB], Kahan (&ai)[TB]) {
   const int nbf = ds.nbf;
-  const float d_in = ds.ap.d_in;
   const float qxf = ds.qx[q], qyf = ds.qy[c];
   float q2f, qa = 0.0f, qb = 0.0f;
   {
@@ -201,7 +182,8 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
       if (i < nt) {
-        const float B = fmaf(qxf, kx2[i], qyf * ky2[i]);
+        // (+ 0: no negative zero where t does not vanish with B)
+        const float B = RADIAL ? fmaf(qxf, kx2[i], qyf * ky2[i]) : fmaf(qxf, kx2[i], qyf * ky2[i]) + 0.0f;
         const float base = cb[i] - q2f;
         // d of Q -/+ k, the larger first: the apertures are zero from 0 down, one from d_in up
         const float near = base + fabsf(B), far = base - fabsf(B);
@@ -227,28 +209,10 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
             }
             t = B < 0.0f ? -ts : ts;
           }
-          // One phasor where one aperture is zero, whatever the other's value
-          // (normalising takes it out), and where both are one; the general
-          // form at an outer edge, with the smaller aperture in its soft band,
-          // and where the sine vanishes.
-          const bool both = far >= d_in;
-          const bool general = (fabsf(near) < margin) | ((far > -margin) & (far < d_in)) | (both & (s == floorf(s)));
-          float2 z = overlap_unit(G, both, s, t, __float_as_uint(B) & 0x80000000u);
-          if (general) {
-            df dn{near, 0.0f}, dfar{far, 0.0f};
-            if ((fabsf(near) < kApMargin) | (fabsf(far) < kApMargin)) {
-              const df qx = df_in_branch(df{qxf, ds.qxl[q]}), qy = df_in_branch(df{qyf, ds.qyl[c]});
-              const df kx{0.5f * kx2[i], km[i].kxl}, ky{0.5f * ky2[i], km[i].kyl};
-              df qk2 = df_mul(df_add(df_mul(qx, kx), df_mul(qy, ky)), df{2.0f, 0.0f});
-              if (B < 0.0f) qk2 = df_neg(qk2);
-              const df bd = df_sub(df{km[i].cb, km[i].cbl}, df_add(df_mul(qx, qx), df_mul(qy, qy)));
-              dn = df_add(bd, qk2);
-              dfar = df_sub(bd, qk2);
-            }
-            float2 g = gamma_hat_st(km[i].ak, aperture_from_d(dn, ds.ap), aperture_from_d(dfar, ds.ap), s, t);
-            if (B < 0.0f) g.x = -g.x;
-            z = mul_conj(G, g);
-          }
+          const float2 z = overlap_term(G, near, far, B, s, t, margin, km[i].ak, ds.ap, [&](df& dm, df& dp) {
+            exact_d(df{qxf, ds.qxl[q]}, df{qyf, ds.qyl[c]}, df{0.5f * kx2[i], km[i].kxl}, df{0.5f * ky2[i], km[i].kyl},
+                    df{km[i].cb, km[i].cbl}, dm, dp);
+          });
           ar[i].add(z.x);
           ai[i].add(z.y);
         }
