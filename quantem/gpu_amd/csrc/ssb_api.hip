@@ -521,9 +521,7 @@ static int prepare_g_typed(ssb_plan* p, const void* data, int dtype, void* strea
   HIP_TRY(launch_gather_rowfft(p->n, dtype, data, p->D, p->det_cols, p->bf_rows, p->bf_cols, p->info, p->nbf_hint,
                                p->tw, p->tune_gather_pairs, p->gain, p->H, s),
           "gather_rowfft");
-  HIP_TRY(launch_trotter_slots(p->n, true, p->H, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics, p->tw,
-                               p->S_part, p->Gt, false, p->tune_trotter, s),
-          "colfft");
+  HIP_TRY(launch_columns_store(p->n, p->H, p->info, geom_ptrs(p), p->tw, p->Gt, s), "colfft");
   p->gcols = p->n / 2 + 1;
   p->g_nbf = p->nbf_hint;
   return QSSB_OK;
@@ -571,6 +569,13 @@ int ssb_import_g(ssb_plan* p, const void* g_in, int nbf, int gcols, void* stream
   return QSSB_OK;
 }
 
+// The quadratic chi in half turns.
+static QuadTurns quad_turns(const ssb_plan* p, double c10, double c12, double phi12) {
+  const double lam = p->wavelength;
+  return QuadTurns{(float)(lam * c10), (float)(lam * c12 * std::cos(2.0 * phi12)),
+                   (float)(lam * c12 * std::sin(2.0 * phi12))};
+}
+
 int ssb_object(ssb_plan* p, double c10, double c12, double phi12, void* obj_out, float* phase_out, void* stream) {
   int rc = check_plan(p);
   if (rc) return rc;
@@ -581,11 +586,17 @@ int ssb_object(ssb_plan* p, double c10, double c12, double phi12, void* obj_out,
     if (rc) return rc;
   }
   const QuadChi m = quad_chi(p, c10, c12, phi12);
-  HIP_TRY(launch_phasors(p->n, p->info, p->nbf_hint, geom_ptrs(p), m, p->rowph, p->colph, p->echi, s), "phasors");
   int groups = object_groups(p->n);
-  if (p->gcols == p->n / 2 + 1) {
+  const bool tiles = p->gcols == p->n / 2 + 1 && optics_isotropic(p->optics);
+  if (!tiles)
+    HIP_TRY(launch_phasors(p->n, p->info, p->nbf_hint, geom_ptrs(p), m, p->rowph, p->colph, p->echi, s), "phasors");
+  if (tiles) {
+    HIP_TRY(launch_object_tiles(p->n, p->Gt, p->info, geom_ptrs(p), quad_turns(p, c10, c12, phi12), p->optics, p->S_part,
+                                s, &groups),
+            "trotter");
+  } else if (p->gcols == p->n / 2 + 1) {
     HIP_TRY(launch_trotter_slots(p->n, false, p->Gt, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics, p->tw,
-                                 p->S_part, nullptr, true, 0, s, &groups),
+                                 p->S_part, 0, s, &groups),
             "trotter");
   } else {
     HIP_TRY(launch_trotter_full(p->n, p->Gt, p->info, geom_ptrs(p), p->rowph, m, p->optics, p->S_part, s),
@@ -1103,8 +1114,9 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
   // than one pass, so one pass is the default.  Stage marks with the split:
   // 5 -> 6 the first half's gather and the phasors, 6 -> 7 both trotters
   // and the second gather.
-  const bool two = p->tune_split == 1 &&
-                   trotter_wave_path(p->n, true, p->optics, true, false, p->tune_trotter);
+  const bool columns = columns_path(p->n, p->optics);
+  const QuadTurns turns = quad_turns(p, c10, c12, phi12);
+  const bool two = p->tune_split == 1 && trotter_wave_path(p->n, true, p->optics, p->tune_trotter);
   if (two) {
     if (!p->pstream) HIP_TRY(hipStreamCreateWithFlags(&p->pstream, hipStreamNonBlocking), "second stream");
     if (!p->pev_a) HIP_TRY(hipEventCreateWithFlags(&p->pev_a, hipEventDisableTiming), "split event");
@@ -1124,25 +1136,31 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
             "phasors");
     mark(6);
     HIP_TRY(launch_trotter_slots(p->n, true, p->H, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics,
-                                 p->tw, p->S_part, nullptr, true, p->tune_trotter, s, &groups, 0, 2),
+                                 p->tw, p->S_part, p->tune_trotter, s, &groups, 0, 2),
             "colfft_trotter");
     HIP_TRY(hipStreamWaitEvent(s, p->pev_b, 0), "split wait");
     HIP_TRY(launch_trotter_slots(p->n, true, p->H, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics,
-                                 p->tw, p->S_part, nullptr, true, p->tune_trotter, s, &groups, 1, 2),
+                                 p->tw, p->S_part, p->tune_trotter, s, &groups, 1, 2),
             "colfft_trotter");
   } else {
-    // The gather's threads also write the phasor tables (one launch fewer;
-    // geometry and phasors on a second stream beside the gather measured
-    // slower: the cross-stream event pair costs more than they would hide).
+    // The gather's threads also write the phasor tables, where the trotter
+    // reads them (one launch fewer; geometry and phasors on a second stream
+    // beside the gather measured slower: the cross-stream event pair costs
+    // more than they would hide).
     const PhasorJob job{p->info, geom_ptrs(p), m, p->n, p->rowph, p->colph, p->echi};
     HIP_TRY(launch_gather_rowfft(p->n, dtype, data, p->D, p->det_cols, p->bf_rows, p->bf_cols, p->info,
                                  p->nbf_hint, p->tw, p->tune_gather_pairs, p->gain, p->H, s,
-                                 sup ? p->sup_box : nullptr, sup ? p->sup_C : nullptr, 0, 1, &job),
+                                 sup ? p->sup_box : nullptr, sup ? p->sup_C : nullptr, 0, 1, columns ? nullptr : &job),
             "gather_rowfft");
     mark(6);
-    HIP_TRY(launch_trotter_slots(p->n, true, p->H, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics,
-                                 p->tw, p->S_part, nullptr, true, p->tune_trotter, s, &groups),
-            "colfft_trotter");
+    if (columns)
+      HIP_TRY(launch_columns_trotter(p->n, p->H, p->info, geom_ptrs(p), turns, p->optics, p->tw, p->S_part,
+                                     p->tune_trotter, s, &groups),
+              "colfft_trotter");
+    else
+      HIP_TRY(launch_trotter_slots(p->n, true, p->H, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics,
+                                   p->tw, p->S_part, p->tune_trotter, s, &groups),
+              "colfft_trotter");
   }
   mark(7);
   HIP_TRY(launch_finish_object(p->n, p->S_part, groups, p->info, p->tw, p->S,

@@ -26,6 +26,63 @@ __device__ __forceinline__ float2 cmul_mi(float2 a) {
   return INV ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
 }
 
+// R-point DFT in registers, R = 2, 4, 8 or 16, in place and in natural order.
+template <bool INV>
+__device__ __forceinline__ void dft4(float2 a, float2 b, float2 c, float2 d, float2 (&y)[4]) {
+  const float2 apc = cadd(a, c), amc = csub(a, c);
+  const float2 bpd = cadd(b, d), bmd = cmul_mi<INV>(csub(b, d));
+  y[0] = cadd(apc, bpd);
+  y[1] = cadd(amc, bmd);
+  y[2] = csub(apc, bpd);
+  y[3] = csub(amc, bmd);
+}
+
+template <int R, bool INV>
+__device__ __forceinline__ void dft_regs(float2 (&x)[R]) {
+  static_assert(R == 2 || R == 4 || R == 8 || R == 16, "radix");
+  if constexpr (R == 2) {
+    const float2 a = x[0], b = x[1];
+    x[0] = cadd(a, b);
+    x[1] = csub(a, b);
+  } else if constexpr (R == 4) {
+    float2 y[4];
+    dft4<INV>(x[0], x[1], x[2], x[3], y);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = y[k];
+  } else {
+    // R = 4 Q: Q-strided radix 4, twiddles e^{+-2 pi i k j / R}, radix Q
+    constexpr int Q = R / 4;
+    float2 z[Q][4];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) dft4<INV>(x[j], x[j + Q], x[j + 2 * Q], x[j + 3 * Q], z[j]);
+#pragma unroll
+    for (int j = 1; j < Q; ++j)
+#pragma unroll
+      for (int k = 1; k < 4; ++k) {
+        constexpr float c16[5] = {1.0f, 0.92387953251128676f, 0.70710678118654752f, 0.38268343236508977f, 0.0f};
+        const int t = k * j * (16 / R);   // sixteenths of a turn, up to 9
+        auto cosine = [&](int v) {
+          v &= 15;
+          v = v > 8 ? 16 - v : v;
+          return v > 4 ? -c16[8 - v] : c16[v];
+        };
+        z[j][k] = cmul(z[j][k], make_float2(cosine(t), INV ? cosine(t + 12) : cosine(t + 4)));
+      }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (Q == 2) {
+        x[k] = cadd(z[0][k], z[1][k]);
+        x[k + 4] = csub(z[0][k], z[1][k]);
+      } else {
+        float2 y[4];
+        dft4<INV>(z[0][k], z[1][k], z[2][k], z[3][k], y);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[k + 4 * j] = y[j];
+      }
+    }
+  }
+}
+
 // Kahan-compensated FP32 accumulator (one real component).
 struct Kahan {
   float s, c;

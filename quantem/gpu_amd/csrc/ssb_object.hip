@@ -44,8 +44,7 @@ __global__ void __launch_bounds__(BLOCK)
 k_trotter_slots(const float2* __restrict__ src, const BfInfo* __restrict__ info, GeomPtrs gp,
                 const float2* __restrict__ rowph_g, const float2* __restrict__ colph_g,
                 const float2* __restrict__ echi_g, ApIso ap, df rout2, Optics o,
-                const float2* __restrict__ tw_g, int groups, float2* __restrict__ S_part, float2* __restrict__ Gt,
-                int do_trotter) {
+                const float2* __restrict__ tw_g, int groups, float2* __restrict__ S_part) {
   constexpr int HALF = N / 2;
   constexpr int NSG = HALF / SG;
   constexpr int P = SG * N / BLOCK;      // points per thread
@@ -141,17 +140,15 @@ k_trotter_slots(const float2* __restrict__ src, const BfInfo* __restrict__ info,
       qyS[tid] = gp.qy[col];
       qySl[tid] = gp.qyl[col];
     }
-    if (do_trotter) {
-      if (sg == 0 && tid < N) {
-        const df qx{gp.qx[tid], gp.qxl[tid]};
-        const df qh{gp.qy[HALF], gp.qyl[HALF]};   // not qyS: written in this same phase
-        if (!ISO) q2halfc[tid] = df_add(df_mul(qx, qx), df_mul(qh, qh));
-        ehalfc[tid] = echi_g[(long long)HALF * N + tid];
-      }
-      if (tid < SG) {
-        const int j = sg * SG + tid;
-        enyqr[tid] = echi_g[(long long)((N - j) & (N - 1)) * N + HALF];
-      }
+    if (sg == 0 && tid < N) {
+      const df qx{gp.qx[tid], gp.qxl[tid]};
+      const df qh{gp.qy[HALF], gp.qyl[HALF]};   // not qyS: written in this same phase
+      if (!ISO) q2halfc[tid] = df_add(df_mul(qx, qx), df_mul(qh, qh));
+      ehalfc[tid] = echi_g[(long long)HALF * N + tid];
+    }
+    if (tid < SG) {
+      const int j = sg * SG + tid;
+      enyqr[tid] = echi_g[(long long)((N - j) & (N - 1)) * N + HALF];
     }
     __syncthreads();
     // per-point constants
@@ -179,15 +176,11 @@ k_trotter_slots(const float2* __restrict__ src, const BfInfo* __restrict__ info,
       const float kxh = gp.kx[b], kyh = gp.ky[b];
       const df kx{kxh, gp.kxl[b]}, ky{kyh, gp.kyl[b]};
       const float ak = gp.ak[b];
-      float2 rowA = make_float2(1.f, 0.f);
+      const float2 rowA = rowph_g[(long long)b * N + q];
       float2 colp[P];
-      float2 colHalf = make_float2(1.f, 0.f);
-      if (do_trotter) {
-        rowA = rowph_g[(long long)b * N + q];
 #pragma unroll
-        for (int i = 0; i < P; ++i) colp[i] = colph_g[(long long)b * GCOLS + sg * SG + s0 + i * SSTEP];
-        colHalf = colph_g[(long long)b * GCOLS + HALF];
-      }
+      for (int i = 0; i < P; ++i) colp[i] = colph_g[(long long)b * GCOLS + sg * SG + s0 + i * SSTEP];
+      const float2 colHalf = colph_g[(long long)b * GCOLS + HALF];
       float2 gHalf = make_float2(0.f, 0.f);
       if (!FROM_H && sg == 0) gHalf = src[((long long)b * GCOLS + HALF) * N + q];
       asm volatile("" ::: "memory");
@@ -196,25 +189,6 @@ k_trotter_slots(const float2* __restrict__ src, const BfInfo* __restrict__ info,
       if (FROM_H) fft_lds_il<N, SG, BLOCK, TSTRIDE, false>(abuf[cur], tileT, tw);
       const float2* tile = FROM_H ? tileT : abuf[cur];
       constexpr int TS = FROM_H ? TSTRIDE : N;
-      if (!do_trotter) {
-        if (Gt) {
-          float2* gb = Gt + (long long)b * GCOLS * N;
-#pragma unroll
-          for (int i = 0; i < P; ++i) {
-            const int s = s0 + i * SSTEP;
-            const int j = sg * SG + s;
-            const float2 z = tile[s * TS + q];
-            if (j == 0) {
-              const float2 zm = tile[s * TS + qm];
-              gb[q] = make_float2(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y));
-              gb[(long long)HALF * N + q] = make_float2(0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x));
-            } else {
-              gb[(long long)j * N + q] = z;
-            }
-          }
-        }
-        continue;
-      }
       // ISO row terms of d(Q -/+ k), -qx^2 +/- 2 qx kx, as float32 estimates
       // (the double-float terms are formed only for points near the soft edge)
       const df kx2{2.0f * kx.hi, 2.0f * kx.lo};
@@ -303,30 +277,23 @@ k_trotter_slots(const float2* __restrict__ src, const BfInfo* __restrict__ info,
             aiB[i].add(GB.y * gr - GB.x * gi);
           }
         }
-        if (Gt) {
-          float2* gb = Gt + (long long)b * GCOLS * N;
-          gb[(long long)j * N + q] = GA;
-          if (j == 0) gb[(long long)HALF * N + q] = GB;
-        }
         // one point at a time: keeps the scheduler from overlapping the
         // points' temporaries, which would spill the accumulators
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (do_trotter) {
-      float2* sp = S_part + (long long)g * N * N;
+    float2* sp = S_part + (long long)g * N * N;
 #pragma unroll
-      for (int i = 0; i < P; ++i) {
-        const int s = s0 + i * SSTEP;
-        const int j = sg * SG + s;
-        const int colB = (j == 0) ? HALF : N - j;
-        const int rowB = (j == 0) ? q : qm;
-        const float2 outA = make_float2(arA[i].s - arA[i].c, aiA[i].s - aiA[i].c);
-        const bool mirror = (j != 0) && (q != HALF);
-        sp[(long long)j * N + q] = outA;
-        sp[(long long)colB * N + rowB] =
-            mirror ? make_float2(-outA.x, outA.y) : make_float2(arB[i].s - arB[i].c, aiB[i].s - aiB[i].c);
-      }
+    for (int i = 0; i < P; ++i) {
+      const int s = s0 + i * SSTEP;
+      const int j = sg * SG + s;
+      const int colB = (j == 0) ? HALF : N - j;
+      const int rowB = (j == 0) ? q : qm;
+      const float2 outA = make_float2(arA[i].s - arA[i].c, aiA[i].s - aiA[i].c);
+      const bool mirror = (j != 0) && (q != HALF);
+      sp[(long long)j * N + q] = outA;
+      sp[(long long)colB * N + rowB] =
+          mirror ? make_float2(-outA.x, outA.y) : make_float2(arB[i].s - arB[i].c, aiB[i].s - aiB[i].c);
     }
   }
 }
@@ -1007,26 +974,32 @@ hipError_t launch_phasors(int N, const BfInfo* info, int nbf_hint, const GeomPtr
 // At N = 256 variants 0 and 1 are the wave-local kernel (the object path of
 // a reconstruction: row-transformed stack, isotropic sampling) with
 // kWaveColumnsDefault columns per wave and with the other count, and 2..4
-// are the workgroup-tile shapes below; elsewhere the tile shapes only.
-int trotter_variants(int N) { return N == 1024 ? 1 : (N == 256 ? 5 : 3); }
+// are the workgroup-tile shapes below; at N = 128 the tile shapes only.
+// From N = 512 on equal sampling goes through ssb_columns.hip (columns_path),
+// whose variants are numbers of BF groups.
+int trotter_variants(int N) { return N >= 512 ? columns_variants(N) : (N == 256 ? 5 : 3); }
 
 static int wave_columns(int variant) { return variant == 0 ? kWaveColumnsDefault : 3 - kWaveColumnsDefault; }
 
-int trotter_groups_max(int N) { return N == 256 ? kWaveTrotterGroups : object_groups(N); }
+int trotter_groups_max(int N) {
+  int g = N == 256 ? kWaveTrotterGroups : object_groups(N);
+  g = object_tile_groups(N) > g ? object_tile_groups(N) : g;
+  for (int v = 0; N >= 512 && v < columns_variants(N); ++v) g = columns_groups(N, v) > g ? columns_groups(N, v) : g;
+  return g;
+}
 
-bool trotter_wave_path(int N, bool from_h, const Optics& o, bool do_trotter, bool has_gt, int variant) {
-  return N == 256 && from_h && optics_isotropic(o) && do_trotter && !has_gt && (variant == 0 || variant == 1);
+bool trotter_wave_path(int N, bool from_h, const Optics& o, int variant) {
+  return N == 256 && from_h && optics_isotropic(o) && (variant == 0 || variant == 1);
 }
 
 hipError_t launch_trotter_slots(int N, bool from_h, const float2* src, const BfInfo* info, const GeomPtrs& gp,
                                 const float2* rowph, const float2* colph, const float2* echi, const Optics& o,
-                                const float2* tw, float2* S_part, float2* Gt, bool do_trotter, int variant,
-                                hipStream_t s, int* groups_used, int part, int parts) {
+                                const float2* tw, float2* S_part, int variant, hipStream_t s, int* groups_used,
+                                int part, int parts) {
   df rout2;
   const ApIso ap = iso_aperture(o, rout2);
-  const int dt = do_trotter ? 1 : 0;
   const bool iso = optics_isotropic(o);
-  if (trotter_wave_path(N, from_h, o, do_trotter, Gt != nullptr, variant)) {
+  if (trotter_wave_path(N, from_h, o, variant)) {
     constexpr int groups = kWaveTrotterGroups;
     // (the item order gives each XCD groups / parts / 8 BF groups)
     if (parts < 1 || part < 0 || part >= parts || groups % (8 * parts)) return hipErrorInvalidValue;
@@ -1047,59 +1020,53 @@ hipError_t launch_trotter_slots(int N, bool from_h, const float2* src, const BfI
   if (parts != 1) return hipErrorInvalidValue;
   // workgroup-tile shapes: at N = 256 their variants follow the wave-local ones
   if (N == 256 && variant > 0) variant = variant >= 2 ? variant - 2 : 0;
-  // a resident stack at N = 256: 32 BF groups (2048 items, two rounds of four
-  // workgroups per CU, so the heavy-first order can even out the CUs)
-  const int groups = (!from_h && N == 256) ? 2 * object_groups(N) : object_groups(N);
+  if (iso && (!from_h || N >= 512)) return hipErrorInvalidValue;   // ssb_columns.hip's
+  const int groups = object_groups(N);
   if (groups_used) *groups_used = groups;
 #define QSSB_SLOTS_ONE(NN, SGV, BL, FH, IS)                                                                 \
   hipLaunchKernelGGL((k_trotter_slots<NN, SGV, BL, FH, IS>), dim3(grid), dim3(BL), 0, s, src, info, gp, rowph, \
-                     colph, echi, ap, rout2, o, tw, groups, S_part, Gt, dt)
+                     colph, echi, ap, rout2, o, tw, groups, S_part)
 #define QSSB_SLOTS(NN, SGV, BL)                                                                \
   do {                                                                                        \
     const unsigned grid = grid_items((long long)groups * ((NN / 2) / SGV), 65536);            \
-    if (from_h && iso) QSSB_SLOTS_ONE(NN, SGV, BL, true, true);                               \
-    else if (from_h) QSSB_SLOTS_ONE(NN, SGV, BL, true, false);                                \
-    else if (iso) QSSB_SLOTS_ONE(NN, SGV, BL, false, true);                                   \
+    if (from_h) QSSB_SLOTS_ONE(NN, SGV, BL, true, false);                                     \
     else QSSB_SLOTS_ONE(NN, SGV, BL, false, false);                                           \
   } while (0)
-#define QSSB_SLOTS_TUNED(NN, SGV, BL)                                                          \
+#define QSSB_SLOTS_ISO(NN, SGV, BL)                                                            \
   do {                                                                                        \
     const unsigned grid = grid_items((long long)groups * ((NN / 2) / SGV), 65536);            \
     QSSB_SLOTS_ONE(NN, SGV, BL, true, true);                                                  \
   } while (0)
-  const bool tuned = from_h && iso && variant > 0;
   switch (N) {
     case 128:
-      if (tuned && variant == 1) QSSB_SLOTS_TUNED(128, 2, 256);
-      else if (tuned && variant == 2) QSSB_SLOTS_TUNED(128, 8, 256);
+      if (iso && variant == 1) QSSB_SLOTS_ISO(128, 2, 256);
+      else if (iso && variant == 2) QSSB_SLOTS_ISO(128, 8, 256);
+      else if (iso) QSSB_SLOTS_ISO(128, 4, 256);
       else QSSB_SLOTS(128, 4, 256);
       break;
     case 256:
-      if (tuned && variant == 1) QSSB_SLOTS_TUNED(256, 4, 256);
-      else if (tuned && variant == 2) QSSB_SLOTS_TUNED(256, 2, 512);
+      if (iso && variant == 1) QSSB_SLOTS_ISO(256, 4, 256);
+      else if (iso && variant == 2) QSSB_SLOTS_ISO(256, 2, 512);
+      else if (iso) QSSB_SLOTS_ISO(256, 2, 256);
       else QSSB_SLOTS(256, 2, 256);
       break;
     case 512:
-      if (tuned && variant == 1) QSSB_SLOTS_TUNED(512, 2, 1024);
-      else if (tuned && variant == 2) QSSB_SLOTS_TUNED(512, 4, 512);
-      else QSSB_SLOTS(512, 2, 512);
+      QSSB_SLOTS(512, 2, 512);
       break;
     case 1024:
       if (from_h) {
         // one slot per tile would split the 16-byte staging copies across rows
         const unsigned grid = grid_items((long long)groups * ((1024 / 2) / 2), 65536);
-        if (iso) QSSB_SLOTS_ONE(1024, 2, 1024, true, true);
-        else QSSB_SLOTS_ONE(1024, 2, 1024, true, false);
+        QSSB_SLOTS_ONE(1024, 2, 1024, true, false);
       } else {
         const unsigned grid = grid_items((long long)groups * ((1024 / 2) / 1), 65536);
-        if (iso) QSSB_SLOTS_ONE(1024, 1, 1024, false, true);
-        else QSSB_SLOTS_ONE(1024, 1, 1024, false, false);
+        QSSB_SLOTS_ONE(1024, 1, 1024, false, false);
       }
       break;
     default:
       return hipErrorInvalidValue;
   }
-#undef QSSB_SLOTS_TUNED
+#undef QSSB_SLOTS_ISO
 #undef QSSB_SLOTS
 #undef QSSB_SLOTS_ONE
   return hipGetLastError();

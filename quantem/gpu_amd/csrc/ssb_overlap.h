@@ -232,6 +232,37 @@ __device__ __forceinline__ void exact_d(df qx, df qy, df kx, df ky, df cb, df& d
   dp = df_sub(base, qk2);
 }
 
+// What the terms of one BF pixel share under a quadratic chi: 2 k, Rout^2 -
+// |k|^2, t as a linear form of q, the margin of overlap_term and A(k).  reach:
+// |u|^2 up to which an aperture or its margin can be met (kReach above Rout^2).
+struct QuadPixel {
+  float kx2, ky2, cb, tx, ty, margin, ak;
+};
+constexpr float kReachRel = 1.00002f, kReachAbs = 3e-4f;
+
+__device__ __forceinline__ QuadPixel quad_pixel(const GeomPtrs& gp, int b, const QuadTurns& ev, df rout2) {
+  QuadPixel p;
+  const df kx{gp.kx[b], gp.kxl[b]}, ky{gp.ky[b], gp.kyl[b]};
+  p.kx2 = 2.0f * kx.hi;
+  p.ky2 = 2.0f * ky.hi;
+  p.cb = df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky))).hi;
+  p.tx = fmaf(ev.k0 + ev.m12c, p.kx2, ev.m12s * p.ky2);
+  p.ty = fmaf(ev.k0 - ev.m12c, p.ky2, ev.m12s * p.kx2);
+  p.ak = gp.ak[b];
+  p.margin = edge_margin(p.ak);
+  return p;
+}
+
+// Whether the apertures around k and -k can reach the frequencies
+// [x0, x1] x [y0, y1].
+__device__ __forceinline__ bool apertures_reach(const QuadPixel& p, float rout2, float x0, float x1, float y0,
+                                                float y1) {
+  const float kx = 0.5f * p.kx2, ky = 0.5f * p.ky2;
+  const float ax = fmaxf(fmaxf(x0 - kx, kx - x1), 0.0f), ay = fmaxf(fmaxf(y0 - ky, ky - y1), 0.0f);
+  const float bx = fmaxf(fmaxf(x0 + kx, -kx - x1), 0.0f), by = fmaxf(fmaxf(y0 + ky, -ky - y1), 0.0f);
+  return p.ak != 0.0f && fminf(fmaf(ax, ax, ay * ay), fmaf(bx, bx, by * by)) < fmaf(rout2, kReachRel, kReachAbs);
+}
+
 // chi(u) split into its even part E and odd part O (ChiPoly).
 __device__ __forceinline__ void chi_parts(const ChiPoly& cp, float ux, float uy, float& E, float& O) {
   const float r2 = ux * ux + uy * uy;

@@ -79,65 +79,11 @@ struct WaveIfft {
     return ((lane >> 4) + 4 * p) % R + R * (lane & 15) + 16 * R * r;
   }
 
-  __device__ static __forceinline__ void radix4(float2 a, float2 b, float2 c, float2 d, float2 (&y)[4]) {
-    const float2 apc = cadd(a, c), amc = csub(a, c);
-    const float2 bpd = cadd(b, d), bmd = cmul_mi<true>(csub(b, d));
-    y[0] = cadd(apc, bpd);
-    y[1] = cadd(amc, bmd);
-    y[2] = csub(apc, bpd);
-    y[3] = csub(amc, bmd);
-  }
-
-  // inverse R-point DFT in place
-  __device__ static __forceinline__ void dft(float2 (&x)[R]) {
-    if constexpr (R == 2) {
-      const float2 a = x[0], b = x[1];
-      x[0] = cadd(a, b);
-      x[1] = csub(a, b);
-    } else if constexpr (R == 4) {
-      float2 y[4];
-      radix4(x[0], x[1], x[2], x[3], y);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) x[k] = y[k];
-    } else {
-      // R = 4 Q: Q-strided radix 4, twiddles e^{2 pi i k j / R}, radix Q
-      constexpr int Q = R / 4;
-      float2 z[Q][4];
-#pragma unroll
-      for (int j = 0; j < Q; ++j) radix4(x[j], x[j + Q], x[j + 2 * Q], x[j + 3 * Q], z[j]);
-#pragma unroll
-      for (int j = 1; j < Q; ++j)
-#pragma unroll
-        for (int k = 1; k < 4; ++k) {
-          constexpr float c16[5] = {1.0f, 0.92387953251128676f, 0.70710678118654752f, 0.38268343236508977f, 0.0f};
-          const int t = k * j * (16 / R);   // sixteenths of a turn, up to 9
-          auto cosine = [&](int v) {
-            v &= 15;
-            v = v > 8 ? 16 - v : v;
-            return v > 4 ? -c16[8 - v] : c16[v];
-          };
-          z[j][k] = cmul(z[j][k], make_float2(cosine(t), cosine(t + 12)));
-        }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if constexpr (Q == 2) {
-          x[k] = cadd(z[0][k], z[1][k]);
-          x[k + 4] = csub(z[0][k], z[1][k]);
-        } else {
-          float2 y[4];
-          radix4(z[0][k], z[1][k], z[2][k], z[3][k], y);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) x[k + 4 * j] = y[j];
-        }
-      }
-    }
-  }
-
   __device__ __forceinline__ void run(float2 (&x)[S][R], float2* __restrict__ xb, int lane, float2 (&o)[P][4]) const {
     wave_fence();
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      dft(x[s]);
+      dft_regs<R, true>(x[s]);
       xb[(s * R) * SP + lane] = x[s][0];
 #pragma unroll
       for (int k = 1; k < R; ++k) xb[(s * R + k) * SP + lane] = cmul(x[s][k], w1[k]);
@@ -160,7 +106,7 @@ struct WaveIfft {
       wave_fence();
 #pragma unroll
       for (int p = 0; p < P; ++p) {
-        radix4(v[p][0], v[p][1], v[p][2], v[p][3], o[p]);
+        dft4<true>(v[p][0], v[p][1], v[p][2], v[p][3], o[p]);
         if (ns < 16) {
           const int base = ((lane >> 4) + 4 * p) * SP + (jj / ns) * ns * 4 + k;
 #pragma unroll
