@@ -17,6 +17,7 @@
 #ifndef QUANTEM_SSB_H
 #define QUANTEM_SSB_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
@@ -168,6 +169,21 @@ const char* ssb_last_error(void);
 int ssb_plan_create(int scan_n, int det_rows, int det_cols, int max_bf, double wavelength_A,
                     double semiangle_rad, double ang_row_rad, double ang_col_rad,
                     double scan_sampling_row_A, double scan_sampling_col_A, ssb_plan** plan);
+
+/*
+ * The same with the caller's device memory: alloc(bytes, stream, ctx) returns
+ * memory of the current device, ordered like work on `stream` (NULL: none
+ * left); release(ptr, ctx) takes it back, called with the plan's device idle.
+ * Both may be called from any thread that calls into the plan, until
+ * ssb_plan_destroy has returned.  Blocks above 1 GiB come from the device
+ * itself.  `stream` orders the creation's uploads; the call waits for it.
+ */
+typedef void* (*ssb_alloc_fn)(size_t bytes, void* stream, void* ctx);
+typedef void (*ssb_release_fn)(void* ptr, void* ctx);
+int ssb_plan_create_with(int scan_n, int det_rows, int det_cols, int max_bf, double wavelength_A,
+                         double semiangle_rad, double ang_row_rad, double ang_col_rad,
+                         double scan_sampling_row_A, double scan_sampling_col_A, ssb_alloc_fn alloc,
+                         ssb_release_fn release, void* ctx, void* stream, ssb_plan** plan);
 
 /*
  * Override the detector reciprocal sampling (1/Angstrom per pixel) used for

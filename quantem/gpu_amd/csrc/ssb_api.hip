@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../../include/quantem_ssb.h"
@@ -49,6 +50,43 @@ hipError_t dmalloc(T** p, size_t count) {
 
 void dfree(void* p) {
   if (p) (void)hipFree(p);
+}
+
+// A plan's buffers: the caller's memory up to kLentBytes a block, which caps
+// what a plan leaves in a caller's cache when it goes, else the device's, and
+// the caller's after all (who may empty that cache) when the device has none left.
+constexpr size_t kLentBytes = (size_t)1 << 30;
+
+template <typename T>
+hipError_t palloc(ssb_plan* p, T** out, size_t count, hipStream_t s) {
+  const size_t bytes = count * sizeof(T) > 0 ? count * sizeof(T) : 1;
+  hipError_t e = hipErrorOutOfMemory;
+  if (!p->alloc || bytes > kLentBytes) e = hipMalloc(reinterpret_cast<void**>(out), bytes);
+  if (e != hipErrorOutOfMemory || !p->alloc) return e;
+  (void)hipGetLastError();
+  for (void*& slot : p->lent) {
+    if (slot) continue;
+    void* q = p->alloc(bytes, s, p->alloc_ctx);
+    if (!q) return hipErrorOutOfMemory;
+    slot = q;
+    *out = reinterpret_cast<T*>(q);
+    return hipSuccess;
+  }
+  return hipErrorOutOfMemory;   // (a plan has fewer buffers than slots)
+}
+
+// Like hipFree it waits for the device: work on any stream may use the block,
+// and the caller's memory is ordered on one stream only.
+void pfree(ssb_plan* p, void* q) {
+  if (!q) return;
+  for (void*& slot : p->lent) {
+    if (slot != q) continue;
+    slot = nullptr;
+    (void)hipDeviceSynchronize();
+    p->release(q, p->alloc_ctx);
+    return;
+  }
+  (void)hipFree(q);
 }
 
 hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
@@ -131,6 +169,15 @@ const char* ssb_last_error(void) { return g_last_error.c_str(); }
 int ssb_plan_create(int scan_n, int det_rows, int det_cols, int max_bf, double wavelength_A,
                     double semiangle_rad, double ang_row_rad, double ang_col_rad, double scan_sampling_row_A,
                     double scan_sampling_col_A, ssb_plan** out) {
+  return ssb_plan_create_with(scan_n, det_rows, det_cols, max_bf, wavelength_A, semiangle_rad, ang_row_rad,
+                              ang_col_rad, scan_sampling_row_A, scan_sampling_col_A, nullptr, nullptr, nullptr,
+                              nullptr, out);
+}
+
+int ssb_plan_create_with(int scan_n, int det_rows, int det_cols, int max_bf, double wavelength_A,
+                         double semiangle_rad, double ang_row_rad, double ang_col_rad, double scan_sampling_row_A,
+                         double scan_sampling_col_A, ssb_alloc_fn alloc, ssb_release_fn release, void* ctx,
+                         void* stream, ssb_plan** out) {
   g_last_error.clear();
   if (!out) return fail(QSSB_ERR_ARG, "plan output pointer is NULL");
   *out = nullptr;
@@ -144,7 +191,11 @@ int ssb_plan_create(int scan_n, int det_rows, int det_cols, int max_bf, double w
   if (!(wavelength_A > 0) || !(semiangle_rad > 0) || !(ang_row_rad > 0) || !(ang_col_rad > 0) ||
       !(scan_sampling_row_A > 0) || !(scan_sampling_col_A > 0))
     return fail(QSSB_ERR_ARG, "optics and sampling must be positive");
+  if (!alloc != !release) return fail(QSSB_ERR_ARG, "alloc and release come together");
   ssb_plan* p = new ssb_plan();
+  p->alloc = alloc;
+  p->release = release;
+  p->alloc_ctx = ctx;
   p->n = scan_n;
   p->det_rows = det_rows;
   p->det_cols = det_cols;
@@ -182,35 +233,53 @@ int ssb_plan_create(int scan_n, int det_rows, int det_cols, int max_bf, double w
     o.angx = to_df(ang_col_rad);
   }
   const int n = scan_n;
-  hipError_t e = hipSuccess;
-  if (e == hipSuccess) e = dmalloc(&p->dp_partial, (size_t)p->max_ranges * p->D);
-  if (e == hipSuccess) e = dmalloc(&p->dp_sums, (size_t)p->D);
-  if (e == hipSuccess) e = dmalloc(&p->dp_mean, (size_t)p->D);
-  if (e == hipSuccess) e = dmalloc(&p->dp_dcpix, (size_t)p->D);
-  if (e == hipSuccess) e = dmalloc(&p->bf_rows, (size_t)max_bf);
-  if (e == hipSuccess) e = dmalloc(&p->bf_cols, (size_t)max_bf);
-  if (e == hipSuccess) e = dmalloc(&p->info, 1);
-  if (e == hipSuccess) e = dmalloc(&p->kx, (size_t)max_bf);
-  if (e == hipSuccess) e = dmalloc(&p->kxl, (size_t)max_bf);
-  if (e == hipSuccess) e = dmalloc(&p->ky, (size_t)max_bf);
-  if (e == hipSuccess) e = dmalloc(&p->kyl, (size_t)max_bf);
-  if (e == hipSuccess) e = dmalloc(&p->ak, (size_t)max_bf);
-  if (e == hipSuccess) e = dmalloc(&p->qx, (size_t)n);
-  if (e == hipSuccess) e = dmalloc(&p->qxl, (size_t)n);
-  if (e == hipSuccess) e = dmalloc(&p->qy, (size_t)n);
-  if (e == hipSuccess) e = dmalloc(&p->qyl, (size_t)n);
-  if (e == hipSuccess) e = dmalloc(&p->tw, (size_t)n);
-  if (e == hipSuccess) e = dmalloc(&p->S_part, (size_t)p->max_groups * n * n);
-  if (e == hipSuccess) e = dmalloc(&p->S, (size_t)n * n);
-  if (e == hipSuccess) e = dmalloc(&p->rowph, (size_t)max_bf * n);
-  if (e == hipSuccess) e = dmalloc(&p->colph, (size_t)max_bf * (n / 2 + 1));
-  if (e == hipSuccess) e = dmalloc(&p->echi, (size_t)n * n);
+  // one block for what every plan has, the uploaded tables first: an
+  // allocation and a free cost 20 and 60 us, an upload 20
+  auto layout = [&](char* base) {
+    size_t at = 0;
+    auto part = [&](auto** ptr, size_t count) {
+      *ptr = reinterpret_cast<std::remove_reference_t<decltype(*ptr)>>(base + at);
+      at += (count * sizeof(**ptr) + 255) / 256 * 256;
+      return at;
+    };
+    part(&p->qx, n);
+    part(&p->qxl, n);
+    part(&p->qy, n);
+    part(&p->qyl, n);
+    part(&p->tw, n);
+    part(&p->info, 1);
+    part(&p->dp_partial, (size_t)p->max_ranges * p->D);
+    part(&p->dp_sums, p->D);
+    part(&p->dp_mean, p->D);
+    part(&p->dp_dcpix, p->D);
+    part(&p->bf_rows, max_bf);
+    part(&p->bf_cols, max_bf);
+    part(&p->kx, max_bf);
+    part(&p->kxl, max_bf);
+    part(&p->ky, max_bf);
+    part(&p->kyl, max_bf);
+    part(&p->ak, max_bf);
+    part(&p->S_part, (size_t)p->max_groups * n * n);
+    part(&p->S, (size_t)n * n);
+    part(&p->rowph, (size_t)max_bf * n);
+    part(&p->colph, (size_t)max_bf * (n / 2 + 1));
+    return part(&p->echi, (size_t)n * n);
+  };
+  const size_t bytes = layout(nullptr);
+  hipStream_t s = as_stream(stream);
+  hipError_t e = hipGetDevice(&p->device);
+  if (e == hipSuccess) e = palloc(p, &p->block, bytes, s);
   if (e != hipSuccess) {
     ssb_plan_destroy(p);
     return hip_fail(e, "ssb_plan_create allocation");
   }
-  std::vector<float> qx(n), qy(n), qxl(n), qyl(n);
-  std::vector<float2> tw(n);
+  layout(p->block);
+  std::vector<char> host((char*)p->info + sizeof(BfInfo) - p->block);   // info: zero
+  float* qx = reinterpret_cast<float*>(host.data());
+  float* qxl = qx + (p->qxl - p->qx);
+  float* qy = qx + (p->qy - p->qx);
+  float* qyl = qx + (p->qyl - p->qx);
+  float2* tw = reinterpret_cast<float2*>(host.data() + ((char*)p->tw - p->block));
   for (int i = 0; i < n; ++i) {
     const int k = (i < (n + 1) / 2) ? i : i - n;   // numpy fftfreq ordering
     const df fx = to_df((double)k / (n * scan_sampling_row_A));
@@ -222,13 +291,8 @@ int ssb_plan_create(int scan_n, int det_rows, int det_cols, int max_bf, double w
     const double a = -2.0 * M_PI * (double)i / (double)n;
     tw[i] = make_float2((float)std::cos(a), (float)std::sin(a));
   }
-  BfInfo zero{};
-  if (e == hipSuccess) e = hipMemcpy(p->qx, qx.data(), n * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->qy, qy.data(), n * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->qxl, qxl.data(), n * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->qyl, qyl.data(), n * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->tw, tw.data(), n * sizeof(float2), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->info, &zero, sizeof(BfInfo), hipMemcpyHostToDevice);
+  e = hipMemcpyAsync(p->block, host.data(), host.size(), hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     ssb_plan_destroy(p);
     return hip_fail(e, "ssb_plan_create upload");
@@ -260,42 +324,14 @@ int ssb_set_scan_frequencies(ssb_plan* p, const float* qrow_host, const float* q
 
 int ssb_plan_destroy(ssb_plan* p) {
   if (!p) return QSSB_OK;
-  dfree(p->dp_partial);
-  dfree(p->dp_partial_wide);
-  dfree(p->dp_sums);
-  dfree(p->dp_mean);
-  dfree(p->dp_dcpix);
-  dfree(p->gain);
-  dfree(p->bf_rows);
-  dfree(p->bf_cols);
+  int dev = p->device;
+  (void)hipGetDevice(&dev);
+  if (dev != p->device) (void)hipSetDevice(p->device);
+  for (void* q : {(void*)p->block, (void*)p->dp_partial_wide, (void*)p->gain, (void*)p->H, (void*)p->Gt, (void*)p->T,
+                  (void*)p->xt, (void*)p->sup_part, (void*)p->sup_box, (void*)p->sup_C})
+    pfree(p, q);
+  if (dev != p->device) (void)hipSetDevice(dev);
   if (p->ev_stream) (void)hipEventDestroy(p->ev_stream);
-  dfree(p->info);
-  dfree(p->kx);
-  dfree(p->kxl);
-  dfree(p->ky);
-  dfree(p->kyl);
-  dfree(p->ak);
-  dfree(p->qx);
-  dfree(p->qxl);
-  dfree(p->qy);
-  dfree(p->qyl);
-  dfree(p->tw);
-  dfree(p->H);
-  dfree(p->S_part);
-  dfree(p->S);
-  dfree(p->rowph);
-  dfree(p->colph);
-  dfree(p->echi);
-  dfree(p->Gt);
-  dfree(p->T);
-  dfree(p->M1);
-  dfree(p->M2);
-  dfree(p->var_part);
-  dfree(p->loss);
-  dfree(p->xt);
-  dfree(p->sup_part);
-  dfree(p->sup_box);
-  dfree(p->sup_C);
   if (p->xexec) (void)hipGraphExecDestroy(p->xexec);
   if (p->xgraph) (void)hipGraphDestroy(p->xgraph);
   if (p->gev_in) (void)hipEventDestroy(p->gev_in);
@@ -314,13 +350,13 @@ static bool dtype_unsigned_int(int dtype) {
 }
 
 // partial-sum buffer of the stream pass for this sample type
-static int dp_partial_for(ssb_plan* p, int dtype, void** out) {
+static int dp_partial_for(ssb_plan* p, int dtype, hipStream_t s, void** out) {
   if (!dtype_wide_partials(dtype)) {
     *out = p->dp_partial;
     return QSSB_OK;
   }
   if (!p->dp_partial_wide) {
-    hipError_t e = hipMalloc(&p->dp_partial_wide, (size_t)p->max_ranges * p->D * 8);
+    hipError_t e = palloc(p, reinterpret_cast<double**>(&p->dp_partial_wide), (size_t)p->max_ranges * p->D, s);
     if (e != hipSuccess) {
       p->dp_partial_wide = nullptr;
       return hip_fail(e, "mean DP partial allocation");
@@ -339,9 +375,9 @@ static int mean_dp_typed(ssb_plan* p, const void* data, int dtype, int64_t frame
   if (sums_out && dtype == QSSB_DTYPE_F32)
     return fail(QSSB_ERR_ARG, "float32 frames have no integer sums; pass sums_out = NULL");
   void* partial = nullptr;
-  rc = dp_partial_for(p, dtype, &partial);
-  if (rc) return rc;
   hipStream_t s = as_stream(stream);
+  rc = dp_partial_for(p, dtype, s, &partial);
+  if (rc) return rc;
   HIP_TRY(launch_mean_dp(dtype, data, frames, p->D, partial, p->max_ranges, p->tune_stream_wg, p->gain, p->dp_sums,
                          p->dp_mean, p->dp_dcpix, s),
           "mean_dp");
@@ -372,12 +408,12 @@ int ssb_set_detector_gain(ssb_plan* p, const float* gain, void* stream) {
   if (!gain) {
     if (p->gain) {
       HIP_TRY(hipStreamSynchronize(s), "set_detector_gain sync");
-      dfree(p->gain);
+      pfree(p, p->gain);
       p->gain = nullptr;
     }
     return QSSB_OK;
   }
-  if (!p->gain) HIP_TRY(dmalloc(&p->gain, (size_t)p->D), "detector gain allocation");
+  if (!p->gain) HIP_TRY(palloc(p, &p->gain, (size_t)p->D, s), "detector gain allocation");
   HIP_TRY(hipMemcpyAsync(p->gain, gain, (size_t)p->D * 4, hipMemcpyDeviceToDevice, s), "set_detector_gain");
   return QSSB_OK;
 }
@@ -476,24 +512,24 @@ int ssb_get_geometry(ssb_plan* p, float* kx_out, float* ky_out, float* ak_out, i
 }
 
 // Row-transformed stack H[b][R_r][slot] for `cap` BF pixels (grown on demand).
-static int alloc_h(ssb_plan* p, int cap) {
+static int alloc_h(ssb_plan* p, int cap, hipStream_t s) {
   if (p->H_cap >= cap) return QSSB_OK;
-  dfree(p->H);
+  pfree(p, p->H);
   p->H = nullptr;
   p->H_cap = 0;
-  hipError_t e = dmalloc(&p->H, (size_t)cap * p->n * (p->n / 2));
+  hipError_t e = palloc(p, &p->H, (size_t)cap * p->n * (p->n / 2), s);
   if (e != hipSuccess) return hip_fail(e, "row-transformed stack allocation");
   p->H_cap = cap;
   return QSSB_OK;
 }
 
-static int alloc_gt(ssb_plan* p, int gcols, int nbf) {
+static int alloc_gt(ssb_plan* p, int gcols, int nbf, hipStream_t s) {
   const size_t need = (size_t)nbf * gcols * p->n * sizeof(float2);
   if (p->Gt_bytes < need) {
-    dfree(p->Gt);
+    pfree(p, p->Gt);
     p->Gt = nullptr;
     p->Gt_bytes = 0;
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->Gt), need);
+    hipError_t e = palloc(p, &p->Gt, need / sizeof(float2), s);
     if (e != hipSuccess) return hip_fail(e, "resident G allocation");
     p->Gt_bytes = need;
   }
@@ -514,9 +550,9 @@ static int prepare_g_typed(ssb_plan* p, const void* data, int dtype, void* strea
     if (info.status != 0 || info.nbf < 1) return fail(QSSB_ERR_STATE, "no valid bright-field selection");
     p->nbf_hint = info.nbf;
   }
-  rc = alloc_gt(p, p->n / 2 + 1, p->nbf_hint);
+  rc = alloc_gt(p, p->n / 2 + 1, p->nbf_hint, s);
   if (rc) return rc;
-  rc = alloc_h(p, p->nbf_hint);
+  rc = alloc_h(p, p->nbf_hint, s);
   if (rc) return rc;
   HIP_TRY(launch_gather_rowfft(p->n, dtype, data, p->D, p->det_cols, p->bf_rows, p->bf_cols, p->info, p->nbf_hint,
                                p->tw, p->tune_gather_pairs, p->gain, p->H, s),
@@ -558,7 +594,7 @@ int ssb_import_g(ssb_plan* p, const void* g_in, int nbf, int gcols, void* stream
   if (gcols != p->n && gcols != p->n / 2 + 1)
     return fail(QSSB_ERR_ARG, "G must have N or N/2+1 columns");
   if (nbf != p->nbf_hint) return fail(QSSB_ERR_ARG, "G first dimension must match the BF selection");
-  rc = alloc_gt(p, gcols, nbf);
+  rc = alloc_gt(p, gcols, nbf, as_stream(stream));
   if (rc) return rc;
   const long long total = (long long)nbf * p->n * gcols;
   hipLaunchKernelGGL(k_import_g, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, as_stream(stream),
@@ -625,25 +661,20 @@ static ChiPoly chi_poly(const ssb_plan* p, const double* mags, const double* ang
 
 // Workspace of the exact phase path, for its even and its general form alike
 // (a later call of the other form, under capture too, allocates nothing).
-static int alloc_loss(ssb_plan* p) {
+static int alloc_loss(ssb_plan* p, hipStream_t s) {
   if (p->T) return QSSB_OK;
   const size_t nn = (size_t)p->n * p->n;
   const size_t planes = std::max(phase_splits(p->n), loss_splits(p->n));
-  hipError_t e = dmalloc(&p->T, std::max(phase_workspace_floats2(p->n), loss_chunk_bf(p->n) * nn));
-  if (e == hipSuccess) e = dmalloc(&p->M1, planes * nn);
-  if (e == hipSuccess) e = dmalloc(&p->M2, planes * nn);
-  if (e == hipSuccess) e = dmalloc(&p->var_part, nn / 64);
-  if (e == hipSuccess) e = dmalloc(&p->loss, 1);
+  const size_t t = std::max(phase_workspace_floats2(p->n), loss_chunk_bf(p->n) * nn);
+  hipError_t e = palloc(p, &p->T, t + 2 * planes * nn + nn / 64 + 1, s);   // one block
   if (e != hipSuccess) {
-    dfree(p->T);
-    dfree(p->M1);
-    dfree(p->M2);
-    dfree(p->var_part);
-    dfree(p->loss);
-    p->T = p->M1 = p->M2 = nullptr;
-    p->var_part = p->loss = nullptr;
+    p->T = nullptr;
     return hip_fail(e, "exact phase workspace allocation");
   }
+  p->M1 = p->T + t;
+  p->M2 = p->M1 + planes * nn;
+  p->var_part = reinterpret_cast<float*>(p->M2 + planes * nn);
+  p->loss = p->var_part + nn / 64;
   return QSSB_OK;
 }
 
@@ -698,7 +729,7 @@ int ssb_phase_loss(ssb_plan* p, double c10, double c12, double phi12, float* pha
     rc = ensure_geometry(p, s);
     if (rc) return rc;
   }
-  rc = alloc_loss(p);
+  rc = alloc_loss(p, s);
   if (rc) return rc;
   const double mags[2] = {c10, c12}, angles[2] = {0.0, phi12};
   HIP_TRY(enqueue_phase(p, mags, angles, true, phase_out, loss_out ? loss_out : p->loss, s), "phase_moments");
@@ -877,7 +908,7 @@ int ssb_phase_loss_full(ssb_plan* p, const double* mags_host, const double* angl
     rc = ensure_geometry(p, s);
     if (rc) return rc;
   }
-  rc = alloc_loss(p);
+  rc = alloc_loss(p, s);
   if (rc) return rc;
   HIP_TRY(enqueue_phase(p, mags_host, angles_host, false, phase_out, loss_out ? loss_out : p->loss, s),
           "phase_moments_full");
@@ -893,7 +924,7 @@ int ssb_batch_phase_loss(ssb_plan* p, int n_trials, const double* mags_host, con
   if (!mags_host || !angles_host || !losses_out) return fail(QSSB_ERR_ARG, "trial arrays must not be NULL");
   if (!p->gcols) return fail(QSSB_ERR_STATE, "no resident Fourier stack");
   hipStream_t s = as_stream(stream);
-  rc = alloc_loss(p);
+  rc = alloc_loss(p, s);
   if (rc) return rc;
   const double rot0 = p->rotation;
   bool have_geometry = p->geometry_valid;
@@ -947,15 +978,15 @@ int ssb_batch_phase_loss_graph(ssb_plan* p, int n_trials, const double* mags_hos
   if (!mags_host || !angles_host || !losses_out) return fail(QSSB_ERR_ARG, "trial arrays must not be NULL");
   if (!p->gcols) return fail(QSSB_ERR_STATE, "no resident Fourier stack");
   hipStream_t s = as_stream(stream);
-  rc = alloc_loss(p);
+  rc = alloc_loss(p, s);
   if (rc) return rc;
   if (p->xt_cap < n_trials) {
     HIP_TRY(hipStreamSynchronize(s), "batch graph sync");
     if (p->gstream) HIP_TRY(hipStreamSynchronize(p->gstream), "batch graph sync");
-    dfree(p->xt);
+    pfree(p, p->xt);
     p->xt = nullptr;
     p->xt_cap = 0;
-    HIP_TRY(dmalloc(&p->xt, (size_t)n_trials), "batch table allocation");
+    HIP_TRY(palloc(p, &p->xt, (size_t)n_trials, s), "batch table allocation");
     p->xt_cap = n_trials;
     if (p->xexec) (void)hipGraphExecDestroy(p->xexec);
     if (p->xgraph) (void)hipGraphDestroy(p->xgraph);
@@ -1017,16 +1048,16 @@ int ssb_batch_phase_loss_graph(ssb_plan* p, int n_trials, const double* mags_hos
 }
 
 // Superset sample sums, box and the compact per-frame copy (allocated on first use).
-static int alloc_superset(ssb_plan* p) {
+static int alloc_superset(ssb_plan* p, hipStream_t s) {
   if (p->sup_C) return QSSB_OK;
   const size_t frames = (size_t)p->n * p->n;
-  hipError_t e = dmalloc(&p->sup_part, (size_t)superset_part_count() * p->D);
-  if (e == hipSuccess) e = dmalloc(&p->sup_box, 1);
-  if (e == hipSuccess) e = dmalloc(&p->sup_C, frames * kSupMaxPixels);
+  hipError_t e = palloc(p, &p->sup_part, (size_t)superset_part_count() * p->D, s);
+  if (e == hipSuccess) e = palloc(p, &p->sup_box, 1, s);
+  if (e == hipSuccess) e = palloc(p, &p->sup_C, frames * kSupMaxPixels, s);
   if (e != hipSuccess) {
-    dfree(p->sup_part);
-    dfree(p->sup_box);
-    dfree(p->sup_C);
+    pfree(p, p->sup_part);
+    pfree(p, p->sup_box);
+    pfree(p, p->sup_C);
     p->sup_part = nullptr;
     p->sup_box = nullptr;
     p->sup_C = nullptr;
@@ -1043,7 +1074,7 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
   if (!data) return fail(QSSB_ERR_ARG, "data is NULL");
   if (!dtype_size(dtype)) return fail(QSSB_ERR_ARG, "unknown sample type " + std::to_string(dtype));
   void* partial = nullptr;
-  rc = dp_partial_for(p, dtype, &partial);
+  rc = dp_partial_for(p, dtype, s, &partial);
   if (rc) return rc;
   if (after == p) return fail(QSSB_ERR_ARG, "a plan cannot be ordered after itself");
   if (after) {
@@ -1066,7 +1097,7 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
   const bool sup = dtype == QSSB_DTYPE_U16 && p->tune_superset == 1 && p->det_cols % 8 == 0 &&
                    (reinterpret_cast<uintptr_t>(data) & 15u) == 0;
   if (sup) {
-    rc = alloc_superset(p);
+    rc = alloc_superset(p, s);
     if (rc) return rc;
   }
   mark(0);
@@ -1101,7 +1132,7 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
   rc = ensure_geometry(p, s);
   if (rc) return rc;
   p->gcols = 0;
-  rc = alloc_h(p, p->max_bf);
+  rc = alloc_h(p, p->max_bf, s);
   if (rc) return rc;
   mark(5);
   const QuadChi m = quad_chi(p, c10, c12, phi12);

@@ -37,7 +37,15 @@ struct ssb_plan {
   bool geometry_valid = false;
   double rotation = 0;
   Optics optics{};
-  // device buffers
+  // where the buffers come from: the caller's memory (ssb_plan_create_with) or
+  // the device; `lent` are the blocks to give back
+  ssb_alloc_fn alloc = nullptr;
+  ssb_release_fn release = nullptr;
+  void* alloc_ctx = nullptr;
+  int device = 0;
+  void* lent[16] = {};
+  // device buffers; those every plan has are parts of one block
+  char* block = nullptr;
   uint32_t* dp_partial = nullptr;
   void* dp_partial_wide = nullptr;   // 64-bit partials of 32-bit samples (allocated on first use)
   unsigned long long* dp_sums = nullptr;

@@ -32,11 +32,16 @@ _fp = ctypes.POINTER(ctypes.c_float)
 _dp = ctypes.POINTER(ctypes.c_double)
 _pp = ctypes.POINTER(ctypes.c_void_p)
 
+AllocFn = ctypes.CFUNCTYPE(_vp, ctypes.c_size_t, _vp, _vp)
+ReleaseFn = ctypes.CFUNCTYPE(None, _vp, _vp)
+
 # name -> argtypes; every function returns int
 SIGNATURES: dict[str, list] = {
     "ssb_version": [],
     "ssb_plan_create": [_c_int, _c_int, _c_int, _c_int, _c_double, _c_double, _c_double, _c_double,
                         _c_double, _c_double, _pp],
+    "ssb_plan_create_with": [_c_int, _c_int, _c_int, _c_int, _c_double, _c_double, _c_double, _c_double,
+                             _c_double, _c_double, AllocFn, ReleaseFn, _vp, _vp, _pp],
     "ssb_plan_destroy": [_vp],
     "ssb_set_detector_sampling": [_vp, _c_double, _c_double],
     "ssb_set_scan_frequencies": [_vp, _fp, _fp],

@@ -118,6 +118,28 @@ class PlanSpec:
     scan_sampling_col_A: float
 
 
+# A plan's buffers come from torch's caching allocator, which keeps them when a
+# session ends (torch.cuda.empty_cache() and torch itself, when it runs short,
+# give them back): allocating and freeing them on the device took two thirds of
+# a short session.  The allocator orders a block by one stream; the plan waits
+# for the device before it releases one.
+@_abi.AllocFn
+def _alloc(nbytes, stream, _ctx):
+    try:
+        torch = _torch()
+        return torch.cuda.caching_allocator_alloc(nbytes, torch.cuda.current_device(), stream or 0)
+    except Exception:      # no exception crosses the C boundary: NULL is out of memory
+        return None
+
+
+@_abi.ReleaseFn
+def _release(ptr, _ctx):
+    try:
+        _torch().cuda.caching_allocator_delete(ptr)
+    except Exception:
+        pass
+
+
 class SSBPlan:
     """Owns one native plan (device buffers for one scan/detector geometry)."""
 
@@ -130,9 +152,10 @@ class SSBPlan:
         self.device = dev
         handle = ctypes.c_void_p()
         with torch.cuda.device(self.device):
-            _abi.call("ssb_plan_create", spec.scan_n, spec.det_rows, spec.det_cols, spec.max_bf,
+            _abi.call("ssb_plan_create_with", spec.scan_n, spec.det_rows, spec.det_cols, spec.max_bf,
                       spec.wavelength_A, spec.semiangle_rad, spec.ang_row_rad, spec.ang_col_rad,
-                      spec.scan_sampling_row_A, spec.scan_sampling_col_A, ctypes.byref(handle))
+                      spec.scan_sampling_row_A, spec.scan_sampling_col_A, _alloc, _release, None,
+                      _abi.stream_handle(torch.cuda.current_stream(dev)), ctypes.byref(handle))
         self._h = handle
 
     @property

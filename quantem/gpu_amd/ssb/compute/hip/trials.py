@@ -41,8 +41,12 @@ class TrialBatch:
         handles = (ctypes.c_void_p * len(self.engines))(*[e.plan.handle.value for e in self.engines])
         out = ctypes.c_void_p()
         with torch.cuda.device(dev):
-            _abi.call("ssb_trials_create", ctypes.cast(handles, _abi._pp), len(self.engines), self.max_trials,
-                      ctypes.byref(out))
+            args = (ctypes.cast(handles, _abi._pp), len(self.engines), self.max_trials, ctypes.byref(out))
+            try:
+                _abi.call("ssb_trials_create", *args)
+            except MemoryError:
+                torch.cuda.empty_cache()   # what ended sessions left in torch's cache
+                _abi.call("ssb_trials_create", *args)
         self._h = out
         self.n_trials = 0
         self.out = torch.empty((len(self.engines), self.max_trials), dtype=torch.float32, device=dev)
