@@ -16,24 +16,33 @@
 // Three kernels:
 //   k_bslz4_index   one thread per chunk: validates the header and walks the
 //                   block sizes into a descriptor table (bounds-checked);
-//   k_bslz4_parse   one thread per block: walks the block's LZ4 sequence
-//                   headers (every length and offset checked) into a table
-//                   of {literal start, literal length, offset, match length}
-//                   per sequence;
+//   k_bslz4_parse   only for blocks too large to stage in LDS, one thread per
+//                   block: walks the block's LZ4 sequence headers (every
+//                   length and offset checked) into a table of {literal
+//                   start, literal length, offset, match length} per sequence;
 //   k_bslz4_decode  one 64-lane workgroup per block: stages the compressed
-//                   block in LDS as whole words and decodes it in LDS in
-//                   rounds of up to 64 table entries (one lane per
-//                   sequence: all of the round's literal runs at once, then
-//                   its matches in order; a match of offset d < length is
-//                   out[o + t] = out[o - d + t mod d], a run of one byte is
-//                   written with 16-byte stores; a block whose sequences
-//                   overflow the table is walked here instead), then inverts
-//                   the bit-shuffle, 32 elements per lane step (two 8x8
-//                   bit-matrix transposes by delta swaps and byte permutes
-//                   per 8 elements), with 16-byte stores.
+//                   block in LDS as whole words, finds its sequences there, and
+//                   decodes it in LDS in rounds of up to 64 sequences (one
+//                   lane per sequence: all of the round's literal runs at
+//                   once, then its matches in order; a match of offset d <
+//                   length is out[o + t] = out[o - d + t mod d], a run of one
+//                   byte is written with 16-byte stores; a block with more
+//                   sequences than are kept is walked here instead), then inverts
+//                   the bit-shuffle, 32 elements per lane step (two 16 x 16
+//                   bit matrices transposed together), with 16-byte stores.
+// Where the sequences of a block start is a chain through its bytes, but where
+// each would end if it started there is not: the lanes find that for every
+// byte at once (lz4_next), and the chain is one LDS read for two sequences.
+// A thread walking one block from memory waits for a line every few sequences
+// and for the longest of its wave's 64 blocks: at 16384 frames of 192 x 192
+// (38 sequences a block, median 7) such a pass took 398 us beside the
+// decode's 718; now the decode takes 868 us in all, bound by its vector
+// instructions (2550 a block).  Workgroups that fetch their next block ahead
+// are slower (1378 us): the hardware's dispatch evens out the blocks better.
 // Malformed input never reads or writes out of bounds: it sets a bit in the
 // status word and the block is skipped.
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "ssb_internal.h"
@@ -47,8 +56,72 @@ constexpr int kMaxCompBytes = kMaxBlockBytes + kMaxBlockBytes / 255 + 16;  // LZ
 // Compressed blocks up to this size (less the alignment bytes around them)
 // are staged in LDS (detector frames compress 10-20x); larger ones are
 // parsed from global memory.  The small staging buffer leaves room for
-// about twice as many workgroups per CU.
+// about twice as many workgroups per CU, and the ends of a staged block's
+// sequences fit where it will be decoded (4 bytes for each of its own).
 constexpr int kStageBytes = 2048;
+static_assert(4 * kStageBytes <= kMaxBlockBytes && kStageBytes == 64 * 32, "lz4_next's table and run_255's bits");
+
+__device__ __forceinline__ bool staged_block(const uint8_t* src, int csize) {
+  return (int)(reinterpret_cast<uintptr_t>(src) & 3u) + csize <= kStageBytes;
+}
+
+// A length of 15 in the token goes on in bytes of 255 and one other.  Lane l of
+// `ones` has a bit for every byte 32 l.. of a staged block that is 255 (none at
+// or past its end); the number of them from byte x < 2048 on, up to 32, which
+// no valid length exceeds.  Every lane of the wave calls it together.
+__device__ __forceinline__ int run_255(unsigned ones, int x) {
+  const int g = x >> 5;
+  const unsigned lo = __shfl(ones, g, 64), next = __shfl(ones, g + 1, 64);
+  const unsigned m = ~__builtin_amdgcn_alignbit(g == 63 ? 0u : next, lo, x & 31);
+  return m ? __builtin_ctz(m) : 32;
+}
+
+constexpr unsigned kSeqEnd = 0xFFFEu, kSeqBad = 0xFFFFu;
+
+// Where the sequence that starts at byte p < cs of a staged block ends:
+// kSeqEnd when its literals end the block, kSeqBad for one that no block of cs
+// bytes can hold.  Without branches, so that calls overlap their reads.
+__device__ __forceinline__ unsigned lz4_next(const uint8_t* in, unsigned ones, int cs, int p) {
+  const int token = in[p];
+  const int q = p + 1 + run_255(ones, min(p + 1, kStageBytes - 1));
+  const int b = in[min(q, cs - 1)];
+  const bool lng = token >= 0xF0;
+  const int lit = lng ? 15 + 255 * (q - p - 1) + b : token >> 4;
+  int ip = lng ? q + 1 : p + 1;
+  bool bad = (lng && (q >= cs || b == 255)) || lit > cs - ip;
+  ip = bad ? cs : ip + lit;
+  const bool end = ip == cs;
+  ip = min(ip + 2, cs);
+  const int r = run_255(ones, min(ip, kStageBytes - 1));
+  if ((token & 15) == 15) {
+    ip += r;
+    if (r == 32 && ip < cs) bad |= in[ip] == 255;
+    ip += 1;
+  }
+  return bad ? kSeqBad : (end ? kSeqEnd : (ip < cs ? (unsigned)ip : kSeqBad));   // the last one has literals only
+}
+
+// The sequence at p, which lz4_next has found sound: {literal start | literal
+// length << 16, offset | match length << 16}, 0 for the last one's match.
+__device__ __forceinline__ uint2 lz4_sequence(const uint8_t* in, unsigned ones, int cs, int p) {
+  const int token = in[p];
+  const int r = run_255(ones, min(p + 1, kStageBytes - 1));
+  int ip = p + 1, lit = token >> 4;
+  if (lit == 15) {
+    lit += 255 * r + in[ip + r];
+    ip += r + 1;
+  }
+  const unsigned x = (unsigned)(ip | (lit << 16));
+  ip += lit;
+  const bool last = ip == cs;
+  const int at = min(ip, cs - 2);                     // (a block of one byte: its token, masked below)
+  const int off = in[max(at, 0)] | (in[min(max(at, 0) + 1, cs - 1)] << 8);
+  ip += 2;
+  int ml = token & 15;
+  const int r2 = run_255(ones, min(ip, kStageBytes - 1));
+  if (!last && ml == 15) ml += 255 * r2 + in[ip + r2];
+  return make_uint2(x, last ? 0u : (unsigned)(off | ((ml + 4) << 16)));
+}
 
 struct BlockDesc {
   long long src;   // byte offset of the block's payload in the compressed buffer
@@ -151,7 +224,7 @@ __device__ __forceinline__ long long seq_slot(long long d, int k, int cap) {
 // length and offset checked as in the decode) and stores sequence k as
 // {literal start | literal length << 16, offset | match length << 16}
 // (offset and match length 0 for the block's last sequence).  nseq[d] is
-// the count, 0 for unused slots and raw tails, -1 when the block has more
+// the count, 0 for unused slots, raw tails and blocks that the decode stages, -1 when the block has more
 // sequences than the table holds (the decode kernel then parses it), -2
 // for a malformed block (its status bit set).  Each thread reads its block
 // through a 32-byte window of aligned vector loads.
@@ -161,7 +234,7 @@ k_bslz4_parse(const uint8_t* __restrict__ comp, long long comp_bytes, const Bloc
   const long long d = (long long)blockIdx.x * 256 + threadIdx.x;
   if (d >= n_desc) return;
   const BlockDesc bd = table[d];
-  if (bd.elems == 0 || bd.csize < 0) {
+  if (bd.elems == 0 || bd.csize < 0 || staged_block(comp + bd.src, bd.csize)) {
     nseq[d] = 0;
     return;
   }
@@ -255,7 +328,8 @@ constexpr int kShortLit = 16;
 
 // The copies of one round of up to 64 sequences, lane j holding sequence j
 // ({literal start | length << 16, offset | match length << 16}; 0 beyond n),
-// output from op0; returns the round's output bytes.  Literal bytes come
+// output from op0; returns the round's output bytes, or, with CHECK, -1 when
+// a length runs past osz or an offset before the start.  Literal bytes come
 // from src[0, src_end) (LDS or global).  Every literal run of the round is
 // copied at once (its destination follows from the lengths before it: a
 // wave prefix sum), then the matches in order, each one read of its source
@@ -263,8 +337,8 @@ constexpr int kShortLit = 16;
 // the literals of later sequences, written first, are never read early.
 // The workgroup is one wave, whose LDS operations complete in issue order,
 // so the phases need only compiler ordering fences.
-template <typename Src>
-__device__ __forceinline__ int lz4_round(uint2 e, int n, int op0, int lane, const Src* src, int src_end,
+template <bool CHECK, typename Src>
+__device__ __forceinline__ int lz4_round(uint2 e, int n, int op0, int osz, int lane, const Src* src, int src_end,
                                          uint8_t* cout) {
   const int lit_l = (int)(e.x >> 16), lip_l = (int)(e.x & 0xFFFFu);
   const int ml_l = (int)(e.y >> 16), off_l = (int)(e.y & 0xFFFFu);
@@ -277,6 +351,11 @@ __device__ __forceinline__ int lz4_round(uint2 e, int n, int op0, int lane, cons
     if (lane >= sh) incl += y;
   }
   const int lop = op0 + incl - len;                   // this lane's sequence starts here
+  if (CHECK) {
+    const int end = lop + lit_l;
+    const bool bad = act && (end + ml_l > osz || (ml_l > 0 && (off_l == 0 || off_l > end)));
+    if (__any(bad)) return -1;
+  }
   if (act && lit_l < kShortLit) {
     uint8_t b[kShortLit - 1];                         // read together (clamped inside src), then written
 #pragma unroll
@@ -369,13 +448,13 @@ k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const Blo
       }
       continue;
     }
-    const int n = nseq[d];
-    if (n == -2) continue;                             // malformed: flagged by the parse
     const int cs = bd.csize;
     const int osz = bd.elems * 2;
     const uint8_t* gsrc = comp + bd.src;
     const int s0 = (int)(reinterpret_cast<uintptr_t>(gsrc) & 3u);
-    const bool staged = s0 + cs <= kStageBytes;        // uniform
+    const bool staged = staged_block(gsrc, cs);        // uniform
+    const int n = staged ? 0 : nseq[d];
+    if (n == -2) continue;                             // malformed: flagged by the parse
     __syncthreads();                                   // previous block's readers are done
     if (staged) {
       // the payload and the bytes around it up to whole 4-byte words, each
@@ -397,16 +476,76 @@ k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const Blo
       __syncthreads();
     }
     int err = 0;
-    if (n >= 0) {
+    bool walk = n < 0;                                 // more sequences than are kept
+    if (staged) {
+      const uint8_t* const in = cin + s0;
+      // ends of the sequences at every byte, of the one and of the one after
+      unsigned* const ends = reinterpret_cast<unsigned*>(cout);
+      unsigned ones = 0u;
+      for (int g = 0; 64 * g < cs; ++g) {
+        const int p = 64 * g + lane;
+        const unsigned long long m = __ballot(in[min(p, cs - 1)] == 255 && p < cs);
+        ones = (lane >> 1) == g ? (unsigned)(m >> (32 * (lane & 1))) : ones;
+      }
+#pragma unroll 2
+      for (int p0 = 0; p0 < cs; p0 += 64) {
+        const int p = p0 + lane;
+        const unsigned e = lz4_next(in, ones, cs, min(p, cs - 1));
+        if (p < cs) ends[p] = e;
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll 4
+      for (int p = lane; p < cs; p += 64) {
+        const unsigned a = ends[p] & 0xFFFFu;
+        ends[p] = a | ((a < (unsigned)cs ? ends[a] : 0u) << 16);
+      }
+      asm volatile("" ::: "memory");
+      // the chain: sequence 64 c + l starts at start[c] of lane l
+      constexpr int KEPT = 8;
+      int start[KEPT], count = 0;
+      unsigned at = cs > 0 ? 0u : kSeqBad;
+#pragma unroll
+      for (int c = 0; c < KEPT; ++c) {
+        start[c] = 0;
+        for (int l = 0; l < 64 && at < kSeqEnd; l += 2) {
+          const unsigned e2 = (unsigned)__builtin_amdgcn_readfirstlane((int)ends[at]);
+          const unsigned e1 = e2 & 0xFFFFu;
+          start[c] = lane == l ? (int)at : start[c];
+          start[c] = lane == l + 1 ? (int)e1 : start[c];
+          count += e1 < kSeqEnd ? 2 : 1;
+          at = e1 < kSeqEnd ? e2 >> 16 : e1;
+        }
+      }
+      asm volatile("" ::: "memory");
+      if (at == kSeqBad) {
+        err = kErrStream;
+      } else if (at != kSeqEnd) {
+        walk = true;
+      } else {
+        int op = 0;
+#pragma unroll 1
+        for (int r0 = 0; r0 < count && !err; r0 += 64) {
+          int p = start[0];
+#pragma unroll
+          for (int c = 1; c < KEPT; ++c) p = r0 == 64 * c ? start[c] : p;
+          const int m = min(64, count - r0);
+          const uint2 e = lz4_sequence(in, ones, cs, lane < m ? p : 0);
+          const int got = lz4_round<true>(lane < m ? e : make_uint2(0u, 0u), m, op, osz, lane, in, cs, cout);
+          op += got;
+          if (got < 0) err = kErrStream;
+        }
+        if (op != osz) err = kErrStream;
+      }
+    } else if (!walk) {
       int op = 0;
       for (int r0 = 0; r0 < n; r0 += 64) {
         const int m = min(64, n - r0);
         const uint2 e = (lane < m) ? seqs[seq_slot(d, r0 + lane, cap)] : make_uint2(0u, 0u);
-        op += staged ? lz4_round(e, m, op, lane, cin + s0, cs, cout) : lz4_round(e, m, op, lane, gsrc, cs, cout);
+        op += lz4_round<false>(e, m, op, osz, lane, gsrc, cs, cout);
       }
-    } else {
-      // more sequences than the table holds: every lane walks the same
-      // headers here and the copies follow each header
+    }
+    if (walk) {
+      // every lane walks the same headers here and the copies follow each header
       auto parse = [&](auto byte_at, int& ip, int& op) -> int {
         while (true) {
           if (ip >= cs) return kErrStream;
@@ -459,12 +598,12 @@ k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const Blo
       continue;                                        // uniform: every lane saw the same stream
     }
     __syncthreads();
-    // inverse bit-shuffle, 8 elements per group: the 16 plane bytes of the
-    // group form two 8x8 bit matrices (planes 0-7 and 8-15, byte = plane,
-    // bit = element); each is transposed in a 64-bit word by three delta
-    // swaps, after which byte i holds element i's low or high byte, and
-    // v_perm interleaves them into the output words.  With whole words per
-    // plane, a lane takes 4 groups: one LDS word per plane, 64 bytes out.
+    // inverse bit-shuffle.  With whole words per plane, a lane takes 32
+    // elements, one LDS word per plane, 64 bytes out.  Else 8 elements per
+    // group: the 16 plane bytes of the group form two 8x8 bit matrices (planes
+    // 0-7 and 8-15, byte = plane, bit = element); each is transposed in a
+    // 64-bit word by three delta swaps, after which byte i holds element i's
+    // low or high byte, and v_perm interleaves them into the output words.
     const int planeb = bd.elems / 8;
     auto group = [&](const unsigned (&bt)[16]) -> uint4 {
       unsigned long long m[2];
@@ -498,13 +637,36 @@ k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const Blo
         unsigned wd[16];
 #pragma unroll
         for (int b = 0; b < 16; ++b) wd[b] = c32[b * pw + g4];
+        // two 16 x 16 bit matrices, of the words' halves, transposed together
+        // (112 operations for 32 elements; 8 x 8 ones a group took 480)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const unsigned x = wd[i], y = wd[i + 8];
+          wd[i] = __builtin_amdgcn_perm(y, x, 0x06020400u);
+          wd[i + 8] = __builtin_amdgcn_perm(y, x, 0x07030501u);
+        }
+        auto swap = [&](auto dist, unsigned m) {
+          constexpr int sh = decltype(dist)::value;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            if (i & sh) continue;
+            const unsigned x = wd[i], y = wd[i + sh];
+            wd[i] = (m & x) | (~m & (y << sh));
+            wd[i + sh] = (m & (x >> sh)) | (~m & y);
+          }
+        };
+        swap(std::integral_constant<int, 4>{}, 0x0F0F0F0Fu);
+        swap(std::integral_constant<int, 2>{}, 0x33333333u);
+        swap(std::integral_constant<int, 1>{}, 0x55555555u);
+        // word p now holds elements p and 16 + p
         uint4* o = reinterpret_cast<uint4*>(out + bd.dst + 32LL * g4);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          unsigned bt[16];
-#pragma unroll
-          for (int b = 0; b < 16; ++b) bt[b] = (wd[b] >> (8 * k)) & 0xFFu;
-          o[k] = group(bt);
+          const unsigned sel = k < 2 ? 0x05040100u : 0x07060302u;
+          const int e = 8 * (k & 1);
+          o[k] = make_uint4(__builtin_amdgcn_perm(wd[e + 1], wd[e], sel), __builtin_amdgcn_perm(wd[e + 3], wd[e + 2], sel),
+                            __builtin_amdgcn_perm(wd[e + 5], wd[e + 4], sel),
+                            __builtin_amdgcn_perm(wd[e + 7], wd[e + 6], sel));
         }
       }
     } else {
