@@ -1140,14 +1140,13 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
   // With QSSB_TUNE_SPLIT 1: two halves of the BF list (raster order, so
   // disjoint detector rows), the second half's gather (HBM-bound) on the
   // plan's second stream beside the first half's trotter (VALU-bound).
-  // Measured at 256x256x128x128 the two compete for the CUs (the trotter
-  // holds one 8-wave workgroup per CU at 225 VGPRs) and the pair is slower
-  // than one pass, so one pass is the default.  Stage marks with the split:
-  // 5 -> 6 the first half's gather and the phasors, 6 -> 7 both trotters
-  // and the second gather.
+  // Measured at 256x256x128x128 the two compete for the CUs and the pair is
+  // slower than one pass, so one pass is the default.  Stage marks with the
+  // split: 5 -> 6 the first half's gather, 6 -> 7 both trotters and the
+  // second gather.
   const bool columns = columns_path(p->n, p->optics);
   const QuadTurns turns = quad_turns(p, c10, c12, phi12);
-  const bool two = p->tune_split == 1 && trotter_wave_path(p->n, true, p->optics, p->tune_trotter);
+  const bool two = p->tune_split == 1 && p->n == 256 && columns;
   if (two) {
     if (!p->pstream) HIP_TRY(hipStreamCreateWithFlags(&p->pstream, hipStreamNonBlocking), "second stream");
     if (!p->pev_a) HIP_TRY(hipEventCreateWithFlags(&p->pev_a, hipEventDisableTiming), "split event");
@@ -1163,15 +1162,13 @@ static int recon_typed(ssb_plan* p, const ssb_plan* after, const void* data, int
                                  sup ? p->sup_box : nullptr, sup ? p->sup_C : nullptr, 1, 2),
             "gather_rowfft");
     HIP_TRY(hipEventRecord(p->pev_b, p->pstream), "split event");
-    HIP_TRY(launch_phasors(p->n, p->info, p->nbf_hint, geom_ptrs(p), m, p->rowph, p->colph, p->echi, s),
-            "phasors");
     mark(6);
-    HIP_TRY(launch_trotter_slots(p->n, true, p->H, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics,
-                                 p->tw, p->S_part, p->tune_trotter, s, &groups, 0, 2),
+    HIP_TRY(launch_columns_trotter(p->n, p->H, p->info, geom_ptrs(p), turns, p->optics, p->tw, p->S_part,
+                                   p->tune_trotter, s, &groups, 0, 2),
             "colfft_trotter");
     HIP_TRY(hipStreamWaitEvent(s, p->pev_b, 0), "split wait");
-    HIP_TRY(launch_trotter_slots(p->n, true, p->H, p->info, geom_ptrs(p), p->rowph, p->colph, p->echi, p->optics,
-                                 p->tw, p->S_part, p->tune_trotter, s, &groups, 1, 2),
+    HIP_TRY(launch_columns_trotter(p->n, p->H, p->info, geom_ptrs(p), turns, p->optics, p->tw, p->S_part,
+                                   p->tune_trotter, s, &groups, 1, 2),
             "colfft_trotter");
   } else {
     // The gather's threads also write the phasor tables, where the trotter

@@ -230,27 +230,32 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
 // m in registers (over Q = K / 16 neighbouring lanes where K > 16), twiddles,
 // one exchange through the wave's own LDS, then 16-point DFTs over jj, so that
 // lane col * K + k1 ends with the rows k1 + K r of its column and every r of
-// the wave is a tile of K rows and S columns.  A workgroup takes the 16 columns
-// of one 128-byte line of H and keeps step over it with a barrier a BF pixel
-// (without: the lines are fetched again).  BF pixels whose apertures miss the
-// line's columns are passed over.  STORE: no sums, the stack is written.
+// the wave is a tile of K rows and S columns.  A workgroup loads its waves'
+// columns together (a 128-byte line of every row of H; half a line at 512),
+// one BF pixel ahead, and deals them out through LDS: with a wave's own loads,
+// 32 or 16 bytes of every line, the lines went through the caches eight times
+// (N = 256: 151 us a reconstruction for 112, 512: 412 for 263; the workgroup
+// kernels before: 119 and 867).  BF pixels whose apertures miss the workgroup's
+// columns are passed over.  STORE: no sums, the stack is written.
+// Two to three waves a SIMD (64 registers of sums) and the exchanges bound it:
+// 800 BF pixels at 256 move 150 MB in 93 us.
 // ------------------------------------------------------------------------
+// Workgroup barrier for LDS only: this wave's LDS operations complete, then
+// s_barrier; its global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 template <int N>
 struct ColumnFft {
   static constexpr int S = 1024 / N, K = N / 16, HALF = N / 2;
   static constexpr int Q = K > 16 ? K / 16 : 1;
-  static constexpr int SP = 17;                 // padded sequence stride
-  static constexpr int LDS = 64 * SP;           // float2 of LDS a wave
+  static constexpr int SP = 17;                 // padded stride of the 16-value sequences
+  // padded column stride: the 32 lanes of a staging write (whole rows of the
+  // workgroup's columns) meet every bank once
+  static constexpr int CS = K * SP + (K == 64 ? 8 : (K == 32 ? 4 : (K == 16 ? 2 : 10)));
+  static constexpr int LDS = S * CS;            // float2 of LDS a wave
 
-  // load e (0..15) of a lane, from H's column base: row jj + 16 h + 16 Q e of
-  // column lane / 16 Q, or (K = 8) row jj + 16 (e & 7) of column lane / 16 + 4 (e >> 3)
-  __device__ static __forceinline__ unsigned load_lane(int lane, bool one) {
-    const int row = (lane / Q & 15) + 16 * (lane % Q);
-    return row * HALF + (one ? 0 : lane / (16 * Q));
-  }
-  __device__ static constexpr int load_step(int e, bool one) {
-    return K == 8 ? 16 * (e & 7) * HALF + (one ? 0 : 4 * (e >> 3)) : 16 * Q * e * HALF;
-  }
+  // where row and column (of the wave's S) of the staged values lie
+  __device__ static __forceinline__ int place(int row, int col) { return col * CS + (row >> 4) * SP + (row & 15); }
 
   __device__ static __forceinline__ float2 dpp(float2 v, bool far) {
     auto mv = [&](float x) {
@@ -276,26 +281,32 @@ struct ColumnFft {
     }
   }
 
-  // x: the loads; on return x[r] = element lane % K + K r of column lane / K
+  // From the staged values; x[r] = element lane % K + K r of column lane / K.
   __device__ static __forceinline__ void run(float2 (&x)[16], const float2* __restrict__ twl, float2* __restrict__ ex,
                                              int lane) {
     const float2* tw = twl + lane;
-    asm volatile("" ::: "memory");
     if constexpr (K == 8) {
       const int jj = lane & 15;
+      float2* e = ex + (lane >> 4) * CS + jj;
+#pragma unroll
+      for (int m = 0; m < 16; ++m) x[m] = e[(m >> 3) * 4 * CS + (m & 7) * SP];
+      asm volatile("" ::: "memory");
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         float2 y[8];
 #pragma unroll
         for (int m = 0; m < 8; ++m) y[m] = x[8 * u + m];
         dft_regs<8, false>(y);
-        float2* e = ex + ((lane >> 4) + 4 * u) * 8 * SP + jj;
-        e[0] = y[0];
+        float2* eu = e + 4 * u * CS;
+        eu[0] = y[0];
 #pragma unroll
-        for (int k = 1; k < 8; ++k) e[k * SP] = cmul(y[k], tw[64 * k]);
+        for (int k = 1; k < 8; ++k) eu[k * SP] = cmul(y[k], tw[64 * k]);
       }
     } else {
       const int h = lane % Q, jj = (lane / Q) & 15, col = lane / (16 * Q);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) x[m] = ex[col * CS + (Q * m + h) * SP + jj];
+      asm volatile("" ::: "memory");
       dft_regs<16, false>(x);
       if constexpr (Q > 1) {
 #pragma unroll
@@ -315,13 +326,13 @@ struct ColumnFft {
           x[k] = (h & 1) ? csub(o, x[k]) : cadd(x[k], o);
         }
       }
-      float2* e = ex + (col * K + (Q > 1 ? base_k1(lane) : 0)) * SP + jj;   // k1 = ka + base_k1
+      float2* e = ex + col * CS + (Q > 1 ? base_k1(lane) : 0) * SP + jj;   // k1 = ka + base_k1
 #pragma unroll
       for (int k = 0; k < 16; ++k) e[k * SP] = cmul(x[k], tw[64 * k]);
     }
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < 16; ++j) x[j] = ex[lane * SP + j];
+    for (int j = 0; j < 16; ++j) x[j] = ex[(lane / K) * CS + (lane % K) * SP + j];
     asm volatile("" ::: "memory");
     dft_regs<16, false>(x);
   }
@@ -356,7 +367,7 @@ constexpr int column_waves(int N) { return N == 128 ? 2 : 4; }
 template <int N, bool STORE>
 __global__ void __launch_bounds__(64 * column_waves(N), STORE ? 2 : 3)
 k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtrs gp, QuadTurns ev, ApIso ap,
-          df rout2, const float2* __restrict__ tw_g, int groups, float2* __restrict__ out) {
+          df rout2, const float2* __restrict__ tw_g, int groups, int part, int parts, float2* __restrict__ out) {
   typedef ColumnFft<N> Fft;
   constexpr int S = Fft::S, K = Fft::K, HALF = N / 2, GCOLS = HALF + 1;
   constexpr int NW = column_waves(N), CG = S * NW;   // columns a workgroup
@@ -370,48 +381,63 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
   Fft::twiddles(twl, tw_g, tid, 64 * NW);
   __syncthreads();
   float2* ex = exS[w];
+  // part `part` of `parts`: BF pixels [lo, hi) into its share of the groups
+  const int nbf = info->nbf;
+  const int lo = (int)((long long)nbf * part / parts), hi = (int)((long long)nbf * (part + 1) / parts);
+  const int gpp = groups / parts;
   // workgroups go round the 8 XCDs: XCD x takes the groups x, x + 8, ..., the
-  // low columns (the long items) first; the items of column N/2 come last, a
-  // group a wave
-  const int items = groups * NCG;
-  int cg = NCG, gl = ((int)blockIdx.x - items) * NW + w;
-  if ((int)blockIdx.x < items) {
-    const int per = groups / 8 * LG, k8 = blockIdx.x >> 3;
-    const int line = k8 / per, rem = k8 - line * per;
-    cg = line * LG + rem % LG;
-    gl = rem / LG * 8 + (blockIdx.x & 7);
-  }
-  const bool last = cg == NCG;
-  if (gl >= groups) return;                             // (only waves of column N/2, which meet no barrier)
-  const int n = group_count(gl, groups, info->nbf);  // BF pixels gl + i groups
-  const int jbase = last ? 0 : cg * CG + S * w;
+  // low columns (the long items) first, column N/2 last
+  const int per = gpp / 8 * LG, k8 = blockIdx.x >> 3;
+  const int line = k8 / per, rem = k8 - line * per;
+  const bool last = line * LG >= NCG;                // one item a group, of the columns that hold slot 0
+  const int cg = last ? 0 : line * LG + rem % LG;
+  const int gl = (last ? k8 - NCG / LG * per : rem / LG) * 8 + (blockIdx.x & 7);
+  const int n = group_count(gl, gpp, hi - lo);
+  const int bg = lo + gl;                            // BF pixels bg + i gpp
+  const int jbase = cg * CG + S * w;
   const int col = lane / K, k1 = lane % K;
   const int j = last ? HALF : jbase + col;           // the lane's column after the transform
   const bool first_col = jbase == 0;                 // wave-uniform: it holds slot 0
-  const bool live = !last || col == 0;
+  const bool live = !last || (w == 0 && col == 0);
 
-  const unsigned loff = Fft::load_lane(lane, last);
-  float2 h[16];
+  // the workgroup's rows of CG columns, 16 bytes a lane and load, whole pieces
+  // of H's lines, to the waves' columns through LDS
+  constexpr int ROWS = 64 * NW / (CG / 2), VEC = N / ROWS;
+  static_assert(VEC == 8, "8 loads a lane");
+  const int lrow = tid / (CG / 2), lcol = tid % (CG / 2) * 2;
+  const unsigned loff = lrow * (HALF / 2) + lcol / 2;
+  float4 h[VEC];
   auto fetch = [&](int b) {
-    const float2* hb = H + (long long)b * N * HALF + jbase;
+    const float4* hb = reinterpret_cast<const float4*>(H + (long long)b * N * HALF + cg * CG);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float2* he = hb + Fft::load_step(e, last);
+    for (int e = 0; e < VEC; ++e) {
+      const float4* he = hb + e * ROWS * (HALF / 2);
       asm volatile("" : "+s"(he));   // a scalar address and one lane offset for all
       h[e] = he[loff];
+    }
+  };
+  float2* const st0 = exS[lcol / S] + Fft::place(lrow, lcol % S);
+  float2* const st1 = exS[(lcol + 1) / S] + Fft::place(lrow, (lcol + 1) % S);
+  auto stage = [&]() {
+    lds_barrier();                                   // every wave is done with the pixel before
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      constexpr int step = ROWS / 16 * Fft::SP;
+      static_assert(ROWS % 16 == 0, "a load moves whole sequences on");
+      st0[e * step] = make_float2(h[e].x, h[e].y);
+      st1[e * step] = make_float2(h[e].z, h[e].w);
     }
   };
 
   if constexpr (STORE) {
     if (n == 0) return;
-    fetch(gl);
+    fetch(bg);
     for (int i = 0; i < n; ++i) {
-      const int b = gl + i * groups;
+      const int b = bg + i * gpp;
+      stage();
+      fetch(min(b + gpp, bg + (n - 1) * gpp));
+      lds_barrier();
       float2 x[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) x[e] = h[e];
-      __builtin_amdgcn_s_barrier();
-      fetch(min(b + groups, gl + (n - 1) * groups));
       Fft::run(x, twl, ex, lane);
       float2* gb = out + (long long)b * GCOLS * N;
       if (first_col) {
@@ -439,24 +465,27 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
     for (int r = 0; r < 16; ++r) acc[r].init();
     nyq.init();
     for (int c0 = 0; c0 < n; c0 += 64) {
-      const QuadPixel pl = quad_pixel(gp, gl + min(c0 + lane, n - 1) * groups, ev, rout2);
+      const QuadPixel pl = quad_pixel(gp, bg + min(c0 + lane, n - 1) * gpp, ev, rout2);
       // the same for every wave of the workgroup
       unsigned long long mask =
           __ballot(c0 + lane < n && apertures_reach(pl, rout2.hi, -INFINITY, INFINITY, y0, y1));
       if (!mask) continue;
       int l = __builtin_ctzll(mask);
-      fetch(gl + (c0 + l) * groups);
+      fetch(bg + (c0 + l) * gpp);
       while (true) {
         const QuadPixel p = pixel_of_lane(pl, l);
-        const int b = gl + (c0 + l) * groups;
+        const int b = bg + (c0 + l) * gpp;
         mask &= mask - 1;
         l = mask ? __builtin_ctzll(mask) : l;
+        stage();
+        fetch(bg + (c0 + l) * gpp);               // the next pixel's, while this one's are summed
+        lds_barrier();
+        if (last && w != 0) {
+          if (!mask) break;
+          continue;
+        }
         float2 x[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) x[e] = h[e];
         Fft::run(x, twl, ex, lane);
-        if (!last) __builtin_amdgcn_s_barrier();
-        fetch(gl + (c0 + l) * groups);
         if (first_col) Fft::put(x, ex, lane);
         const float Bq = qy * p.ky2, tq = qy * p.ty;
         const float cq = live ? p.cb - qy * qy : -INFINITY;
@@ -485,7 +514,7 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
       }
     }
     if (!live) return;
-    float2* sp = out + (long long)gl * N * N;
+    float2* sp = out + (long long)(part * gpp + gl) * N * N;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int q = k1 + K * r;
@@ -500,16 +529,20 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
 // ------------------------------------------------------------------------
 // Launch
 // ------------------------------------------------------------------------
-// From H: N = 512 and 1024.  A wave's loads take 32 bytes of every 128-byte
-// line of H at N <= 256 and keep few waves busy there (16 points a lane are
-// 8 waves a CU at 256): 151 us against k_trotter_wave's 119 at N = 256 and 114
-// against k_trotter_slots' 53 at 128, but NEW_512 us against 867 at 512.
-bool columns_path(int N, const Optics& o) { return N >= 512 && optics_isotropic(o); }
+// From H: N >= 256.  At 128 a wave's 16 points a lane keep few waves busy: 94 us
+// in 64 groups and 49 in 192, with 9 and 22 us to sum the planes, against
+// k_trotter_slots' 53 and 9.
+bool columns_path(int N, const Optics& o) { return N >= 256 && optics_isotropic(o); }
 
-// BF groups (partial planes): the tuner's candidates, the default first.
-int columns_variants(int N) { return N == 512 ? 3 : 1; }
+// BF groups (partial planes): the tuner's candidates, the default first.  Whole
+// rounds of the 8 XCDs in each of two parts.  At N = 256 (800 BF pixels) 64, 96
+// and 128 take 112, 93 and 91 us, their sums 8, 10 and 13; at 512 32, 64 and
+// 128 take 263, 277 and 305, their sums 14, 24 and 54.
+int columns_variants(int N) { return N == 512 ? 3 : (N == 256 ? 5 : 1); }
 int columns_groups(int N, int variant) {
-  return N == 512 ? 32 >> (variant > 0 && variant < 3 ? variant : 0) : 8;
+  static const int g256[5] = {96, 64, 48, 32, 16};
+  if (variant < 0 || variant >= columns_variants(N)) variant = 0;
+  return N == 512 ? 32 >> variant : (N == 256 ? g256[variant] : 8);
 }
 // 4096 waves where the partial planes are few: four a SIMD, all in flight at once
 // (with three a SIMD a third of them made a second round: 60 us for 53 at N = 256)
@@ -540,15 +573,17 @@ hipError_t launch_object_tiles(int N, const float2* Gt, const BfInfo* info, cons
 
 hipError_t launch_columns_trotter(int N, const float2* H, const BfInfo* info, const GeomPtrs& gp, const QuadTurns& ev,
                                   const Optics& o, const float2* tw, float2* S_part, int variant, hipStream_t s,
-                                  int* groups_used) {
+                                  int* groups_used, int part, int parts) {
   df rout2;
   const ApIso ap = iso_aperture(o, rout2);
-  const int groups = columns_groups(N, variant), nw = column_waves(N);   // groups: whole rounds of the 8 XCDs
-  const unsigned grid = (unsigned)(groups * (N / 2 / (1024 / N * nw)) + (groups + nw - 1) / nw);
+  const int groups = columns_groups(N, variant), nw = column_waves(N);
+  if (parts < 1 || part < 0 || part >= parts || groups % (8 * parts)) return hipErrorInvalidValue;
+  const unsigned grid = (unsigned)(groups / parts * (N / 2 / (1024 / N * nw) + 1));
 #define QSSB_CALL(NN)                                                                                               \
   hipLaunchKernelGGL((k_columns<NN, false>), dim3(grid), dim3(64 * column_waves(NN)), 0, s, H, info, gp, ev, ap, rout2, \
-                     tw, groups, S_part)
+                     tw, groups, part, parts, S_part)
   switch (N) {
+    case 256: QSSB_CALL(256); break;
     case 512: QSSB_CALL(512); break;
     case 1024: QSSB_CALL(1024); break;
     default: return hipErrorInvalidValue;
@@ -565,7 +600,7 @@ hipError_t launch_columns_store(int N, const float2* H, const BfInfo* info, cons
   const unsigned grid = (unsigned)(groups * (N / 2 / (1024 / N * column_waves(N))));
 #define QSSB_CALL(NN)                                                                                                \
   hipLaunchKernelGGL((k_columns<NN, true>), dim3(grid), dim3(64 * column_waves(NN)), 0, s, H, info, gp, QuadTurns{}, ApIso{}, df{0.f, 0.f}, \
-                     tw, groups, Gt)
+                     tw, groups, 0, 1, Gt)
   QSSB_BY_SIZE(QSSB_CALL)
 #undef QSSB_CALL
   return hipGetLastError();

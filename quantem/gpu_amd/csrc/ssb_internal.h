@@ -246,22 +246,19 @@ hipError_t launch_phasors(int N, const BfInfo* info, int nbf_hint, const GeomPtr
 // Trotter over Hermitian slot columns: from the row-transformed stack H
 // (fused scan-column FFT; from_h) or, with unequal detector sampling, from the
 // resident stack Gt[b][c][q], c = 0..N/2.  Writes partial planes S_part[g][c][q].
-// variant: kernel of the reconstruction path's trotter, 0 (default) to
-// trotter_variants(N) - 1 (at N = 256, 0 and 1 are the wave-local kernel and
-// 2..4 the tile shapes); other paths always use variant 0.  groups_used receives
-// the number of partial planes written (launch_finish_object's `groups`).
+// variant: tile shape of a reconstruction at N = 128 with equal sampling, 0
+// (default) to trotter_variants(N) - 1; other paths always use variant 0.
+// groups_used receives the number of partial planes written
+// (launch_finish_object's `groups`).
 int trotter_variants(int N);
 hipError_t launch_trotter_slots(int N, bool from_h, const float2* src, const BfInfo* info, const GeomPtrs& gp,
                                 const float2* rowph, const float2* colph, const float2* echi, const Optics& o,
                                 const float2* tw, float2* S_part, int variant, hipStream_t s,
-                                int* groups_used = nullptr, int part = 0, int parts = 1);
-// Whether launch_trotter_slots takes the wave-local kernel (which can run
-// in BF parts: part p of `parts` sums its share of the BF pixels into its
-// share of the partial planes).
-bool trotter_wave_path(int N, bool from_h, const Optics& o, int variant);
+                                int* groups_used = nullptr);
 // The same for equal detector sampling: from a resident Hermitian stack, and
 // where columns_path holds from H, in columns_groups(N, variant) BF groups,
-// variant < columns_variants(N).
+// variant < columns_variants(N); part p of `parts` sums its share of the BF
+// pixels into its share of the partial planes.
 bool columns_path(int N, const Optics& o);
 int columns_variants(int N);
 int columns_groups(int N, int variant);
@@ -270,7 +267,7 @@ hipError_t launch_object_tiles(int N, const float2* Gt, const BfInfo* info, cons
                                const Optics& o, float2* S_part, hipStream_t s, int* groups_used);
 hipError_t launch_columns_trotter(int N, const float2* H, const BfInfo* info, const GeomPtrs& gp, const QuadTurns& ev,
                                   const Optics& o, const float2* tw, float2* S_part, int variant, hipStream_t s,
-                                  int* groups_used);
+                                  int* groups_used, int part = 0, int parts = 1);
 // H to the resident stack Gt[b][c][q], c <= N/2.
 hipError_t launch_columns_store(int N, const float2* H, const BfInfo* info, const GeomPtrs& gp, const float2* tw,
                                 float2* Gt, hipStream_t s);

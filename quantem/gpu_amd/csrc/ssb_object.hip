@@ -299,484 +299,6 @@ k_trotter_slots(const float2* __restrict__ src, const BfInfo* __restrict__ info,
 }
 
 // ------------------------------------------------------------------------
-// Wave-local fused column FFT + trotter of the reconstruction (row-transformed
-// stack H, isotropic detector sampling).  A workgroup of NW waves takes one
-// BF group and NW * CPW adjacent slot columns (8 waves x 2 columns: the 128
-// bytes of every row of H that one cache line holds), and each wave owns CPW
-// of those columns for every BF pixel of the group.  Lane l holds rows
-// l + 64 m (m < R = N / 64): one 16- or 8-byte load per row brings the
-// wave's columns.  The column FFT needs no workgroup barrier: an R-point DFT
-// in registers (stride-64 elements) with twiddles w_N^(l k1), then 64-point
-// Stockham radix-4 stages over the CPW R sequences through the wave's own
-// LDS (every lane reads its operands before any lane writes), so
-// X[k1 + R k2] = Z_k1[k2]; the last stage's outputs stay in the registers of
-// the lane that computed them, lane l holding q = wave_qlane(l) + 64 r.
-// Per point the trotter term is that of k_trotter_slots (same double-float
-// apertures, phasors and guard), with Kahan FP32 sums over the group's BF
-// pixels.  The aperture of a point far from the soft edge is decided from
-// a float32 estimate of d (error < 2e-5 for |terms| < 32, inside the 1e-4
-// margin of aperture_sum); only points near the edge evaluate d in
-// double-float.  Outputs B of the mirror points are written as -conj(A);
-// column N/2 (slot 0) is accumulated with A; the Nyquist-row outputs
-// S(N/2, N - j) are summed after the BF loop, one BF pixel per lane, from
-// the G_b(N/2, j) lane 0 holds.  The column terms of d for each (BF pixel,
-// column) are computed once per workgroup into LDS, 64 BF pixels at a time;
-// H and the phasors of the next BF pixel are loaded while this one is
-// transformed.  Items (BF group, column group) start heavy-first on each
-// XCD: the low slot columns hold more points inside the apertures.
-// ------------------------------------------------------------------------
-constexpr int kWaveColumnsDefault = 2;   // slot columns per wave of the default variant
-constexpr int kWaveTrotterGroups = 64;
-constexpr int kWaveChunk = 64;           // BF pixels per column-term table / Nyquist pass
-
-__device__ __forceinline__ void wave_lds_fence() { asm volatile("" ::: "memory"); }
-
-// Workgroup barrier for LDS only: this wave's LDS operations complete, then
-// s_barrier.  Unlike __syncthreads it does not drain the wave's global loads,
-// so prefetches of H stay in flight across it (their uses wait for them).
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-
-// Column terms of d(Q -/+ k) for one (BF pixel, column): (Rout^2 - |k|^2) -
-// qy^2 +/- 2 qy ky (isotropic sampling).
-struct ColTerm {
-  df A, B;
-};
-
-__device__ __forceinline__ ColTerm col_term(df rout2, df kx, df ky, df qy) {
-  const df cbv = df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky)));
-  const df base = df_sub(cbv, df_mul(qy, qy));
-  const df qk = df_mul(qy, df{2.0f * ky.hi, 2.0f * ky.lo});
-  return ColTerm{df_add(base, qk), df_sub(base, qk)};
-}
-
-// After the wave-local column FFT, lane l holds frequencies
-// q = wave_qlane(l) + 64 r (r = 0..3) of each of its columns: the outputs of the
-// last Stockham stage stay in the registers of the lane that computed them.
-// Per-row tables in LDS are stored in that order, entry 64 r + l for lane l.
-__device__ __forceinline__ int wave_qlane(int lane) { return (lane >> 4) + 4 * (lane & 15); }
-
-// Column c of one row's load: a float4 holds two adjacent slot columns.
-__device__ __forceinline__ float2 column_of(float4 v, int c) {
-  return c ? make_float2(v.z, v.w) : make_float2(v.x, v.y);
-}
-__device__ __forceinline__ float2 column_of(float2 v, int) { return v; }
-
-// Per-BF operands of one wave other than H (loaded one BF pixel ahead).
-template <int R, int CPW>
-struct WaveBf {
-  float2 rowA[R];       // e^{i qx a_b} at the lane's frequencies
-  float2 colp[CPW];     // e^{i qy b_b} at the wave's columns
-  float2 colHalf;       // ... at column N/2
-  float kx, kxl, ak;
-};
-
-template <int N, int R, int CPW>
-__device__ __forceinline__ void wave_bf_load(WaveBf<R, CPW>& o, const float2* __restrict__ rowph_g,
-                                             const float2* __restrict__ colph_g, const GeomPtrs& gp, int b,
-                                             int lane, int j0) {
-  constexpr int HALF = N / 2, GCOLS = HALF + 1;
-#pragma unroll
-  for (int m = 0; m < R; ++m) o.rowA[m] = rowph_g[(long long)b * N + wave_qlane(lane) + 64 * m];
-#pragma unroll
-  for (int c = 0; c < CPW; ++c) o.colp[c] = colph_g[(long long)b * GCOLS + j0 + c];
-  o.colHalf = colph_g[(long long)b * GCOLS + HALF];
-  o.kx = gp.kx[b];
-  o.kxl = gp.kxl[b];
-  o.ak = gp.ak[b];
-}
-
-// Normalised overlap weight and the term G * conj(g) of one point.
-__device__ __forceinline__ float2 trotter_point(float2 G, float am, float app, float2 echi, float2 eth, float ak) {
-  const float wr = (am - app) * echi.x;
-  const float wi = -(am + app) * echi.y;
-  float gr = ak * (eth.x * wr - eth.y * wi);
-  float gi = ak * (eth.x * wi + eth.y * wr);
-  const float mag2 = gr * gr + gi * gi;
-  const float sc = (mag2 > 1e-16f) ? rsqrtf(mag2) : 1e8f;
-  gr *= sc;
-  gi *= sc;
-  return make_float2(G.x * gr + G.y * gi, G.y * gr - G.x * gi);
-}
-
-// One wave's share of a work item: BF pixels [b0, b1) for the CPW slot
-// columns j0, j0 + 1, ...; SLOT0 for the wave holding slot 0, whose first
-// column packs the real columns 0 and N/2.  Every wave of the workgroup calls
-// it with the same BF range (the barriers of the column-term tables match).
-template <int N, int CPW, int NW, bool SLOT0>
-__device__ __forceinline__ void wave_trotter_item(const float2* __restrict__ H, const GeomPtrs& gp,
-                                                  const float2* __restrict__ rowph_g,
-                                                  const float2* __restrict__ colph_g,
-                                                  const float2* __restrict__ echi_g, const ApIso& ap, df rout2,
-                                                  const float2* __restrict__ tw, float2* __restrict__ xb,
-                                                  float2* __restrict__ nyqz,
-                                                  ColTerm (*colT)[CPW * NW + 1],
-                                                  const float2 (*echiS)[N], const df* __restrict__ qxS,
-                                                  const df* __restrict__ q2xS, int cg, int w, int tid, int b0, int b1,
-                                                  float2* __restrict__ sp) {
-  constexpr int HALF = N / 2;
-  constexpr int R = N / 64;
-  constexpr int SP = 65;                 // padded sequence stride in the wave's LDS
-  constexpr int CG = CPW * NW;
-  constexpr int NBH = SLOT0 ? R : 1;     // column N/2 accumulators (slot 0 only)
-  static_assert(CPW == 1 || CPW == 2, "one or two columns per wave");
-  const int lane = tid & 63;
-  const int j0 = cg * CG + CPW * w;
-  Kahan aR[CPW][R], aI[CPW][R], hR[NBH], hI[NBH];
-#pragma unroll
-  for (int c = 0; c < CPW; ++c)
-#pragma unroll
-    for (int m = 0; m < R; ++m) {
-      aR[c][m].init();
-      aI[c][m].init();
-    }
-#pragma unroll
-  for (int i = 0; i < NBH; ++i) {
-    hR[i].init();
-    hI[i].init();
-  }
-  // Nyquist-row sums (wave-uniform), value + running error term
-  df nyR[CPW], nyI[CPW];
-#pragma unroll
-  for (int c = 0; c < CPW; ++c) {
-    nyR[c] = df{0.f, 0.f};
-    nyI[c] = df{0.f, 0.f};
-  }
-  // one load per row brings the wave's CPW columns (16 or 8 bytes)
-  using HV = typename std::conditional<CPW == 2, float4, float2>::type;
-  const HV* hrow = reinterpret_cast<const HV*>(H + (long long)lane * HALF + j0);
-  constexpr long long ROWS64 = 64LL * HALF / CPW;   // HV between rows l and l + 64
-  constexpr long long PER_B = (long long)N * HALF / CPW;
-  HV h[R];
-  // the per-BF operands other than H are loaded one BF pixel ahead with two
-  // columns per wave; with one (a register budget of 168) at the top of the
-  // BF pixel's iteration, where the column FFT covers their latency
-  constexpr bool BF_AHEAD = CPW == 2;
-  WaveBf<R, CPW> nx;
-  if (b0 < b1) {
-#pragma unroll
-    for (int m = 0; m < R; ++m) h[m] = hrow[(long long)b0 * PER_B + m * ROWS64];
-    if (BF_AHEAD) wave_bf_load<N, R, CPW>(nx, rowph_g, colph_g, gp, b0, lane, j0);
-  }
-  for (int c0 = b0; c0 < b1; c0 += kWaveChunk) {
-    const int n = min(kWaveChunk, b1 - c0);
-    // column terms of the chunk's BF pixels at the workgroup's CG columns
-    // and column N/2, computed once for all waves
-    lds_barrier();
-    for (int e = tid; e < n * (CG + 1); e += 64 * NW) {
-      const int bi = e / (CG + 1), ci = e - (e / (CG + 1)) * (CG + 1);
-      const int b = c0 + bi;
-      const int col = (ci < CG) ? cg * CG + ci : HALF;
-      colT[bi][ci] = col_term(rout2, df{gp.kx[b], gp.kxl[b]}, df{gp.ky[b], gp.kyl[b]},
-                              df{gp.qy[col], gp.qyl[col]});
-    }
-    lds_barrier();
-    for (int b = c0; b < c0 + n; ++b) {
-      WaveBf<R, CPW> cu;
-      if constexpr (BF_AHEAD) {
-        cu = nx;
-        if (b + 1 < b1) wave_bf_load<N, R, CPW>(nx, rowph_g, colph_g, gp, b + 1, lane, j0);
-      } else {
-        wave_bf_load<N, R, CPW>(cu, rowph_g, colph_g, gp, b, lane, j0);
-      }
-      // column FFT: in-register radix-4 over m, twiddle, into the wave's LDS.
-      // The exchange runs across the lanes of this wave only: a compiler
-      // memory barrier at each phase boundary keeps every LDS access in
-      // program order (the hardware keeps a wave's LDS operations in order).
-      wave_lds_fence();
-#pragma unroll
-      for (int c = 0; c < CPW; ++c) {
-        float2 x[R];
-#pragma unroll
-        for (int m = 0; m < R; ++m) x[m] = column_of(h[m], c);
-        const float2 apc = cadd(x[0], x[2]), amc = csub(x[0], x[2]);
-        const float2 bpd = cadd(x[1], x[3]), bmd = cmul_mi<false>(csub(x[1], x[3]));
-        xb[(c * R + 0) * SP + lane] = cadd(apc, bpd);
-        xb[(c * R + 1) * SP + lane] = cmul(cadd(amc, bmd), tw[lane & (N - 1)]);
-        xb[(c * R + 2) * SP + lane] = cmul(csub(apc, bpd), tw[(2 * lane) & (N - 1)]);
-        xb[(c * R + 3) * SP + lane] = cmul(csub(amc, bmd), tw[(3 * lane) & (N - 1)]);
-      }
-      // H of the next BF pixel: issued once this one's rows are consumed
-      if (b + 1 < b1) {
-#pragma unroll
-        for (int m = 0; m < R; ++m) h[m] = hrow[(long long)(b + 1) * PER_B + m * ROWS64];
-      }
-      // 64-point Stockham radix-4 stages over the 2R sequences (two
-      // butterflies per lane): all operands are read before any is written.
-      // The last stage's butterfly p of lane l is column p at frequencies
-      // q = wave_qlane(l) + 64 r; it stays in registers (slot 0's wave also
-      // stores it, for the mirror rows N - q its column 0 needs).
-      float2 zq[CPW][4];
-#pragma unroll
-      for (int ns = 1; ns < 64; ns *= 4) {
-        wave_lds_fence();
-        float2 v[CPW][4];
-#pragma unroll
-        for (int p = 0; p < CPW; ++p) {
-          const int it = lane + 64 * p;
-          const int sq = it >> 4, jj = it & 15, k = jj & (ns - 1);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float2 xv = xb[sq * SP + jj + 16 * r];
-            if (ns > 1 && r > 0) xv = cmul(xv, tw[(4 * r * k * (16 / ns)) & (N - 1)]);
-            v[p][r] = xv;
-          }
-        }
-        wave_lds_fence();
-#pragma unroll
-        for (int p = 0; p < CPW; ++p) {
-          const int it = lane + 64 * p;
-          const int sq = it >> 4, jj = it & 15, k = jj & (ns - 1);
-          const int base = sq * SP + (jj / ns) * ns * 4 + k;
-          const float2 apc = cadd(v[p][0], v[p][2]), amc = csub(v[p][0], v[p][2]);
-          const float2 bpd = cadd(v[p][1], v[p][3]), bmd = cmul_mi<false>(csub(v[p][1], v[p][3]));
-          const float2 o[4] = {cadd(apc, bpd), cadd(amc, bmd), csub(apc, bpd), csub(amc, bmd)};
-          if (ns < 16 || SLOT0) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) xb[base + r * ns] = o[r];
-          }
-          if (ns == 16) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) zq[p][r] = o[r];
-          }
-        }
-      }
-      wave_lds_fence();
-      // G_b(N/2, j0 + c) for the deferred Nyquist pass (lane 0 holds q = N/2 at r = 2)
-      static_assert(HALF == 128, "q = N/2 is lane 0's r = 2");
-      if (lane == 0) {
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) nyqz[CPW * (b - c0) + c] = zq[c][2];
-      }
-      ColTerm ct[CPW];
-#pragma unroll
-      for (int c = 0; c < CPW; ++c) ct[c] = colT[b - c0][CPW * w + c];
-      const float ak = cu.ak;
-      const df kx2{2.0f * cu.kx, 2.0f * cu.kxl};
-      // LDS operands of the lane's points at q = wave_qlane(lane) + 64 m
-      // (table entry 64 m + lane), read one row ahead so that no point waits
-      // on its own reads
-      struct RowOps {
-        df qx, q2x;
-        float2 e[CPW];
-      };
-      auto row_ops = [&](int m, RowOps& o) {
-        const int i = lane + 64 * m;
-        o.qx = qxS[i];
-        o.q2x = q2xS[i];
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) o.e[c] = echiS[CPW * w + c][i];
-      };
-      RowOps next_ops;
-      row_ops(0, next_ops);
-#pragma unroll
-      for (int m = 0; m < R; ++m) {
-        const int q = wave_qlane(lane) + 64 * m;
-        const RowOps ops = next_ops;
-        if (m + 1 < R) row_ops(m + 1, next_ops);
-        const df qx = ops.qx;
-        const df q2x = ops.q2x;
-        const float uq = row_estimate_minus(qx, kx2, q2x);
-        const float vq = row_estimate_plus(qx, kx2, q2x);
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) {
-          const float2 z = zq[c][m];
-          float2 GA;
-          if (SLOT0 && c == 0) {
-            const int qq = (N - q) & (N - 1);
-            const float2 zm = xb[(qq & 3) * SP + (qq >> 2)];
-            GA = make_float2(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y));
-          } else {
-            GA = z;
-          }
-          float am, app;
-          iso_aperture_pair(uq, vq, qx, kx2, q2x, ct[c].A, ct[c].B, ap, am, app);
-          if (am != 0.0f || app != 0.0f) {
-            const float2 t = trotter_point(GA, am, app, ops.e[c], cmul(cu.rowA[m], cu.colp[c]), ak);
-            aR[c][m].add(t.x);
-            aI[c][m].add(t.y);
-          }
-          if constexpr (SLOT0) {
-            if (c == 0) {
-              // output B of slot 0: column N/2 at row q
-              const int qq = (N - q) & (N - 1);
-              const float2 zm = xb[(qq & 3) * SP + (qq >> 2)];
-              const float2 GB = make_float2(0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x));
-              const ColTerm th = colT[b - c0][CG];
-              float bm, bp;
-              iso_aperture_pair(uq, vq, qx, kx2, q2x, th.A, th.B, ap, bm, bp);
-              if (bm != 0.0f || bp != 0.0f) {
-                const float2 t = trotter_point(GB, bm, bp, echiS[CG][lane + 64 * m], cmul(cu.rowA[m], cu.colHalf), ak);
-                hR[m].add(t.x);
-                hI[m].add(t.y);
-              }
-            }
-          }
-          // one point at a time: keeps the scheduler from overlapping the
-          // points' temporaries
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    }
-    // Nyquist-row terms of the chunk: lane i takes BF pixel c0 + i
-    wave_lds_fence();
-    {
-      float2 t[CPW];
-#pragma unroll
-      for (int c = 0; c < CPW; ++c) t[c] = make_float2(0.f, 0.f);
-      if (lane < n) {
-        const int b = c0 + lane;
-        const float ak = gp.ak[b];
-        const df u = df_mul(qxS[HALF], df{2.0f * gp.kx[b], 2.0f * gp.kxl[b]});
-        const df rowTA = df_sub(u, q2xS[HALF]);
-        const df rowTB = df_neg(df_add(q2xS[HALF], u));
-        const float2 rA = rowph_g[(long long)b * N + HALF];
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) {
-          const int j = j0 + c;
-          if (j == 0) continue;          // slot 0: column N/2 holds this point
-          const ColTerm ctn = colT[lane][CPW * w + c];
-          const float bm = aperture_sum(rowTA, ctn.B, ap);
-          const float bp = aperture_sum(rowTB, ctn.A, ap);
-          if (bm != 0.0f || bp != 0.0f) {
-            const float2 echiB = echi_g[(long long)((N - j) & (N - 1)) * N + HALF];
-            const float2 eB = cmul(rA, cconj(colph_g[(long long)b * (HALF + 1) + j]));
-            t[c] = trotter_point(cconj(nyqz[CPW * lane + c]), bm, bp, echiB, eB, ak);
-          }
-        }
-      }
-      // compensated xor tree over the lanes: two_sum's error term is exact,
-      // so every lane holds the same (sum, error) pair
-#pragma unroll
-      for (int c = 0; c < CPW; ++c) {
-        df re{t[c].x, 0.f}, im{t[c].y, 0.f};
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-          const df ro{__shfl_xor(re.hi, off, 64), __shfl_xor(re.lo, off, 64)};
-          const df io{__shfl_xor(im.hi, off, 64), __shfl_xor(im.lo, off, 64)};
-          const df rs = two_sum(re.hi, ro.hi), is = two_sum(im.hi, io.hi);
-          re = df{rs.hi, (re.lo + ro.lo) + rs.lo};
-          im = df{is.hi, (im.lo + io.lo) + is.lo};
-        }
-        const df rs = two_sum(nyR[c].hi, re.hi), is = two_sum(nyI[c].hi, im.hi);
-        nyR[c] = df{rs.hi, (nyR[c].lo + re.lo) + rs.lo};
-        nyI[c] = df{is.hi, (nyI[c].lo + im.lo) + is.lo};
-      }
-    }
-    wave_lds_fence();
-  }
-#pragma unroll
-  for (int m = 0; m < R; ++m) {
-    const int q = wave_qlane(lane) + 64 * m;
-    const int qm = (N - q) & (N - 1);
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      const int j = j0 + c;
-      const float2 outA = make_float2(aR[c][m].s - aR[c][m].c, aI[c][m].s - aI[c][m].c);
-      sp[(long long)j * N + q] = outA;
-      if (j == 0) {
-        if constexpr (SLOT0) sp[(long long)HALF * N + q] = make_float2(hR[m].s - hR[m].c, hI[m].s - hI[m].c);
-      } else if (q != HALF) {
-        sp[(long long)(N - j) * N + qm] = make_float2(-outA.x, outA.y);
-      } else {
-        sp[(long long)(N - j) * N + HALF] = make_float2(nyR[c].hi + nyR[c].lo, nyI[c].hi + nyI[c].lo);
-      }
-    }
-  }
-}
-
-template <int N, int CPW, int NW, int WAVES_PER_SIMD>
-__global__ void __launch_bounds__(64 * NW, WAVES_PER_SIMD)
-k_trotter_wave(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtrs gp,
-               const float2* __restrict__ rowph_g, const float2* __restrict__ colph_g,
-               const float2* __restrict__ echi_g, ApIso ap, df rout2, const float2* __restrict__ tw_g, int groups,
-               float2* __restrict__ S_part, int part, int parts) {
-  constexpr int HALF = N / 2;
-  constexpr int R = N / 64;
-  static_assert(R == 4, "the in-register pass is radix 4");
-  constexpr int W = NW;
-  constexpr int CG = CPW * W;            // slot columns per workgroup
-  constexpr int NCG = HALF / CG;
-  // LG workgroups share the 16 slot columns of one 128-byte line of H
-  constexpr int LG = 16 / CG;
-  constexpr int NL = NCG / LG;           // line groups (8)
-  static_assert(CG <= 16 && 16 % CG == 0 && NL == 8, "workgroup columns must tile a line of H");
-  constexpr int SP = 65;
-  __shared__ float2 tw[N];
-  __shared__ float2 xbuf[W][CPW * R * SP];
-  __shared__ float2 nyqz[W][CPW * kWaveChunk];
-  __shared__ ColTerm colT[kWaveChunk][CG + 1];
-  __shared__ float2 echiS[CG + 1][N];    // e^{i chi} of the CG columns and of column N/2
-  __shared__ df qxS[N], q2xS[N];
-  const int tid = threadIdx.x;
-  const int w = tid >> 6;
-  // qxS, q2xS and echiS in lane order: entry 64 r + l is frequency
-  // wave_qlane(l) + 64 r (entry N/2 is q = N/2 itself)
-  for (int i = tid; i < N; i += 64 * W) {
-    tw[i] = tw_g[i];
-    const int q = wave_qlane(i & 63) + (i & ~63);
-    const df qx{gp.qx[q], gp.qxl[q]};
-    qxS[i] = qx;
-    q2xS[i] = df_mul(qx, qx);
-  }
-  // part `part` of `parts`: BF pixels [lo, hi) into partial planes
-  // [part * gpp, (part + 1) * gpp), gpp = groups / parts
-  const int nbf_all = info->nbf;
-  const int lo = (int)((long long)nbf_all * part / parts);
-  const int hi = (int)((long long)nbf_all * (part + 1) / parts);
-  const int gpp = groups / parts;
-  const long long items = (long long)gpp * NCG;
-  for (long long item = blockIdx.x; item < items; item += gridDim.x) {
-    // Workgroups go round-robin over the 8 XCDs and, within one, start in
-    // order as CUs free up.  XCD x takes the BF groups x, x + 8, ...; its
-    // items run line by line of H in increasing slot order -- the low slot
-    // columns hold more points inside the apertures, so the long items start
-    // first and the short ones fill in at the end -- and the LG items that
-    // share a line of H are consecutive (read once per L2).
-    const int xcd = (int)(item & 7);
-    const long long k8 = item >> 3;
-    const int gx = gpp / 8;                // BF groups per XCD
-    const int line = (int)(k8 / (gx * LG));
-    const int rem = (int)(k8 % (gx * LG));
-    const int gl = (rem / LG) * 8 + xcd;
-    const int cg = line * LG + rem % LG;
-    const int g = part * gpp + gl;
-    int b0, b1;
-    group_range(gl, gpp, hi - lo, b0, b1);
-    b0 += lo;
-    b1 += lo;
-    __syncthreads();
-    {
-      // all of a thread's loads are issued before its LDS stores
-      constexpr int FILL = ((CG + 1) * N + 64 * W - 1) / (64 * W);
-      float2 ev[FILL];
-#pragma unroll
-      for (int k = 0; k < FILL; ++k) {
-        const int i = tid + k * 64 * W;
-        if (i < (CG + 1) * N) {
-          const int c = i / N, e = i - (i / N) * N;
-          const int col = (c < CG) ? cg * CG + c : HALF;
-          ev[k] = echi_g[(long long)col * N + wave_qlane(e & 63) + (e & ~63)];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < FILL; ++k) {
-        const int i = tid + k * 64 * W;
-        if (i < (CG + 1) * N) echiS[i / N][i - (i / N) * N] = ev[k];
-      }
-    }
-    // (the first column-term table's barrier orders these writes)
-    float2* sp = S_part + (long long)g * N * N;
-    if (cg == 0 && w == 0)
-      wave_trotter_item<N, CPW, NW, true>(H, gp, rowph_g, colph_g, echi_g, ap, rout2, tw, xbuf[w], nyqz[w], colT, echiS, qxS,
-                                 q2xS, cg, w, tid, b0, b1, sp);
-    else
-      wave_trotter_item<N, CPW, NW, false>(H, gp, rowph_g, colph_g, echi_g, ap, rout2, tw, xbuf[w], nyqz[w], colT, echiS, qxS,
-                                  q2xS, cg, w, tid, b0, b1, sp);
-  }
-}
-
-// ------------------------------------------------------------------------
 // Trotter from a full (non-Hermitian) stack Gt[b][c][q], c < N: each full
 // column is its own output (test seam for imported full-plane stacks).
 // ------------------------------------------------------------------------
@@ -968,59 +490,27 @@ hipError_t launch_phasors(int N, const BfInfo* info, int nbf_hint, const GeomPtr
 }
 
 // Tile shapes (SG slot columns, BLOCK threads) of the fused column FFT +
-// trotter on the row-transformed stack (the reconstruction path); variant 0
-// is the default, the others are the tuner's candidates.  SG is even there:
-// each lane's 16-byte staging copy moves two adjacent slots of a row of H.
-// At N = 256 variants 0 and 1 are the wave-local kernel (the object path of
-// a reconstruction: row-transformed stack, isotropic sampling) with
-// kWaveColumnsDefault columns per wave and with the other count, and 2..4
-// are the workgroup-tile shapes below; at N = 128 the tile shapes only.
-// From N = 512 on equal sampling goes through ssb_columns.hip (columns_path),
-// whose variants are numbers of BF groups.
-int trotter_variants(int N) { return N >= 512 ? columns_variants(N) : (N == 256 ? 5 : 3); }
-
-static int wave_columns(int variant) { return variant == 0 ? kWaveColumnsDefault : 3 - kWaveColumnsDefault; }
+// trotter on the row-transformed stack (the reconstruction path); at N = 128
+// with equal sampling variant 0 is the default, the others are the tuner's
+// candidates.  SG is even there: each lane's 16-byte staging copy moves two
+// adjacent slots of a row of H.  From N = 256 on equal sampling goes through
+// ssb_columns.hip (columns_path), whose variants are numbers of BF groups.
+int trotter_variants(int N) { return N >= 256 ? columns_variants(N) : 3; }
 
 int trotter_groups_max(int N) {
-  int g = N == 256 ? kWaveTrotterGroups : object_groups(N);
+  int g = object_groups(N);
   g = object_tile_groups(N) > g ? object_tile_groups(N) : g;
-  for (int v = 0; N >= 512 && v < columns_variants(N); ++v) g = columns_groups(N, v) > g ? columns_groups(N, v) : g;
+  for (int v = 0; N >= 256 && v < columns_variants(N); ++v) g = columns_groups(N, v) > g ? columns_groups(N, v) : g;
   return g;
-}
-
-bool trotter_wave_path(int N, bool from_h, const Optics& o, int variant) {
-  return N == 256 && from_h && optics_isotropic(o) && (variant == 0 || variant == 1);
 }
 
 hipError_t launch_trotter_slots(int N, bool from_h, const float2* src, const BfInfo* info, const GeomPtrs& gp,
                                 const float2* rowph, const float2* colph, const float2* echi, const Optics& o,
-                                const float2* tw, float2* S_part, int variant, hipStream_t s, int* groups_used,
-                                int part, int parts) {
+                                const float2* tw, float2* S_part, int variant, hipStream_t s, int* groups_used) {
   df rout2;
   const ApIso ap = iso_aperture(o, rout2);
   const bool iso = optics_isotropic(o);
-  if (trotter_wave_path(N, from_h, o, variant)) {
-    constexpr int groups = kWaveTrotterGroups;
-    // (the item order gives each XCD groups / parts / 8 BF groups)
-    if (parts < 1 || part < 0 || part >= parts || groups % (8 * parts)) return hipErrorInvalidValue;
-    // one column per wave in 4-wave workgroups (3 per CU at <= 168 VGPRs),
-    // or two per wave in 8-wave workgroups (one per CU)
-    const int cpw = wave_columns(variant);
-    const int nw = cpw == 1 ? 4 : 8;
-    const unsigned grid = grid_items((long long)(groups / parts) * ((256 / 2) / (cpw * nw)), 65536);
-    if (cpw == 1)
-      hipLaunchKernelGGL((k_trotter_wave<256, 1, 4, 3>), dim3(grid), dim3(64 * 4), 0, s, src, info, gp, rowph, colph,
-                         echi, ap, rout2, tw, groups, S_part, part, parts);
-    else
-      hipLaunchKernelGGL((k_trotter_wave<256, 2, 8, 2>), dim3(grid), dim3(64 * 8), 0, s, src, info, gp, rowph, colph,
-                         echi, ap, rout2, tw, groups, S_part, part, parts);
-    if (groups_used) *groups_used = groups;
-    return hipGetLastError();
-  }
-  if (parts != 1) return hipErrorInvalidValue;
-  // workgroup-tile shapes: at N = 256 their variants follow the wave-local ones
-  if (N == 256 && variant > 0) variant = variant >= 2 ? variant - 2 : 0;
-  if (iso && (!from_h || N >= 512)) return hipErrorInvalidValue;   // ssb_columns.hip's
+  if (iso && (!from_h || N != 128)) return hipErrorInvalidValue;   // ssb_columns.hip's
   const int groups = object_groups(N);
   if (groups_used) *groups_used = groups;
 #define QSSB_SLOTS_ONE(NN, SGV, BL, FH, IS)                                                                 \
@@ -1045,10 +535,7 @@ hipError_t launch_trotter_slots(int N, bool from_h, const float2* src, const BfI
       else QSSB_SLOTS(128, 4, 256);
       break;
     case 256:
-      if (iso && variant == 1) QSSB_SLOTS_ISO(256, 4, 256);
-      else if (iso && variant == 2) QSSB_SLOTS_ISO(256, 2, 512);
-      else if (iso) QSSB_SLOTS_ISO(256, 2, 256);
-      else QSSB_SLOTS(256, 2, 256);
+      QSSB_SLOTS(256, 2, 256);
       break;
     case 512:
       QSSB_SLOTS(512, 2, 512);
