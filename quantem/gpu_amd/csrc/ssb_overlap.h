@@ -149,6 +149,8 @@ __device__ __forceinline__ void sincos_half_turns(float r, float& s, float& c) {
 // bit): the other side is meant.  The caller takes points whose s is a whole
 // number (the sine vanishes) and small A(k) through gamma_hat_st.
 __device__ __forceinline__ float2 overlap_unit(float2 G, bool both, float s, float t, unsigned flip) {
+  // (contracted, t's last product would round here by where this is inlined)
+#pragma clang fp contract(off)
   const float a = t + (both ? -0.5f : -s);
   const float n = rintf(a);
   float sn, cs;
