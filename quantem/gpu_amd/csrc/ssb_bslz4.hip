@@ -16,12 +16,13 @@
 // Three kernels:
 //   k_bslz4_index   one thread per chunk: validates the header and walks the
 //                   block sizes into a descriptor table (bounds-checked);
-//   k_bslz4_parse   only for blocks too large to stage in LDS, one thread per
-//                   block: walks the block's LZ4 sequence headers (every
-//                   length and offset checked) into a table of {literal
-//                   start, literal length, offset, match length} per sequence;
+//   k_bslz4_parse   one thread per block: walks the block's LZ4 sequence
+//                   headers (every length and offset checked) into a table of
+//                   {literal start, literal length, offset, match length} per
+//                   sequence; of blocks that the decode searches itself, none;
 //   k_bslz4_decode  one 64-lane workgroup per block: stages the compressed
-//                   block in LDS as whole words, finds its sequences there, and
+//                   block in LDS as whole words, finds its sequences there or
+//                   reads them from the table, and
 //                   decodes it in LDS in rounds of up to 64 sequences (one
 //                   lane per sequence: all of the round's literal runs at
 //                   once, then its matches in order; a match of offset d <
@@ -33,12 +34,7 @@
 // Where the sequences of a block start is a chain through its bytes, but where
 // each would end if it started there is not: the lanes find that for every
 // byte at once (lz4_next), and the chain is one LDS read for two sequences.
-// A thread walking one block from memory waits for a line every few sequences
-// and for the longest of its wave's 64 blocks: at 16384 frames of 192 x 192
-// (38 sequences a block, median 7) such a pass took 398 us beside the
-// decode's 718; now the decode takes 868 us in all, bound by its vector
-// instructions (2550 a block).  Workgroups that fetch their next block ahead
-// are slower (1378 us): the hardware's dispatch evens out the blocks better.
+// kSearchBytes says which way is taken.
 // Malformed input never reads or writes out of bounds: it sets a bit in the
 // status word and the block is skipped.
 #include <cstring>
@@ -60,6 +56,16 @@ constexpr int kMaxCompBytes = kMaxBlockBytes + kMaxBlockBytes / 255 + 16;  // LZ
 // sequences fit where it will be decoded (4 bytes for each of its own).
 constexpr int kStageBytes = 2048;
 static_assert(4 * kStageBytes <= kMaxBlockBytes && kStageBytes == 64 * 32, "lz4_next's table and run_255's bits");
+
+// Up to this many compressed bytes in all, the decode searches its staged blocks
+// for their sequences; beyond, the parse does.  A thread that walks its block
+// from memory waits for a line every few sequences, and its wave for the
+// longest of 64 blocks: ~400 us however few the blocks, and little more for
+// many.  The search costs the decode, which its vector instructions bound, 4 us
+// per MB of sparse blocks and 10 of dense ones: 16384 frames of 192 x 192 (44 MB, 38 sequences a
+// block, median 7) take 868 us, 685 and 398 with the parse; 65536 of 128 x 128
+// (129 MB, 200 a block) 2548 and 471, 3780 with the search.
+constexpr long long kSearchBytes = 48ll << 20;
 
 __device__ __forceinline__ bool staged_block(const uint8_t* src, int csize) {
   return (int)(reinterpret_cast<uintptr_t>(src) & 3u) + csize <= kStageBytes;
@@ -224,17 +230,18 @@ __device__ __forceinline__ long long seq_slot(long long d, int k, int cap) {
 // length and offset checked as in the decode) and stores sequence k as
 // {literal start | literal length << 16, offset | match length << 16}
 // (offset and match length 0 for the block's last sequence).  nseq[d] is
-// the count, 0 for unused slots, raw tails and blocks that the decode stages, -1 when the block has more
+// the count, 0 for unused slots, raw tails and blocks that the decode searches, -1 when the block has more
 // sequences than the table holds (the decode kernel then parses it), -2
 // for a malformed block (its status bit set).  Each thread reads its block
 // through a 32-byte window of aligned vector loads.
 __global__ void __launch_bounds__(256)
 k_bslz4_parse(const uint8_t* __restrict__ comp, long long comp_bytes, const BlockDesc* __restrict__ table,
-              long long n_desc, int cap, uint2* __restrict__ seqs, int* __restrict__ nseq, int* __restrict__ status) {
+              long long n_desc, int search, int cap, uint2* __restrict__ seqs, int* __restrict__ nseq,
+              int* __restrict__ status) {
   const long long d = (long long)blockIdx.x * 256 + threadIdx.x;
   if (d >= n_desc) return;
   const BlockDesc bd = table[d];
-  if (bd.elems == 0 || bd.csize < 0 || staged_block(comp + bd.src, bd.csize)) {
+  if (bd.elems == 0 || bd.csize < 0 || (search && staged_block(comp + bd.src, bd.csize))) {
     nseq[d] = 0;
     return;
   }
@@ -423,6 +430,7 @@ __device__ __forceinline__ int lz4_round(uint2 e, int n, int op0, int osz, int l
   return __builtin_amdgcn_readlane(incl, 63);
 }
 
+template <bool SEARCH>
 __global__ void __launch_bounds__(64)
 k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const BlockDesc* __restrict__ table,
                long long n_desc, int cap, const uint2* __restrict__ seqs, const int* __restrict__ nseq,
@@ -453,7 +461,8 @@ k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const Blo
     const uint8_t* gsrc = comp + bd.src;
     const int s0 = (int)(reinterpret_cast<uintptr_t>(gsrc) & 3u);
     const bool staged = staged_block(gsrc, cs);        // uniform
-    const int n = staged ? 0 : nseq[d];
+    const bool search = SEARCH && staged;
+    const int n = search ? 0 : nseq[d];
     if (n == -2) continue;                             // malformed: flagged by the parse
     __syncthreads();                                   // previous block's readers are done
     if (staged) {
@@ -477,7 +486,7 @@ k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const Blo
     }
     int err = 0;
     bool walk = n < 0;                                 // more sequences than are kept
-    if (staged) {
+    if (search) {
       const uint8_t* const in = cin + s0;
       // ends of the sequences at every byte, of the one and of the one after
       unsigned* const ends = reinterpret_cast<unsigned*>(cout);
@@ -541,7 +550,8 @@ k_bslz4_decode(const uint8_t* __restrict__ comp, long long comp_bytes, const Blo
       for (int r0 = 0; r0 < n; r0 += 64) {
         const int m = min(64, n - r0);
         const uint2 e = (lane < m) ? seqs[seq_slot(d, r0 + lane, cap)] : make_uint2(0u, 0u);
-        op += lz4_round<false>(e, m, op, osz, lane, gsrc, cs, cout);
+        op += staged ? lz4_round<false>(e, m, op, osz, lane, cin + s0, cs, cout)
+                     : lz4_round<false>(e, m, op, osz, lane, gsrc, cs, cout);
       }
     }
     if (walk) {
@@ -741,14 +751,19 @@ hipError_t launch_bslz4_decode_u16(const uint8_t* comp, long long comp_bytes, co
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (n_desc == 0) return hipSuccess;
+  const bool search = comp_bytes <= kSearchBytes;
   hipLaunchKernelGGL(k_bslz4_parse, dim3((unsigned)((n_desc + 255) / 256)), dim3(256), 0, s, comp, comp_bytes, table,
-                     n_desc, cap, seqs, nseq, status);
+                     n_desc, search ? 1 : 0, cap, seqs, nseq, status);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   const long long npad = (n_desc + 127) / 128 * 128;   // a multiple of 8: workgroup w stays on XCD w mod 8
   const unsigned grid = (unsigned)(npad < 262144 ? npad : 262144);
-  hipLaunchKernelGGL(k_bslz4_decode, dim3(grid), dim3(64), 0, s, comp, comp_bytes, table, n_desc, cap, seqs, nseq,
-                     out, status);
+  if (search)
+    hipLaunchKernelGGL(k_bslz4_decode<true>, dim3(grid), dim3(64), 0, s, comp, comp_bytes, table, n_desc, cap, seqs,
+                       nseq, out, status);
+  else
+    hipLaunchKernelGGL(k_bslz4_decode<false>, dim3(grid), dim3(64), 0, s, comp, comp_bytes, table, n_desc, cap, seqs,
+                       nseq, out, status);
   return hipGetLastError();
 }
 

@@ -117,3 +117,27 @@ def test_malformed_sequences_are_refused(cuda, kind):
         decode_u16([_chunk([good]), _chunk([MALFORMED[kind]]), _chunk([good])], (1, 64, 64))
     out = decode_u16([_chunk([good])], (1, 64, 64)).cpu().numpy()
     np.testing.assert_array_equal(out.ravel(), np.asarray(_expect(good)).ravel())
+
+
+def test_a_large_buffer_is_parsed_ahead(cuda):
+    """Beyond 48 MiB of compressed bytes the sequences come from the parse: the
+    same frames, and a malformed block still refused."""
+    from quantem.gpu_amd.ssb.compute.hip.bslz4 import Bslz4Chunks
+    rng = np.random.default_rng(9)
+    kinds = [_chunk([_fill(rng, n, lit)]) for n, lit in ((2, 0), (64, 40), (65, 900), (300, 100), (640, 0))]
+    kinds.append(_chunk([_seq(rng.integers(0, 256, 6000).astype(np.uint8).tobytes(), 5, BLOCK - 6009) + END]))
+    order = np.concatenate([np.arange(6), rng.integers(4, 6, 17000)])
+    buf = np.frombuffer(b"".join(kinds[i] for i in order), dtype=np.uint8).copy()
+    sizes = np.array([len(kinds[i]) for i in order], dtype=np.int64)
+    assert buf.size > 48 << 20
+    want = [np.asarray(_expect(k[16:])).reshape(64, 64) for k in kinds]
+    out = Bslz4Chunks((buf, sizes), (1, 64, 64)).decode().cpu().numpy()
+    for i in list(range(40)) + list(range(len(order) - 40, len(order))):
+        np.testing.assert_array_equal(out[i], want[order[i]])
+    for k in range(6):
+        ids = np.flatnonzero(order == k)
+        assert (out[ids].astype(np.int64).sum(axis=(1, 2)) == want[k].astype(np.int64).sum()).all()
+    bad = buf.copy()
+    bad[16 + 2:16 + 4] = 0xFF                                        # the first block's offset
+    with pytest.raises(ValueError, match="malformed"):
+        Bslz4Chunks((bad, sizes), (1, 64, 64)).decode()
