@@ -477,7 +477,9 @@ def trials_leg(dev, data, cfg, n_trials: int = 512, reps: int = 5, seed: int = 3
 
 
 SEARCH_PROFILE = REPO / "profiles" / "trials_search_512x256x128.md"
-VALU_LANES_PER_S = 1024 * 16 * 2.4e9   # 256 CUs x 4 SIMDs, one wave64 VALU instruction per 4 cycles, 2.4 GHz
+# 256 CUs x 4 SIMDs, one wave64 VALU instruction per 4 cycles, 2.4 GHz: nominal, instructions
+# issue in 3.2 cycles in the search (a fraction above 1)
+VALU_LANES_PER_S = 1024 * 16 * 2.4e9
 
 
 def read_profile_figure(path: Path, key: str) -> float | None:

@@ -3,8 +3,9 @@
 Three knobs of the native library (``ssb_tune_*`` in ``include/quantem_ssb.h``)
 change launch shapes only -- the workgroup count of the raw-data stream pass
 (exact integer sums, bit-identical), the number of FFT pairs per gather
-workgroup and the tile shape of the fused column FFT + trotter (the same
-arithmetic in another instantiation, equal to float rounding).  ``autotune`` times every
+workgroup and the groups of bright-field pixels (128 x 128 scans: the tile
+shape) of the fused column FFT + trotter (the same arithmetic summed in
+another order or instantiation, equal to float rounding).  ``autotune`` times every
 candidate of each knob in turn (coordinate descent, the others held at their
 best so far) on the caller's own resident data with the per-stage hipEvents
 of ``ssb_recon_u16``, keeps the fastest, and can store the choice in a JSON
