@@ -124,16 +124,15 @@ class PlanSpec:
 # a short session.  The allocator orders a block by one stream; the plan waits
 # for the device before it releases one.
 @_abi.AllocFn
-def _alloc(nbytes, stream, _ctx):
+def _alloc(nbytes, stream, device):
     try:
-        torch = _torch()
-        return torch.cuda.caching_allocator_alloc(nbytes, torch.cuda.current_device(), stream or 0)
+        return _torch().cuda.caching_allocator_alloc(nbytes, device or 0, stream or 0)
     except Exception:      # no exception crosses the C boundary: NULL is out of memory
         return None
 
 
 @_abi.ReleaseFn
-def _release(ptr, _ctx):
+def _release(ptr, _device):
     try:
         _torch().cuda.caching_allocator_delete(ptr)
     except Exception:
@@ -154,7 +153,7 @@ class SSBPlan:
         with torch.cuda.device(self.device):
             _abi.call("ssb_plan_create_with", spec.scan_n, spec.det_rows, spec.det_cols, spec.max_bf,
                       spec.wavelength_A, spec.semiangle_rad, spec.ang_row_rad, spec.ang_col_rad,
-                      spec.scan_sampling_row_A, spec.scan_sampling_col_A, _alloc, _release, None,
+                      spec.scan_sampling_row_A, spec.scan_sampling_col_A, _alloc, _release, dev.index,
                       _abi.stream_handle(torch.cuda.current_stream(dev)), ctypes.byref(handle))
         self._h = handle
 
