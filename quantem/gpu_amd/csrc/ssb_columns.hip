@@ -65,12 +65,12 @@ struct Kahan2 {
 
 // The term of one point, row q + dq and column col + dcol (sign -1: of -qy),
 // given B = 2 q.k and base = Rout^2 - |k|^2 - |q|^2.
-__device__ __forceinline__ float2 quad_term(float2 G, float B, float base, float s, float t, const QuadPixel& p,
-                                            const ApIso& ap, const GeomPtrs& gp, df rout2, int b, int q, int dq, int col,
-                                            int dcol, float sign) {
+__device__ __forceinline__ float2 quad_term(float2 G, float B, float base, float s, float t, bool whole,
+                                            const QuadPixel& p, const ApIso& ap, const GeomPtrs& gp, df rout2, int b,
+                                            int q, int dq, int col, int dcol, float sign) {
   const float near = base + fabsf(B), far = base - fabsf(B);
   t = B < 0.0f ? -t : t;
-  return overlap_term(G, near, far, B, s, t, p.margin, p.ak, ap, [&](df& dm, df& dp) {
+  return overlap_term(G, near, far, B, s, t, whole, p.margin, p.ak, ap, [&](df& dm, df& dp) {
     asm volatile("" : "+v"(q), "+v"(col));   // no addresses kept ahead of the branch
     q += dq;
     col += dcol;
@@ -80,8 +80,21 @@ __device__ __forceinline__ float2 quad_term(float2 G, float B, float base, float
   });
 }
 
+// s of overlap_unit, qx (sxx qx + sxy) + syy, given sxx = k0 + m12c, sxy = 2 m12s qy
+// and syy = half_sum_qy(ev, qy).  Both squares are rounded alike and not contracted
+// into the sum: where C10 and C12 cancel (on the diagonals without C10, on an axis
+// with |C10| = |C12|) s is zero, not what rounding leaves, whose sign the term
+// would take.
+__device__ __forceinline__ float half_sum(float sxx, float sxy, float syy, float qx) {
+#pragma clang fp contract(off)
+  const float a = qx * fmaf(qx, sxx, sxy);
+  return a + syy;
+}
+__device__ __forceinline__ float half_sum_qy(const QuadTurns& ev, float qy) {
+  return half_sum(ev.k0 - ev.m12c, 0.0f, 0.0f, qy);
+}
 __device__ __forceinline__ float half_sum(const QuadTurns& ev, float qx, float qy) {
-  return fmaf(qx, fmaf(qx, ev.k0 + ev.m12c, 2.0f * qy * ev.m12s), qy * qy * (ev.k0 - ev.m12c));
+  return half_sum(ev.k0 + ev.m12c, 2.0f * qy * ev.m12s, half_sum_qy(ev, qy), qx);
 }
 
 }  // namespace
@@ -186,13 +199,14 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
       for (int i = 0; i < 4; ++i) {
         const float B = B_of(i, p), base = p.cb - q2[i];
         if (base + fabsf(B) > -p.margin)
-          acc[i].add(quad_term(cur.G[i], B, base, s[i], fmaf(qx[i], p.tx, qy[i] * p.ty), p, ap, gp, rout2, b, lr, row0[i],
-                               lc, col0[i], 1.0f));
+          acc[i].add(quad_term(cur.G[i], B, base, s[i], fmaf(qx[i], p.tx, qy[i] * p.ty), near_whole(s[i]), p, ap, gp,
+                               rout2, b, lr, row0[i], lc, col0[i], 1.0f));
         __builtin_amdgcn_sched_barrier(0);
       }
       if (nmask >> l & 1) {
         // the Nyquist row's partners, columns N - j: their own frequencies (q_N/2, -qy)
         const float B = fmaf(nqx, p.kx2, nqy * p.ky2) + 0.0f, base = p.cb - nq2;
+        const float ns = half_sum(ev, nqx, nqy);
         float2 G = cur.G[0];
         int c = col0[0];
 #pragma unroll
@@ -203,8 +217,8 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
           }
         }
         if (lr == 0 && base + fabsf(B) > -p.margin)
-          nyq.add(quad_term(cconj(G), B, base, half_sum(ev, nqx, nqy), fmaf(nqx, p.tx, nqy * p.ty), p, ap, gp, rout2, b, HALF,
-                            0, lc, c, -1.0f));
+          nyq.add(quad_term(cconj(G), B, base, ns, fmaf(nqx, p.tx, nqy * p.ty), near_whole(ns), p, ap, gp, rout2, b,
+                            HALF, 0, lc, c, -1.0f));
       }
       if (!mask) break;
       cur = nxt;
@@ -459,7 +473,14 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
     float y0, y1;
     wave_range(gp.qy[last ? HALF : cg * CG + lane % CG], y0, y1);
     const float qn = as_const(gp.qx)[HALF];
-    const float sxx = ev.k0 + ev.m12c, sxy = 2.0f * qy * ev.m12s, syy = qy * qy * (ev.k0 - ev.m12c);
+    const float sxy = 2.0f * qy * ev.m12s, syy = half_sum_qy(ev, qy);
+    const float sxx = ev.k0 + ev.m12c;
+    // whether a point of the wave, the mean's apart, has s near a whole number: s is
+    // the point's alone, and without one its terms need not ask (a scalar branch)
+    bool whole = false;
+    for (int r = 0; r < 16; ++r)
+      whole |= near_whole(half_sum(sxx, sxy, syy, qxS[k1 + K * r])) && (j != 0 || k1 + K * r != 0);
+    const bool ask = __any(whole);
     Kahan2 acc[16], nyq;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r].init();
@@ -498,17 +519,25 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
             const float2 m = Fft::mirror(r, ex, lane);
             x[r] = last ? unpack_half(x[r], m) : unpack_first(x[r], m);
           }
+          const float s = half_sum(sxx, sxy, syy, qx);
+          whole = false;
+          if (ask) {
+            float at = s;
+            asm volatile("" : "+v"(at));             // not ahead of the branch
+            whole = near_whole(at);
+          }
           if (base + fabsf(B) > -p.margin)
-            acc[r].add(quad_term(x[r], B, base, fmaf(qx, fmaf(qx, sxx, sxy), syy), fmaf(qx, p.tx, tq), p, ap, gp, rout2,
-                                 b, k1, K * r, j, 0, 1.0f));
+            acc[r].add(quad_term(x[r], B, base, s, fmaf(qx, p.tx, tq), whole, p, ap, gp, rout2, b, k1, K * r, j, 0,
+                                 1.0f));
           __builtin_amdgcn_sched_barrier(0);               // one point at a time
         }
         if (!last && apertures_reach(p, rout2.hi, qn, qn, -y1, -y0)) {
           // the Nyquist row's partners, columns N - j: their own frequencies (q_N/2, -qy)
           const float B = fmaf(qn, p.kx2, -Bq) + 0.0f, base = fmaf(-qn, qn, cq);
+          const float ns = half_sum(ev, qn, -qy);
           if (k1 == 0 && base + fabsf(B) > -p.margin)
-            nyq.add(quad_term(cconj(x[8]), B, base, fmaf(qn, fmaf(qn, sxx, -sxy), syy), fmaf(qn, p.tx, -tq), p, ap, gp,
-                              rout2, b, HALF, 0, j, 0, -1.0f));
+            nyq.add(quad_term(cconj(x[8]), B, base, ns, fmaf(qn, p.tx, -tq), near_whole(ns), p, ap, gp, rout2, b, HALF,
+                              0, j, 0, -1.0f));
         }
         if (!mask) break;
       }

@@ -111,6 +111,13 @@ struct PhasorJob {
   float2* echi;
 };
 
+// chi(Q), the squares rounded alike: zero where mxx = -myy and |x| = |y|, as exactly.
+__device__ __forceinline__ float chi_plane(const QuadChi& m, float x, float y) {
+#pragma clang fp contract(off)
+  const float a = m.mxx * (x * x), b = m.myy * (y * y);
+  return fmaf(2.0f * m.mxy * x, y, a + b);
+}
+
 // The items [gid, gid + stride, ...) of a phasor job.
 __device__ __forceinline__ void phasor_work(const PhasorJob& j, long long gid, long long stride) {
   const QuadChi m = j.m;
@@ -124,7 +131,7 @@ __device__ __forceinline__ void phasor_work(const PhasorJob& j, long long gid, l
     const int c = (int)(idx / N), q = (int)(idx - (long long)c * N);
     const float x = j.gp.qx[q], y = j.gp.qy[c];
     float sn, cs;
-    sincosf(m.mxx * x * x + 2.0f * m.mxy * x * y + m.myy * y * y, &sn, &cs);
+    sincosf(chi_plane(m, x, y), &sn, &cs);
     j.echi[idx] = make_float2(cs, sn);
   }
   for (long long idx = gid; idx < total; idx += stride) {

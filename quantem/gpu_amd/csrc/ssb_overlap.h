@@ -146,8 +146,9 @@ __device__ __forceinline__ void sincos_half_turns(float r, float& s, float& c) {
 // exchanging k and -k turns Gamma^ into -conj(Gamma^): one form, on the side
 // where A(Q-k) is the larger, serves all.  Returns G * conj(Gamma^): `both`
 // apertures 1 or A(Q-k) alone for `t` taken on that side, `flip` (a sign
-// bit): the other side is meant.  The caller takes points whose s is a whole
-// number (the sine vanishes) and small A(k) through gamma_hat_st.
+// bit): the other side is meant.  It is normalised without the guard of
+// gamma_hat, so the caller takes the points where Gamma can be that small
+// through gamma_hat_st.
 __device__ __forceinline__ float2 overlap_unit(float2 G, bool both, float s, float t, unsigned flip) {
   // (contracted, t's last product would round here by where this is inlined)
 #pragma clang fp contract(off)
@@ -159,6 +160,14 @@ __device__ __forceinline__ float2 overlap_unit(float2 G, bool both, float s, flo
   cs = __uint_as_float(__float_as_uint(cs) ^ flip);
   const float x = fmaf(G.x, cs, G.y * sn), y = fmaf(G.y, cs, -(G.x * sn));
   return make_float2(__uint_as_float(__float_as_uint(x) ^ turn), __uint_as_float(__float_as_uint(y) ^ turn));
+}
+
+// a + b, a not contracted into it: the C12 term m12c (qx - qy) (qx + qy) of s
+// cancels a C10 term of its size to zero on an axis, and is zero on the diagonals.
+// What rounding would leave has a sign, which overlap_unit would take.
+__device__ __forceinline__ float add_cancelling(float a, float b) {
+#pragma clang fp contract(off)
+  return a + b;
 }
 
 // The general form of the same, with the guard of gamma_hat.
@@ -188,23 +197,30 @@ __device__ __forceinline__ float2 gamma_hat_st(float ak, float am, float app, fl
 // says which of the two is the nearer (negative: Q + k); s, t as in
 // overlap_unit, t on the nearer side.  One phasor serves where one aperture
 // is zero, whatever the other's value (normalising takes it out), and where
-// both are one; the general form at an outer edge and with the smaller
-// aperture in its soft band, where the sine vanishes, and for a BF pixel whose
-// small A(k) can meet the guard elsewhere (margin = infinity).  There both d
+// both are one; the general form at an outer edge and with the smaller aperture
+// in its soft band, and wherever |Gamma| can meet the guard of gamma_hat, 1e-8:
+// with both apertures one it is 2 A(k) |sin(pi s)|, at least 1.5e-7 for s further
+// than kNearWhole from a whole number and A(k) from kSmallAk up (s is that near
+// under no aberration, tiny ones, and on lines of the plane where C10 and C12
+// cancel; next to 1 float32 itself is no finer than 6e-8).  A BF pixel of smaller
+// A(k) goes there with all its points (margin = infinity).  whole: near_whole(s),
+// if the caller cannot know that it isn't.  There both d
 // come in double-float from exact(dn, df) within kEdgeMargin of an edge and
 // with both apertures in their bands, where their values or their difference
 // decide; inside one aperture and well inside the other's band the estimates
 // give the ratio to 2e-6.  B must not be a negative zero unless t is zero.
 constexpr float kEdgeMargin = 1e-4f;   // far above the estimates' error (2e-5 for terms below 32)
-constexpr float kSmallAk = 1e-3f;
+constexpr float kSmallAk = 1.2e-2f;
+constexpr float kNearWhole = 2e-6f;
+__device__ __forceinline__ bool near_whole(float s) { return fabsf(s - rintf(s)) <= kNearWhole; }
 __device__ __forceinline__ float edge_margin(float ak) { return ak < kSmallAk ? INFINITY : kEdgeMargin; }
 
 template <typename Exact>
 __device__ __forceinline__ float2 overlap_term(float2 G, float near, float far, float B, float s, float t,
-                                               float margin, float ak, const ApIso& ap, Exact exact) {
+                                               bool whole, float margin, float ak, const ApIso& ap, Exact exact) {
   const float inner = ap.d_in + kEdgeMargin;
   const bool both = far >= inner;
-  const bool general = (fabsf(near) < margin) | ((far > -margin) & (far < inner)) | (both & (s == floorf(s)));
+  const bool general = (fabsf(near) < margin) | ((far > -margin) & (far < inner)) | (both & whole);
   float2 z = overlap_unit(G, both, s, t, __float_as_uint(B) & 0x80000000u);
   if (general) {
     df dn{near, 0.0f}, dfar{far, 0.0f};

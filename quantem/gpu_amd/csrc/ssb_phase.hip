@@ -193,7 +193,7 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
 #pragma unroll
   for (int m = 0; m < R; ++m) asm volatile("" : "+v"(qx[m]));   // arrived here
   const float qn = as_const(gp.qx)[HALF];
-  const float k0 = ch.k0, k4 = ch.k4, m12c = ch.m12c, m12s = ch.m12s;
+  const float k0 = ch.k0, k4 = ch.k4, m12c = ch.m12c, m12s = ch.m12s, m12s2 = 2.0f * m12s;
 
   // what a point needs of its BF pixel
   struct Pixel {
@@ -222,10 +222,10 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
         const float w4 = fmaf(k4, q2, px.u);
         t = fmaf(qxv, px.vx, fmaf(qyv, px.vy, B * fmaf(k4, q2, w4)));
         s = fmaf(q2, w4, k4 * (B * B));
-        s = fmaf(fmaf(qxv, qxv, -(qyv * qyv)), m12c, fmaf(2.0f * qxv * qyv, m12s, s));
+        s = add_cancelling((qxv - qyv) * (qxv + qyv) * m12c, fmaf(qxv * qyv, m12s2, s));
       }
       t = B < 0.0f ? -t : t;
-      z = overlap_term(G, near, far, B, s, t, px.margin, px.ak, ap, [&](df& dm, df& dp) {
+      z = overlap_term(G, near, far, B, s, t, near_whole(s), px.margin, px.ak, ap, [&](df& dm, df& dp) {
         const df kx{0.5f * px.kx2, as_const(gp.kxl)[b]}, ky{0.5f * px.ky2, as_const(gp.kyl)[b]};
         exact_d(df{qxv, gp.qxl[q]}, df{qyv, gp.qyl[col]}, kx, ky, df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky))),
                 dm, dp);

@@ -155,10 +155,11 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
     const df qx{qxf, ds.qxl[q]}, qy{qyf, ds.qyl[c]};
     const df q2 = df_add(df_mul(qx, qx), df_mul(qy, qy));
     q2f = live ? q2.hi + q2.lo : 1e30f;   // idle lanes: outside every aperture
-  }
-  if (!RADIAL) {
-    qa = qxf * qxf - qyf * qyf;
-    qb = 2.0f * qxf * qyf;
+    if (!RADIAL) {
+      const df a = df_sub(df_mul(qx, qx), df_mul(qy, qy));
+      qa = a.hi + a.lo;
+      qb = 2.0f * qxf * qyf;
+    }
   }
   float k4[TB];
 #pragma unroll
@@ -198,7 +199,7 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
             if (kind == kChiAstig) {
               ts = fmaf(qxf, km[i].vx, qyf * km[i].vy);
               ts = B < 0.0f ? ts - t : ts + t;
-              s = fmaf(qa, ch[i].m12c, fmaf(qb, ch[i].m12s, s));
+              s = add_cancelling(qa * ch[i].m12c, fmaf(qb, ch[i].m12s, s));
             } else {
               const float kxh = 0.5f * kx2[i], kyh = 0.5f * ky2[i], chik = km[i].chik;
               const float cm = chi_even(tch[i], qxf - kxh, qyf - kyh) - chik;
@@ -209,7 +210,7 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
             }
             t = B < 0.0f ? -ts : ts;
           }
-          const float2 z = overlap_term(G, near, far, B, s, t, margin, km[i].ak, ds.ap, [&](df& dm, df& dp) {
+          const float2 z = overlap_term(G, near, far, B, s, t, near_whole(s), margin, km[i].ak, ds.ap, [&](df& dm, df& dp) {
             exact_d(df{qxf, ds.qxl[q]}, df{qyf, ds.qyl[c]}, df{0.5f * kx2[i], km[i].kxl}, df{0.5f * ky2[i], km[i].kyl},
                     df{km[i].cb, km[i].cbl}, dm, dp);
           });

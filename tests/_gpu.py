@@ -55,6 +55,47 @@ def scaled_error(obj, ref):
 OBJ_SCALED = 2e-6
 
 
+def undecided_points(g: O.Geometry, c10, c12, phi12):
+    """Bool [N, N]: points where float32 cannot decide some pixel's normalised
+    overlap, which jumps there.  The plan's detector centre is float32, so an
+    aperture moves by up to 1e-6 of its soft edge: the nearer aperture within
+    2e-6 of the edge's foot (no overlap, or a unit vector), or both apertures in
+    their soft edges with |Gamma| / A(k) below 1e-5, its direction off by a tenth."""
+    n = g.qx.size
+    out = np.zeros((n, n), bool)
+    mags, angs = np.zeros(14), np.zeros(14)
+    mags[:2], angs[1] = (c10, c12), phi12
+
+    def edge(u, v):          # unclipped
+        r = np.hypot(u, v)
+        phi = np.arctan2(v, u)
+        width = np.hypot(np.cos(phi) * g.ang_y_rad, np.sin(phi) * g.ang_x_rad)
+        return (g.semiangle_rad - r * g.wavelength) / width + 0.5
+
+    def chi(u, v):
+        return O.chi_full(u, v, g.wavelength, mags, angs)
+
+    for kx, ky in zip(g.kx, g.ky):
+        qx, qy = g.qx.reshape(-1, 1), g.qy.reshape(1, -1)
+        em, ep = edge(qx - kx, qy - ky), edge(qx + kx, qy + ky)
+        out |= np.abs(np.maximum(em, ep)) < 2e-6
+        am, ap = np.clip(em, 0.0, 1.0), np.clip(ep, 0.0, 1.0)
+        i, j = np.nonzero((np.minimum(am, ap) > 0) & (np.abs(am - ap) < 1e-5) & (np.minimum(am, ap) < 1))
+        x, y = g.qx.reshape(-1)[i], g.qy.reshape(-1)[j]
+        ck = chi(np.array([kx]), np.array([ky]))
+        gamma = am[i, j] * np.exp(-1j * (chi(x - kx, y - ky) - ck)) - ap[i, j] * np.exp(1j * (chi(x + kx, y + ky) - ck))
+        small = np.abs(gamma) < 1e-5
+        out[i[small], j[small]] = True
+    out[0, 0] = False        # the mean
+    return out
+
+
+def decided_error(obj, ref, undecided):
+    """``scaled_error`` with the undecided points taken out of both spectra."""
+    o, r = (np.where(undecided, 0, np.fft.fft2(np.asarray(v, np.complex128))) for v in (obj, ref))
+    return scaled_error(np.fft.ifft2(o), np.fft.ifft2(r))
+
+
 def engine_for_data(torch, data_np, *, semiangle_mrad, det_sampling, step, voltage_kV=300,
                     max_bf=4096):
     n, det = data_np.shape[0], data_np.shape[2:]
