@@ -337,7 +337,8 @@ int ssb_batch_phase_loss(ssb_plan* plan, int n_trials, const double* mags_host, 
  * ssb_batch_phase_loss as a captured hipGraph: the per-trial kernels read
  * their rotation and aberration coefficients from a plan-owned device table,
  * so the sequence is captured once (again when the count, the pattern of
- * higher-order trials or losses_out change) and replayed for each new batch
+ * higher-order trials, losses_out, the place, size or layout of the resident
+ * stack or the detector sampling change) and replayed for each new batch
  * after the table upload, on the plan's own stream ordered after and before
  * `stream`.  Losses are bit-identical to ssb_batch_phase_loss (every trial
  * recomputes its geometry).  Synchronises `stream` once for the upload.

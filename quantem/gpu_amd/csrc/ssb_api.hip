@@ -1024,7 +1024,8 @@ int ssb_batch_phase_loss_graph(ssb_plan* p, int n_trials, const double* mags_hos
   HIP_TRY(hipMemcpyAsync(p->xt, p->xt_host.data(), sizeof(ExactTrial) * n_trials, hipMemcpyHostToDevice, s),
           "batch table upload");
   HIP_TRY(hipStreamSynchronize(s), "batch table upload");   // the host table may change after return
-  if (!p->xexec || pattern != p->xt_pattern || p->xgraph_out != losses_out) {
+  const StackKey stack{p->Gt, p->g_nbf, p->nbf_hint, p->gcols, p->recip_y, p->recip_x};
+  if (!p->xexec || pattern != p->xt_pattern || p->xgraph_out != losses_out || !(stack == p->xgraph_stack)) {
     if (p->xexec) (void)hipGraphExecDestroy(p->xexec);
     if (p->xgraph) (void)hipGraphDestroy(p->xgraph);
     p->xexec = nullptr;
@@ -1037,6 +1038,7 @@ int ssb_batch_phase_loss_graph(ssb_plan* p, int n_trials, const double* mags_hos
     HIP_TRY(hipGraphInstantiate(&p->xexec, p->xgraph, nullptr, nullptr, 0), "batch graph instantiate");
     p->xt_pattern = pattern;
     p->xgraph_out = losses_out;
+    p->xgraph_stack = stack;
   }
   HIP_TRY(hipEventRecord(p->gev_in, s), "batch graph launch");
   HIP_TRY(hipStreamWaitEvent(p->gstream, p->gev_in, 0), "batch graph launch");

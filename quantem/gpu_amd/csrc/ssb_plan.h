@@ -22,6 +22,19 @@ struct ExactTrial {
   double mags[14], angles[14];   // as given (host)
 };
 
+// What the launches of a captured batch hold of the plan by value: the resident
+// stack (a new selection or stack may move it, resize it or change its layout)
+// and the detector sampling.
+struct StackKey {
+  const void* gt = nullptr;
+  int nbf = 0, hint = 0, gcols = 0;
+  double recip_y = 0, recip_x = 0;
+  bool operator==(const StackKey& o) const {
+    return gt == o.gt && nbf == o.nbf && hint == o.hint && gcols == o.gcols && recip_y == o.recip_y &&
+           recip_x == o.recip_x;
+  }
+};
+
 struct ssb_plan {
   int n = 0;
   int det_rows = 0, det_cols = 0, D = 0;
@@ -110,6 +123,7 @@ struct ssb_plan {
   hipGraph_t xgraph = nullptr;
   hipGraphExec_t xexec = nullptr;
   float* xgraph_out = nullptr;
+  StackKey xgraph_stack;
   // stage timing
   std::vector<hipEvent_t> events;   // (NSTAGES + 1) per recorded call
   int timing_calls = 0;
