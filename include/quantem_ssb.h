@@ -366,6 +366,10 @@ int ssb_trials_create(ssb_plan* const* plans, int n_plans, int max_trials, ssb_t
 int ssb_trials_destroy(ssb_trials* trials);
 
 /*
+ * Both entry points below refuse a plan whose stack has been replaced by one of
+ * another size, place or layout since ssb_trials_create (QSSB_ERR_STATE); one that
+ * has taken its place is evaluated from the next call on.
+ *
  * Set n_trials aberration sets from host arrays in the layout of
  * ssb_batch_phase_loss (mags_host[14 t ..], angles_host[14 t ..]; odd-order
  * terms C21, C23, C41, C43, C45 must be zero) with per-trial scan rotations

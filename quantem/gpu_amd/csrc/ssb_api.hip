@@ -560,6 +560,7 @@ static int prepare_g_typed(ssb_plan* p, const void* data, int dtype, void* strea
   HIP_TRY(launch_columns_store(p->n, p->H, p->info, geom_ptrs(p), p->tw, p->Gt, s), "colfft");
   p->gcols = p->n / 2 + 1;
   p->g_nbf = p->nbf_hint;
+  ++p->g_count;
   return QSSB_OK;
 }
 
@@ -602,6 +603,7 @@ int ssb_import_g(ssb_plan* p, const void* g_in, int nbf, int gcols, void* stream
   HIP_TRY(hipGetLastError(), "import_g");
   p->gcols = gcols;
   p->g_nbf = nbf;
+  ++p->g_count;
   return QSSB_OK;
 }
 

@@ -44,6 +44,7 @@ struct ssb_plan {
   int nbf_hint = 0;
   int gcols = 0;            // columns of the resident stack (0 = none)
   int g_nbf = 0;
+  unsigned g_count = 0;     // stacks prepared or imported so far
   double wavelength = 0, semiangle = 0, ang_y = 0, ang_x = 0;
   double sampling_row = 0, sampling_col = 0;
   double recip_y = 0, recip_x = 0;

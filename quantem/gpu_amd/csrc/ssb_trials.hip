@@ -493,6 +493,11 @@ struct ssb_trials {
   std::vector<TrialSet> sets_host;
   std::vector<TrialBf*> tbf;
   std::vector<TrialBfMore*> more;
+  // the pixels and the mean of each plan's stack (the plan's own may be those of
+  // a later selection), and the stack they were copied for
+  std::vector<int*> bf;                  // rows, then columns
+  std::vector<BfInfo*> info;
+  std::vector<unsigned> g_count;
   std::vector<float2*> S;
   std::vector<float2*> W;
   std::vector<float*> part;
@@ -502,6 +507,7 @@ struct ssb_trials {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int graph_trials = 0;                  // n_trials the graph was captured for
+  std::vector<double> graph_recip;       // the plans' detector sampling it holds
   float* graph_out = nullptr;
   unsigned* queue = nullptr;             // work-queue counters of k_trotter_trials (zero between launches)
 };
@@ -520,6 +526,8 @@ void trials_free(ssb_trials* tr) {
   (void)hipFree(tr->sets);
   for (auto* p : tr->tbf) (void)hipFree(p);
   for (auto* p : tr->more) (void)hipFree(p);
+  for (auto* p : tr->bf) (void)hipFree(p);
+  for (auto* p : tr->info) (void)hipFree(p);
   for (auto* p : tr->S) (void)hipFree(p);
   for (auto* p : tr->W) (void)hipFree(p);
   for (auto* p : tr->part) (void)hipFree(p);
@@ -531,6 +539,29 @@ df to_df(double v) {
   return df{hi, (float)(v - (double)hi)};
 }
 
+// The tables and the stack's address were laid out for the stacks that the plans
+// held when the handle was made: refuse others, before any launch.  Another stack
+// of the same size in the same place is taken over, its pixels and mean with it.
+int follow_stacks(ssb_trials* tr, hipStream_t s) {
+  for (size_t i = 0; i < tr->plans.size(); ++i) {
+    const ssb_plan* p = tr->plans[i];
+    const TrialSet& ds = tr->sets_host[i];
+    if (p->Gt != ds.Gt || p->g_nbf != ds.nbf || p->gcols == p->n)
+      return report_error(QSSB_ERR_STATE, "the Fourier stack of plan " + std::to_string(i) +
+                                              " was replaced by one of another size or layout; make a new trials handle");
+    if (p->g_count == tr->g_count[i]) continue;
+    if (!p->gcols)   // replaced and selected anew since: the pixels are gone
+      return report_error(QSSB_ERR_STATE, "no resident Fourier stack");
+    const size_t bytes = sizeof(int) * (size_t)ds.nbf;
+    hipError_t e = hipMemcpyAsync(tr->bf[i], p->bf_rows, bytes, hipMemcpyDeviceToDevice, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(tr->bf[i] + ds.nbf, p->bf_cols, bytes, hipMemcpyDeviceToDevice, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(tr->info[i], p->info, sizeof(BfInfo), hipMemcpyDeviceToDevice, s);
+    if (e != hipSuccess) return report_hip_error(e, "trials pixels");
+    tr->g_count[i] = p->g_count;
+  }
+  return QSSB_OK;
+}
+
 // Enqueue the whole batched evaluation on `s`; out[p * max_trials + t].
 hipError_t enqueue_trials(ssb_trials* tr, float* out, hipStream_t s) {
   const int T = tr->n_trials;
@@ -538,9 +569,10 @@ hipError_t enqueue_trials(ssb_trials* tr, float* out, hipStream_t s) {
     ssb_plan* p = tr->plans[i];
     df rout2;
     (void)iso_aperture(p->optics, rout2);
-    const long long total = (long long)T * p->g_nbf;
-    hipLaunchKernelGGL(k_trial_geometry, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p->bf_rows,
-                       p->bf_cols, p->info, p->g_nbf, T, to_df(p->recip_y), to_df(p->recip_x), p->optics, rout2,
+    const int nbf = tr->sets_host[i].nbf;
+    const long long total = (long long)T * nbf;
+    hipLaunchKernelGGL(k_trial_geometry, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, tr->bf[i],
+                       tr->bf[i] + nbf, tr->info[i], nbf, T, to_df(p->recip_y), to_df(p->recip_x), p->optics, rout2,
                        tr->chis, tr->tbf[i], tr->more[i]);
   }
   long long total_items = 0;
@@ -553,7 +585,7 @@ hipError_t enqueue_trials(ssb_trials* tr, float* out, hipStream_t s) {
                      (int)tr->sets_host.size(), total_items, tr->chis, tr->queue);
   for (size_t i = 0; i < tr->plans.size(); ++i) {
     ssb_plan* p = tr->plans[i];
-    hipError_t e = launch_trials_finish(p->n, T, tr->S[i], p->info, p->tw, tr->W[i], tr->part[i],
+    hipError_t e = launch_trials_finish(p->n, T, tr->S[i], tr->info[i], p->tw, tr->W[i], tr->part[i],
                                         out + (long long)i * tr->max_trials, s);
     if (e != hipSuccess) return e;
   }
@@ -592,11 +624,15 @@ int ssb_trials_create(ssb_plan* const* plans, int n_plans, int max_trials, ssb_t
     const size_t slots = (size_t)((max_trials + kTrialBlock - 1) / kTrialBlock) * p->g_nbf;
     TrialBf* tb = nullptr;
     TrialBfMore* more = nullptr;
+    int* bf = nullptr;
+    BfInfo* info = nullptr;
     float2* S = nullptr;
     float2* W = nullptr;
     float* part = nullptr;
     e = hipMalloc(reinterpret_cast<void**>(&tb), sizeof(TrialBf) * slots);
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&more), sizeof(TrialBfMore) * kTrialBlock * slots);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&bf), sizeof(int) * 2 * (size_t)p->g_nbf);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&info), sizeof(BfInfo));
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&S), sizeof(float2) * (size_t)max_trials * NP);
     if (e == hipSuccess)
       e = hipMalloc(reinterpret_cast<void**>(&W), sizeof(float2) * (size_t)max_trials * p->n * p->n);
@@ -604,6 +640,9 @@ int ssb_trials_create(ssb_plan* const* plans, int n_plans, int max_trials, ssb_t
       e = hipMalloc(reinterpret_cast<void**>(&part), sizeof(float) * 4 * (size_t)max_trials * (p->n / kFinishCount));
     tr->tbf.push_back(tb);
     tr->more.push_back(more);
+    tr->bf.push_back(bf);
+    tr->info.push_back(info);
+    tr->g_count.push_back(p->g_count - 1);   // copied below
     tr->S.push_back(S);
     tr->W.push_back(W);
     tr->part.push_back(part);
@@ -627,9 +666,19 @@ int ssb_trials_create(ssb_plan* const* plans, int n_plans, int max_trials, ssb_t
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&tr->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&tr->ev_in, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&tr->ev_out, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipDeviceSynchronize();   // the selections may be on any stream
   if (e != hipSuccess) {
     trials_free(tr);
     return report_hip_error(e, "ssb_trials_create");
+  }
+  int rc = follow_stacks(tr, tr->stream);
+  if (rc == QSSB_OK) {
+    e = hipStreamSynchronize(tr->stream);
+    if (e != hipSuccess) rc = report_hip_error(e, "ssb_trials_create");
+  }
+  if (rc) {
+    trials_free(tr);
+    return rc;
   }
   *out = tr;
   return QSSB_OK;
@@ -682,6 +731,8 @@ int ssb_trials_set(ssb_trials* tr, int n_trials, const double* mags_host, const 
     tc.sin_a = to_df(std::sin(-rot));
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int rc = follow_stacks(tr, s);
+  if (rc) return rc;
   // the work queue: each dataset's items follow the previous dataset's
   long long item0 = 0;
   for (auto& ds : tr->sets_host) {
@@ -710,12 +761,16 @@ int ssb_trials_phase_variance(ssb_trials* tr, float* out, int use_graph, void* s
   if (e != hipSuccess) return report_hip_error(e, "trials device");
   if (dev != tr->device) return report_error(QSSB_ERR_ARG, "the trials handle belongs to another device");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int rc = follow_stacks(tr, s);
+  if (rc) return rc;
   if (!use_graph) {
     e = enqueue_trials(tr, out, s);
     if (e != hipSuccess) return report_hip_error(e, "trials");
     return QSSB_OK;
   }
-  if (!tr->exec || tr->graph_trials != tr->n_trials || tr->graph_out != out) {
+  std::vector<double> recip;
+  for (const ssb_plan* p : tr->plans) recip.insert(recip.end(), {p->recip_y, p->recip_x});
+  if (!tr->exec || tr->graph_trials != tr->n_trials || tr->graph_out != out || tr->graph_recip != recip) {
     if (tr->exec) (void)hipGraphExecDestroy(tr->exec);
     if (tr->graph) (void)hipGraphDestroy(tr->graph);
     tr->exec = nullptr;
@@ -730,6 +785,7 @@ int ssb_trials_phase_variance(ssb_trials* tr, float* out, int use_graph, void* s
     if (e != hipSuccess) return report_hip_error(e, "trials graph instantiate");
     tr->graph_trials = tr->n_trials;
     tr->graph_out = out;
+    tr->graph_recip = recip;
   }
   // the graph runs on the handle's own stream, ordered after and before `s`
   e = hipEventRecord(tr->ev_in, s);

@@ -51,6 +51,10 @@ class TrialBatch:
         self.n_trials = 0
         self.out = torch.empty((len(self.engines), self.max_trials), dtype=torch.float32, device=dev)
 
+    def _check_open(self) -> None:
+        for e in self.engines:
+            e.plan.handle          # raises once the plan is closed
+
     def _stream(self):
         return _abi.stream_handle(self.torch.cuda.current_stream(self.device))
 
@@ -66,6 +70,7 @@ class TrialBatch:
             rot = np.ascontiguousarray(np.asarray(rotations, dtype=np.float64).reshape(-1))
             if rot.size != m.shape[0]:
                 raise ValueError("one rotation per trial is needed")
+        self._check_open()
         with self.torch.cuda.device(self.device):
             _abi.call("ssb_trials_set", self._h, int(m.shape[0]), m.ctypes.data_as(_abi._dp),
                       a.ctypes.data_as(_abi._dp), rot.ctypes.data_as(_abi._dp) if rot is not None else None,
@@ -74,6 +79,7 @@ class TrialBatch:
 
     def phase_variance(self, use_graph: bool = True):
         """``[datasets, T]`` phase-image variances (device tensor, asynchronous)."""
+        self._check_open()
         with self.torch.cuda.device(self.device):
             _abi.call("ssb_trials_phase_variance", self._h, _abi.ptr(self.out), 1 if use_graph else 0,
                       self._stream())

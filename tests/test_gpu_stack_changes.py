@@ -1,6 +1,6 @@
-"""Results that outlive a plan's stack: a captured batch of exact losses, replayed
+"""Handles that outlive a plan's stack: a captured batch of exact losses, replayed
 into the same output after the bright field or the stack has changed, gives what
-the plain batch gives."""
+the plain batch gives; a trials handle follows the stack or refuses it."""
 from __future__ import annotations
 
 import numpy as np
@@ -8,7 +8,7 @@ import pytest
 
 from oracle import ssb_oracle as O
 from tests import _cases as C
-from tests._gpu import make_engine
+from tests._gpu import engine_for_data, make_engine
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +52,67 @@ def test_captured_batch_follows_the_stack(cuda):
         np.testing.assert_array_equal(got, plain)
         eng.set_detector_sampling(1.0 / 32.0, 1.0 / 32.0)
     assert len(seen) >= 10
+
+
+def _prepare(eng, d, radius):
+    eng.mean_dp(d)
+    eng.select_bf(0.0, radius)
+    eng.prepare_g(d)
+    eng.cache_rotation(0.0)
+
+
+def _variance(batch, graph):
+    return batch.phase_variance(use_graph=graph).cpu().numpy().copy()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_trials_follow_or_refuse_another_stack(cuda, graph):
+    """A trials handle takes over a stack of the same size and place, keeps its own
+    pixels under a selection that is not prepared, and refuses a stack of another
+    size or layout before anything is launched."""
+    from quantem.gpu_amd.ssb.compute.hip.trials import TrialBatch
+    d, d2 = (cuda.from_numpy(C.poisson_data(s)).cuda() for s in (123, 321))
+    eng = engine_for_data(cuda, d, semiangle_mrad=21.4, det_sampling=1.0, step=0.5, max_bf=256)
+    trials = _trials(9)
+
+    def fresh():
+        batch = TrialBatch([eng], 9)
+        batch.set(*trials)
+        got = _variance(batch, False)
+        batch.close()
+        return got
+
+    _prepare(eng, d, 3.2)
+    small = TrialBatch([eng], 9)
+    small.set(*trials)
+    want = _variance(small, graph)
+    np.testing.assert_array_equal(want, fresh())
+    eng.recon_u16(d2, 0.0, 0.0, 0.0, bf_radius=2.0)           # another selection, the stack untouched
+    np.testing.assert_array_equal(_variance(small, graph), want)
+    small.set(*trials)
+    np.testing.assert_array_equal(_variance(small, graph), want)
+    _prepare(eng, d2, 3.2)                                    # another stack in the same place
+    want2 = fresh()
+    assert not np.array_equal(want2, want)
+    np.testing.assert_array_equal(_variance(small, graph), want2)
+    eng.set_detector_sampling(1.0 / 18.0, 1.0 / 18.0)
+    eng.cache_rotation(0.0)
+    np.testing.assert_array_equal(_variance(small, graph), fresh())
+    for radius in (4.0, 2.0):                                 # more pixels, fewer
+        _prepare(eng, d, radius)
+        with pytest.raises(ValueError, match="replaced"):
+            small.phase_variance(use_graph=graph)
+        with pytest.raises(ValueError, match="replaced"):
+            small.set(*trials)
+    eng.set_bf([8] * 3, [7, 8, 9], (8.0, 8.0), 1.0)
+    eng.import_g(cuda.zeros((3, 128, 65), dtype=cuda.complex64))
+    three = TrialBatch([eng], 9)
+    three.set(*trials)
+    eng.import_g(cuda.zeros((3, 128, 128), dtype=cuda.complex64))
+    with pytest.raises(ValueError, match="replaced"):
+        three.phase_variance(use_graph=graph)
+    eng.plan.close()
+    with pytest.raises(ValueError, match="closed"):
+        three.phase_variance(use_graph=graph)
+    three.close()
+    small.close()
