@@ -57,8 +57,20 @@ void dfree(void* p) {
 // the caller's after all (who may empty that cache) when the device has none left.
 constexpr size_t kLentBytes = (size_t)1 << 30;
 
+// The plan's device for a scope, whichever the caller's is.
+struct OnDevice {
+  int was = -1;
+  explicit OnDevice(int device) {
+    if (hipGetDevice(&was) != hipSuccess || was == device || hipSetDevice(device) != hipSuccess) was = -1;
+  }
+  ~OnDevice() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
+
 template <typename T>
 hipError_t palloc(ssb_plan* p, T** out, size_t count, hipStream_t s) {
+  const OnDevice on(p->device);
   const size_t bytes = count * sizeof(T) > 0 ? count * sizeof(T) : 1;
   hipError_t e = hipErrorOutOfMemory;
   if (!p->alloc || bytes > kLentBytes) e = hipMalloc(reinterpret_cast<void**>(out), bytes);
@@ -75,18 +87,42 @@ hipError_t palloc(ssb_plan* p, T** out, size_t count, hipStream_t s) {
   return hipErrorOutOfMemory;   // (a plan has fewer buffers than slots)
 }
 
-// Like hipFree it waits for the device: work on any stream may use the block,
-// and the caller's memory is ordered on one stream only.
+// Blocks that are done with, once the device has no work that may use them.
+void give_back(ssb_plan* p) {
+  bool any = false;
+  for (void* d : p->unwaited) any = any || d;
+  if (!any) return;
+  if (hipDeviceSynchronize() != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  for (void*& d : p->unwaited) {
+    if (d) p->release(d, p->alloc_ctx);
+    d = nullptr;
+  }
+}
+
+// Like hipFree it waits for the plan's device: work on any stream may use the
+// block, and the caller's memory is ordered on one stream only.  Where that wait
+// is refused (a capture is open) the block stays until the next one succeeds, and
+// for good when the plan ends before.
 void pfree(ssb_plan* p, void* q) {
   if (!q) return;
+  bool lent = false;
   for (void*& slot : p->lent) {
     if (slot != q) continue;
     slot = nullptr;
-    (void)hipDeviceSynchronize();
-    p->release(q, p->alloc_ctx);
-    return;
+    lent = true;
+    for (void*& d : p->unwaited)
+      if (!d) {
+        d = q;
+        break;
+      }
+    break;
   }
-  (void)hipFree(q);
+  const OnDevice on(p->device);
+  if (!lent) (void)hipFree(q);
+  give_back(p);
 }
 
 hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
@@ -324,13 +360,9 @@ int ssb_set_scan_frequencies(ssb_plan* p, const float* qrow_host, const float* q
 
 int ssb_plan_destroy(ssb_plan* p) {
   if (!p) return QSSB_OK;
-  int dev = p->device;
-  (void)hipGetDevice(&dev);
-  if (dev != p->device) (void)hipSetDevice(p->device);
   for (void* q : {(void*)p->block, (void*)p->dp_partial_wide, (void*)p->gain, (void*)p->H, (void*)p->Gt, (void*)p->T,
                   (void*)p->xt, (void*)p->sup_part, (void*)p->sup_box, (void*)p->sup_C})
     pfree(p, q);
-  if (dev != p->device) (void)hipSetDevice(dev);
   if (p->ev_stream) (void)hipEventDestroy(p->ev_stream);
   if (p->xexec) (void)hipGraphExecDestroy(p->xexec);
   if (p->xgraph) (void)hipGraphDestroy(p->xgraph);

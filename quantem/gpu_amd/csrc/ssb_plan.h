@@ -52,12 +52,13 @@ struct ssb_plan {
   double rotation = 0;
   Optics optics{};
   // where the buffers come from: the caller's memory (ssb_plan_create_with) or
-  // the device; `lent` are the blocks to give back
+  // the device; `lent` are the blocks to give back, `unwaited` those of them that
+  // the plan is done with and the device may not be
   ssb_alloc_fn alloc = nullptr;
   ssb_release_fn release = nullptr;
   void* alloc_ctx = nullptr;
   int device = 0;
-  void* lent[16] = {};
+  void* lent[16] = {}, *unwaited[32] = {};
   // device buffers; those every plan has are parts of one block
   char* block = nullptr;
   uint32_t* dp_partial = nullptr;
