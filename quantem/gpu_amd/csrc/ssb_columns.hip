@@ -27,6 +27,9 @@ __device__ __forceinline__ QuadPixel pixel_of_lane(const QuadPixel& p, int lane)
   o.ty = lane_value(p.ty, lane);
   o.margin = lane_value(p.margin, lane);
   o.ak = lane_value(p.ak, lane);
+  o.kx2l = lane_value(p.kx2l, lane);
+  o.ky2l = lane_value(p.ky2l, lane);
+  o.cbl = lane_value(p.cbl, lane);
   return o;
 }
 
@@ -63,20 +66,17 @@ struct Kahan2 {
   __device__ __forceinline__ float2 sum() const { return make_float2(r.s - r.c, i.s - i.c); }
 };
 
-// The term of one point, row q + dq and column col + dcol (sign -1: of -qy),
-// given B = 2 q.k and base = Rout^2 - |k|^2 - |q|^2.
+// The term of one point, given B = 2 q.k and base = Rout^2 - |k|^2 - |q|^2; point
+// gives its frequency in double-float, in the branch that needs it.
+template <typename Point>
 __device__ __forceinline__ float2 quad_term(float2 G, float B, float base, float s, float t, bool whole,
-                                            const QuadPixel& p, const ApIso& ap, const GeomPtrs& gp, df rout2, int b,
-                                            int q, int dq, int col, int dcol, float sign) {
+                                            const QuadPixel& p, const ApIso& ap, Point point) {
   const float near = base + fabsf(B), far = base - fabsf(B);
   t = B < 0.0f ? -t : t;
-  return overlap_term(G, near, far, B, s, t, whole, p.margin, p.ak, ap, [&](df& dm, df& dp) {
-    asm volatile("" : "+v"(q), "+v"(col));   // no addresses kept ahead of the branch
-    q += dq;
-    col += dcol;
-    const df kx{0.5f * p.kx2, as_const(gp.kxl)[b]}, ky{0.5f * p.ky2, as_const(gp.kyl)[b]};
-    exact_d(df{gp.qx[q], gp.qxl[q]}, df{sign * gp.qy[col], sign * gp.qyl[col]}, kx, ky,
-            df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky))), dm, dp);
+  return overlap_term(G, near, far, B, s, t, whole, p.margin, p.ak, ap, [&](float& dm, float& dp) {
+    df x, y;
+    point(x, y);
+    exact_d(x, y, square_of(x, y), df{p.kx2, p.kx2l}, df{p.ky2, p.ky2l}, df{p.cb, p.cbl}, dm, dp);
   });
 }
 
@@ -127,6 +127,16 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
   const int n = group_count(g, groups, info->nbf);   // BF pixels g + i groups
   float2* sp = S_part + (long long)g * N * N;
 
+  // a lane's four frequencies in double-float, for the points at an edge (from LDS: the
+  // wave waits less than for the tables)
+  __shared__ float4 own[4 * 256];
+  auto own_point = [&](int i, float sign, df& x, df& y) {
+    int at = i * 256 + threadIdx.x;
+    asm volatile("" : "+v"(at));                     // in the branch, not ahead of it
+    const float4 v = own[at];
+    x = df{v.x, v.y};
+    y = df{sign * v.z, sign * v.w};
+  };
   int row0[4], col0[4];                              // the tiles' first row and column (wave-uniform)
   float qx[4], qy[4], q2[4], s[4], x0[4], x1[4], y0[4], y1[4];
   const int lr = last ? lane : lane & 15, lc = last ? 0 : lane >> 4;
@@ -142,6 +152,7 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
     // (at N = 128 the rows of column N/2 fill two of the four)
     q2[i] = last && (t - SETS) * 256 + 64 * i >= N ? INFINITY : fmaf(qx[i], qx[i], qy[i] * qy[i]);
     s[i] = half_sum(ev, qx[i], qy[i]);
+    own[i * 256 + threadIdx.x] = make_float4(qx[i], gp.qxl[row0[i] + lr], qy[i], gp.qyl[col0[i] + lc]);
   }
   // the tile of the rows from N/2, whose first row has partners of its own
   const int ny = last || rt != 0 ? -1 : (2 - turn) & 3;
@@ -167,7 +178,7 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
   };
   auto B_of = [&](int i, const QuadPixel& p) { return fmaf(qx[i], p.kx2, qy[i] * p.ky2) + 0.0f; };   // no negative zero
   for (int c0 = 0; c0 < n; c0 += 64) {
-    const QuadPixel pl = quad_pixel(gp, g + min(c0 + lane, n - 1) * groups, ev, rout2);
+    const QuadPixel pl = quad_pixel(gp, g + min(c0 + lane, n - 1) * groups, ev, rout2, ap);
     bool reach = ny >= 0 && apertures_reach(pl, rout2.hi, qn, qn, ny0, ny1);
     unsigned long long nmask = __ballot(reach);
 #pragma unroll
@@ -199,8 +210,8 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
       for (int i = 0; i < 4; ++i) {
         const float B = B_of(i, p), base = p.cb - q2[i];
         if (base + fabsf(B) > -p.margin)
-          acc[i].add(quad_term(cur.G[i], B, base, s[i], fmaf(qx[i], p.tx, qy[i] * p.ty), near_whole(s[i]), p, ap, gp,
-                               rout2, b, lr, row0[i], lc, col0[i], 1.0f));
+          acc[i].add(quad_term(cur.G[i], B, base, s[i], fmaf(qx[i], p.tx, qy[i] * p.ty), near_whole(s[i]), p, ap,
+                               [&](df& x, df& y) { own_point(i, 1.0f, x, y); }));
         __builtin_amdgcn_sched_barrier(0);
       }
       if (nmask >> l & 1) {
@@ -208,17 +219,15 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
         const float B = fmaf(nqx, p.kx2, nqy * p.ky2) + 0.0f, base = p.cb - nq2;
         const float ns = half_sum(ev, nqx, nqy);
         float2 G = cur.G[0];
-        int c = col0[0];
 #pragma unroll
         for (int i = 1; i < 4; ++i) {
           if (i == ny) {
             G = cur.G[i];
-            c = col0[i];
           }
         }
         if (lr == 0 && base + fabsf(B) > -p.margin)
-          nyq.add(quad_term(cconj(G), B, base, ns, fmaf(nqx, p.tx, nqy * p.ty), near_whole(ns), p, ap, gp, rout2, b,
-                            HALF, 0, lc, c, -1.0f));
+          nyq.add(quad_term(cconj(G), B, base, ns, fmaf(nqx, p.tx, nqy * p.ty), near_whole(ns), p, ap,
+                            [&](df& x, df& y) { own_point(ny, -1.0f, x, y); }));
       }
       if (!mask) break;
       cur = nxt;
@@ -387,11 +396,20 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
   constexpr int NW = column_waves(N), CG = S * NW;   // columns a workgroup
   constexpr int NCG = HALF / CG, LG = 16 / CG;       // workgroups that share a line of H
   __shared__ float2 twl[Fft::TW];
-  __shared__ float qxS[N];
+  // the frequencies of the rows and of the workgroup's columns, for the points at an
+  // edge in double-float (at 512 the rows' low words would cost a workgroup a CU)
+  constexpr bool LOWS = N != 512 && !STORE;
+  __shared__ float qxS[STORE ? 1 : N], qxlS[LOWS ? N : 1];
+  __shared__ float2 qyS[CG];
   __shared__ float2 exS[NW][Fft::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  for (int i = tid; i < N; i += 64 * NW) qxS[i] = gp.qx[i];
+  if constexpr (!STORE) {
+    for (int i = tid; i < N; i += 64 * NW) {
+      qxS[i] = gp.qx[i];
+      if (LOWS) qxlS[LOWS ? i : 0] = gp.qxl[i];
+    }
+  }
   Fft::twiddles(twl, tw_g, tid, 64 * NW);
   __syncthreads();
   float2* ex = exS[w];
@@ -470,6 +488,15 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
     }
   } else {
     const float qy = gp.qy[j];
+    if (tid < CG) qyS[tid] = make_float2(gp.qy[last ? HALF : cg * CG + tid], gp.qyl[last ? HALF : cg * CG + tid]);
+    __syncthreads();
+    auto point = [&](int q, int dq, float sign, df& x, df& y) {
+      int c = last ? 0 : S * w + col;
+      asm volatile("" : "+v"(q), "+v"(c));           // no addresses kept ahead of the branch
+      x = df{qxS[q + dq], LOWS ? qxlS[LOWS ? q + dq : 0] : gp.qxl[q + dq]};
+      const float2 v = qyS[c];
+      y = df{sign * v.x, sign * v.y};
+    };
     float y0, y1;
     wave_range(gp.qy[last ? HALF : cg * CG + lane % CG], y0, y1);
     const float qn = as_const(gp.qx)[HALF];
@@ -486,7 +513,7 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
     for (int r = 0; r < 16; ++r) acc[r].init();
     nyq.init();
     for (int c0 = 0; c0 < n; c0 += 64) {
-      const QuadPixel pl = quad_pixel(gp, bg + min(c0 + lane, n - 1) * gpp, ev, rout2);
+      const QuadPixel pl = quad_pixel(gp, bg + min(c0 + lane, n - 1) * gpp, ev, rout2, ap);
       // the same for every wave of the workgroup
       unsigned long long mask =
           __ballot(c0 + lane < n && apertures_reach(pl, rout2.hi, -INFINITY, INFINITY, y0, y1));
@@ -527,8 +554,8 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
             whole = near_whole(at);
           }
           if (base + fabsf(B) > -p.margin)
-            acc[r].add(quad_term(x[r], B, base, s, fmaf(qx, p.tx, tq), whole, p, ap, gp, rout2, b, k1, K * r, j, 0,
-                                 1.0f));
+            acc[r].add(quad_term(x[r], B, base, s, fmaf(qx, p.tx, tq), whole, p, ap,
+                                 [&](df& x, df& y) { point(k1, K * r, 1.0f, x, y); }));
           __builtin_amdgcn_sched_barrier(0);               // one point at a time
         }
         if (!last && apertures_reach(p, rout2.hi, qn, qn, -y1, -y0)) {
@@ -536,8 +563,8 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
           const float B = fmaf(qn, p.kx2, -Bq) + 0.0f, base = fmaf(-qn, qn, cq);
           const float ns = half_sum(ev, qn, -qy);
           if (k1 == 0 && base + fabsf(B) > -p.margin)
-            nyq.add(quad_term(cconj(x[8]), B, base, ns, fmaf(qn, p.tx, -tq), near_whole(ns), p, ap, gp, rout2, b, HALF,
-                              0, j, 0, -1.0f));
+            nyq.add(quad_term(cconj(x[8]), B, base, ns, fmaf(qn, p.tx, -tq), near_whole(ns), p, ap,
+                              [&](df& x, df& y) { point(HALF, 0, -1.0f, x, y); }));
         }
         if (!mask) break;
       }

@@ -235,6 +235,7 @@ struct ApIso {
   float d_out;      // d below which A == 0 (negative margin)
   float rout;       // Rout
   float scale;      // lambda / ang
+  float edge;       // distance in d from the edges up to which overlap_term's estimates do not decide
 };
 
 // Number of BF groups (partial planes) of the object-path trotter's tile

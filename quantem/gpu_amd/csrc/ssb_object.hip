@@ -474,6 +474,7 @@ ApIso iso_aperture(const Optics& o, df& rout2_df) {
   // exact 0/1 outside the band, with a relative margin above FP32 noise
   a.d_in = (rin > 0.0) ? (float)((r2 - rin * rin) * (1.0 + 1e-5)) : INFINITY;
   a.d_out = (float)(-r2 * 1e-5);
+  a.edge = (float)(r2 > 25.0 ? 4e-6 * r2 : 1e-4);
   return a;
 }
 

@@ -205,49 +205,60 @@ __device__ __forceinline__ float2 gamma_hat_st(float ak, float am, float app, fl
 // cancel; next to 1 float32 itself is no finer than 6e-8).  A BF pixel of smaller
 // A(k) goes there with all its points (margin = infinity).  whole: near_whole(s),
 // if the caller cannot know that it isn't.  There both d
-// come in double-float from exact(dn, df) within kEdgeMargin of an edge and
-// with both apertures in their bands, where their values or their difference
-// decide; inside one aperture and well inside the other's band the estimates
-// give the ratio to 2e-6.  B must not be a negative zero unless t is zero.
-constexpr float kEdgeMargin = 1e-4f;   // far above the estimates' error (2e-5 for terms below 32)
+// come from exact(dn, df), to float32 of themselves: the float32 estimates, whose error grows
+// with the terms and weighs by the width of the band, would give an aperture in its
+// band to 1e-6 at 20 mrad and 1.25 mrad a pixel and to 1e-5 at 40 mrad and 0.25.
+// They only say whether a point is within ap.edge of an edge, at least 1e-4 and
+// 4e-6 Rout^2: they add up, for |Q| up to 2 Rout, to 2.5e-6 Rout^2.  B must not be a
+// negative zero unless t is zero.
 constexpr float kSmallAk = 1.2e-2f;
 constexpr float kNearWhole = 2e-6f;
 __device__ __forceinline__ bool near_whole(float s) { return fabsf(s - rintf(s)) <= kNearWhole; }
-__device__ __forceinline__ float edge_margin(float ak) { return ak < kSmallAk ? INFINITY : kEdgeMargin; }
+__device__ __forceinline__ float edge_margin(float ak, const ApIso& ap) { return ak < kSmallAk ? INFINITY : ap.edge; }
 
 template <typename Exact>
 __device__ __forceinline__ float2 overlap_term(float2 G, float near, float far, float B, float s, float t,
                                                bool whole, float margin, float ak, const ApIso& ap, Exact exact) {
-  const float inner = ap.d_in + kEdgeMargin;
+  const float inner = ap.d_in + ap.edge;
   const bool both = far >= inner;
   const bool general = (fabsf(near) < margin) | ((far > -margin) & (far < inner)) | (both & whole);
   float2 z = overlap_unit(G, both, s, t, __float_as_uint(B) & 0x80000000u);
   if (general) {
-    df dn{near, 0.0f}, dfar{far, 0.0f};
-    // the estimates do away from every edge of a lens whose other aperture is one
-    if (!(both | ((near >= inner) & (far >= kEdgeMargin) & (far <= ap.d_in - kEdgeMargin))) | (margin > kEdgeMargin)) {
+    float dn = near, dfar = far;
+    if (!both) {
       exact(dn, dfar);
       if (B < 0.0f) {
-        const df x = dn;
+        const float x = dn;
         dn = dfar;
         dfar = x;
       }
     }
-    float2 g = gamma_hat_st(ak, aperture_from_d(dn, ap), aperture_from_d(dfar, ap), s, t);
+    float2 g = gamma_hat_st(ak, aperture_from_d(df{dn, 0.0f}, ap), aperture_from_d(df{dfar, 0.0f}, ap), s, t);
     if (B < 0.0f) g.x = -g.x;
     z = make_float2(fmaf(G.x, g.x, G.y * g.y), fmaf(G.y, g.x, -(G.x * g.y)));
   }
   return z;
 }
 
-// d of Q - k and Q + k in double-float; q and k through the branch they are
-// needed in (nothing of it is formed ahead of it).
-__device__ __forceinline__ void exact_d(df qx, df qy, df kx, df ky, df cb, df& dm, df& dp) {
-  const df x = df_in_branch(qx), y = df_in_branch(qy);
-  const df qk2 = df_mul(df_add(df_mul(x, kx), df_mul(y, ky)), df{2.0f, 0.0f});
-  const df base = df_sub(cb, df_add(df_mul(x, x), df_mul(y, y)));
-  dm = df_add(base, qk2);
-  dp = df_sub(base, qk2);
+// |q|^2 in double-float.
+__device__ __forceinline__ df square_of(df x, df y) {
+#pragma clang fp contract(off)
+  const df xx = two_prod(x.hi, x.hi), yy = two_prod(y.hi, y.hi), q2 = two_sum(xx.hi, yy.hi);
+  return df{q2.hi, q2.lo + (xx.lo + yy.lo) + 2.0f * (x.hi * x.lo + y.hi * y.lo)};
+}
+
+// d of Q - k and Q + k from double-float q, |q|^2, 2 k and Rout^2 - |k|^2, rounded once
+// but for terms of 1e-14: the leading products and sums exactly, the rest in
+// float32 (a third of the work of double-float throughout).  Equal where Q.k is
+// zero.
+__device__ __forceinline__ void exact_d(df x, df y, df q2, df kx2, df ky2, df cb, float& dm, float& dp) {
+#pragma clang fp contract(off)
+  const df xk = two_prod(x.hi, kx2.hi), yk = two_prod(y.hi, ky2.hi), qk2 = two_sum(xk.hi, yk.hi);
+  const float qkl = qk2.lo + (xk.lo + yk.lo) + ((x.hi * kx2.lo + y.hi * ky2.lo) + (x.lo * kx2.hi + y.lo * ky2.hi));
+  const df base = two_sum(cb.hi, -q2.hi);
+  const float bl = base.lo + (cb.lo - q2.lo);
+  dm = (base.hi + qk2.hi) + (bl + qkl);
+  dp = (base.hi - qk2.hi) + (bl - qkl);
 }
 
 // What the terms of one BF pixel share under a quadratic chi: 2 k, Rout^2 -
@@ -255,19 +266,25 @@ __device__ __forceinline__ void exact_d(df qx, df qy, df kx, df ky, df cb, df& d
 // |u|^2 up to which an aperture or its margin can be met (kReach above Rout^2).
 struct QuadPixel {
   float kx2, ky2, cb, tx, ty, margin, ak;
+  float kx2l, ky2l, cbl;   // low words, for exact_d
 };
 constexpr float kReachRel = 1.00002f, kReachAbs = 3e-4f;
 
-__device__ __forceinline__ QuadPixel quad_pixel(const GeomPtrs& gp, int b, const QuadTurns& ev, df rout2) {
+__device__ __forceinline__ QuadPixel quad_pixel(const GeomPtrs& gp, int b, const QuadTurns& ev, df rout2,
+                                                const ApIso& ap) {
   QuadPixel p;
   const df kx{gp.kx[b], gp.kxl[b]}, ky{gp.ky[b], gp.kyl[b]};
   p.kx2 = 2.0f * kx.hi;
   p.ky2 = 2.0f * ky.hi;
-  p.cb = df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky))).hi;
+  p.kx2l = 2.0f * kx.lo;
+  p.ky2l = 2.0f * ky.lo;
+  const df cb = df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky)));
+  p.cb = cb.hi;
+  p.cbl = cb.lo;
   p.tx = fmaf(ev.k0 + ev.m12c, p.kx2, ev.m12s * p.ky2);
   p.ty = fmaf(ev.k0 - ev.m12c, p.ky2, ev.m12s * p.kx2);
   p.ak = gp.ak[b];
-  p.margin = edge_margin(p.ak);
+  p.margin = edge_margin(p.ak, ap);
   return p;
 }
 

@@ -195,12 +195,18 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
   const float qn = as_const(gp.qx)[HALF];
   const float k0 = ch.k0, k4 = ch.k4, m12c = ch.m12c, m12s = ch.m12s, m12s2 = 2.0f * m12s;
 
+  // the low words of qx where registers are left for them
+  constexpr int LOWS = R <= 4 ? R : 0;
+  float qxl[LOWS ? LOWS : 1];
+#pragma unroll
+  for (int m = 0; m < LOWS; ++m) qxl[m] = gp.qxl[lane + 64 * m];
+  auto low_of = [&](int m) { return LOWS ? qxl[LOWS ? m : 0] : gp.qxl[lane + 64 * m]; };
+
   // what a point needs of its BF pixel
   struct Pixel {
-    float kx2, ky2, cb, u, vx, vy, margin, ak, chik;
+    float kx2, ky2, cb, u, vx, vy, margin, ak, chik, kxl, kyl, cbl;
   } px;
-  int b = 0;
-  auto term = [&](float2 G, int q, float qxv, int col, float qyv) {
+  auto term = [&](float2 G, int m, float qxv, int col, float qyv) {   // row lane + 64 m
     const float B = fmaf(qxv, px.kx2, qyv * px.ky2) + 0.0f;   // no negative zero
     const float q2 = fmaf(qxv, qxv, qyv * qyv);
     const float base = px.cb - q2;
@@ -225,10 +231,9 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
         s = add_cancelling((qxv - qyv) * (qxv + qyv) * m12c, fmaf(qxv * qyv, m12s2, s));
       }
       t = B < 0.0f ? -t : t;
-      z = overlap_term(G, near, far, B, s, t, near_whole(s), px.margin, px.ak, ap, [&](df& dm, df& dp) {
-        const df kx{0.5f * px.kx2, as_const(gp.kxl)[b]}, ky{0.5f * px.ky2, as_const(gp.kyl)[b]};
-        exact_d(df{qxv, gp.qxl[q]}, df{qyv, gp.qyl[col]}, kx, ky, df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky))),
-                dm, dp);
+      z = overlap_term(G, near, far, B, s, t, near_whole(s), px.margin, px.ak, ap, [&](float& dm, float& dp) {
+        const df x = df_in_branch(df{qxv, low_of(m)}), y = df_in_branch(df{qyv, as_const(gp.qyl)[col]});
+        exact_d(x, y, square_of(x, y), df{px.kx2, 2.0f * px.kxl}, df{px.ky2, 2.0f * px.kyl}, df{px.cb, px.cbl}, dm, dp);
       });
     }
     return z;
@@ -244,22 +249,26 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
   };
   fetch(i0);
   for (int i = i0; i < i1; ++i) {
-    b = b_begin + i;
+    const int b = b_begin + i;
     const float kx = as_const(gp.kx)[b], ky = as_const(gp.ky)[b];   // scalar loads
     const float kxl = as_const(gp.kxl)[b], kyl = as_const(gp.kyl)[b];
     px.kx2 = 2.0f * kx;
     px.ky2 = 2.0f * ky;
+    px.kxl = kxl;
+    px.kyl = kyl;
     {
       const df kxd{kx, kxl}, kyd{ky, kyl};
-      px.cb = df_sub(rout2, df_add(df_mul(kxd, kxd), df_mul(kyd, kyd))).hi;
+      const df cb = df_sub(rout2, df_add(df_mul(kxd, kxd), df_mul(kyd, kyd)));
+      px.cb = cb.hi;
+      px.cbl = cb.lo;
     }
     px.u = fmaf(2.0f * k4, fmaf(kx, kx, ky * ky), k0);
     px.vx = 2.0f * fmaf(m12c, kx, m12s * ky);
     px.vy = 2.0f * fmaf(m12s, kx, -(m12c * ky));
     px.ak = as_const(gp.ak)[b];
-    px.margin = edge_margin(px.ak);
+    px.margin = edge_margin(px.ak, ap);
     if (px.ak == 0.0f) px.cb = -1e30f;   // no overlap at all (ak takes part in no other form)
-    if (px.ak == 0.0f) px.margin = kEdgeMargin;
+    if (px.ak == 0.0f) px.margin = ap.edge;
     px.chik = 0.0f;
     if constexpr (GENERAL) {
       float odd;
@@ -279,14 +288,14 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
       const float qy = as_const(gp.qy)[j];
 #pragma unroll
       for (int m = 0; m < R; ++m) {
-        c[s][m] = term(g[s][m], lane + 64 * m, qx[m], j, qy);
+        c[s][m] = term(g[s][m], m, qx[m], j, qy);
         __builtin_amdgcn_sched_barrier(0);   // one point at a time
       }
       if (j != 0) {
         if (nyq) {
           // the Nyquist row (lane 0, m = R / 2): its partner, column N - j, is
           // evaluated at its own grid frequency (q_N/2, -qy)
-          const float2 cb = term(cconj(g[s][R / 2]), lane + 64 * (R / 2), qx[R / 2], N - j, -qy);
+          const float2 cb = term(cconj(g[s][R / 2]), R / 2, qx[R / 2], N - j, -qy);
           if (lane == 0) {
             const float2 ca = c[s][R / 2];
             Hrow[(long long)i * HALF + j] = make_float2(0.5f * (ca.x + cb.x), 0.5f * (ca.y - cb.y));
@@ -305,7 +314,7 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
       const float2* gh = Gt + ((long long)b * GCOLS + HALF) * N;
       const float qy = as_const(gp.qy)[HALF];
 #pragma unroll
-      for (int m = 0; m < R; ++m) h[m] = term(gh[lane + 64 * m], lane + 64 * m, qx[m], HALF, qy);
+      for (int m = 0; m < R; ++m) h[m] = term(gh[lane + 64 * m], m, qx[m], HALF, qy);
       if (lane == 0) c[0][0] = make_float2(info->dc_re, info->dc_im);
       wave_fence();
       float2 pc[R], ph[R];

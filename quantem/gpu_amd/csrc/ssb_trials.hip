@@ -70,7 +70,7 @@ struct __attribute__((aligned(32))) TrialBf {
 struct __attribute__((aligned(32))) TrialBfMore {
   float ak, chik;      // A(k), chi(k) in radians
   float cb, cbl;       // Rout^2 - |k|^2 as double-float
-  float kxl, kyl;      // low words of k
+  float kx2l, ky2l;    // low words of 2 k
   float vx, vy;        // 2 M k of the C12 matrix, half turns
 };
 
@@ -104,7 +104,7 @@ __device__ __forceinline__ float chi_even(const TrialChi& tc, float ux, float uy
 
 __global__ void __launch_bounds__(256)
 k_trial_geometry(const int* __restrict__ bf_rows, const int* __restrict__ bf_cols, const BfInfo* __restrict__ info,
-                 int nbf, int T, df recip_y, df recip_x, Optics o, df rout2,
+                 int nbf, int T, df recip_y, df recip_x, Optics o, ApIso ap, df rout2,
                  const TrialChi* __restrict__ chis, TrialBf* __restrict__ out, TrialBfMore* __restrict__ more) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (long long)T * nbf) return;
@@ -126,14 +126,14 @@ k_trial_geometry(const int* __restrict__ bf_rows, const int* __restrict__ bf_col
   r.ky2[i] = 2.0f * ky.hi;
   r.cb[i] = ak == 0.0f ? -1e30f : cb.hi;
   r.u[i] = fmaf(2.0f * tc.k4, k2, tc.k0);
-  r.margin[i] = ak == 0.0f ? kEdgeMargin : edge_margin(ak);
+  r.margin[i] = ak == 0.0f ? ap.edge : edge_margin(ak, ap);
   TrialBfMore m;
   m.ak = ak;
   m.chik = chi_even(tc, kx.hi, ky.hi);
   m.cb = cb.hi;
   m.cbl = cb.lo;
-  m.kxl = kx.lo;
-  m.kyl = ky.lo;
+  m.kx2l = 2.0f * kx.lo;
+  m.ky2l = 2.0f * ky.lo;
   m.vx = 2.0f * (tc.m12c * kx.hi + tc.m12s * ky.hi);
   m.vy = 2.0f * (tc.m12s * kx.hi - tc.m12c * ky.hi);
   more[slot * kTrialBlock + i] = m;
@@ -150,11 +150,13 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
                                            Kahan (&ar)[TB], Kahan (&ai)[TB]) {
   const int nbf = ds.nbf;
   const float qxf = ds.qx[q], qyf = ds.qy[c];
-  float q2f, qa = 0.0f, qb = 0.0f;
+  const float qxl = ds.qxl[q], qyl = ds.qyl[c];
+  float q2f, q2l, qa = 0.0f, qb = 0.0f;
   {
-    const df qx{qxf, ds.qxl[q]}, qy{qyf, ds.qyl[c]};
+    const df qx{qxf, qxl}, qy{qyf, qyl};
     const df q2 = df_add(df_mul(qx, qx), df_mul(qy, qy));
-    q2f = live ? q2.hi + q2.lo : 1e30f;   // idle lanes: outside every aperture
+    q2f = live ? q2.hi : 1e30f;   // idle lanes: outside every aperture
+    q2l = q2.lo;
     if (!RADIAL) {
       const df a = df_sub(df_mul(qx, qx), df_mul(qy, qy));
       qa = a.hi + a.lo;
@@ -210,9 +212,9 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
             }
             t = B < 0.0f ? -ts : ts;
           }
-          const float2 z = overlap_term(G, near, far, B, s, t, near_whole(s), margin, km[i].ak, ds.ap, [&](df& dm, df& dp) {
-            exact_d(df{qxf, ds.qxl[q]}, df{qyf, ds.qyl[c]}, df{0.5f * kx2[i], km[i].kxl}, df{0.5f * ky2[i], km[i].kyl},
-                    df{km[i].cb, km[i].cbl}, dm, dp);
+          const float2 z = overlap_term(G, near, far, B, s, t, near_whole(s), margin, km[i].ak, ds.ap, [&](float& dm, float& dp) {
+            exact_d(df_in_branch(df{qxf, qxl}), df_in_branch(df{qyf, qyl}), df{q2f, q2l}, df{kx2[i], km[i].kx2l},
+                    df{ky2[i], km[i].ky2l}, df{km[i].cb, km[i].cbl}, dm, dp);
           });
           ar[i].add(z.x);
           ai[i].add(z.y);
@@ -568,11 +570,11 @@ hipError_t enqueue_trials(ssb_trials* tr, float* out, hipStream_t s) {
   for (size_t i = 0; i < tr->plans.size(); ++i) {
     ssb_plan* p = tr->plans[i];
     df rout2;
-    (void)iso_aperture(p->optics, rout2);
+    const ApIso ap = iso_aperture(p->optics, rout2);
     const int nbf = tr->sets_host[i].nbf;
     const long long total = (long long)T * nbf;
     hipLaunchKernelGGL(k_trial_geometry, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, tr->bf[i],
-                       tr->bf[i] + nbf, tr->info[i], nbf, T, to_df(p->recip_y), to_df(p->recip_x), p->optics, rout2,
+                       tr->bf[i] + nbf, tr->info[i], nbf, T, to_df(p->recip_y), to_df(p->recip_x), p->optics, ap, rout2,
                        tr->chis, tr->tbf[i], tr->more[i]);
   }
   long long total_items = 0;
