@@ -118,6 +118,9 @@ struct WaveIfft {
   }
 };
 
+// (a + b) / 2 rounded once, whatever a + b is.
+__device__ __forceinline__ float mean2(float a, float b) { return fmaf(0.5f, a, 0.5f * b); }
+
 // Whether a BF pixel's apertures can reach the Nyquist row: |Q -/+ k| >=
 // |q_N/2| - |kx| there.
 __device__ __forceinline__ bool reaches_nyquist(float qn, float kx, const ApIso& ap) {
@@ -139,21 +142,26 @@ __device__ __forceinline__ float atan_unit(float q) {
   return fmaf(p * u, q, q);
 }
 
-// a / b to the last place or two, for finite b that is no denormal.
+// a / b to the last place or two, for kQuotientLo <= b <= kQuotientHi (the hardware's
+// reciprocal knows no denormals, neither given nor returned).
+constexpr float kQuotientLo = 0x1p-125f, kQuotientHi = 0x1p125f;
 __device__ __forceinline__ float quotient(float a, float b) {
   const float inv = __builtin_amdgcn_rcpf(b);
   const float q = a * inv;
   return fmaf(fmaf(-q, b, a), inv, q);
 }
 
-// atan2 for finite arguments by the octants; where x > |y| it is
-// atan_unit(quotient(y, x)), to which it then reduces bit for bit.
+// atan2 by the octants, for arguments of any size; where x > |y| it is
+// atan_unit(quotient(y, x)), to which it then reduces bit for bit (both operands
+// come to the exponent of the larger first: the same mantissas).
 __device__ __forceinline__ float phase_of(float y, float x) {
   const float ay = fabsf(y), ax = fabsf(x);
   const bool steep = ay > ax;                                   // (fmaxf and fminf would lose a NaN)
   const float mx = steep ? ay : ax, mn = steep ? ax : ay;
-  float q = quotient(mn, mx);
+  const int ex = __builtin_amdgcn_frexp_expf(mx);
+  float q = quotient(ldexpf(mn, -ex), ldexpf(mx, -ex));
   q = mx > 0.0f || mn != mn ? q : mx;   // 0 / 0 -> 0
+  q = mx == INFINITY ? (mn < mx ? 0.0f : (mn == mx ? 1.0f : mn)) : q;
   float a = atan_unit(q);
   a = steep ? 1.5707963267948966f - a : a;
   a = x < 0.0f ? 3.1415926535897931f - a : a;
@@ -298,8 +306,8 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
           const float2 cb = term(cconj(g[s][R / 2]), R / 2, qx[R / 2], N - j, -qy);
           if (lane == 0) {
             const float2 ca = c[s][R / 2];
-            Hrow[(long long)i * HALF + j] = make_float2(0.5f * (ca.x + cb.x), 0.5f * (ca.y - cb.y));
-            c[s][R / 2] = make_float2(0.5f * (ca.x - cb.x), 0.5f * (ca.y + cb.y));
+            Hrow[(long long)i * HALF + j] = make_float2(mean2(ca.x, cb.x), mean2(ca.y, -cb.y));
+            c[s][R / 2] = make_float2(mean2(ca.x, -cb.x), mean2(ca.y, cb.y));
           }
         }
         // Y = -i C
@@ -336,10 +344,10 @@ k_phase_cols(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, Geo
 #pragma unroll
       for (int m = 0; m < R; ++m) {
         // D = (C - conj C(-Q)) / 2 and H = (C + conj C(-Q)) / 2 of both columns
-        const float2 d0 = make_float2(0.5f * (c[0][m].x - pc[m].x), 0.5f * (c[0][m].y + pc[m].y));
-        const float2 dh = make_float2(0.5f * (h[m].x - ph[m].x), 0.5f * (h[m].y + ph[m].y));
-        const float2 h0 = make_float2(0.5f * (c[0][m].x + pc[m].x), 0.5f * (c[0][m].y - pc[m].y));
-        const float2 hh = make_float2(0.5f * (h[m].x + ph[m].x), 0.5f * (h[m].y - ph[m].y));
+        const float2 d0 = make_float2(mean2(c[0][m].x, -pc[m].x), mean2(c[0][m].y, pc[m].y));
+        const float2 dh = make_float2(mean2(h[m].x, -ph[m].x), mean2(h[m].y, ph[m].y));
+        const float2 h0 = make_float2(mean2(c[0][m].x, pc[m].x), mean2(c[0][m].y, -pc[m].y));
+        const float2 hh = make_float2(mean2(h[m].x, ph[m].x), mean2(h[m].y, -ph[m].y));
         // Y0 + i Yh = -i D0 + Dh, and H0 + i Hh
         c[0][m] = make_float2(d0.y + dh.x, dh.y - d0.x);
         eg[0][m] = make_float2(h0.x - hh.y, h0.y + hh.x);
@@ -503,7 +511,7 @@ k_phase_rows(const float2* __restrict__ T, const float2* __restrict__ EG, const 
           eb = egv[2 * a + 1];
         }
       }
-      float h[4][2];
+      float h[4][2], lo = INFINITY, hi = 0.0f;
       bool easy = true;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -511,7 +519,10 @@ k_phase_rows(const float2* __restrict__ T, const float2* __restrict__ EG, const 
         h[r][0] = ea.x + (odd ? -ea.y : ea.y) + f[p][r];
         h[r][1] = eb.x + (odd ? -eb.y : eb.y) - f[p][r];
         easy &= (h[r][0] > fabsf(o[p][r].x)) & (h[r][1] > fabsf(o[p][r].y));
+        lo = fminf(lo, fminf(h[r][0], h[r][1]));
+        hi = fmaxf(hi, fmaxf(h[r][0], h[r][1]));
       }
+      easy &= (lo >= kQuotientLo) & (hi <= kQuotientHi);
       // a bright field brighter than its modulation leaves the first octants only
       float ph[4][2];
       if (__all(easy)) {
