@@ -10,7 +10,8 @@ candidate of each knob in turn (coordinate descent, the others held at their
 best so far) on the caller's own resident data with the per-stage hipEvents
 of ``ssb_recon_u16``, keeps the fastest, and can store the choice in a JSON
 cache keyed by device, scan size, detector size and BF count so later runs
-reuse it (``load_cached``).  The reference has no counterpart: its launch
+reuse it (``load_cached``).  An entry says which meaning of the ``trotter``
+values it was measured with; values of another meaning are left out.  The reference has no counterpart: its launch
 shapes are fixed per scan size (``cuda/kernels/fft256.py:1051-1058``).
 """
 from __future__ import annotations
@@ -29,6 +30,13 @@ KNOBS = {"stream_wg": 0, "gather_pairs": 1, "trotter": 2, "split": 4}
 # the recon stages whose time each knob changes
 STAGE = {"stream_wg": ("mean_dp_stream",), "gather_pairs": ("gather_rowfft",), "trotter": ("colfft_trotter",),
          "split": ("gather_rowfft", "colfft_trotter")}
+
+
+# what the values of "trotter" stand for, by scan size: groups of bright-field
+# pixels from 256 on (before, and in entries that say nothing, kernels and tile
+# shapes), tile shapes at 128
+def trotter_meaning(scan_n: int) -> str:
+    return "bf_groups" if scan_n >= 256 else "tile_shape"
 
 
 def candidates(scan_n: int, knob: str) -> list[int]:
@@ -61,17 +69,22 @@ def _read_cache(path: Path) -> dict:
 
 
 def load_cached(engine, nbf: int, path: Path | None = None) -> dict | None:
-    """Apply a cached choice for this device/shape, if one exists; returns it."""
+    """Apply a cached choice for this device/shape, if one exists; returns what
+    was applied."""
     torch = engine.torch
     s = engine.plan.spec
     key = cache_key(torch.cuda.get_device_name(engine.plan.device), s.scan_n, (s.det_rows, s.det_cols), nbf)
-    entry = _read_cache(path or cache_path()).get(key)
-    if not entry:
-        return None
+    entry = usable(_read_cache(path or cache_path()).get(key), s.scan_n)
     for knob, value in entry.items():
-        if knob in KNOBS:
-            engine.tune_set(KNOBS[knob], int(value))
-    return entry
+        engine.tune_set(KNOBS[knob], int(value))
+    return entry or None
+
+
+def usable(entry: dict | None, scan_n: int) -> dict:
+    """The knobs of a cache entry whose values mean what they mean now."""
+    entry = entry or {}
+    same = entry.get("trotter_meaning", "tile_shape") == trotter_meaning(scan_n)
+    return {k: v for k, v in entry.items() if k in KNOBS and (same or k != "trotter")}
 
 
 def _time_stage(engine, run, stages, repeats: int) -> float:
@@ -132,7 +145,7 @@ def autotune(engine, data, c10: float = 0.0, repeats: int = 5, knobs=tuple(KNOBS
         key = cache_key(torch.cuda.get_device_name(engine.plan.device), n, (s.det_rows, s.det_cols), engine.num_bf)
         p = path or cache_path()
         entries = _read_cache(p)
-        entries[key] = best
+        entries[key] = {**best, "trotter_meaning": trotter_meaning(n)}
         p.parent.mkdir(parents=True, exist_ok=True)
         p.write_text(json.dumps(entries, indent=1, sort_keys=True))
     return {"config": best, "ms": {k: {str(v): t for v, t in d.items()} for k, d in table.items()},
