@@ -512,7 +512,10 @@ hipError_t launch_trotter_slots(int N, bool from_h, const float2* src, const BfI
   const ApIso ap = iso_aperture(o, rout2);
   const bool iso = optics_isotropic(o);
   if (iso && (!from_h || N != 128)) return hipErrorInvalidValue;   // ssb_columns.hip's
-  const int groups = object_groups(N);
+  // a resident stack at N = 256: 32 BF groups (2048 items, two rounds of four
+  // workgroups a CU, so that the heavy-first order can even out the CUs: an object
+  // of 800 BF pixels takes 181 us, in 16 groups 193)
+  const int groups = (!from_h && N == 256) ? 2 * object_groups(N) : object_groups(N);
   if (groups_used) *groups_used = groups;
 #define QSSB_SLOTS_ONE(NN, SGV, BL, FH, IS)                                                                 \
   hipLaunchKernelGGL((k_trotter_slots<NN, SGV, BL, FH, IS>), dim3(grid), dim3(BL), 0, s, src, info, gp, rowph, \
