@@ -593,7 +593,10 @@ bool columns_path(int N, const Optics& o) { return N >= 256 && optics_isotropic(
 // BF groups (partial planes): the tuner's candidates, the default first.  Whole
 // rounds of the 8 XCDs in each of two parts.  At N = 256 (800 BF pixels) 64, 96
 // and 128 take 112, 93 and 91 us, their sums 8, 10 and 13; at 512 32, 64 and
-// 128 take 263, 277 and 305, their sums 14, 24 and 54.
+// 128 take 263, 277 and 305, their sums 14, 24 and 54.  Fewer groups keep fewer
+// waves in flight and are there for small selections: whole reconstructions of 48 x 48
+// frames with 800 BF pixels take 290, 313, 336, 401 and 589 us with the candidates at
+// 256 and 996, 1185 and 1565 us at 512.
 int columns_variants(int N) { return N == 512 ? 3 : (N == 256 ? 5 : 1); }
 int columns_groups(int N, int variant) {
   static const int g256[5] = {96, 64, 48, 32, 16};

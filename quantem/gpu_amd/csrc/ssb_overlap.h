@@ -32,22 +32,10 @@ __device__ __forceinline__ float aperture_from_d(df d, const ApIso& a) {
   return fminf(fmaxf(e, 0.0f), 1.0f);
 }
 
-// aperture_from_d(a + b) for d given as two double-float terms: the float32
-// sum of their high words is within a few 1e-6 of d for the magnitudes here
-// (|a|, |b| < 32), so outside the soft band by more than 1e-4 the value is
-// exactly 1 or 0 without the double-float addition; inside, the same
-// double-float evaluation as aperture_from_d.
-__device__ __forceinline__ float aperture_sum(const df& a, const df& b, const ApIso& ap) {
-  constexpr float kMargin = 1e-4f;
-  const float est = a.hi + b.hi;
-  if (est >= ap.d_in + kMargin) return 1.0f;
-  if (est <= ap.d_out - kMargin) return 0.0f;
-  return aperture_from_d(df_add(a, b), ap);
-}
-
 // The aperture from a float32 estimate of d when it lies beyond the 1e-4
-// margin of the soft band (the value aperture_sum gives there); false when
-// the estimate is too close to the band to decide.
+// margin of the soft band (exactly 0 or 1 there: the estimate is within a few
+// 1e-6 of d for terms below 32 in magnitude); false when it is too close to the
+// band to decide.
 __device__ __forceinline__ bool aperture_decided(float est, const ApIso& ap, float& a) {
   constexpr float kMargin = 1e-4f;
   a = (est >= ap.d_in + kMargin) ? 1.0f : 0.0f;
@@ -70,9 +58,9 @@ __device__ __forceinline__ float row_estimate_plus(df qx, df kx2, df q2x) { retu
 
 // Isotropic aperture pair A(Q - k), A(Q + k) from d = row + col: decided
 // from the estimates uq, vq of the row terms wherever d lies beyond the soft
-// band's margin (exactly the value aperture_sum gives), otherwise from the
-// double-float row terms, which are formed inside that branch only -- the
-// few points near the soft edge pay for them, the rest do not.
+// band's margin, otherwise from the double-float row terms, which are formed
+// inside that branch only -- the few points near the soft edge pay for them,
+// the rest do not.
 __device__ __forceinline__ void iso_aperture_pair(float uq, float vq, df qx, df kx2, df q2x, const df& colA,
                                                   const df& colB, const ApIso& ap, float& am, float& app) {
   const bool da = aperture_decided(uq + colA.hi, ap, am);
