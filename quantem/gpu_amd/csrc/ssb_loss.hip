@@ -305,14 +305,18 @@ k_rowifft_moments(const float2* __restrict__ T, const BfInfo* __restrict__ info,
 // Pass 3: combine the splits (fixed order), mean phase, per-pixel variance,
 // per-block variance sums; then one block sums those in fixed order.
 // ------------------------------------------------------------------------
-// A workgroup owns 64 pixels, its four waves a quarter of the splits each.
+// WAVES waves share the splits of 64 pixels (4: few pixels, many splits), a
+// workgroup has 4 / WAVES such sets.
+template <int WAVES>
 __global__ void __launch_bounds__(256)
 k_moments_finish(const float2* __restrict__ M1, const float2* __restrict__ M2, int nsplit, int NN,
                  const BfInfo* __restrict__ info, float* __restrict__ phase, float* __restrict__ var_part) {
   __shared__ float2 part[4][64][2];
+  __shared__ float sums[4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int idx = blockIdx.x * 64 + lane;   // N * N is a multiple of 64
-  const int s0 = nsplit * w / 4, s1 = nsplit * (w + 1) / 4;
+  const int share = w % WAVES;
+  const int idx = (blockIdx.x * (4 / WAVES) + w / WAVES) * 64 + lane;   // N * N is a multiple of 256
+  const int s0 = nsplit * share / WAVES, s1 = nsplit * (share + 1) / WAVES;
   Kahan a1, a2;
   a1.init();
   a2.init();
@@ -323,22 +327,32 @@ k_moments_finish(const float2* __restrict__ M1, const float2* __restrict__ M2, i
     a1.add(a.x - a.y);
     a2.add(c.x - c.y);
   }
-  part[w][lane][0] = make_float2(a1.s, a1.c);
-  part[w][lane][1] = make_float2(a2.s, a2.c);
-  __syncthreads();
-  if (w != 0) return;
-  for (int k = 1; k < 4; ++k) {
-    const float2 u = part[k][lane][0], v = part[k][lane][1];
-    a1.add(u.x - u.y);
-    a2.add(v.x - v.y);
+  if constexpr (WAVES > 1) {
+    part[w][lane][0] = make_float2(a1.s, a1.c);
+    part[w][lane][1] = make_float2(a2.s, a2.c);
+    __syncthreads();
+    if (share == 0) {
+      for (int k = 1; k < WAVES; ++k) {
+        const float2 u = part[w + k][lane][0], v = part[w + k][lane][1];
+        a1.add(u.x - u.y);
+        a2.add(v.x - v.y);
+      }
+    }
   }
   const float inv = 1.0f / (float)(info->nbf > 0 ? info->nbf : 1);
   const float mean = (a1.s - a1.c) * inv;
-  if (phase) phase[idx] = mean;
-  // the block's variances in a tree of fixed order
+  // the block's variances in a tree of fixed order, then its sets'
   float v = (a2.s - a2.c) * inv - mean * mean;
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  if (lane == 0) var_part[blockIdx.x] = v;
+  if (phase && share == 0) phase[idx] = mean;
+  if (lane == 0) sums[w] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    Kahan k;
+    k.init();
+    for (int i = 0; i < 4; i += WAVES) k.add(sums[i]);
+    var_part[blockIdx.x] = k.s - k.c;
+  }
 }
 
 __global__ void __launch_bounds__(256)
@@ -449,8 +463,13 @@ hipError_t launch_phase_moments(int N, const float2* Gt, int gcols, const BfInfo
 hipError_t launch_moments_finish(int N, int nsplit, const BfInfo* info, const float2* M1, const float2* M2,
                                  float* var_part, float* phase, float* loss, hipStream_t s) {
   const int NN = N * N;
-  const int parts = NN / 64;
-  hipLaunchKernelGGL(k_moments_finish, dim3(parts), dim3(256), 0, s, M1, M2, nsplit, NN, info, phase, var_part);
+  // four waves a pixel set where the splits are many: at 16 the sets of a wave each
+  // already have loads enough in flight
+  const int parts = nsplit > 16 ? NN / 64 : NN / 256;
+  if (nsplit > 16)
+    hipLaunchKernelGGL(k_moments_finish<4>, dim3(parts), dim3(256), 0, s, M1, M2, nsplit, NN, info, phase, var_part);
+  else
+    hipLaunchKernelGGL(k_moments_finish<1>, dim3(parts), dim3(256), 0, s, M1, M2, nsplit, NN, info, phase, var_part);
   hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(256), 0, s, var_part, parts, NN, loss);
   return hipGetLastError();
 }

@@ -583,17 +583,25 @@ hipError_t launch_phase_even(int N, const float2* Gt, const BfInfo* info, int nb
                              float2* M1, float2* M2, float* var_part, float* phase, float* loss, hipStream_t s) {
   df rout2;
   const ApIso ap = iso_aperture(o, rout2);
-  const int chunk = phase_chunk_bf(N), nsplit = phase_splits(N);
+  const int chunk = phase_chunk_bf(N);
+  const int nb = nbf > 0 ? nbf : 1;
+  // Small selections.  A split costs the finishing kernel two planes: at least two BF
+  // pixels each (a loss of 13 pixels at 128 x 128 takes 47 us in 128 splits, 22 in 7, 27
+  // in 4; of 81 at 256 x 256 49 us in 32 and 51 in 21).  And waves enough for a few
+  // rounds, whose first loads hide behind each other (81 pixels at 256 x 256: 57 us with
+  // 2048 waves of two pixels, 46 with one pixel a wave; at 1024, one wave a SIMD, more
+  // rounds cost 193 -> 199).
+  const int nsplit = phase_splits(N) < (nb + 1) / 2 ? phase_splits(N) : (nb + 1) / 2;
+  const int fill = N == 1024 ? 2048 : 8192;
   const int half = N / 2;
   float2* T = ws;
   float2* EG = T + (size_t)chunk * half * N;
   float2* Hrow = EG + (size_t)chunk * N;
-  const int nb = nbf > 0 ? nbf : 1;
 #define QSSB_PHASE(NN, SC, SR, ROWS)                                                                              \
   do {                                                                                                            \
-    int groups = cnt / 4; /* four BF pixels a wave */                                                             \
+    int groups = cnt / 4; /* four BF pixels a wave, fewer to have `fill` waves */                                 \
+    if (groups < fill / (half / SC)) groups = fill / (half / SC);                                                 \
     if (groups > cnt) groups = cnt;                                                                               \
-    if (groups < 1) groups = 1;                                                                                   \
     const unsigned g1 = (unsigned)(((long long)groups * (half / SC) + 3) / 4);                                    \
     if (ch.general)                                                                                               \
       hipLaunchKernelGGL((k_phase_cols<NN, SC, true>), dim3(g1), dim3(256), 0, s, Gt, info, gp, ch, ch_dev, ap, rout2, \
