@@ -642,8 +642,8 @@ int ssb_import_g(ssb_plan* p, const void* g_in, int nbf, int gcols, void* stream
 // The quadratic chi in half turns.
 static QuadTurns quad_turns(const ssb_plan* p, double c10, double c12, double phi12) {
   const double lam = p->wavelength;
-  return QuadTurns{(float)(lam * c10), (float)(lam * c12 * std::cos(2.0 * phi12)),
-                   (float)(lam * c12 * std::sin(2.0 * phi12))};
+  const double c = c12 * std::cos(2.0 * phi12);
+  return QuadTurns{to_df(lam * (c10 + c)), to_df(lam * (c10 - c)), to_df(lam * c12 * std::sin(2.0 * phi12))};
 }
 
 int ssb_object(ssb_plan* p, double c10, double c12, double phi12, void* obj_out, float* phase_out, void* stream) {

@@ -80,22 +80,18 @@ __device__ __forceinline__ float2 quad_term(float2 G, float B, float base, float
   });
 }
 
-// s of overlap_unit, qx (sxx qx + sxy) + syy, given sxx = k0 + m12c, sxy = 2 m12s qy
-// and syy = half_sum_qy(ev, qy).  Both squares are rounded alike and not contracted
-// into the sum: where C10 and C12 cancel (on the diagonals without C10, on an axis
-// with |C10| = |C12|) s is zero, not what rounding leaves, whose sign the term
-// would take.
-__device__ __forceinline__ float half_sum(float sxx, float sxy, float syy, float qx) {
+// k q^2 less its whole turns (2: the period of e^{i pi s}), for s of overlap_unit: s =
+// turn_part(sxx, qx) + turn_part(syy, qy) + qx cross_part(sxy, qy).  Each part is rounded at its
+// remainder, not at its tens of turns.  Odd in k: where C10 and C12 cancel (on the
+// diagonals without C10, on an axis with |C10| = |C12|) s is zero, not what rounding
+// leaves, whose sign the term would take.
+__device__ __forceinline__ float turn_part(df k, df q) {
 #pragma clang fp contract(off)
-  const float a = qx * fmaf(qx, sxx, sxy);
-  return a + syy;
+  const df v = df_mul(k, df_mul(q, q));
+  const float n = rintf(0.5f * v.hi);
+  return (v.hi - 2.0f * n) + v.lo;
 }
-__device__ __forceinline__ float half_sum_qy(const QuadTurns& ev, float qy) {
-  return half_sum(ev.k0 - ev.m12c, 0.0f, 0.0f, qy);
-}
-__device__ __forceinline__ float half_sum(const QuadTurns& ev, float qx, float qy) {
-  return half_sum(ev.k0 + ev.m12c, 2.0f * qy * ev.m12s, half_sum_qy(ev, qy), qx);
-}
+__device__ __forceinline__ float cross_part(df k, df q) { return 2.0f * df_mul(k, q).hi; }
 
 }  // namespace
 
@@ -151,18 +147,20 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
     wave_range(qy[i], y0[i], y1[i]);
     // (at N = 128 the rows of column N/2 fill two of the four)
     q2[i] = last && (t - SETS) * 256 + 64 * i >= N ? INFINITY : fmaf(qx[i], qx[i], qy[i] * qy[i]);
-    s[i] = half_sum(ev, qx[i], qy[i]);
-    own[i * 256 + threadIdx.x] = make_float4(qx[i], gp.qxl[row0[i] + lr], qy[i], gp.qyl[col0[i] + lc]);
+    const df x{qx[i], gp.qxl[row0[i] + lr]}, y{qy[i], gp.qyl[col0[i] + lc]};
+    s[i] = fmaf(qx[i], cross_part(ev.sxy, y), turn_part(ev.sxx, x) + turn_part(ev.syy, y));
+    own[i * 256 + threadIdx.x] = make_float4(x.hi, x.lo, y.hi, y.lo);
   }
   // the tile of the rows from N/2, whose first row has partners of its own
   const int ny = last || rt != 0 ? -1 : (2 - turn) & 3;
-  float nqx = 0.f, nqy = 0.f, nq2 = 0.f, ny0 = 0.f, ny1 = 0.f;
+  float nqx = 0.f, nqy = 0.f, nq2 = 0.f, ns = 0.f, ny0 = 0.f, ny1 = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (i == ny) {
       nqx = qx[i];
       nqy = -qy[i];
       nq2 = q2[i];
+      ns = fmaf(nqx, 4.0f * nqy * ev.sxy.hi, s[i]);   // its term in qx qy the other way round
       ny0 = -y1[i];
       ny1 = -y0[i];
     }
@@ -217,7 +215,6 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
       if (nmask >> l & 1) {
         // the Nyquist row's partners, columns N - j: their own frequencies (q_N/2, -qy)
         const float B = fmaf(nqx, p.kx2, nqy * p.ky2) + 0.0f, base = p.cb - nq2;
-        const float ns = half_sum(ev, nqx, nqy);
         float2 G = cur.G[0];
 #pragma unroll
         for (int i = 1; i < 4; ++i) {
@@ -288,9 +285,10 @@ struct ColumnFft {
     return make_float2(mv(v.x), mv(v.y));
   }
 
-  // The lanes' twiddles, 64 a row (one address, no bank conflicts): rows 0..15
-  // w_N^(jj k1) of output ka, rows 16.. w_K^(h ka) where lanes share a DFT.
-  static constexpr int TW = 64 * (Q > 1 ? 32 : (K == 8 ? 8 : 16));
+  // The lanes' twiddles, 64 a row (one address, no bank conflicts): w_N^(jj k1) of
+  // output ka; after them w_K^(h ka) where lanes share a DFT, Q a row (lanes of one h
+  // read one address).
+  static constexpr int TW1 = 64 * (K == 8 ? 8 : 16), TW = TW1 + (Q > 1 ? 16 * Q : 0);
   __device__ static __forceinline__ int base_k1(int lane) {
     const int h = lane % Q;
     return Q == 4 ? 16 * (((h & 1) << 1) | (h >> 1)) : 16 * h;
@@ -298,9 +296,9 @@ struct ColumnFft {
   __device__ static __forceinline__ void twiddles(float2* __restrict__ twl, const float2* __restrict__ tw, int tid,
                                                   int threads) {
     for (int i = tid; i < TW; i += threads) {
-      const int lane = i & 63, k = i >> 6;
+      const int lane = i & 63, k = i >> 6, u = i - TW1;
       const int jj = K == 8 ? lane & 15 : (lane / Q) & 15;
-      twl[i] = k < 16 ? tw[((k + (K == 8 ? 0 : base_k1(lane))) * jj) & (N - 1)] : tw[(16 * (k - 16) * (lane % Q)) & (N - 1)];
+      twl[i] = tw[(i < TW1 ? (k + (K == 8 ? 0 : base_k1(lane))) * jj : 16 * (u / Q) * (u % Q)) & (N - 1)];
     }
   }
 
@@ -333,7 +331,7 @@ struct ColumnFft {
       dft_regs<16, false>(x);
       if constexpr (Q > 1) {
 #pragma unroll
-        for (int k = 1; k < 16; ++k) x[k] = cmul(x[k], tw[64 * (16 + k)]);
+        for (int k = 1; k < 16; ++k) x[k] = cmul(x[k], twl[TW1 + k * Q + h]);
         if constexpr (Q == 4) {
 #pragma unroll
           for (int k = 0; k < 16; ++k) {
@@ -396,18 +394,18 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
   constexpr int NW = column_waves(N), CG = S * NW;   // columns a workgroup
   constexpr int NCG = HALF / CG, LG = 16 / CG;       // workgroups that share a line of H
   __shared__ float2 twl[Fft::TW];
-  // the frequencies of the rows and of the workgroup's columns, for the points at an
-  // edge in double-float (at 512 the rows' low words would cost a workgroup a CU)
-  constexpr bool LOWS = N != 512 && !STORE;
-  __shared__ float qxS[STORE ? 1 : N], qxlS[LOWS ? N : 1];
+  // the rows' frequencies (high and low words) and parts of s, the columns' frequencies
+  __shared__ float qxS[STORE ? 1 : N], qxlS[STORE ? 1 : N], sxS[STORE ? 1 : N];
   __shared__ float2 qyS[CG];
   __shared__ float2 exS[NW][Fft::LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   if constexpr (!STORE) {
     for (int i = tid; i < N; i += 64 * NW) {
-      qxS[i] = gp.qx[i];
-      if (LOWS) qxlS[LOWS ? i : 0] = gp.qxl[i];
+      const df x{gp.qx[i], gp.qxl[i]};
+      qxS[i] = x.hi;
+      qxlS[i] = x.lo;
+      sxS[i] = turn_part(ev.sxx, x);
     }
   }
   Fft::twiddles(twl, tw_g, tid, 64 * NW);
@@ -493,20 +491,20 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
     auto point = [&](int q, int dq, float sign, df& x, df& y) {
       int c = last ? 0 : S * w + col;
       asm volatile("" : "+v"(q), "+v"(c));           // no addresses kept ahead of the branch
-      x = df{qxS[q + dq], LOWS ? qxlS[LOWS ? q + dq : 0] : gp.qxl[q + dq]};
+      x = df{qxS[q + dq], qxlS[q + dq]};
       const float2 v = qyS[c];
       y = df{sign * v.x, sign * v.y};
     };
     float y0, y1;
     wave_range(gp.qy[last ? HALF : cg * CG + lane % CG], y0, y1);
     const float qn = as_const(gp.qx)[HALF];
-    const float sxy = 2.0f * qy * ev.m12s, syy = half_sum_qy(ev, qy);
-    const float sxx = ev.k0 + ev.m12c;
+    const df yd{qy, gp.qyl[j]};
+    const float sxy = cross_part(ev.sxy, yd), sy = turn_part(ev.syy, yd);
     // whether a point of the wave, the mean's apart, has s near a whole number: s is
     // the point's alone, and without one its terms need not ask (a scalar branch)
     bool whole = false;
     for (int r = 0; r < 16; ++r)
-      whole |= near_whole(half_sum(sxx, sxy, syy, qxS[k1 + K * r])) && (j != 0 || k1 + K * r != 0);
+      whole |= near_whole(fmaf(qxS[k1 + K * r], sxy, sxS[k1 + K * r] + sy)) && (j != 0 || k1 + K * r != 0);
     const bool ask = __any(whole);
     Kahan2 acc[16], nyq;
 #pragma unroll
@@ -546,7 +544,7 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
             const float2 m = Fft::mirror(r, ex, lane);
             x[r] = last ? unpack_half(x[r], m) : unpack_first(x[r], m);
           }
-          const float s = half_sum(sxx, sxy, syy, qx);
+          const float s = fmaf(qx, sxy, sxS[k1 + K * r] + sy);
           whole = false;
           if (ask) {
             float at = s;
@@ -561,7 +559,7 @@ k_columns(const float2* __restrict__ H, const BfInfo* __restrict__ info, GeomPtr
         if (!last && apertures_reach(p, rout2.hi, qn, qn, -y1, -y0)) {
           // the Nyquist row's partners, columns N - j: their own frequencies (q_N/2, -qy)
           const float B = fmaf(qn, p.kx2, -Bq) + 0.0f, base = fmaf(-qn, qn, cq);
-          const float ns = half_sum(ev, qn, -qy);
+          const float ns = fmaf(qn, -sxy, sxS[HALF] + sy);
           if (k1 == 0 && base + fabsf(B) > -p.margin)
             nyq.add(quad_term(cconj(x[8]), B, base, ns, fmaf(qn, p.tx, -tq), near_whole(ns), p, ap,
                               [&](df& x, df& y) { point(HALF, 0, -1.0f, x, y); }));

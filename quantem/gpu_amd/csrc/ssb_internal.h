@@ -84,9 +84,11 @@ struct EvenChi {
   ChiPoly cp;
 };
 
-// A quadratic one: chi / pi = k0 r2 + m12c (ux^2 - uy^2) + m12s 2 ux uy.
+// A quadratic one: chi / pi = sxx ux^2 + syy uy^2 + 2 sxy ux uy (C10, C12), in
+// double-float: a coefficient's rounding is the same for every BF pixel, and does not
+// average out of their sum as the terms' own does.
 struct QuadTurns {
-  float k0, m12c, m12s;
+  df sxx, syy, sxy;
 };
 
 // Matrix of the quadratic aberration phase chi(u) = u^T M u,
@@ -111,11 +113,13 @@ struct PhasorJob {
   float2* echi;
 };
 
-// chi(Q), the squares rounded alike: zero where mxx = -myy and |x| = |y|, as exactly.
+// chi(Q), rounded once but for the term in x y; zero where mxx = -myy and |x| = |y|,
+// as exactly.
 __device__ __forceinline__ float chi_plane(const QuadChi& m, float x, float y) {
-#pragma clang fp contract(off)
-  const float a = m.mxx * (x * x), b = m.myy * (y * y);
-  return fmaf(2.0f * m.mxy * x, y, a + b);
+  const df a = df_mul(df{m.mxx, 0.0f}, df_mul(df{x, 0.0f}, df{x, 0.0f}));
+  const df b = df_mul(df{m.myy, 0.0f}, df_mul(df{y, 0.0f}, df{y, 0.0f}));
+  const df s = df_add(a, b);
+  return s.hi + fmaf(2.0f * m.mxy * x, y, s.lo);
 }
 
 // The items [gid, gid + stride, ...) of a phasor job.

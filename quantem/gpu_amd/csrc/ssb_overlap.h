@@ -269,8 +269,8 @@ __device__ __forceinline__ QuadPixel quad_pixel(const GeomPtrs& gp, int b, const
   const df cb = df_sub(rout2, df_add(df_mul(kx, kx), df_mul(ky, ky)));
   p.cb = cb.hi;
   p.cbl = cb.lo;
-  p.tx = fmaf(ev.k0 + ev.m12c, p.kx2, ev.m12s * p.ky2);
-  p.ty = fmaf(ev.k0 - ev.m12c, p.ky2, ev.m12s * p.kx2);
+  p.tx = 2.0f * df_add(df_mul(ev.sxx, kx), df_mul(ev.sxy, ky)).hi;
+  p.ty = 2.0f * df_add(df_mul(ev.syy, ky), df_mul(ev.sxy, kx)).hi;
   p.ak = gp.ak[b];
   p.margin = edge_margin(p.ak, ap);
   return p;
