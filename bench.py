@@ -477,9 +477,9 @@ def trials_leg(dev, data, cfg, n_trials: int = 512, reps: int = 5, seed: int = 3
 
 
 SEARCH_PROFILE = REPO / "profiles" / "trials_search_512x256x128.md"
-# 256 CUs x 4 SIMDs, one wave64 VALU instruction per 4 cycles, 2.4 GHz: nominal, instructions
-# issue in 3.2 cycles in the search (a fraction above 1)
-VALU_LANES_PER_S = 1024 * 16 * 2.4e9
+# what chains of independent 32-bit operations sustain on this card with 8 waves a
+# SIMD: 2.6 cycles a wave64 instruction (fused multiply-adds 3.05, 5.2e13 lanes/s)
+VALU_LANES_PER_S = 6.0e13
 
 
 def read_profile_figure(path: Path, key: str) -> float | None:
@@ -498,8 +498,9 @@ def read_profile_figure(path: Path, key: str) -> float | None:
 def search_unit_roofline(units_per_s: float) -> dict:
     """The batched search against its VALU issue bound: VALU (and
     transcendental) lane-instructions per search unit from the committed
-    counter summary of the same launch, the bound = FP32 VALU lane rate
-    (packed FP32 unused) / instructions per unit, frac = achieved / bound."""
+    counter summary of the same launch, the bound = the measured issue rate of
+    independent operations (packed FP32 unused) / instructions per unit, frac =
+    achieved / bound."""
     per = read_profile_figure(SEARCH_PROFILE, "valu_lane_instructions_per_unit")
     trans = read_profile_figure(SEARCH_PROFILE, "trans_f32_lane_instructions_per_unit")
     if not per:

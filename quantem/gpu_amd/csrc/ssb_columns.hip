@@ -258,7 +258,8 @@ k_object_tiles(const float2* __restrict__ Gt, const BfInfo* __restrict__ info, G
 // kernels before: 119 and 867).  BF pixels whose apertures miss the workgroup's
 // columns are passed over.  STORE: no sums, the stack is written.
 // Two to three waves a SIMD (64 registers of sums) and the exchanges bound it:
-// 800 BF pixels at 256 move 150 MB in 93 us.
+// 800 BF pixels at 256 move 150 MB in 96 us, at 512 take 303 (93 and 263 with
+// the lens' soft band from float32 estimates, wrong by up to 1e-5 of a term).
 // ------------------------------------------------------------------------
 // Workgroup barrier for LDS only: this wave's LDS operations complete, then
 // s_barrier; its global loads stay in flight.

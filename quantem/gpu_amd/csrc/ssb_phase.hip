@@ -26,8 +26,8 @@
 //
 // 16 trials of C10, C30 and rotation at 256 x 256, 800 BF pixels: 8.70 ms on
 // the general path (complex planes, chi at Q - k and Q + k, workgroup
-// barriers in every FFT stage), 3.36 ms here; 64 quadratic trials at
-// 128 x 128: 9.70 and 4.15 ms.  A trial at 256 x 256 takes k_phase_cols 88 us
+// barriers in every FFT stage), 3.35 ms here; 64 quadratic trials at
+// 128 x 128: 9.70 and 4.05 ms.  A trial at 256 x 256 takes k_phase_cols 88 us
 // (420 MB, the rate of a large copy) and k_phase_rows 109 us (210 MB; its LDS
 // exchanges and the arctangents bound it, at 4 waves a SIMD).
 #include "ssb_internal.h"

@@ -240,8 +240,9 @@ __device__ __forceinline__ void trial_sums(const TrialSet& ds, const TrialChi* _
 // soon as one of its points needs it, so the points lie in square tiles.  512
 // trials of C10, C30 and rotation at 256 x 256, 800 BF pixels: 66.9 ms with
 // two sincosf and a normalisation a point; 32.4 ms with one phasor and the
-// whole soft bands in the general form; 9.0 ms with the general form at the
-// outer edges and the lens' own band alone, on 8 x 8 tiles.  At most 128
+// whole soft bands in the general form; 9.2 ms with the general form at the
+// outer edges, in the lens' own band and near whole s alone, on 8 x 8 tiles (the
+// band's apertures in double-float are 0.2 ms of it).  At most 128
 // registers (4 waves per SIMD): the BF pixel's scalars and the next G hide
 // behind the other waves.
 template <int TB>

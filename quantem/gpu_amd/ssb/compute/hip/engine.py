@@ -78,7 +78,9 @@ def normalize_scan(data):
     """Crop/pad a resident ``[H, W, k_r, k_c]`` scan (any supported sample
     type) to the supported square size with the mean-frame padding of
     ``cuda/backend.py:229-269`` (returns ``data`` itself when it is already
-    supported)."""
+    supported).  The work is queued on the current stream of ``data``'s device:
+    a caller that uses the result, or overwrites ``data``, on another stream
+    orders that stream behind it."""
     torch = _torch()
     if not isinstance(data, torch.Tensor) or not data.is_cuda:
         raise ValueError("data must be a torch tensor on the GPU")
